@@ -8,12 +8,13 @@
 // z = z1 + N(r1); plain GMG-FCG takes over when the defect stalls.
 //
 // Tensors are channels-last [batch][z][y][x][c] in FP32.  Convolutions are
-// implicit GEMMs on v_mfma_f32_16x16x16bf16_1k: M = voxels (tiles of 16),
-// N = output channels (tiles of 16), K = 27 taps x input channels (chunks of
+// implicit GEMMs on v_mfma_f32_16x16x16bf16_1k over voxels (tiles of 16),
+// output channels (tiles of 16) and 27 taps x input channels (chunks of
 // 16); activations and weights are rounded to BF16 when they enter the
 // matrix cores, products accumulate in FP32.  Weight gradients are implicit
-// GEMMs on the same instruction (voxels as K) with per-chunk partials reduced
+// GEMMs on the same instruction (voxels as K) with per-block partials reduced
 // in a fixed order.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <random>
@@ -37,275 +38,527 @@ __device__ __forceinline__ short bf16_bits(float f) {
   return (short)(u >> 16);
 }
 
+// ---- tiles of the convolutions ----------------------------------------------------------------
+// A workgroup works on a box of bz x by x bx voxels of one sample; the input channels of the box
+// and of the one-voxel halo around it are staged in LDS as BF16, one plane of 16 channels after
+// another: lds[chunk][halo voxel][16].  With 32 bytes per voxel the 16 lanes of an MFMA operand
+// (16 voxels) times its four channel groups read 512 consecutive bytes wherever the tap shifts
+// them, so no tap has bank conflicts and every value is rounded to BF16 once per box instead of
+// once per tap.
+struct Div1 {  // n / d for d >= 1
+  FastDiv f;
+};
+inline Div1 div1(unsigned d) { return Div1{d >= 2 ? fast_div(d) : FastDiv{1u, 0u, 0}}; }
+__device__ __forceinline__ unsigned fdiv(unsigned n, Div1 d) {
+  return d.f.d == 1u ? n : fdiv(n, d.f);
+}
+
+struct ConvGeom {
+  int n;                   // voxels per axis
+  int bz, by, bx;          // box
+  int vol, hvol;           // voxels of the box, of the box with its halo
+  int nbox;                // boxes of all samples
+  Div1 dnx, dny, dnz;      // boxes per axis
+  Div1 dbx, dby, dhx, dhy; // box and halo extents
+};
+
+// how a convolution's blocks are split (conv_plan)
+struct ConvPlan {
+  ConvGeom g;
+  int mt, nt, wm;  // voxel and channel tiles per wave, waves along the voxels
+  int nch, ntt;    // chunks of input channels, tiles of output channels
+};
+
+// The input of a convolution: channels [0, c0) from p0, [c0, c0 + c1) from p1.  up: p0 lives
+// on the grid of n / 2 voxels per axis and is upsampled (nearest), the decoder's concatenation
+// [upsampled, skip], which is then never stored.
+struct ConvIn {
+  const float *p0, *p1;
+  int c0, c1, up;
+};
+
+// box `t` of the geometry: sample and first voxel
+__device__ __forceinline__ void conv_box(const ConvGeom &G, int t, int &b, int &z0, int &y0,
+                                         int &x0) {
+  unsigned u = (unsigned)t, q = fdiv(u, G.dnx);
+  x0 = (int)(u - q * G.dnx.f.d) * G.bx;
+  u = q;
+  q = fdiv(u, G.dny);
+  y0 = (int)(u - q * G.dny.f.d) * G.by;
+  u = q;
+  q = fdiv(u, G.dnz);
+  z0 = (int)(u - q * G.dnz.f.d) * G.bz;
+  b = (int)q;
+}
+
+// Stages channels [16 ch0, 16 (ch0 + nch)) of the box at (b, z0, y0, x0) and its halo; zero
+// outside the grid and beyond the last channel.  Four entries of four channels per thread in
+// flight together.
+__device__ __forceinline__ void conv_stage(const ConvGeom &G, const ConvIn &in, int ch0, int nch,
+                                           Div1 dq, int b, int z0, int y0, int x0, short *lds) {
+  const int Q = nch * 4, total = G.hvol * Q, ct = in.c0 + in.c1, n = G.n, h = n >> 1;
+  const bool vec = ((in.c0 | in.c1) & 3) == 0;
+  constexpr int U = 4;
+  for (int e0 = threadIdx.x; e0 < total; e0 += U * 256) {
+    float f[U][4];
+    int dst[U];
+    bool live[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int e = e0 + u * 256;
+      const unsigned ec = (unsigned)min(e, total - 1);
+      const unsigned pos = fdiv(ec, dq), q = ec - pos * (unsigned)Q;
+      const unsigned t = fdiv(pos, G.dhx);
+      const int hx = (int)(pos - t * G.dhx.f.d);
+      const unsigned hz = fdiv(t, G.dhy);
+      const int hy = (int)(t - hz * G.dhy.f.d);
+      const int z = z0 + (int)hz - 1, y = y0 + hy - 1, x = x0 + hx - 1;
+      const int c = ch0 * 16 + (int)q * 4;
+      dst[u] = e < total ? (int)(((q >> 2) * (unsigned)G.hvol + pos) * 16u + (q & 3u) * 4u) : -1;
+      live[u] = z >= 0 && y >= 0 && x >= 0 && z < n && y < n && x < n && c < ct;
+      const bool second = c >= in.c0;
+      const int cs = second ? in.c1 : in.c0, cc = second ? c - in.c0 : c;
+      const float *src = second ? in.p1 : in.p0;
+      long vox;
+      if (in.up && !second)
+        vox = (((long)b * h + (z >> 1)) * h + (y >> 1)) * h + (x >> 1);
+      else
+        vox = (((long)b * n + z) * n + y) * n + x;
+      if (vec) {
+        const float4 v = live[u] ? *(const float4 *)(src + vox * cs + cc)
+                                 : make_float4(0.f, 0.f, 0.f, 0.f);
+        f[u][0] = v.x;
+        f[u][1] = v.y;
+        f[u][2] = v.z;
+        f[u][3] = v.w;
+      } else {  // channel counts that are no multiple of 4 (one source)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          f[u][j] = live[u] && c + j < ct ? in.p0[vox * in.c0 + c + j] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (dst[u] >= 0) {
+        v4s s;
+#pragma unroll
+        for (int j = 0; j < 4; j++) s[j] = bf16_bits(f[u][j]);
+        *(v4s *)(lds + dst[u]) = s;
+      }
+  }
+}
+
 // ---- convolution forward / input gradient (implicit GEMM on MFMA) --------------------
 
 // out[v][o] = bias[o] + sum_t sum_c in[v + off(t) * sgn][c] * W[t][c][o]
-// with W given in BF16 as wk[t][o][c] (the K index c contiguous).  sgn = +1
-// for the forward convolution; sgn = -1 with wk = W^T computes the input
-// gradient (taps mirrored).  One wavefront: 16 voxels x all output channels.
-template <int NT>
-__global__ __launch_bounds__(256) void k_conv_mfma(int batch, int n, int ci, int co,
-                                                   const float *__restrict__ in,
-                                                   const short *__restrict__ wk,
-                                                   const float *__restrict__ bias, float *out,
-                                                   int relu, int sgn) {
-  long nv = (long)n * n * n;
-  long total = batch * nv;
-  long tile = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  long v0 = tile * 16;
-  if (v0 >= total) return;  // wave-uniform
-  int lane = threadIdx.x & 63;
-  int i = lane & 15, g = lane >> 4;
-  long v = v0 + i;
-  bool vin = v < total;
-  int b = 0, z = 0, y = 0, x = 0;
-  if (vin) {
-    b = (int)(v / nv);
-    long r = v % nv;
-    z = (int)(r / ((long)n * n));
-    y = (int)((r / n) % n);
-    x = (int)(r % n);
+// with W as MFMA fragments wf[t][chunk of 16 c][tile of 16 o][lane][4] (k_wfrag).  sgn = +1 for
+// the forward convolution; sgn = -1 with the transposed weights' fragments computes the input
+// gradient (taps mirrored).  mask (an activation of the output's layout): the result is zero
+// where it is <= 0, the ReLU's backward pass.
+//
+// The weights are the MFMA's row operand and the voxels its column operand, so a lane ends with
+// four consecutive channels of one voxel and stores them with one 16-byte access.  A wave holds
+// MT x NT tiles of 16 voxels x 16 channels, which share each voxel operand (LDS) and each weight
+// fragment (512 contiguous bytes, from L1/L2, fetched a group of iterations ahead).  Products
+// accumulate tap by tap and, within a tap, 16 channels at a time in ascending order.
+// Batch 32, 32^3, [32 up, 16 skip] -> 16 channels: 227 us, 96 TFLOP/s, bound by LDS reads and the
+// staging (2559 us and 215 us for the concatenation as one wave per 16 voxels without LDS, which
+// rounded the inputs and fetched single 2-byte weights anew for each of the 27 taps).
+template <int MT, int NT>
+__global__ __launch_bounds__(256) void k_conv(ConvGeom G, ConvIn in, int nch, Div1 dq, int no,
+                                              int ntt, const short *__restrict__ wf,
+                                              const float *__restrict__ bias,
+                                              const float *__restrict__ mask,
+                                              float *__restrict__ out, int relu, int sgn,
+                                              int wm) {
+  extern __shared__ __align__(16) short lds[];
+  const int box = (int)xcd_block(blockIdx.x, gridDim.x);
+  if (box >= G.nbox) return;  // the whole block
+  int b, z0, y0, x0;
+  conv_box(G, box, b, z0, y0, x0);
+  conv_stage(G, in, 0, nch, dq, b, z0, y0, x0, lds);
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int mw = w % wm, nw = w / wm;
+  const int hx = (int)G.dhx.f.d, hy = (int)G.dhy.f.d;
+  int abase[MT];
+  long vout[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) {
+    const int m = (mw * MT + mt) * 16 + i;
+    const unsigned mc = (unsigned)(m < G.vol ? m : 0);
+    const unsigned t = fdiv(mc, G.dbx);
+    const int xx = (int)(mc - t * G.dbx.f.d);
+    const unsigned zz = fdiv(t, G.dby);
+    const int yy = (int)(t - zz * G.dby.f.d);
+    abase[mt] = ((((int)zz + 1) * hy + yy + 1) * hx + xx + 1) * 16 + 4 * g;
+    const int z = z0 + (int)zz, y = y0 + yy, x = x0 + xx;
+    vout[mt] = m < G.vol && z < G.n && y < G.n && x < G.n
+                   ? (((long)b * G.n + z) * G.n + y) * G.n + x
+                   : -1;
   }
-  v4f acc[NT];
-  for (int t = 0; t < NT; t++) acc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
-  bool vec_ok = (ci % 4) == 0;
-  for (int tap = 0; tap < 27; tap++) {
-    int dz = (tap / 9 - 1) * sgn, dy = ((tap / 3) % 3 - 1) * sgn, dx = (tap % 3 - 1) * sgn;
-    int zz = z + dz, yy = y + dy, xx = x + dx;
-    bool ok = vin && zz >= 0 && zz < n && yy >= 0 && yy < n && xx >= 0 && xx < n;
-    const float *ip = in + ((long)b * nv + ((long)zz * n + yy) * n + xx) * ci;
-    for (int c0 = 0; c0 < ci; c0 += 16) {
-      int cb = c0 + 4 * g;
-      v4s a;
-      if (ok && vec_ok && cb < ci) {
-        float4 f = *(const float4 *)(ip + cb);
-        a[0] = bf16_bits(f.x);
-        a[1] = bf16_bits(f.y);
-        a[2] = bf16_bits(f.z);
-        a[3] = bf16_bits(f.w);
-      } else {
-        for (int j = 0; j < 4; j++) a[j] = (ok && cb + j < ci) ? bf16_bits(ip[cb + j]) : (short)0;
-      }
-      for (int t = 0; t < NT; t++) {
-        int o = t * 16 + i;
-        v4s bw;
-        const short *wp = wk + ((long)tap * co + o) * ci + cb;
-        for (int j = 0; j < 4; j++) bw[j] = (o < co && cb + j < ci) ? wp[j] : (short)0;
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bw, acc[t], 0, 0, 0);
+  v4f acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[mt][t] = (v4f){0.f, 0.f, 0.f, 0.f};
+  const int nit = 27 * nch;
+  const v4s *wp = (const v4s *)wf + (long)nw * NT * 64 + lane;
+  // weight fragments of PF iterations (tap, chunk) are in flight ahead of their use
+  constexpr int PF = MT == 1 || NT == 1 ? 9 : 3;  // divides the 27 taps
+  v4s bw[PF][NT];
+#pragma unroll
+  for (int u = 0; u < PF; u++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) bw[u][t] = wp[((long)min(u, nit - 1) * ntt + t) * 64];
+  __syncthreads();
+  int tz = -1, ty = -1, tx = -1, ch = 0;  // offset of the tap, channel chunk
+  for (int it = 0; it < nit; it += PF) {
+#pragma unroll
+    for (int u = 0; u < PF; u++) {
+      const int off = (((tz * hy + ty) * hx + tx) * sgn + ch * G.hvol) * 16;
+      v4s a[MT];
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) a[mt] = *(const v4s *)(lds + abase[mt] + off);
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+          acc[mt][t] =
+              __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bw[u][t], a[mt], acc[mt][t], 0, 0, 0);
+      const int nx = min(it + u + PF, nit - 1);
+#pragma unroll
+      for (int t = 0; t < NT; t++) bw[u][t] = wp[((long)nx * ntt + t) * 64];
+      if (++ch == nch) {
+        ch = 0;
+        if (++tx == 2) {
+          tx = -1;
+          if (++ty == 2) {
+            ty = -1;
+            tz++;
+          }
+        }
       }
     }
   }
-  // D[4g+v][i]: voxel v0 + 4g + q, channel t*16 + i
-  for (int t = 0; t < NT; t++) {
-    int o = t * 16 + i;
-    if (o >= co) continue;
-    float bo = bias ? bias[o] : 0.f;
-    for (int q = 0; q < 4; q++) {
-      long vv = v0 + 4 * g + q;
-      if (vv >= total) continue;
-      float val = acc[t][q] + bo;
-      if (relu && val < 0.f) val = 0.f;
-      out[vv * co + o] = val;
+  // D[4g + q][i]: channel 4g + q of the tile, voxel i
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) {
+    if (vout[mt] < 0) continue;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      const int o = (nw * NT + t) * 16 + 4 * g;
+      if ((no & 3) == 0) {
+        if (o >= no) continue;
+        float4 r = make_float4(acc[mt][t][0], acc[mt][t][1], acc[mt][t][2], acc[mt][t][3]);
+        if (bias) {
+          r.x += bias[o];
+          r.y += bias[o + 1];
+          r.z += bias[o + 2];
+          r.w += bias[o + 3];
+        }
+        if (relu) {
+          if (r.x < 0.f) r.x = 0.f;
+          if (r.y < 0.f) r.y = 0.f;
+          if (r.z < 0.f) r.z = 0.f;
+          if (r.w < 0.f) r.w = 0.f;
+        }
+        if (mask) {
+          const float4 k = *(const float4 *)(mask + vout[mt] * no + o);
+          if (k.x <= 0.f) r.x = 0.f;
+          if (k.y <= 0.f) r.y = 0.f;
+          if (k.z <= 0.f) r.z = 0.f;
+          if (k.w <= 0.f) r.w = 0.f;
+        }
+        *(float4 *)(out + vout[mt] * no + o) = r;
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          if (o + q >= no) continue;
+          float r = acc[mt][t][q] + (bias ? bias[o + q] : 0.f);
+          if (relu && r < 0.f) r = 0.f;
+          if (mask && mask[vout[mt] * no + o + q] <= 0.f) r = 0.f;
+          out[vout[mt] * no + o + q] = r;
+        }
+      }
     }
   }
 }
 
 // ---- weight gradients: gW[t][c][o] = sum_v in[v + off(t)][c] * gout[v][o] -------------
-// An implicit GEMM on v_mfma_f32_16x16x16bf16_1k per tap: M = input channels (tiles of 16),
-// N = output channels (tiles of 16), K = voxels (16 per product).  A block takes one tap and a
-// chunk of kWgVox voxels; it stages kWgChunk voxels at a time in LDS (the tap-shifted inputs
-// and the output gradients, rounded to BF16), and each wave accumulates up to kWgTiles
-// (c, o) tiles in FP32.  Blocks of the 27 taps of a chunk are adjacent in the grid, so the
-// chunk's values are read from HBM once and from L2 by the other taps.  The centre tap's
-// blocks also sum gout per channel in FP32 (the bias gradient).  Every block writes its sums
-// as a partial [chunk][27 ci co + co], reduced over the chunks in a fixed order.
+// An implicit GEMM on v_mfma_f32_16x16x16bf16_1k: M = 16 input channels, N = output channels,
+// K = voxels.  A block takes 16 input channels and every P-th box: it stages the box's inputs
+// with their halo as the convolution does and the box's output gradients, both rounded to BF16,
+// and accumulates the 16 x co products of all 27 taps in FP32 registers, 7 taps to a wave, over
+// its boxes.  The operands need four voxels of one channel per lane while LDS holds 16 channels
+// of a voxel: ds_read_tr16 transposes on the way (a lane reads four channels of voxel
+// 4g + lane % 16 / 4; it receives channel lane % 16 of voxels 4g .. 4g + 3).  So an input value
+// is read from device memory once (2.5 times with its halo) instead of once per tap, and a
+// wave's gradient operand serves its seven taps.  The blocks of the first channel chunk also sum
+// gout in FP32 (the bias gradient).  Every block writes its sums as a partial
+// [block][27 ci co + co]; k_wgrad_reduce adds them in a fixed order.
+// Batch 32, 32^3, 48 x 16 channels: 213 us (3592 us with one tap per block, which read the
+// inputs 27 times and gathered the operands from LDS two bytes at a time).
 
-constexpr int kWgChunk = 64;  // voxels staged per LDS round
-constexpr int kWgVox = 4096;  // voxels per block (partial sum)
-constexpr int kWgTiles = 4;   // (c, o) tiles per wave: 16 tiles of 16 x 16 for 4 waves
+constexpr int kWgVox = 256;  // voxels of a box, 16 K steps
 
-__global__ __launch_bounds__(256) void k_conv_wgrad(int batch, int n, int ci, int co,
-                                                    const float *__restrict__ in,
-                                                    const float *__restrict__ gout,
-                                                    float *partial) {
-  __shared__ short sin[kWgChunk * 96];  // [voxel][c], c padded to a multiple of 16
-  __shared__ short sg[kWgChunk * 64];   // [voxel][o]
-  __shared__ long soff[kWgChunk];       // element offset of the shifted input voxel, -1: zero
-  __shared__ float sb[256];
-  const int cip = (ci + 15) & ~15, cop = (co + 15) & ~15;
-  const int tap = (int)(blockIdx.x % 27);
-  const long chunk = blockIdx.x / 27;
-  const long nv = (long)n * n * n, total = batch * nv;
-  const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-  const int nto = cop / 16, ntiles = (cip / 16) * nto;
-  v4f acc[kWgTiles];
-  for (int t = 0; t < kWgTiles; t++) acc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.f;  // centre tap: this thread's channel o = threadIdx.x % cop
-  const long vbeg = chunk * kWgVox, vend = min(vbeg + kWgVox, total);
-  for (long vs = vbeg; vs < vend; vs += kWgChunk) {
-    __syncthreads();
-    if (threadIdx.x < kWgChunk) {
-      const long v = vs + threadIdx.x;
-      long off = -1;
-      if (v < vend) {
-        const int b = (int)(v / nv);
-        const long r = v % nv;
-        const int z = (int)(r / ((long)n * n)) + dz, y = (int)((r / n) % n) + dy,
-                  x = (int)(r % n) + dx;
-        if (z >= 0 && z < n && y >= 0 && y < n && x >= 0 && x < n)
-          off = ((long)b * nv + ((long)z * n + y) * n + x) * ci;
+typedef __attribute__((address_space(3))) v4s lds_v4s;
+__device__ __forceinline__ v4s lds_read_tr(const short *p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)p);
+}
+
+template <int NTO>
+__global__ __launch_bounds__(256) void k_conv_wgrad(ConvGeom G, ConvIn in, int ncc, int co,
+                                                    const float *__restrict__ gout, int P,
+                                                    float *__restrict__ partial) {
+  extern __shared__ __align__(16) short lds[];
+  constexpr int Q = NTO * 4;
+  short *sa = lds;                                // [halo voxel][16]
+  short *sg = sa + (long)G.hvol * 16;             // [o tile][voxel of the box][16]
+  short *sz = sg + NTO * kWgVox * 16;             // 4 zeros: the input of voxels outside the grid
+  float *sb = (float *)(sz + 8);                  // [256][4] bias partial sums
+  unsigned short *pt = (unsigned short *)(sb + 1024);  // halo position of a voxel, 0xffff: none
+  const int cc = (int)(blockIdx.x % (unsigned)ncc), p = (int)(blockIdx.x / (unsigned)ncc);
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
+  const int hx = (int)G.dhx.f.d, hy = (int)G.dhy.f.d, ct = in.c0 + in.c1;
+  if (tid < 4) sz[tid] = 0;
+  v4f acc[7][NTO];
+  int toff[7];
+#pragma unroll
+  for (int t = 0; t < 7; t++) {
+    const int tap = min(w + 4 * t, 26);
+    toff[t] = (((tap / 9 - 1) * hy + (tap / 3) % 3 - 1) * hx + tap % 3 - 1) * 16;
+#pragma unroll
+    for (int k = 0; k < NTO; k++) acc[t][k] = (v4f){0.f, 0.f, 0.f, 0.f};
+  }
+  float bs[4] = {0.f, 0.f, 0.f, 0.f};
+  const Div1 d4 = Div1{FastDiv{4u, 0x80000000u, 1}};  // (n * 2^31 >> 32) >> 1 = n / 4
+  for (int box = p; box < G.nbox; box += P) {
+    int b, z0, y0, x0;
+    conv_box(G, box, b, z0, y0, x0);
+    __syncthreads();  // the previous box has been read
+    conv_stage(G, in, cc, 1, d4, b, z0, y0, x0, sa);
+    // the output gradients: thread tid takes the channels 4 (tid % Q) .. + 3 of every box voxel
+    // tid / Q + k 256 / Q
+    const int q = tid % Q;
+#pragma unroll 4
+    for (int m = tid / Q; m < kWgVox; m += 256 / Q) {
+      const unsigned mc = (unsigned)(m < G.vol ? m : 0), t = fdiv(mc, G.dbx);
+      const int xx = (int)(mc - t * G.dbx.f.d);
+      const unsigned zz = fdiv(t, G.dby);
+      const int yy = (int)(t - zz * G.dby.f.d);
+      const int z = z0 + (int)zz, y = y0 + yy, x = x0 + xx;
+      const bool ok = m < G.vol && z < G.n && y < G.n && x < G.n;
+      const long v = (((long)b * G.n + z) * G.n + y) * G.n + x;
+      float f[4];
+      if ((co & 3) == 0) {
+        const float4 r = ok && 4 * q < co ? *(const float4 *)(gout + v * co + 4 * q)
+                                          : make_float4(0.f, 0.f, 0.f, 0.f);
+        f[0] = r.x;
+        f[1] = r.y;
+        f[2] = r.z;
+        f[3] = r.w;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++) f[j] = ok && 4 * q + j < co ? gout[v * co + 4 * q + j] : 0.f;
       }
-      soff[threadIdx.x] = off;
+      v4s s;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        bs[j] += f[j];
+        s[j] = bf16_bits(f[j]);
+      }
+      *(v4s *)(sg + ((long)(q >> 2) * kWgVox + m) * 16 + (q & 3) * 4) = s;
+      if (q == 0)
+        pt[m] = ok ? (unsigned short)((((int)zz + 1) * hy + yy + 1) * hx + xx + 1) : 0xffff;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < kWgChunk * cip; e += blockDim.x) {
-      const int k = e / cip, c = e - k * cip;
-      const long off = soff[k];
-      sin[e] = bf16_bits(off >= 0 && c < ci ? in[off + c] : 0.f);
-    }
-    for (int e = threadIdx.x; e < kWgChunk * cop; e += blockDim.x) {
-      const int k = e / cop, o = e - k * cop;
-      const long v = vs + k;
-      const float val = v < vend && o < co ? gout[v * co + o] : 0.f;
-      bsum += val;
-      sg[e] = bf16_bits(val);
-    }
-    __syncthreads();
-#pragma unroll 1
-    for (int k0 = 0; k0 < kWgChunk; k0 += 16) {
+#pragma unroll 2
+    for (int ks = 0; ks < kWgVox; ks += 16) {
+      const int m = ks + 4 * g + (l16 >> 2);
+      const unsigned pos = pt[m];
+      const short *ab = sa + (int)pos * 16 + 4 * (l16 & 3);
+      v4s bb[NTO];
 #pragma unroll
-      for (int t = 0; t < kWgTiles; t++) {
-        const int tile = w + 4 * t;
-        if (tile >= ntiles) break;  // wave-uniform
-        const int c0 = (tile / nto) * 16, o0 = (tile % nto) * 16;
-        v4s a, bb;
+      for (int k = 0; k < NTO; k++)
+        bb[k] = lds_read_tr(sg + ((long)k * kWgVox + m) * 16 + 4 * (l16 & 3));
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          a[j] = sin[(k0 + 4 * g + j) * cip + c0 + i];   // A[c0 + i][voxel 4g + j]
-          bb[j] = sg[(k0 + 4 * g + j) * cop + o0 + i];   // B[voxel 4g + j][o0 + i]
-        }
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, acc[t], 0, 0, 0);
+      for (int t = 0; t < 7; t++) {
+        const v4s a = lds_read_tr(pos == 0xffffu ? sz : ab + toff[t]);
+#pragma unroll
+        for (int k = 0; k < NTO; k++)
+          acc[t][k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb[k], acc[t][k], 0, 0, 0);
       }
     }
   }
-  const long npair = (long)ci * co, stride = 27 * npair + co;
-  float *part = partial + chunk * stride;
-  // D[4g + q][i]: input channel c0 + 4g + q, output channel o0 + i
+  const long npair = (long)ct * co, stride = 27 * npair + co;
+  float *part = partial + (long)p * stride;
+  // D[4g + q][l16]: input channel 16 cc + 4g + q, output channel 16 k + l16
 #pragma unroll
-  for (int t = 0; t < kWgTiles; t++) {
-    const int tile = w + 4 * t;
-    if (tile >= ntiles) break;
-    const int c0 = (tile / nto) * 16, o = (tile % nto) * 16 + i;
-    for (int q = 0; q < 4; q++) {
-      const int c = c0 + 4 * g + q;
-      if (c < ci && o < co) part[tap * npair + (long)c * co + o] = acc[t][q];
-    }
+  for (int t = 0; t < 7; t++) {
+    const int tap = w + 4 * t;
+    if (tap >= 27) break;
+#pragma unroll
+    for (int k = 0; k < NTO; k++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int c = cc * 16 + 4 * g + q, o = k * 16 + l16;
+        if (c < ct && o < co) part[tap * npair + (long)c * co + o] = acc[t][k][q];
+      }
   }
-  if (tap == 13) {  // bias: threads with the same channel summed in thread order
-    sb[threadIdx.x] = bsum;
+  if (cc == 0) {  // bias: the threads of one channel group summed in thread order
+#pragma unroll
+    for (int j = 0; j < 4; j++) sb[tid * 4 + j] = bs[j];
     __syncthreads();
-    if (threadIdx.x < co) {
+    if (tid < co) {
       float s = 0.f;
-      for (int k = threadIdx.x; k < 256; k += cop) s += sb[k];
-      part[27 * npair + threadIdx.x] = s;
+      for (int k = tid >> 2; k < 256; k += Q) s += sb[k * 4 + (tid & 3)];
+      part[27 * npair + tid] = s;
     }
   }
 }
 
-// gW[t][c][o] and gb[o] = sums over the chunks (fixed order) of the partials
-__global__ void k_wgrad_reduce(long nchunks, int np27, int co, const float *partial, float *gw,
-                               float *gb) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np27 + co) return;
-  const long stride = (long)np27 + co;
-  float s = 0.f;
-  for (long c = 0; c < nchunks; c++) s += partial[c * stride + p];
-  if (p < np27) gw[p] = s;
-  else gb[p - np27] = s;
+// The gradients of all layers from their partials, one launch: grad[off + e] = the sum over the
+// layer's P partials in a fixed order (eight consecutive ranges, each in ascending order).
+struct WgLayer {
+  long part, off;  // first partial value, first gradient value
+  int np, P, blk;  // values per partial, partials, first block of the layer
+};
+struct WgTable {
+  WgLayer l[9];
+};
+constexpr int kWrSeg = 8;
+
+__global__ __launch_bounds__(64 * kWrSeg) void k_wgrad_reduce(WgTable T,
+                                                              const float *__restrict__ partial,
+                                                              float *__restrict__ grad) {
+  __shared__ float s[kWrSeg][64];
+  int l = 0;
+  while (l < 8 && (int)blockIdx.x >= T.l[l + 1].blk) l++;
+  const WgLayer L = T.l[l];
+  const int e = ((int)blockIdx.x - L.blk) * 64 + (threadIdx.x & 63), seg = threadIdx.x >> 6;
+  const int per = (L.P + kWrSeg - 1) / kWrSeg, c1 = min((seg + 1) * per, L.P);
+  float a = 0.f;
+  if (e < L.np) {
+    const float *q = partial + L.part + e;
+    int c = seg * per;
+    for (; c + 8 <= c1; c += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = q[(long)(c + u) * L.np];
+#pragma unroll
+      for (int u = 0; u < 8; u++) a += v[u];
+    }
+    for (; c < c1; c++) a += q[(long)c * L.np];
+  }
+  s[seg][threadIdx.x & 63] = a;
+  __syncthreads();
+  if (seg == 0 && e < L.np) {
+    float r = 0.f;
+#pragma unroll
+    for (int k = 0; k < kWrSeg; k++) r += s[k][threadIdx.x & 63];
+    grad[L.off + e] = r;
+  }
 }
 
-// ---- elementwise / resampling ------------------------------------------------------------
+// ---- elementwise / resampling (four channels per thread) -----------------------------------
 
-__global__ void k_relu_bwd(long m, const float *act, float *g) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < m && act[i] <= 0.f) g[i] = 0.f;
+// voxel v of the grid of n per axis: batch, z, y, x
+__device__ __forceinline__ void vox_coords(long v, int n, long &b, int &z, int &y, int &x) {
+  long t = v / n;
+  x = (int)(v - t * n);
+  long u = t / n;
+  y = (int)(t - u * n);
+  b = u / n;
+  z = (int)(u - b * n);
 }
 
-// average pool 2x2x2: out (n/2) from in (n)
+// average pool 2x2x2: out (n/2) from in (n), c channels (a multiple of 4)
 __global__ void k_pool(int batch, int n, int c, const float *in, float *out) {
-  int h = n / 2;
-  long total = (long)batch * h * h * h * c;
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int h = n / 2, c4 = c / 4;
+  const long total = (long)batch * h * h * h * c4;
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= total) return;
-  int k = (int)(e % c);
-  long pv = e / c;
-  int x = (int)(pv % h), y = (int)((pv / h) % h), z = (int)((pv / ((long)h * h)) % h);
-  int b = (int)(pv / ((long)h * h * h));
-  float s = 0.f;
+  const int k = (int)(e % c4);
+  long b;
+  int z, y, x;
+  vox_coords(e / c4, h, b, z, y, x);
+  float4 f[8];
+#pragma unroll
   for (int d = 0; d < 8; d++) {
-    int zz = 2 * z + (d >> 2), yy = 2 * y + ((d >> 1) & 1), xx = 2 * x + (d & 1);
-    s += in[(((long)b * n + zz) * n * n + (long)yy * n + xx) * c + k];
+    const int zz = 2 * z + (d >> 2), yy = 2 * y + ((d >> 1) & 1), xx = 2 * x + (d & 1);
+    f[d] = *(const float4 *)(in + (((b * n + zz) * n + yy) * n + xx) * c + 4 * k);
   }
-  out[e] = 0.125f * s;
-}
-
-// gin (n) += gout (n/2) / 8
-__global__ void k_pool_bwd(int batch, int n, int c, const float *gout, float *gin) {
-  long total = (long)batch * n * n * n * c;
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  int k = (int)(e % c);
-  long v = e / c;
-  int x = (int)(v % n), y = (int)((v / n) % n), z = (int)((v / ((long)n * n)) % n);
-  int b = (int)(v / ((long)n * n * n));
-  int h = n / 2;
-  gin[e] += 0.125f * gout[(((long)b * h + z / 2) * h * h + (long)(y / 2) * h + x / 2) * c + k];
-}
-
-// cat (n, cu+cs) = [nearest-upsampled up (n/2, cu), skip (n, cs)]
-__global__ void k_upcat(int batch, int n, int cu, int cs, const float *up, const float *skip,
-                        float *cat) {
-  int ct = cu + cs;
-  long total = (long)batch * n * n * n * ct;
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  int k = (int)(e % ct);
-  long v = e / ct;
-  if (k >= cu) {
-    cat[e] = skip[v * cs + (k - cu)];
-    return;
-  }
-  int x = (int)(v % n), y = (int)((v / n) % n), z = (int)((v / ((long)n * n)) % n);
-  int b = (int)(v / ((long)n * n * n));
-  int h = n / 2;
-  cat[e] = up[(((long)b * h + z / 2) * h * h + (long)(y / 2) * h + x / 2) * cu + k];
-}
-
-// backward of upcat: gup (n/2, cu) = sum over the 8 children; gskip (n, cs) += skip part
-__global__ void k_upcat_bwd_up(int batch, int n, int cu, int cs, const float *gcat, float *gup) {
-  int h = n / 2;
-  long total = (long)batch * h * h * h * cu;
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  int k = (int)(e % cu);
-  long pv = e / cu;
-  int x = (int)(pv % h), y = (int)((pv / h) % h), z = (int)((pv / ((long)h * h)) % h);
-  int b = (int)(pv / ((long)h * h * h));
-  float s = 0.f;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
   for (int d = 0; d < 8; d++) {
-    int zz = 2 * z + (d >> 2), yy = 2 * y + ((d >> 1) & 1), xx = 2 * x + (d & 1);
-    s += gcat[(((long)b * n + zz) * n * n + (long)yy * n + xx) * (cu + cs) + k];
+    s.x += f[d].x;
+    s.y += f[d].y;
+    s.z += f[d].z;
+    s.w += f[d].w;
   }
-  gup[e] = s;
+  *(float4 *)(out + e * 4) = make_float4(0.125f * s.x, 0.125f * s.y, 0.125f * s.z, 0.125f * s.w);
 }
 
-__global__ void k_upcat_bwd_skip(long nvox, int cu, int cs, const float *gcat, float *gskip) {
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nvox * cs) return;
-  long v = e / cs;
-  int k = (int)(e % cs);
-  gskip[e] = gcat[v * (cu + cs) + cu + k];
+// gradient of an upsampled layer (n/2, cu) from that of the concatenation (n, cu + cs): the sum
+// over the 8 children, zero where the layer's activation is <= 0
+__global__ void k_up_bwd(int batch, int n, int cu, int cs, const float *gcat, const float *act,
+                         float *gup) {
+  const int h = n / 2, c4 = cu / 4;
+  const long total = (long)batch * h * h * h * c4;
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= total) return;
+  const int k = (int)(e % c4);
+  long b;
+  int z, y, x;
+  vox_coords(e / c4, h, b, z, y, x);
+  float4 f[8];
+#pragma unroll
+  for (int d = 0; d < 8; d++) {
+    const int zz = 2 * z + (d >> 2), yy = 2 * y + ((d >> 1) & 1), xx = 2 * x + (d & 1);
+    f[d] = *(const float4 *)(gcat + (((b * n + zz) * n + yy) * n + xx) * (cu + cs) + 4 * k);
+  }
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int d = 0; d < 8; d++) {
+    s.x += f[d].x;
+    s.y += f[d].y;
+    s.z += f[d].z;
+    s.w += f[d].w;
+  }
+  const float4 a = *(const float4 *)(act + e * 4);
+  if (a.x <= 0.f) s.x = 0.f;
+  if (a.y <= 0.f) s.y = 0.f;
+  if (a.z <= 0.f) s.z = 0.f;
+  if (a.w <= 0.f) s.w = 0.f;
+  *(float4 *)(gup + e * 4) = s;
+}
+
+// gradient of a layer that feeds the skip connection and the pool: the skip part of gcat
+// (n, cu + cs) plus gpool (n/2, cs) / 8, zero where the layer's activation is <= 0
+__global__ void k_skip_bwd(int batch, int n, int cu, int cs, const float *gcat,
+                           const float *gpool, const float *act, float *g) {
+  const int h = n / 2, c4 = cs / 4;
+  const long total = (long)batch * n * n * n * c4;
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= total) return;
+  const int k = (int)(e % c4);
+  const long v = e / c4;
+  long b;
+  int z, y, x;
+  vox_coords(v, n, b, z, y, x);
+  float4 s = *(const float4 *)(gcat + v * (cu + cs) + cu + 4 * k);
+  const float4 p = *(const float4 *)(gpool + (((b * h + z / 2) * h + y / 2) * h + x / 2) * cs +
+                                     4 * k);
+  const float4 a = *(const float4 *)(act + e * 4);
+  s.x += 0.125f * p.x;
+  s.y += 0.125f * p.y;
+  s.z += 0.125f * p.z;
+  s.w += 0.125f * p.w;
+  if (a.x <= 0.f) s.x = 0.f;
+  if (a.y <= 0.f) s.y = 0.f;
+  if (a.z <= 0.f) s.z = 0.f;
+  if (a.w <= 0.f) s.w = 0.f;
+  *(float4 *)(g + e * 4) = s;
 }
 
 // MSE: g = 2 (y - t) / m; per-block partial sums of (y - t)^2
@@ -327,12 +580,16 @@ __global__ __launch_bounds__(256) void k_mse(long m, const float *y, const float
   if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
 }
 
-__global__ void k_sum_partials(int np, const double *p, double *out, double scale) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < np; i++) s += p[i];
-    *out = s * scale;
+// *out = scale * the sum of 256 partials, by pairs
+__global__ __launch_bounds__(256) void k_sum_partials(const double *p, double *out, double scale) {
+  __shared__ double s[256];
+  s[threadIdx.x] = p[threadIdx.x];
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+    __syncthreads();
   }
+  if (threadIdx.x == 0) *out = s[0] * scale;
 }
 
 // Adam (Kingma & Ba 2015) on the FP32 master parameters
@@ -348,17 +605,39 @@ __global__ void k_adam(long np, float *theta, const float *g, float *m, float *v
   theta[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
-// BF16 weight copies: wf[t][o][c] (forward) and wg[t][c][o] (input gradient)
-__global__ void k_wcopies(int ci, int co, const float *W, short *wf, short *wg) {
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long tot = 27L * ci * co;
-  if (e >= tot) return;
-  int t = (int)(e / ((long)ci * co));
-  int c = (int)((e / co) % ci);
-  int o = (int)(e % co);
-  short b = bf16_bits(W[e]);  // W[t][c][o]
-  wf[((long)t * co + o) * ci + c] = b;
-  wg[((long)t * ci + c) * co + o] = b;
+// The BF16 weight fragments of k_conv, all layers in one launch, zero beyond ci and co:
+// forward   wf[t][chunk of c][tile of o][lane][j] = W[t][c = 16 chunk + 4 (lane / 16) + j]
+//                                                    [o = 16 tile + lane % 16]
+// transposed wg[t][chunk of o][tile of c][lane][j] = W[t][c = 16 tile + lane % 16]
+//                                                    [o = 16 chunk + 4 (lane / 16) + j]
+struct WfLayer {
+  long w, f;        // first weight, first fragment value
+  int ci, co, blk;  // channels, first block of the layer
+};
+struct WfTable {
+  WfLayer l[9];
+};
+__global__ __launch_bounds__(256) void k_wfrag(WfTable T, const float *__restrict__ theta,
+                                               short *wf, short *wg) {
+  int l = 0;
+  while (l < 8 && (int)blockIdx.x >= T.l[l + 1].blk) l++;
+  const WfLayer L = T.l[l];
+  const int nc = (L.ci + 15) / 16, no = (L.co + 15) / 16;
+  const int e = ((int)blockIdx.x - L.blk) * 256 + threadIdx.x;
+  if (e >= 27 * nc * no * 256) return;
+  const int j = e & 3, lane = (e >> 2) & 63, f = e >> 8;
+  const int k = 4 * (lane >> 4) + j, i = lane & 15;
+  const float *W = theta + L.w;
+  {
+    const int ot = f % no, ch = (f / no) % nc, t = f / (no * nc), c = ch * 16 + k, o = ot * 16 + i;
+    wf[L.f + e] =
+        c < L.ci && o < L.co ? bf16_bits(W[((long)t * L.ci + c) * L.co + o]) : (short)0;
+  }
+  {
+    const int tt = f % nc, ch = (f / nc) % no, t = f / (no * nc), c = tt * 16 + i, o = ch * 16 + k;
+    wg[L.f + e] =
+        c < L.ci && o < L.co ? bf16_bits(W[((long)t * L.ci + c) * L.co + o]) : (short)0;
+  }
 }
 
 }  // namespace flgpu
@@ -370,15 +649,21 @@ struct flgpu_unet {
   int cin = 2;
   long np = 0;
   long woff[flgpu::NL], boff[flgpu::NL];
+  long foff[flgpu::NL];  // first weight fragment value of a layer
+  flgpu::WfTable wft;
+  unsigned wf_blocks = 0;
   float *theta = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr;
-  short *wf = nullptr, *wg = nullptr;  // BF16 copies, same offsets as W blocks
+  short *wf = nullptr, *wg = nullptr;  // BF16 weight fragments (k_wfrag)
   int step = 0;
-  // activation storage for the current (batch, n)
+  // activation storage and launch plans for the current (batch, n)
   int cap_batch = 0, cap_n = 0;
-  float *a[flgpu::NL] = {}, *p0 = nullptr, *p1 = nullptr, *c1 = nullptr, *c0 = nullptr;
+  float *a[flgpu::NL] = {}, *p0 = nullptr, *p1 = nullptr;
   float *g[flgpu::NL] = {}, *gp0 = nullptr, *gp1 = nullptr, *gc1 = nullptr, *gc0 = nullptr;
-  float *gskip0 = nullptr, *gskip1 = nullptr, *partial = nullptr;
-  long partial_cap = 0;
+  float *partial = nullptr;
+  flgpu::ConvPlan fwd[flgpu::NL], bwd[flgpu::NL];
+  flgpu::ConvGeom wgeom[3];
+  flgpu::WgTable wgt;
+  unsigned wr_blocks = 0;
   double *lpart = nullptr;
 };
 
@@ -388,14 +673,92 @@ flgpu_ctx *unet_ctx(const flgpu_unet *u) { return u->ctx; }
 
 static long vox(int batch, int n) { return (long)batch * n * n * n; }
 
+static int layer_cin(const flgpu_unet *u, int l) { return l == 0 ? u->cin : L_CIN[l]; }
+static int tiles16(int c) { return (c + 15) / 16; }
+
+// The box of at most vcap voxels, with at most hcap voxels including its halo, that costs least
+// for n voxels per axis: every block costs its vcap voxels of products, also where the box or
+// its part inside the grid is smaller, and about 0.3 of that per halo voxel staged.  Extents
+// that divide the grid evenly win, so odd grids get boxes of their own.
+static ConvGeom conv_geom(int batch, int n, int vcap, int hcap) {
+  std::vector<int> ext;
+  for (int k = 1; k <= n; k++) {
+    const int e = (n + k - 1) / k;
+    if (ext.empty() || ext.back() != e) ext.push_back(e);
+  }
+  double best = -1.0;
+  int bz = 1, by = 1, bx = 1;
+  for (int ex : ext)
+    for (int ey : ext)
+      for (int ez : ext) {
+        if ((long)ex * ey * ez > vcap) continue;
+        const long hv = (long)(ex + 2) * (ey + 2) * (ez + 2);
+        if (hv > hcap) continue;
+        const double boxes = (double)((n + ex - 1) / ex) * ((n + ey - 1) / ey) * ((n + ez - 1) / ez);
+        const double cost = boxes * (vcap + 0.3 * hv);
+        if (best < 0.0 || cost < best) {
+          best = cost;
+          bz = ez;
+          by = ey;
+          bx = ex;
+        }
+      }
+  ConvGeom G;
+  G.n = n;
+  G.bz = bz;
+  G.by = by;
+  G.bx = bx;
+  G.vol = bz * by * bx;
+  G.hvol = (bz + 2) * (by + 2) * (bx + 2);
+  const int nx = (n + bx - 1) / bx, ny = (n + by - 1) / by, nz = (n + bz - 1) / bz;
+  const long nbox = (long)batch * nx * ny * nz;
+  FLGPU_REQUIRE(nbox < 0x7fffffffL / 27, "too many voxels for the convolution's index range");
+  G.nbox = (int)nbox;
+  G.dnx = div1(nx);
+  G.dny = div1(ny);
+  G.dnz = div1(nz);
+  G.dbx = div1(bx);
+  G.dby = div1(by);
+  G.dhx = div1(bx + 2);
+  G.dhy = div1(by + 2);
+  return G;
+}
+
+// bytes of LDS per block: two blocks fit a CU's 160 KB
+constexpr int kConvLds = 80 * 1024;
+
+// How a convolution with nch chunks of input channels and ntt tiles of output channels is
+// split: four waves share a box, wm of them along its voxels and 4 / wm along its channel tiles.
+// A wave with more voxel tiles (mt) reuses a weight fragment more often, so the largest mt is
+// taken that still gives every CU two blocks; grids too small for that (one sample: 64 boxes
+// of 64 voxels at 16^3, 8 at 8^3) are split further, over the channel tiles too.
+static ConvPlan conv_plan(const flgpu_unet *u, int batch, int n, int nch, int ntt) {
+  const int hcap = kConvLds / (32 * nch), cus = u->ctx->cus;
+  ConvPlan p;
+  for (p.mt = 4; p.mt >= 1; p.mt /= 2) {
+    if (p.mt * ntt > 16 && p.mt > 1) continue;  // registers of the accumulators
+    p.wm = 4;
+    p.nt = ntt;
+    p.g = conv_geom(batch, n, 64 * p.mt, hcap);
+    if (p.g.nbox >= 2 * cus || p.mt == 1) break;
+  }
+  while (p.mt == 1 && p.g.nbox < cus && p.wm > 1 && p.nt % 2 == 0) {
+    p.wm /= 2;
+    p.nt /= 2;
+    p.g = conv_geom(batch, n, 16 * p.wm, hcap);
+  }
+  p.nch = nch;
+  p.ntt = ntt;
+  return p;
+}
+
 static void unet_free_acts(flgpu_unet *u) {
   for (int l = 0; l < NL; l++) {
     dev_free(u->a[l]);
     dev_free(u->g[l]);
     u->a[l] = u->g[l] = nullptr;
   }
-  for (float **p : {&u->p0, &u->p1, &u->c1, &u->c0, &u->gp0, &u->gp1, &u->gc1, &u->gc0,
-                    &u->gskip0, &u->gskip1}) {
+  for (float **p : {&u->p0, &u->p1, &u->gp0, &u->gp1, &u->gc1, &u->gc0, &u->partial}) {
     dev_free(*p);
     *p = nullptr;
   }
@@ -407,113 +770,149 @@ static void unet_alloc_acts(flgpu_unet *u, int batch, int n, bool train) {
   unet_free_acts(u);
   int nl[3] = {n, n / 2, n / 4};
   auto fa = [](long cnt) { return (float *)dev_alloc(sizeof(float) * cnt); };
-  for (int l = 0; l < NL; l++) u->a[l] = fa(vox(batch, nl[L_LEVEL[l]]) * L_COUT[l]);
+  for (int l = 0; l < NL; l++) {
+    const int nn = nl[L_LEVEL[l]], ci = tiles16(layer_cin(u, l)), co = tiles16(L_COUT[l]);
+    u->fwd[l] = conv_plan(u, batch, nn, ci, co);
+    u->bwd[l] = conv_plan(u, batch, nn, co, ci);
+    u->a[l] = fa(vox(batch, nn) * L_COUT[l]);
+  }
   u->p0 = fa(vox(batch, nl[1]) * 16);
   u->p1 = fa(vox(batch, nl[2]) * 32);
-  u->c1 = fa(vox(batch, nl[1]) * 96);
-  u->c0 = fa(vox(batch, nl[0]) * 48);
   if (train) {
     for (int l = 0; l < NL; l++) u->g[l] = fa(vox(batch, nl[L_LEVEL[l]]) * L_COUT[l]);
     u->gp0 = fa(vox(batch, nl[1]) * 16);
     u->gp1 = fa(vox(batch, nl[2]) * 32);
     u->gc1 = fa(vox(batch, nl[1]) * 96);
     u->gc0 = fa(vox(batch, nl[0]) * 48);
-    u->gskip0 = fa(vox(batch, nl[0]) * 16);
-    u->gskip1 = fa(vox(batch, nl[1]) * 32);
+    for (int k = 0; k < 3; k++)
+      u->wgeom[k] = conv_geom(batch, nl[k], kWgVox, kConvLds / 64);
+    // P blocks per chunk of input channels: about four blocks per CU (two: 2197 us for a
+    // batch of 32 x 32^3 instead of 1999), all with the same number
+    // of boxes but for the last few
+    long off = 0;
+    int blk = 0;
+    for (int l = 0; l < NL; l++) {
+      const int nbox = u->wgeom[L_LEVEL[l]].nbox, ncc = tiles16(layer_cin(u, l));
+      const int pmax = std::max(1, std::min(nbox, 4 * u->ctx->cus / ncc));
+      const int per = (nbox + pmax - 1) / pmax;
+      WgLayer &W = u->wgt.l[l];
+      W.P = (nbox + per - 1) / per;
+      W.np = 27 * layer_cin(u, l) * L_COUT[l] + L_COUT[l];
+      W.part = off;
+      W.off = u->woff[l];
+      W.blk = blk;
+      off += (long)W.P * W.np;
+      blk += (W.np + 63) / 64;
+    }
+    u->partial = fa(off);
+    u->wr_blocks = (unsigned)blk;
   }
   u->cap_batch = batch;
   u->cap_n = n;
 }
 
-static void conv(flgpu_unet *u, int l, int batch, int n, int ci, const float *in, float *out,
-                 int relu) {
-  int co = L_COUT[l];
-  long total = vox(batch, n);
-  unsigned gsz = grid_for((total + 15) / 16, 4);
-  const short *wk = u->wf + u->woff[l];
-  const float *bias = u->theta + u->boff[l];
-  hipStream_t s = u->ctx->stream;
-  int nt = (co + 15) / 16;
-  switch (nt) {
-    case 1: k_conv_mfma<1><<<gsz, 256, 0, s>>>(batch, n, ci, co, in, wk, bias, out, relu, 1); break;
-    case 2: k_conv_mfma<2><<<gsz, 256, 0, s>>>(batch, n, ci, co, in, wk, bias, out, relu, 1); break;
-    default: k_conv_mfma<4><<<gsz, 256, 0, s>>>(batch, n, ci, co, in, wk, bias, out, relu, 1); break;
-  }
+template <int MT, int NT>
+static void conv_launch(flgpu_unet *u, const ConvPlan &p, const ConvIn &in, int no,
+                        const short *wf, const float *bias, const float *mask, float *out,
+                        int relu, int sgn) {
+  const size_t lds = (size_t)p.nch * p.g.hvol * 32;
+  if (lds > 64 * 1024)
+    FLGPU_HIP(hipFuncSetAttribute((const void *)k_conv<MT, NT>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  k_conv<MT, NT><<<xcd_grid(p.g.nbox), 256, lds, u->ctx->stream>>>(
+      p.g, in, p.nch, div1(p.nch * 4), no, p.ntt, wf, bias, mask, out, relu, sgn, p.wm);
   FLGPU_HIP(hipGetLastError());
 }
 
-// gin = conv^T(gout) through the transposed weights (taps mirrored)
-static void conv_gin(flgpu_unet *u, int l, int batch, int n, int ci, const float *gout,
-                     float *gin) {
-  int co = L_COUT[l];
-  long total = vox(batch, n);
-  unsigned gsz = grid_for((total + 15) / 16, 4);
-  const short *wk = u->wg + u->woff[l];  // [t][c][o]: K index o contiguous
-  hipStream_t s = u->ctx->stream;
-  int nt = (ci + 15) / 16;
-  // roles swap: "input" channels = co (K), "output" channels = ci (N)
-  switch (nt) {
-    case 1: k_conv_mfma<1><<<gsz, 256, 0, s>>>(batch, n, co, ci, gout, wk, nullptr, gin, 0, -1); break;
-    case 2: k_conv_mfma<2><<<gsz, 256, 0, s>>>(batch, n, co, ci, gout, wk, nullptr, gin, 0, -1); break;
-    case 3:
-    case 4: k_conv_mfma<4><<<gsz, 256, 0, s>>>(batch, n, co, ci, gout, wk, nullptr, gin, 0, -1); break;
-    default: k_conv_mfma<6><<<gsz, 256, 0, s>>>(batch, n, co, ci, gout, wk, nullptr, gin, 0, -1); break;
+static void conv_run(flgpu_unet *u, const ConvPlan &p, const ConvIn &in, int no, const short *wf,
+                     const float *bias, const float *mask, float *out, int relu, int sgn) {
+#define FLGPU_CONV(MT, NT)                                                     \
+  if (p.mt == MT && p.nt == NT) {                                              \
+    conv_launch<MT, NT>(u, p, in, no, wf, bias, mask, out, relu, sgn);         \
+    return;                                                                    \
   }
-  FLGPU_HIP(hipGetLastError());
+  FLGPU_CONV(4, 1)
+  FLGPU_CONV(4, 2)
+  FLGPU_CONV(4, 3)
+  FLGPU_CONV(4, 4)
+  FLGPU_CONV(2, 1)
+  FLGPU_CONV(2, 2)
+  FLGPU_CONV(2, 3)
+  FLGPU_CONV(2, 4)
+  FLGPU_CONV(2, 6)
+  FLGPU_CONV(1, 1)
+  FLGPU_CONV(1, 2)
+  FLGPU_CONV(1, 3)
+  FLGPU_CONV(1, 4)
+  FLGPU_CONV(1, 6)
+#undef FLGPU_CONV
+  FLGPU_REQUIRE(false, "no convolution kernel for this layer");
 }
 
-static void conv_wgrad(flgpu_unet *u, int l, int batch, int n, int ci, const float *in,
-                       const float *gout) {
-  int co = L_COUT[l];
-  long total = vox(batch, n);
-  long nchunks = (total + kWgVox - 1) / kWgVox;
-  const int np27 = 27 * ci * co;
-  long need = nchunks * (np27 + (long)co);
-  if (need > u->partial_cap) {
-    dev_free(u->partial);
-    u->partial = (float *)dev_alloc(sizeof(float) * need);
-    u->partial_cap = need;
-  }
-  const int cip = (ci + 15) & ~15, cop = (co + 15) & ~15;
-  FLGPU_REQUIRE(cip <= 96 && cop <= 64 && (cip / 16) * (cop / 16) <= 4 * kWgTiles &&
-                    256 % cop == 0,
-                "layer too wide for the weight-gradient kernel");
+// out = relu(conv(in) + bias) of layer l
+static void conv(flgpu_unet *u, int l, const ConvIn &in, float *out, int relu) {
+  conv_run(u, u->fwd[l], in, L_COUT[l], u->wf + u->foff[l], u->theta + u->boff[l], nullptr, out,
+           relu, 1);
+}
+
+// gin = conv^T(gout) through the transposed weights (taps mirrored), zero where mask <= 0
+static void conv_gin(flgpu_unet *u, int l, const float *gout, const float *mask, float *gin) {
+  const ConvIn in = {gout, nullptr, L_COUT[l], 0, 0};
+  conv_run(u, u->bwd[l], in, layer_cin(u, l), u->wg + u->foff[l], nullptr, mask, gin, 0, -1);
+}
+
+// the partial sums of layer l's weight and bias gradients
+static void conv_wgrad(flgpu_unet *u, int l, const ConvIn &in, const float *gout) {
+  const ConvGeom &G = u->wgeom[L_LEVEL[l]];
+  const WgLayer &W = u->wgt.l[l];
+  const int co = L_COUT[l], nto = tiles16(co), ncc = tiles16(in.c0 + in.c1);
+  const size_t lds = (size_t)G.hvol * 32 + (size_t)nto * kWgVox * 32 + 16 + 4096 + kWgVox * 2;
+  const unsigned grid = (unsigned)(W.P * ncc);
+  float *part = u->partial + W.part;
   hipStream_t s = u->ctx->stream;
-  k_conv_wgrad<<<(unsigned)(nchunks * 27), 256, 0, s>>>(batch, n, ci, co, in, gout, u->partial);
-  k_wgrad_reduce<<<grid_for(np27 + co, 256), 256, 0, s>>>(nchunks, np27, co, u->partial,
-                                                          u->grad + u->woff[l],
-                                                          u->grad + u->boff[l]);
-  FLGPU_HIP(hipGetLastError());
+  auto launch = [&](auto kern) {
+    if (lds > 64 * 1024)
+      FLGPU_HIP(hipFuncSetAttribute((const void *)kern,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    kern<<<grid, 256, lds, s>>>(G, in, ncc, co, gout, W.P, part);
+    FLGPU_HIP(hipGetLastError());
+  };
+  switch (nto) {
+    case 1: launch(k_conv_wgrad<1>); break;
+    case 2: launch(k_conv_wgrad<2>); break;
+    case 4: launch(k_conv_wgrad<4>); break;
+    default: FLGPU_REQUIRE(false, "no weight-gradient kernel for this layer");
+  }
 }
 
 static void refresh_bf16(flgpu_unet *u) {
-  for (int l = 0; l < NL; l++) {
-    int ci = l == 0 ? u->cin : L_CIN[l], co = L_COUT[l];
-    long tot = 27L * ci * co;
-    k_wcopies<<<grid_for(tot, 256), 256, 0, u->ctx->stream>>>(ci, co, u->theta + u->woff[l],
-                                                             u->wf + u->woff[l], u->wg + u->woff[l]);
-  }
+  k_wfrag<<<u->wf_blocks, 256, 0, u->ctx->stream>>>(u->wft, u->theta, u->wf, u->wg);
   FLGPU_HIP(hipGetLastError());
 }
 
 static unsigned ew(long m) { return grid_for(m, 256); }
 
-void unet_forward(flgpu_unet *u, int batch, int n, const float *x) {
+// the decoder's inputs [upsampled, skip] and the plain ones
+static ConvIn conv_in(const float *p, int c) { return ConvIn{p, nullptr, c, 0, 0}; }
+static ConvIn conv_cat(const float *up, int cu, const float *skip, int cs) {
+  return ConvIn{up, skip, cu, cs, 1};
+}
+
+// y: the network's output (FP32, batch n^3 values)
+void unet_forward(flgpu_unet *u, int batch, int n, const float *x, float *y) {
   hipStream_t s = u->ctx->stream;
   int nl[3] = {n, n / 2, n / 4};
-  conv(u, 0, batch, n, u->cin, x, u->a[0], 1);
-  conv(u, 1, batch, n, 16, u->a[0], u->a[1], 1);
-  k_pool<<<ew(vox(batch, nl[1]) * 16), 256, 0, s>>>(batch, n, 16, u->a[1], u->p0);
-  conv(u, 2, batch, nl[1], 16, u->p0, u->a[2], 1);
-  conv(u, 3, batch, nl[1], 32, u->a[2], u->a[3], 1);
-  k_pool<<<ew(vox(batch, nl[2]) * 32), 256, 0, s>>>(batch, nl[1], 32, u->a[3], u->p1);
-  conv(u, 4, batch, nl[2], 32, u->p1, u->a[4], 1);
-  conv(u, 5, batch, nl[2], 64, u->a[4], u->a[5], 1);
-  k_upcat<<<ew(vox(batch, nl[1]) * 96), 256, 0, s>>>(batch, nl[1], 64, 32, u->a[5], u->a[3], u->c1);
-  conv(u, 6, batch, nl[1], 96, u->c1, u->a[6], 1);
-  k_upcat<<<ew(vox(batch, n) * 48), 256, 0, s>>>(batch, n, 32, 16, u->a[6], u->a[1], u->c0);
-  conv(u, 7, batch, n, 48, u->c0, u->a[7], 1);
-  conv(u, 8, batch, n, 16, u->a[7], u->a[8], 0);
+  conv(u, 0, conv_in(x, u->cin), u->a[0], 1);
+  conv(u, 1, conv_in(u->a[0], 16), u->a[1], 1);
+  k_pool<<<ew(vox(batch, nl[1]) * 4), 256, 0, s>>>(batch, n, 16, u->a[1], u->p0);
+  conv(u, 2, conv_in(u->p0, 16), u->a[2], 1);
+  conv(u, 3, conv_in(u->a[2], 32), u->a[3], 1);
+  k_pool<<<ew(vox(batch, nl[2]) * 8), 256, 0, s>>>(batch, nl[1], 32, u->a[3], u->p1);
+  conv(u, 4, conv_in(u->p1, 32), u->a[4], 1);
+  conv(u, 5, conv_in(u->a[4], 64), u->a[5], 1);
+  conv(u, 6, conv_cat(u->a[5], 64, u->a[3], 32), u->a[6], 1);
+  conv(u, 7, conv_cat(u->a[6], 32, u->a[1], 16), u->a[7], 1);
+  conv(u, 8, conv_in(u->a[7], 16), y, 0);
   FLGPU_HIP(hipGetLastError());
 }
 
@@ -523,40 +922,82 @@ void unet_backward(flgpu_unet *u, int batch, int n, const float *x, const float 
   int nl[3] = {n, n / 2, n / 4};
   long v0 = vox(batch, n), v1 = vox(batch, nl[1]), v2 = vox(batch, nl[2]);
   k_mse<<<256, 256, 0, s>>>(v0, u->a[8], t, u->g[8], u->lpart);
-  k_sum_partials<<<1, 1, 0, s>>>(256, u->lpart, u->ctx->red_out + 8, 1.0 / (double)v0);
-  conv_wgrad(u, 8, batch, n, 16, u->a[7], u->g[8]);
-  conv_gin(u, 8, batch, n, 16, u->g[8], u->g[7]);
-  k_relu_bwd<<<ew(v0 * 16), 256, 0, s>>>(v0 * 16, u->a[7], u->g[7]);
-  conv_wgrad(u, 7, batch, n, 48, u->c0, u->g[7]);
-  conv_gin(u, 7, batch, n, 48, u->g[7], u->gc0);
-  k_upcat_bwd_up<<<ew(v1 * 32), 256, 0, s>>>(batch, n, 32, 16, u->gc0, u->g[6]);
-  k_upcat_bwd_skip<<<ew(v0 * 16), 256, 0, s>>>(v0, 32, 16, u->gc0, u->gskip0);
-  k_relu_bwd<<<ew(v1 * 32), 256, 0, s>>>(v1 * 32, u->a[6], u->g[6]);
-  conv_wgrad(u, 6, batch, nl[1], 96, u->c1, u->g[6]);
-  conv_gin(u, 6, batch, nl[1], 96, u->g[6], u->gc1);
-  k_upcat_bwd_up<<<ew(v2 * 64), 256, 0, s>>>(batch, nl[1], 64, 32, u->gc1, u->g[5]);
-  k_upcat_bwd_skip<<<ew(v1 * 32), 256, 0, s>>>(v1, 64, 32, u->gc1, u->gskip1);
-  k_relu_bwd<<<ew(v2 * 64), 256, 0, s>>>(v2 * 64, u->a[5], u->g[5]);
-  conv_wgrad(u, 5, batch, nl[2], 64, u->a[4], u->g[5]);
-  conv_gin(u, 5, batch, nl[2], 64, u->g[5], u->g[4]);
-  k_relu_bwd<<<ew(v2 * 64), 256, 0, s>>>(v2 * 64, u->a[4], u->g[4]);
-  conv_wgrad(u, 4, batch, nl[2], 32, u->p1, u->g[4]);
-  conv_gin(u, 4, batch, nl[2], 32, u->g[4], u->gp1);
+  k_sum_partials<<<1, 256, 0, s>>>(u->lpart, u->ctx->red_out + 8, 1.0 / (double)v0);
+  conv_wgrad(u, 8, conv_in(u->a[7], 16), u->g[8]);
+  conv_gin(u, 8, u->g[8], u->a[7], u->g[7]);
+  conv_wgrad(u, 7, conv_cat(u->a[6], 32, u->a[1], 16), u->g[7]);
+  conv_gin(u, 7, u->g[7], nullptr, u->gc0);
+  k_up_bwd<<<ew(v1 * 8), 256, 0, s>>>(batch, n, 32, 16, u->gc0, u->a[6], u->g[6]);
+  conv_wgrad(u, 6, conv_cat(u->a[5], 64, u->a[3], 32), u->g[6]);
+  conv_gin(u, 6, u->g[6], nullptr, u->gc1);
+  k_up_bwd<<<ew(v2 * 16), 256, 0, s>>>(batch, nl[1], 64, 32, u->gc1, u->a[5], u->g[5]);
+  conv_wgrad(u, 5, conv_in(u->a[4], 64), u->g[5]);
+  conv_gin(u, 5, u->g[5], u->a[4], u->g[4]);
+  conv_wgrad(u, 4, conv_in(u->p1, 32), u->g[4]);
+  conv_gin(u, 4, u->g[4], nullptr, u->gp1);
   // a3 feeds the pool and the skip: gradients add
-  k_pool_bwd<<<ew(v1 * 32), 256, 0, s>>>(batch, nl[1], 32, u->gp1, u->gskip1);
-  k_relu_bwd<<<ew(v1 * 32), 256, 0, s>>>(v1 * 32, u->a[3], u->gskip1);
-  conv_wgrad(u, 3, batch, nl[1], 32, u->a[2], u->gskip1);
-  conv_gin(u, 3, batch, nl[1], 32, u->gskip1, u->g[2]);
-  k_relu_bwd<<<ew(v1 * 32), 256, 0, s>>>(v1 * 32, u->a[2], u->g[2]);
-  conv_wgrad(u, 2, batch, nl[1], 16, u->p0, u->g[2]);
-  conv_gin(u, 2, batch, nl[1], 16, u->g[2], u->gp0);
-  k_pool_bwd<<<ew(v0 * 16), 256, 0, s>>>(batch, n, 16, u->gp0, u->gskip0);
-  k_relu_bwd<<<ew(v0 * 16), 256, 0, s>>>(v0 * 16, u->a[1], u->gskip0);
-  conv_wgrad(u, 1, batch, n, 16, u->a[0], u->gskip0);
-  conv_gin(u, 1, batch, n, 16, u->gskip0, u->g[0]);
-  k_relu_bwd<<<ew(v0 * 16), 256, 0, s>>>(v0 * 16, u->a[0], u->g[0]);
-  conv_wgrad(u, 0, batch, n, u->cin, x, u->g[0]);
+  k_skip_bwd<<<ew(v1 * 8), 256, 0, s>>>(batch, nl[1], 64, 32, u->gc1, u->gp1, u->a[3], u->g[3]);
+  conv_wgrad(u, 3, conv_in(u->a[2], 32), u->g[3]);
+  conv_gin(u, 3, u->g[3], u->a[2], u->g[2]);
+  conv_wgrad(u, 2, conv_in(u->p0, 16), u->g[2]);
+  conv_gin(u, 2, u->g[2], nullptr, u->gp0);
+  k_skip_bwd<<<ew(v0 * 4), 256, 0, s>>>(batch, n, 32, 16, u->gc0, u->gp0, u->a[1], u->g[1]);
+  conv_wgrad(u, 1, conv_in(u->a[0], 16), u->g[1]);
+  conv_gin(u, 1, u->g[1], u->a[0], u->g[0]);
+  conv_wgrad(u, 0, conv_in(x, u->cin), u->g[0]);
+  k_wgrad_reduce<<<u->wr_blocks, 64 * kWrSeg, 0, s>>>(u->wgt, u->partial, u->grad);
   FLGPU_HIP(hipGetLastError());
+}
+
+// Standard normal values from 64-bit random words by Marsaglia's polar method (1964), in the
+// sequence std::normal_distribution<double> gives over std::mt19937_64, so a seed keeps its
+// weights.  The library's version takes two long double logarithms per word to find how many
+// words a double needs (one), 12 to 21 ms for a network; this takes 4.
+struct Normal {
+  std::mt19937_64 rng;
+  bool saved = false;
+  double save = 0.0;
+  explicit Normal(unsigned long seed) : rng(seed) {}
+  double canonical() {
+    const double u = (double)rng() / 18446744073709551616.0;
+    return u >= 1.0 ? std::nextafter(1.0, 0.0) : u;
+  }
+  void reset() { saved = false; }
+  double next() {
+    if (saved) {
+      saved = false;
+      return save;
+    }
+    double x, y, r2;
+    do {
+      x = 2.0 * canonical() - 1.0;
+      y = 2.0 * canonical() - 1.0;
+      r2 = x * x + y * y;
+    } while (r2 > 1.0 || r2 == 0.0);
+    const double m = std::sqrt(-2.0 * std::log(r2) / r2);
+    save = x * m;
+    saved = true;
+    return y * m;
+  }
+};
+
+// He-normal weights for the ReLU layers (a tenth of that for the output layer), zero biases
+static std::vector<float> initial_parameters(int cin, unsigned long seed) {
+  std::vector<float> h;
+  Normal nd(seed);
+  for (int l = 0; l < NL; l++) {
+    const int ci = l == 0 ? cin : L_CIN[l], co = L_COUT[l];
+    const long nw = 27L * ci * co;
+    const double sd = std::sqrt(2.0 / (27.0 * ci));
+    nd.reset();  // each layer has a distribution of its own
+    h.reserve(h.size() + nw + co);
+    for (long i = 0; i < nw; i++) {
+      const double v = nd.next() * sd;
+      h.push_back((float)(l == NL - 1 ? 0.1 * v : v));
+    }
+    h.insert(h.end(), co, 0.f);
+  }
+  return h;
 }
 
 static void check_shape(const flgpu_unet *u, const flgpu_vec *vec, int batch, int n, int ch,
@@ -578,28 +1019,28 @@ extern "C" int flgpu_unet_create(flgpu_ctx *ctx, int cin, unsigned long seed, fl
     flgpu_unet *u = new flgpu_unet;
     u->ctx = ctx;
     u->cin = cin;
+    const std::vector<float> h = initial_parameters(cin, seed);
     long off = 0;
-    std::vector<float> h;
-    std::mt19937_64 rng(seed);
     for (int l = 0; l < NL; l++) {
-      int ci = l == 0 ? cin : L_CIN[l], co = L_COUT[l];
       u->woff[l] = off;
-      long nw = 27L * ci * co;
-      // He-normal initialisation for ReLU layers
-      std::normal_distribution<double> nd(0.0, std::sqrt(2.0 / (27.0 * ci)));
-      for (long i = 0; i < nw; i++) h.push_back((float)(l == NL - 1 ? 0.1 * nd(rng) : nd(rng)));
-      off += nw;
-      u->boff[l] = off;
-      for (int i = 0; i < co; i++) h.push_back(0.f);
-      off += co;
+      u->boff[l] = off + 27L * layer_cin(u, l) * L_COUT[l];
+      off = u->boff[l] + L_COUT[l];
     }
     u->np = off;
+    long fo = 0;
+    for (int l = 0; l < NL; l++) {
+      const int ci = layer_cin(u, l), co = L_COUT[l], nf = 27 * tiles16(ci) * tiles16(co);
+      u->foff[l] = fo;
+      u->wft.l[l] = WfLayer{u->woff[l], fo, ci, co, (int)u->wf_blocks};
+      u->wf_blocks += nf;
+      fo += 256L * nf;
+    }
     u->theta = (float *)dev_alloc(sizeof(float) * off);
     u->m = (float *)dev_alloc(sizeof(float) * off);
     u->v = (float *)dev_alloc(sizeof(float) * off);
     u->grad = (float *)dev_alloc(sizeof(float) * off);
-    u->wf = (short *)dev_alloc(sizeof(short) * off);
-    u->wg = (short *)dev_alloc(sizeof(short) * off);
+    u->wf = (short *)dev_alloc(sizeof(short) * fo);
+    u->wg = (short *)dev_alloc(sizeof(short) * fo);
     u->lpart = (double *)dev_alloc(sizeof(double) * 256);
     FLGPU_HIP(hipMemcpyAsync(u->theta, h.data(), sizeof(float) * off, hipMemcpyHostToDevice,
                              ctx->stream));
@@ -620,7 +1061,7 @@ extern "C" int flgpu_unet_destroy(flgpu_unet *u) {
     FLGPU_HIP(hipStreamSynchronize(u->ctx->stream));
     unet_free_acts(u);
     for (void *p : {(void *)u->theta, (void *)u->m, (void *)u->v, (void *)u->grad, (void *)u->wf,
-                    (void *)u->wg, (void *)u->partial, (void *)u->lpart})
+                    (void *)u->wg, (void *)u->lpart})
       dev_free(p);
     delete u;
     return 0;
@@ -687,8 +1128,7 @@ extern "C" int flgpu_unet_forward(flgpu_unet *u, int batch, int n, const flgpu_v
     check_shape(u, y, batch, n, 1, "y");
     CTX_LOCK(u->ctx);
     unet_alloc_acts(u, batch, n, false);
-    unet_forward(u, batch, n, (const float *)x->d);
-    vcopy(u->ctx, vox(batch, n), FLGPU_F32, u->a[8], FLGPU_F32, y->d);
+    unet_forward(u, batch, n, (const float *)x->d, (float *)y->d);
     return 0;
   });
 }
@@ -703,7 +1143,7 @@ extern "C" int flgpu_unet_loss_grad(flgpu_unet *u, int batch, int n, const flgpu
     check_shape(u, t, batch, n, 1, "t");
     CTX_LOCK(u->ctx);
     unet_alloc_acts(u, batch, n, true);
-    unet_forward(u, batch, n, (const float *)x->d);
+    unet_forward(u, batch, n, (const float *)x->d, u->a[8]);
     unet_backward(u, batch, n, (const float *)x->d, (const float *)t->d);
     fetch_slots(u->ctx, 9);
     *loss = u->ctx->host_out[8];
@@ -726,7 +1166,7 @@ extern "C" int flgpu_unet_train_step(flgpu_unet *u, int batch, int n, const flgp
     check_shape(u, t, batch, n, 1, "t");
     CTX_LOCK(u->ctx);
     unet_alloc_acts(u, batch, n, true);
-    unet_forward(u, batch, n, (const float *)x->d);
+    unet_forward(u, batch, n, (const float *)x->d, u->a[8]);
     unet_backward(u, batch, n, (const float *)x->d, (const float *)t->d);
     u->step += 1;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -839,7 +1279,7 @@ struct UnetHook : LearnedHook {
       vdot_dev(ctx, N, prec, r1, r1, 10);
       k_pack<double><<<grid_for(nv, 256), 256, 0, s>>>(n, (const double *)r1, kd,
                                                        ctx->red_out + 10, xin, 0);
-      unet_forward(u, 1, n, xin);
+      unet_forward(u, 1, n, xin, u->a[8]);
       k_unpack<double><<<grid_for(N, 256), 256, 0, s>>>(n, u->a[8], (double *)c);
     } else {
       vcopy(ctx, N, FLGPU_F64, r1, mprec, lv[top - lc]);
@@ -852,7 +1292,7 @@ struct UnetHook : LearnedHook {
       else
         k_pack<float><<<grid_for(nv, 256), 256, 0, s>>>(n, (const float *)lv[0], kd,
                                                         ctx->red_out + 10, xin, 0);
-      unet_forward(u, 1, n, xin);
+      unet_forward(u, 1, n, xin, u->a[8]);
       if (mprec == FLGPU_F64)
         k_unpack<double><<<grid_for(Nc, 256), 256, 0, s>>>(n, u->a[8], (double *)lv[0]);
       else

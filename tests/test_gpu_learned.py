@@ -74,6 +74,54 @@ def test_unet_gradient_parity():
         assert d <= 3e-2 * np.linalg.norm(go[sl]) + 1e-12, (l, d, np.linalg.norm(go[sl]))
 
 
+@pytest.mark.parametrize("n,batch", [(4, 1), (12, 3), (20, 1)])
+def test_unet_parity_on_ragged_grids(n, batch):
+    """grids whose levels (n, n/2, n/4 down to 1, 3 and 5 voxels) leave partial boxes and halos:
+    the tolerances of the parity tests above"""
+    say(f"unet ragged {batch} x {n}^3")
+    theta = he_theta(n).astype(np.float32).astype(np.float64)
+    net = learned.UNet(2, 0)
+    net.set_params(theta)
+    rng = np.random.default_rng(n + 1)
+    x = rng.normal(size=batch * n ** 3 * 2).astype(np.float32).astype(np.float64)
+    t = rng.normal(size=batch * n ** 3).astype(np.float32).astype(np.float64)
+    xv, tv = GpuVector.from_array(x, F.F32), GpuVector.from_array(t, F.F32)
+    y = net.forward(xv, batch, n).numpy()
+    yo = po.unet_forward(theta, x, batch, n, bf16=True)
+    assert np.abs(y - yo).max() <= 1e-2 * np.abs(yo).max()
+    loss, g = net.loss_grad(xv, tv, batch, n)
+    lo, go = po.unet_loss_grad(theta, x, t, batch, n, bf16=True)
+    assert abs(loss - lo) <= 1e-3 * abs(lo)
+    for l, sl in enumerate(layer_slices()):
+        d = np.linalg.norm(g[sl] - go[sl])
+        assert d <= 3e-2 * np.linalg.norm(go[sl]) + 1e-12, (l, d, np.linalg.norm(go[sl]))
+
+
+@pytest.mark.parametrize("n,batch", [(32, 8), (20, 16), (12, 2)])
+def test_unet_batch_equals_its_samples(n, batch):
+    """a batch is split over the GPU otherwise than one sample, but every output accumulates
+    its products in the same order: the outputs equal bit for bit.  The batch is a power of two,
+    so its gradient is the samples' mean up to the order of the FP32 sums over the voxels, about
+    eps sqrt(voxels) of its size: 3e-5 at 8 x 32^3"""
+    say(f"unet batch {batch} x {n}^3")
+    net = learned.UNet(2, 0)
+    net.set_params(he_theta(11))
+    rng = np.random.default_rng(12)
+    x = rng.normal(size=(batch, n ** 3 * 2))
+    t = rng.normal(size=(batch, n ** 3))
+    xs = [GpuVector.from_array(v, F.F32) for v in x]
+    ts = [GpuVector.from_array(v, F.F32) for v in t]
+    xv, tv = GpuVector.from_array(x.ravel(), F.F32), GpuVector.from_array(t.ravel(), F.F32)
+    one = [net.forward(v, 1, n).numpy() for v in xs]
+    assert np.array_equal(net.forward(xv, batch, n).numpy(), np.concatenate(one))
+    parts = [net.loss_grad(a, b, 1, n) for a, b in zip(xs, ts)]
+    loss, g = net.loss_grad(xv, tv, batch, n)
+    assert abs(loss - np.mean([p[0] for p in parts])) <= 1e-12 * loss
+    gm = np.mean([p[1] for p in parts], axis=0)
+    for l, sl in enumerate(layer_slices()):
+        assert np.linalg.norm(g[sl] - gm[sl]) <= 1e-4 * np.linalg.norm(gm[sl]), l
+
+
 def test_unet_training_reduces_loss():
     say("unet training")
     n = 16
