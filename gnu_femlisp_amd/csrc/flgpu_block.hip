@@ -18,9 +18,11 @@
 // The blocks are symmetric positive definite (principal submatrices of the SPD operator, the
 // Dirichlet vertex an identity row), so their inverses are formed once by Gauss-Jordan without
 // pivoting in FP64 and stored (femlisp's store-p t, blockit.lisp:118-121), per vertex in
-// lattice vertex order as inv[v][j][i] = (A_BB^-1)_ij, identity rows and columns at absent
-// slots.  One iterate then costs per block the block's matrix rows (<ssc> only) and the W x W
-// inverse; order-1 blocks are single DOFs and take one lane each.
+// lattice vertex order as inv[v][i][j] = (A_BB^-1)_ij, rows padded to 16 bytes, identity rows and
+// columns at absent slots.  One iterate then costs per block the residual of its rows (<ssc>
+// only; from the element matrices of the cells around the vertex where the matrix has them,
+// else from its CSR rows) and the W x W inverse; order-1 blocks are single DOFs and take one
+// lane each.
 #include "flgpu_internal.h"
 
 namespace flgpu {
@@ -33,6 +35,7 @@ struct BlkGeom {
   int dim, order, n, M, W, w1, h;
   int par[3];  // colour parity per axis
   int cnt[3];  // vertices of that parity per axis
+  Div1 dcnt[3];
 };
 
 BlkGeom blk_geom(const flgpu_mat *A, int colour) {
@@ -53,6 +56,7 @@ BlkGeom blk_geom(const flgpu_mat *A, int colour) {
     g.par[k] = (colour >> (g.dim - 1 - k)) & 1;
     g.cnt[k] = (g.n + 2 - g.par[k]) / 2;
   }
+  for (int k = 0; k < 3; k++) g.dcnt[k] = div1(g.cnt[k]);
   return g;
 }
 
@@ -101,6 +105,13 @@ __device__ __forceinline__ int blk_key(const BlkGeom &g, const int *a, int s) {
     s /= g.w1;
   }
   return blk_key_d(g, a, dg);
+}
+
+// entries of a stored row of a block's inverse: W padded to 16 bytes
+template <class T>
+__host__ __device__ constexpr int blk_pad(int W) {
+  const int v = 16 / (int)sizeof(T);
+  return (W + v - 1) / v * v;
 }
 
 // Block inverses, one wave per vertex (grid: all (n+1)^dim vertices, colour 0's geometry with
@@ -163,23 +174,55 @@ __global__ __launch_bounds__(64) void k_blk_invert(BlkGeom g, const int *__restr
     }
     __syncthreads();
   }
-  T *out = inv + v * W * W;
-  for (int e = lane; e < W * W; e += 64) {
-    int j = e / W, i = e % W;
-    out[e] = (T)a[i][W + j];
+  const int wp = blk_pad<T>(W);
+  T *out = inv + v * W * wp;
+  for (int e = lane; e < W * wp; e += 64) {
+    int i = e / wp, j = e % wp;
+    out[e] = j < W ? (T)a[i][W + j] : (T)0;
   }
 }
 
-// v broadcast from lane j (j uniform over the wave)
-__device__ __forceinline__ float lane_bcast(float v, int j) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
+// The LDS traffic of one wave is in order; this keeps the compiler from moving accesses across.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-__device__ __forceinline__ double lane_bcast(double v, int j) {
-  long long u = __double_as_longlong(v);
-  int lo = __builtin_amdgcn_readlane((int)(u & 0xffffffffll), j);
-  int hi = __builtin_amdgcn_readlane((int)(u >> 32), j);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
+
+// A block's inverse in the registers of the G lanes that share the block, as 16-byte pieces of
+// its padded rows (piece f = k G + gl), and y = A_BB^-1 r from it: every lane multiplies its
+// pieces with the matching entries of r from LDS, and a slot's lane sums the pieces of its row
+// in order.  All of a block's 16-byte loads are independent and coalesced (27 loads of 4 bytes
+// by 27 of 64 lanes, and 27 broadcasts, as one column per step).
+template <class T, int W, int G>
+struct BlkInverse {
+  static constexpr int VL = 16 / (int)sizeof(T), WP = (W + VL - 1) / VL * VL, CPR = WP / VL,
+                       NC = W * CPR, K = (NC + G - 1) / G;
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+  vec a[K];
+  __device__ __forceinline__ void load(const T *__restrict__ iv, int gl) {
+#pragma unroll
+    for (int k = 0; k < K; k++) a[k] = *(const vec *)(iv + (long)min(k * G + gl, NC - 1) * VL);
+  }
+  // rv: r in LDS, WP values (zero beyond W); part: NC values of LDS
+  __device__ __forceinline__ void multiply(const T *rv, T *part, int gl) const {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const int f = k * G + gl;
+      const vec r = *(const vec *)(rv + (f % CPR) * VL);
+      T p = 0;
+#pragma unroll
+      for (int j = 0; j < VL; j++) p += a[k][j] * r[j];
+      if (f < NC) part[f] = p;
+    }
+  }
+  static __device__ __forceinline__ T row(const T *part, int slot) {
+    T y = 0;
+#pragma unroll
+    for (int j = 0; j < CPR; j++) y += part[slot * CPR + j];
+    return y;
+  }
+};
 
 constexpr int kBlkWaves = 2;  // waves per workgroup of k_blk_sweep
 
@@ -252,7 +295,8 @@ __global__ __launch_bounds__(64 * kBlkWaves) void k_blk_sweep(BlkGeom g, long cn
                                                               const T *__restrict__ inv, T omega,
                                                               T *x, const T *b, T *r) {
   constexpr int W = pow_i(3, DIM), NRUN = W / 3;
-  __shared__ T part[kBlkWaves][64][W + 1];
+  typedef BlkInverse<T, W, 64> Inv;
+  __shared__ __align__(16) T part[kBlkWaves][64 * (W + 1)];
   unsigned lb = xcd_block(blockIdx.x, gridDim.x);
   const int wv = threadIdx.x >> 6;
   long w = (long)lb * kBlkWaves + wv;
@@ -261,12 +305,8 @@ __global__ __launch_bounds__(64 * kBlkWaves) void k_blk_sweep(BlkGeom g, long cn
   int av[3];
   blk_vertex(g, w, av);
   int key = lane < W ? blk_key(g, av, lane) : -1;
-  const T *iv = inv + blk_vertex_id(g, av) * W * W;
-  T ivr[W];
-  auto load_inverse = [&]() {
-#pragma unroll
-    for (int j = 0; j < W; j++) ivr[j] = lane < W ? iv[j * W + lane] : (T)0;
-  };
+  const T *iv = inv + blk_vertex_id(g, av) * W * Inv::WP;
+  Inv A;
   T myr = 0;
   if (SSC) {
     int rs = 0, re = 0;
@@ -295,27 +335,242 @@ __global__ __launch_bounds__(64 * kBlkWaves) void k_blk_sweep(BlkGeom g, long cn
     for (int s = 0; s < W; s++) acc[s] = 0;
     blk_runs<T, DIM, 0, NRUN>(colidx, vals, x, lane, ta, e0, e1, e2, e3, acc);
 #pragma unroll
-    for (int s = 0; s < W; s++) part[wv][lane][s] = acc[s];
-    load_inverse();  // in flight during the reduction, in the registers acc held
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int s = 0; s < W; s++) part[wv][lane * (W + 1) + s] = acc[s];
+    A.load(iv, lane);  // in flight during the reduction, in the registers acc held
+    wave_sync();
     if (key >= 0) {
       T sum = 0;
-      for (int l = 0; l < 64; l++) sum += part[wv][l][lane];
+      for (int l = 0; l < 64; l++) sum += part[wv][l * (W + 1) + lane];
       myr = b[key] - sum;
     }
   } else {
-    load_inverse();
+    A.load(iv, lane);
     if (key >= 0) myr = r[key];
   }
-  T y = 0;
-#pragma unroll
-  for (int j = 0; j < W; j++) y += ivr[j] * lane_bcast(myr, j);
+  wave_sync();  // part is free for r and the products
+  T *rv = part[wv], *pr = part[wv] + 32;
+  if (lane < Inv::WP) rv[lane] = myr;
+  wave_sync();
+  A.multiply(rv, pr, lane);
+  wave_sync();
+  const T y = lane < W ? Inv::row(pr, lane) : (T)0;
   if (key >= 0) {
     if (SSC) r[key] = myr;
     x[key] += omega * y;
   }
+}
+
+// One colour of an iterate with order-2 blocks from the element matrices of the cells around
+// each vertex: (A x)_i over the block's rows i is the sum, over the 2^DIM cells, of the cell's
+// element row times the cell's 3^DIM values of x, so the columns and row bounds of the CSR, which
+// cost two more dependent round trips to memory, are not read.  rows: with ALPHA one reference
+// matrix, scaled by the cell's factor alpha[cell] (a coefficient constant per cell), else
+// every cell's own matrix (`elem`).
+//
+// G = 4^DIM lanes share a block: lane = (cell s around the vertex, node t of that cell within
+// the block), bits per axis, axis 0 most significant.  A lane multiplies its element row
+// (registers) with the cell's part of the x patch (LDS, 5^DIM values around the vertex, zero at
+// Dirichlet points as the eliminated columns are); a node shared by several cells is summed by
+// exchanges across the cell bits, both partners forming the same sum.  The rows, the patch, b,
+// the old x and the block's inverse are all loaded at once, one round trip.
+//
+// Issue, not bytes, bounds the 3D sweep, so everything that depends on the lane alone (offsets
+// from the vertex, the reference row) is formed once per wave; a vertex costs its coordinates
+// (uniform in 3D) and one bit test per axis for what the boundary cuts off.  A wave takes `per`
+// consecutive vertices and loads the next one's values before it works on the current one.
+// Q2 48^3, one fine colour (14 700 blocks): FP32 16.2 us (17.5 us with the indices formed anew
+// for every block); 51 us from the CSR rows, 10.6 KB of entries per block where this reads 32
+// bytes of alpha.
+template <class T, bool SSC, int DIM, bool ALPHA>
+struct BlkCell {
+  static constexpr int W = pow_i(3, DIM), G = pow_i(4, DIM), NP = pow_i(5, DIM);
+  typedef BlkInverse<T, W, G> Inv;
+  typedef typename Inv::vec vec;
+  // what depends on the lane alone
+  int gl, dk, po[2], pp[2][3], ps[3], sb[3], dc, erow, pbase, slot;
+  bool canon, centre;
+  vec e[Inv::CPR];  // element row
+  // what a vertex's loads give
+  struct Vals {
+    int key;
+    bool present, exists, vb;
+    T xo, bo, al, pv[2];
+    Inv A;
+    vec e[ALPHA ? 1 : Inv::CPR];
+  };
+
+  __device__ __forceinline__ void init(const BlkGeom &g, int gl_, const T *__restrict__ rows) {
+    gl = gl_;
+    dk = dc = erow = pbase = slot = 0;
+    canon = centre = true;
+#pragma unroll
+    for (int k = 0; k < DIM; k++) {
+      const int s = (gl >> (DIM + DIM - 1 - k)) & 1, t = (gl >> (DIM - 1 - k)) & 1;
+      const int d = s ? t : -t;
+      sb[k] = s;
+      ps[k] = d + 2;
+      dk = dk * g.M + d;
+      dc = dc * g.n + s - 1;
+      erow = erow * 3 + (s ? t : 2 - t);
+      pbase = pbase * 5 + 2 * s;
+      slot = slot * 3 + d + 1;
+      canon = canon && (s || t);
+      centre = centre && d == 0;
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int q = gl + u * G;
+      po[u] = 0;
+#pragma unroll
+      for (int k = 0; k < DIM; k++) {
+        pp[u][k] = q < NP ? (q / pow_i(5, DIM - 1 - k)) % 5 : 5;  // 5: no such value
+        po[u] = po[u] * g.M + pp[u][k] - 2;
+      }
+    }
+    if (SSC && ALPHA)
+#pragma unroll
+      for (int j = 0; j < Inv::CPR; j++)
+        e[j] = *(const vec *)(rows + erow * Inv::WP + j * Inv::VL);
+  }
+
+  // every load of vertex w of the colour
+  __device__ __forceinline__ Vals load(const BlkGeom &g, unsigned w, bool live,
+                                       const T *__restrict__ rows, const T *__restrict__ alpha,
+                                       const T *__restrict__ inv, const T *x, const T *b,
+                                       const T *r) const {
+    Vals v;
+    int vk = 0, vc = 0, vcl = 0, vid = 0;
+    int in = 1, ex = 1;  // the slot's point is interior, the cell exists
+    int ip[2] = {1, 1};
+    v.vb = false;
+    int av[3] = {0, 0, 0};
+#pragma unroll
+    for (int k = DIM - 1; k >= 0; k--) {
+      const unsigned q = k > 0 ? fdiv(w, g.dcnt[k]) : 0u;
+      av[k] = 2 * (int)(w - q * (unsigned)g.cnt[k]) + g.par[k];
+      w = q;
+    }
+#pragma unroll
+    for (int k = 0; k < DIM; k++) {
+      const int a = av[k];
+      // bit p: the point 2 a - 2 + p lies inside (0, M - 1); bit s: the cell a - 1 + s exists
+      int vm = 0x1f;
+      vm = a == 0 ? vm & 0x18 : vm;
+      vm = a == 1 ? vm & 0x1e : vm;
+      vm = a == g.n ? vm & 0x03 : vm;
+      vm = a == g.n - 1 ? vm & 0x0f : vm;
+      const int em = (a > 0 ? 1 : 0) | (a < g.n ? 2 : 0);
+      in &= vm >> ps[k];
+      ex &= em >> sb[k];
+      ip[0] &= vm >> pp[0][k];
+      ip[1] &= vm >> pp[1][k];
+      v.vb = v.vb || a == 0 || a == g.n;
+      vk = vk * g.M + 2 * a;
+      vc = vc * g.n + a;
+      vcl = vcl * g.n + min(a, g.n - 1);
+      vid = vid * (g.n + 1) + a;
+    }
+    v.exists = ex & 1;
+    v.present = live && (centre || (in & 1));
+    v.key = vk + ((centre || (in & 1)) ? dk : 0);
+    v.xo = x[v.key];
+    v.bo = SSC ? b[v.key] : r[v.key];
+    v.A.load(inv + (long)vid * (W * Inv::WP), gl);
+    if (SSC) {
+      const int cell = v.exists ? vc + dc : vcl;
+      if (ALPHA) {
+        v.al = alpha[cell];
+      } else {
+        const T *rp = rows + (long)cell * (W * Inv::WP) + erow * Inv::WP;
+#pragma unroll
+        for (int j = 0; j < Inv::CPR; j++) v.e[j] = *(const vec *)(rp + j * Inv::VL);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const T t = x[vk + ((ip[u] & 1) ? po[u] : 0)];
+        v.pv[u] = (ip[u] & 1) ? t : (T)0;
+      }
+    }
+    return v;
+  }
+
+  // the update of the vertex whose loads gave v; lds: the block's LDS
+  __device__ __forceinline__ void update(const Vals &v, T omega, T *lds, T *x, T *r) const {
+    T *px = lds, *rv = px + kPatch, *part = rv + Inv::WP;
+    T sum = 0;
+    if (SSC) {
+      px[gl] = v.pv[0];
+      if (gl + G < NP) px[gl + G] = v.pv[1];
+      wave_sync();
+#pragma unroll
+      for (int j = 0; j < W; j++) {
+        // node j of the cell, digits base 3: its place in the patch
+        int o = 0, q = j, mul = 1;
+#pragma unroll
+        for (int k = 0; k < DIM; k++) {
+          o += (q % 3) * mul;
+          q /= 3;
+          mul *= 5;
+        }
+        sum += (ALPHA ? e : v.e)[j / Inv::VL][j % Inv::VL] * px[pbase + o];
+      }
+      if (ALPHA) sum *= v.al;
+      if (!v.exists) sum = 0;
+#pragma unroll
+      for (int k = 0; k < DIM; k++) {
+        const T other = __shfl_xor(sum, 1 << (DIM + DIM - 1 - k), 64);
+        if (!((gl >> (DIM - 1 - k)) & 1)) sum += other;
+      }
+      if (centre && v.vb) sum = v.xo;  // a Dirichlet vertex: identity row
+    }
+    const T res = v.present ? (SSC ? v.bo - sum : v.bo) : (T)0;
+    if (canon) rv[slot] = res;
+    if (gl < Inv::WP - W) rv[W + gl] = 0;
+    wave_sync();
+    v.A.multiply(rv, part, gl);
+    wave_sync();
+    if (canon && v.present) {
+      const T y = Inv::row(part, slot);
+      if (SSC) r[v.key] = res;
+      x[v.key] = v.xo + omega * y;
+    }
+    wave_sync();
+  }
+  static constexpr int kPatch = (NP + Inv::VL - 1) / Inv::VL * Inv::VL;
+  static constexpr int kLds = kPatch + Inv::WP + (Inv::NC + Inv::VL - 1) / Inv::VL * Inv::VL;
+};
+
+template <class T, bool SSC, int DIM, bool ALPHA>
+__global__ __launch_bounds__(256) void k_blk_cell(BlkGeom g, long cnt, int per,
+                                                  const T *__restrict__ rows,
+                                                  const T *__restrict__ alpha,
+                                                  const T *__restrict__ inv, T omega, T *x,
+                                                  const T *b, T *r) {
+  typedef BlkCell<T, SSC, DIM, ALPHA> B;
+  constexpr int NB = 64 / B::G;  // blocks side by side in a wave
+  __shared__ __align__(16) T lds[4 * NB][B::kLds];
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  // the wave's groups of NB blocks [w0, w1)
+  const int groups = (int)((cnt + NB - 1) / NB), w0 = (int)(lb * 4 + wv) * per,
+            w1 = min(w0 + per, groups);
+  if (w0 >= w1) return;
+  const int sub = lane / B::G;
+  B blk;
+  blk.init(g, lane & (B::G - 1), rows);
+  T *my = lds[wv * NB + sub];
+  auto load = [&](int w) {
+    const int id = w * NB + (NB > 1 ? sub : 0);
+    const bool live = NB == 1 || id < (int)cnt;
+    return blk.load(g, (unsigned)(live ? id : 0), live, rows, alpha, inv, x, b, r);
+  };
+  typename B::Vals cur = load(w0);
+  for (int w = w0 + 1; w < w1; w++) {
+    typename B::Vals next = load(w);
+    blk.update(cur, omega, my, x, r);
+    cur = next;
+  }
+  blk.update(cur, omega, my, x, r);
 }
 
 // One colour of an iterate with one-DOF blocks (order 1), one lane per block: gesv! of the
@@ -357,7 +612,8 @@ void blocks_prepare(flgpu_mat *A) {
   for (int k = 0; k < g.dim; k++) N *= g.M;
   FLGPU_REQUIRE(A->nrows == N && A->ncols == N, "matrix size differs from its lattice");
   if (g.W == 1) return;  // one-DOF blocks use the diagonal
-  size_t bytes = (size_t)nv * g.W * g.W * prec_bytes(A->prec);
+  const int wp = A->prec == FLGPU_F64 ? blk_pad<double>(g.W) : blk_pad<float>(g.W);
+  size_t bytes = (size_t)nv * g.W * wp * prec_bytes(A->prec);
   if (!A->blk_inv) {
     A->blk_inv = dev_alloc(bytes);
     layout_changed(A);
@@ -379,7 +635,7 @@ void blocks_drop(flgpu_mat *A) {
 
 template <class T>
 static void block_sweep_t(const flgpu_mat *A, bool ssc, T omega, int backwards, T *x, const T *b,
-                          T *r) {
+                          T *r, bool cells) {
   int ncol = 1 << A->lat_dim;
   for (int k = 0; k < ncol; k++) {
     BlkGeom g = blk_geom(A, backwards ? ncol - 1 - k : k);
@@ -395,6 +651,28 @@ static void block_sweep_t(const flgpu_mat *A, bool ssc, T omega, int backwards, 
         k_blk_point<T, false><<<grid, 256, 0, st>>>(g, cnt, A->rowptr, A->colidx,
                                                     (const T *)A->vals, (const T *)A->diag,
                                                     omega, x, b, r);
+    } else if (cells && (A->cell || A->elem)) {
+      // groups of vertices (one per wave at a time), shared out evenly over at most five
+      // waves per SIMD, the kernel's occupancy
+      const int nb = 64 >> (2 * g.dim);
+      const long groups = (cnt + nb - 1) / nb, waves = 20L * A->ctx->cus;
+      const int per = (int)((groups + waves - 1) / waves);
+      unsigned grid = xcd_grid(grid_for((groups + per - 1) / per, 4));
+      auto launch = [&](auto kern, const void *rows) {
+        kern<<<grid, 256, 0, st>>>(g, cnt, per, (const T *)rows, (const T *)A->cell,
+                                   (const T *)A->blk_inv, omega, x, b, r);
+      };
+#define FLGPU_BLK(DIM)                                                               \
+  if (A->cell)                                                                       \
+    launch(ssc ? k_blk_cell<T, true, DIM, true> : k_blk_cell<T, false, DIM, true>,   \
+           A->kref);                                                                 \
+  else                                                                               \
+    launch(ssc ? k_blk_cell<T, true, DIM, false> : k_blk_cell<T, false, DIM, false>, \
+           A->elem)
+      if (g.dim == 3) FLGPU_BLK(3);
+      else if (g.dim == 2) FLGPU_BLK(2);
+      else FLGPU_BLK(1);
+#undef FLGPU_BLK
     } else {
       unsigned grid = xcd_grid(grid_for(cnt, kBlkWaves));
       auto launch = [&](auto kern) {
@@ -413,14 +691,15 @@ static void block_sweep_t(const flgpu_mat *A, bool ssc, T omega, int backwards, 
 }
 
 void block_sweep(const flgpu_mat *A, bool ssc, double omega, int backwards, void *x,
-                 const void *b, void *r) {
+                 const void *b, void *r, bool cells) {
   BlkGeom g = blk_geom(A, 0);
   if (g.W > 1 && !A->blk_inv) blocks_prepare(const_cast<flgpu_mat *>(A));
   if (A->prec == FLGPU_F64)
-    block_sweep_t<double>(A, ssc, omega, backwards, (double *)x, (const double *)b, (double *)r);
+    block_sweep_t<double>(A, ssc, omega, backwards, (double *)x, (const double *)b, (double *)r,
+                          cells);
   else
     block_sweep_t<float>(A, ssc, (float)omega, backwards, (float *)x, (const float *)b,
-                         (float *)r);
+                         (float *)r, cells);
 }
 
 }  // namespace flgpu
@@ -447,7 +726,9 @@ extern "C" int flgpu_block_iterate(const flgpu_mat *A, int kind, double omega, i
     CTX_LOCK(A->ctx);
     flgpu_mat *M = const_cast<flgpu_mat *>(A);
     if (!M->blk_inv) blocks_prepare(M);
-    block_sweep(A, kind == FLGPU_SMOOTH_SSC, omega, backwards, x->d, b->d, r->d);
+    // a single iterate sums the CSR entries in their order, whatever else A holds, so that a
+    // caller's copy of a lattice matrix gives the same values
+    block_sweep(A, kind == FLGPU_SMOOTH_SSC, omega, backwards, x->d, b->d, r->d, false);
     return 0;
   });
 }

@@ -100,6 +100,13 @@ inline FastDiv fast_div(unsigned d) {
   return FastDiv{d, (unsigned)m, l - 1};
 }
 __device__ __forceinline__ unsigned fdiv(unsigned n, FastDiv f) { return __umulhi(n, f.m) >> f.s; }
+struct Div1 {  // n / d for d >= 1
+  FastDiv f;
+};
+inline Div1 div1(unsigned d) { return Div1{d >= 2 ? fast_div(d) : FastDiv{1u, 0u, 0}}; }
+__device__ __forceinline__ unsigned fdiv(unsigned n, Div1 d) {
+  return d.f.d == 1u ? n : fdiv(n, d.f);
+}
 
 }  // namespace flgpu
 
@@ -182,9 +189,14 @@ struct flgpu_mat {
   // interpolation (tp_kind 1) the entries of the fine nodes of c's block by parity class
   // (k_tp8_fill); 0 where there is no such entry
   void *tp27 = nullptr;
+  // order-2 lattice matrices as sums over their cells (prec, rows padded to 16 bytes: row_pad):
+  // with a coefficient constant per cell the factors cell[c] of one reference element matrix
+  // kref; else, on the levels of a hierarchy with a block smoother, every cell's element
+  // matrix elem[c].  nullptr if not available; never both
+  void *cell = nullptr, *kref = nullptr, *elem = nullptr;
   // block smoothers on a lattice matrix: inverses of the vertex-centred blocks, per vertex in
-  // lattice vertex order, blk_inv[v][j][i] = (A_BB^-1)_ij (prec); nullptr until needed and for
-  // order 1, whose blocks are single DOFs
+  // lattice vertex order, blk_inv[v][i][j] = (A_BB^-1)_ij (prec, rows padded to 16 bytes);
+  // nullptr until needed and for order 1, whose blocks are single DOFs
   void *blk_inv = nullptr;
   // per-block partial sums of the per-cell product's fused dot (spmv_dot), dot_np entries
   double *dot_part = nullptr;
@@ -206,6 +218,9 @@ void mat_finish(flgpu_mat *A);  // SELL + diagonal from the device CSR
 void mat_refresh_values(flgpu_mat *A);  // SELL/diag/colour values after a CSR value change
 void mat_build_transpose(const flgpu_mat *A);
 void drop_alpha(flgpu_mat *A);
+void drop_cells(flgpu_mat *A);  // cell, kref, elem
+// entries of a row of n values padded to 16 bytes
+inline int row_pad(int n, int prec) { return prec == FLGPU_F64 ? (n + 1) & ~1 : (n + 3) & ~3; }
 // the strips and boundary copy of the per-cell <sor> sweep, after alpha is allocated
 void sor_strips_alloc(flgpu_mat *A);
 void tp_prepare(flgpu_mat *T);  // (re)fill tp27 of an interpolation or its transpose
@@ -248,18 +263,22 @@ void stage_first_step(const flgpu_mat *A, int rprec, const void *r, void *b, dou
                       void *xo);
 // vertex-centred block smoothers (flgpu_block.hip): (re)compute the block inverses of a
 // lattice matrix, release them, and one <geometric-ssc> (ssc) / <geometric-psc> iterate
-// (backwards: colours last to first; b may be r)
+// (backwards: colours last to first; b may be r; cells: form the residuals from the matrix's
+// cells where it has them, else always from its CSR rows)
 void blocks_prepare(flgpu_mat *A);
 void blocks_drop(flgpu_mat *A);
 void block_sweep(const flgpu_mat *A, bool ssc, double omega, int backwards, void *x,
-                 const void *b, void *r);
+                 const void *b, void *r, bool cells);
 // `steps` sweeps
 void sor_sweeps(const flgpu_mat *A, double omega, int steps, int backwards, void *x,
                 const void *b, void *r);
 
 // lattices (flgpu_lattice.hip)
+// keep_elem: keep the element matrices of an order-2 lattice (flgpu_mat::elem) when its
+// coefficient is not constant per cell
 flgpu_mat *lattice_assemble(flgpu_ctx *ctx, int dim, int order, int n, const flgpu_vec *kappa,
-                            int nk, double f, int prec, int mode, flgpu_vec **rhs);
+                            int nk, double f, int prec, int mode, flgpu_vec **rhs,
+                            bool keep_elem = false);
 flgpu_mat *lattice_interpolation(flgpu_ctx *ctx, int dim, int order, int nc, int prec);
 flgpu_mat *lattice_projection(flgpu_ctx *ctx, int dim, int order, int nc, int prec);
 void lattice_colouring(flgpu_mat *A, int dim, int order, int n);
@@ -270,6 +289,7 @@ void lattice_dirichlet_identity(flgpu_mat *A, int dim, int order, int n);
 // operator-dependent interpolation values of P (3D Q1) from the fine matrix A
 void lattice_blackbox(const flgpu_mat *A, flgpu_mat *P);
 void lattice_reassemble(flgpu_mat *A, const flgpu_vec *kappa, int nk, int mode);
+void lattice_set_kref(flgpu_mat *A);  // the reference element matrix of the per-cell form
 
 // vectors (flgpu_core.hip)
 flgpu_vec *vec_new(flgpu_ctx *ctx, long n, int prec);

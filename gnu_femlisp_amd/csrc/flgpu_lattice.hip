@@ -358,17 +358,25 @@ __global__ void k_coef(long ncells, int dim, int n, int s, int nq, const double 
 }
 
 // ---- element contractions E[c][ab] = sum_q S[c][q] T[q][ab] ---------------------------
+// Rows of E are ld >= nloc values apart (ElemLayout; ld = nloc: dense matrices).
+struct ElemLayout {
+  int nloc, ld;
+  __device__ __forceinline__ long at(long cell, int ab) const {
+    const int a = ab / nloc;
+    return cell * (long)(nloc * ld) + a * ld + (ab - a * nloc);
+  }
+};
 
 template <class TE>
 __global__ void k_elem_fma(long ncells, int nq, int nloc2, const double *__restrict__ S,
-                           const double *__restrict__ Tt, TE *E) {
+                           const double *__restrict__ Tt, TE *E, ElemLayout L) {
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= ncells * nloc2) return;
   long cell = t / nloc2;
   int ab = (int)(t % nloc2);
   double acc = 0.0;
   for (int q = 0; q < nq; q++) acc += S[cell * nq + q] * Tt[(long)q * nloc2 + ab];
-  E[t] = (TE)acc;
+  E[L.at(cell, ab)] = (TE)acc;
 }
 
 typedef double v4d __attribute__((ext_vector_type(4)));
@@ -381,7 +389,8 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 // (measured on gfx950: the four result rows of a lane are 4 apart).
 __global__ __launch_bounds__(256) void k_elem_mfma_f64(long ncells, int nq, int nloc2,
                                                        const double *__restrict__ S,
-                                                       const double *__restrict__ Tt, double *E) {
+                                                       const double *__restrict__ Tt, double *E,
+                                                       ElemLayout L) {
   long tile = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   long c0 = tile * 16;
   if (c0 >= ncells) return;
@@ -399,7 +408,7 @@ __global__ __launch_bounds__(256) void k_elem_mfma_f64(long ncells, int nq, int 
     }
     for (int v = 0; v < 4; v++) {
       long row = c0 + kq + 4 * v;
-      if (row < ncells && bcol < nloc2) E[row * nloc2 + bcol] = acc[v];
+      if (row < ncells && bcol < nloc2) E[L.at(row, bcol)] = acc[v];
     }
   }
 }
@@ -449,7 +458,8 @@ __device__ __forceinline__ v4f mfma_bf16x3(v4s ah, v4s am, v4s al, v4s bh, v4s b
 // are exact zeros instead of the FP32 accumulator's cancellation error.
 __global__ __launch_bounds__(256) void k_elem_mfma_bf16(long ncells, int nq, int nloc2,
                                                         const double *__restrict__ S,
-                                                        const double *__restrict__ Tt, float *E) {
+                                                        const double *__restrict__ Tt, float *E,
+                                                        ElemLayout L) {
   long tile = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   long c0 = tile * 16;
   if (c0 >= ncells) return;
@@ -482,7 +492,7 @@ __global__ __launch_bounds__(256) void k_elem_mfma_bf16(long ncells, int nq, int
     }
     for (int v = 0; v < 4; v++) {
       long row = c0 + 4 * kg + v;
-      if (row < ncells && bcol < nloc2) E[row * nloc2 + bcol] = acc[v];
+      if (row < ncells && bcol < nloc2) E[L.at(row, bcol)] = acc[v];
     }
   }
 }
@@ -495,7 +505,7 @@ __global__ __launch_bounds__(256) void k_elem_mfma_bf16(long ncells, int nq, int
 // load vector rhs_P = f H^d sum_cells m[loc(P)].
 template <class T, class TE>
 __global__ void k_gather(long N, int dim, int order, int n, DevTable pat, const int *rowptr,
-                         const TE *__restrict__ E, int nloc, T *vals, double rhs_scale,
+                         const TE *__restrict__ E, int nloc, int ld, T *vals, double rhs_scale,
                          const double *__restrict__ mload, T *rhs) {
   long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= N) return;
@@ -511,7 +521,7 @@ __global__ void k_gather(long N, int dim, int order, int n, DevTable pat, const 
     e[k] = lo[k];
     if (P[k] == 0 || P[k] == M - 1) rb = true;
   }
-  long nloc2 = (long)nloc * nloc;
+  long nloc2 = (long)nloc * ld;
   long pos = rowptr[r];
   for (;;) {
     int Q[kMaxDim], clo[kMaxDim], chi[kMaxDim], c[kMaxDim];
@@ -536,7 +546,7 @@ __global__ void k_gather(long N, int dim, int order, int n, DevTable pat, const 
           la = la * nl1 + (P[k] - order * c[k]);
           lb = lb * nl1 + (Q[k] - order * c[k]);
         }
-        acc += (double)E[cell * nloc2 + (long)la * nloc + lb];
+        acc += (double)E[cell * nloc2 + (long)la * ld + lb];
         int k = dim - 1;
         while (k >= 0 && c[k] == chi[k]) {
           c[k] = clo[k];
@@ -816,9 +826,10 @@ static void check_kappa(const flgpu_vec *kappa, int dim, int n, int nk) {
   FLGPU_REQUIRE(kappa->n == ipow(nk, dim), "kappa must hold nk^dim values");
 }
 
-// element matrices of all cells of the level into E (TE = double or float)
+// element matrices of all cells of the level into E (TE = double or float), rows ld apart
 static void element_matrices(flgpu_ctx *ctx, const RefElement &R, int n, const flgpu_vec *kappa,
-                             int nk, int mode, int prec, void *E) {
+                             int nk, int mode, int prec, void *E, int ld) {
+  const ElemLayout L = {R.nloc, ld};
   int dim = R.dim;
   long ncells = ipow(n, dim);
   double H = 1.0 / n;
@@ -835,16 +846,16 @@ static void element_matrices(flgpu_ctx *ctx, const RefElement &R, int n, const f
   if (mode == FLGPU_ASM_MFMA) {
     unsigned g = grid_for((ncells + 15) / 16, 4);
     if (prec == FLGPU_F64)
-      k_elem_mfma_f64<<<g, 256, 0, ctx->stream>>>(ncells, R.nq, R.nloc2, dS, dT, (double *)E);
+      k_elem_mfma_f64<<<g, 256, 0, ctx->stream>>>(ncells, R.nq, R.nloc2, dS, dT, (double *)E, L);
     else
-      k_elem_mfma_bf16<<<g, 256, 0, ctx->stream>>>(ncells, R.nq, R.nloc2, dS, dT, (float *)E);
+      k_elem_mfma_bf16<<<g, 256, 0, ctx->stream>>>(ncells, R.nq, R.nloc2, dS, dT, (float *)E, L);
   } else {
     if (prec == FLGPU_F64)
       k_elem_fma<double><<<grid_for(ncells * R.nloc2, 256), 256, 0, ctx->stream>>>(
-          ncells, R.nq, R.nloc2, dS, dT, (double *)E);
+          ncells, R.nq, R.nloc2, dS, dT, (double *)E, L);
     else
       k_elem_fma<float><<<grid_for(ncells * R.nloc2, 256), 256, 0, ctx->stream>>>(
-          ncells, R.nq, R.nloc2, dS, dT, (float *)E);
+          ncells, R.nq, R.nloc2, dS, dT, (float *)E, L);
   }
   FLGPU_HIP(hipGetLastError());
   FLGPU_HIP(hipStreamSynchronize(ctx->stream));
@@ -914,8 +925,10 @@ static void assemble_values(flgpu_mat *A, const flgpu_vec *kappa, int nk, int mo
   long ncells = ipow(n, dim);
   // E in FP64 for the FP64 path, FP32 for the FP32 (BF16-MFMA) path
   int eprec = A->prec;
-  void *E = dev_alloc(prec_bytes(eprec) * ncells * R.nloc2);
-  element_matrices(ctx, R, n, kappa, nk, mode, eprec, E);
+  // a matrix that keeps its element matrices (elem) has them formed in place
+  const int ld = A->elem ? row_pad(R.nloc, eprec) : R.nloc;
+  void *E = A->elem ? A->elem : dev_alloc(prec_bytes(eprec) * ncells * R.nloc2);
+  element_matrices(ctx, R, n, kappa, nk, mode, eprec, E, ld);
   DevTable dpat = upload_table(ctx, pat);
   double *dm = (double *)dev_alloc(sizeof(double) * R.nloc);
   FLGPU_HIP(hipMemcpyAsync(dm, R.m.data(), sizeof(double) * R.nloc, hipMemcpyHostToDevice,
@@ -924,17 +937,17 @@ static void assemble_values(flgpu_mat *A, const flgpu_vec *kappa, int nk, int mo
   long N = A->nrows;
   if (A->prec == FLGPU_F64)
     k_gather<double, double><<<grid_for(N, 128), 128, 0, ctx->stream>>>(
-        N, dim, order, n, dpat, A->rowptr, (const double *)E, R.nloc, (double *)A->vals, rscale,
+        N, dim, order, n, dpat, A->rowptr, (const double *)E, R.nloc, ld, (double *)A->vals, rscale,
         dm, (double *)rhs_dev);
   else
     k_gather<float, float><<<grid_for(N, 128), 128, 0, ctx->stream>>>(
-        N, dim, order, n, dpat, A->rowptr, (const float *)E, R.nloc, (float *)A->vals, rscale, dm,
+        N, dim, order, n, dpat, A->rowptr, (const float *)E, R.nloc, ld, (float *)A->vals, rscale, dm,
         (float *)rhs_dev);
   FLGPU_HIP(hipGetLastError());
   FLGPU_HIP(hipStreamSynchronize(ctx->stream));
   free_table(dpat);
   dev_free(dm);
-  dev_free(E);
+  if (E != A->elem) dev_free(E);
 }
 
 template <class T>
@@ -943,12 +956,56 @@ __global__ void k_alpha(long ncells, double H, const double *__restrict__ kappa,
   if (c < ncells) alpha[c] = (T)(H * (kappa ? kappa[c] : 1.0));
 }
 
+// kref: the reference element matrix of a constant coefficient (sum_q T_q), padded rows
+void lattice_set_kref(flgpu_mat *A) {
+  RefElement R = ref_element(A->lat_dim, A->lat_order);
+  const int ld = row_pad(R.nloc, A->prec);
+  std::vector<double> k((size_t)R.nloc * ld, 0.0);
+  for (int a = 0; a < R.nloc; a++)
+    for (int b = 0; b < R.nloc; b++)
+      k[(size_t)a * ld + b] = R.T[(size_t)R.nq * R.nloc2 + (size_t)a * R.nloc + b];
+  std::vector<float> k32(k.begin(), k.end());
+  const void *src = A->prec == FLGPU_F64 ? (const void *)k.data() : (const void *)k32.data();
+  if (!A->kref) A->kref = dev_alloc(prec_bytes(A->prec) * k.size());
+  FLGPU_HIP(hipMemcpyAsync(A->kref, src, prec_bytes(A->prec) * k.size(), hipMemcpyHostToDevice,
+                           A->ctx->stream));
+  FLGPU_HIP(hipStreamSynchronize(A->ctx->stream));
+}
+
+// Order 2 with one coefficient value per cell: cell[c] = H^(d-2) kappa_c against kref.
+static void lattice_set_cell(flgpu_mat *A, const flgpu_vec *kappa, int nk) {
+  const int n = A->lat_n, dim = A->lat_dim;
+  if (A->elem || (kappa && nk != n)) {
+    if (A->cell) drop_cells(A);
+    return;
+  }
+  const long ncells = ipow(n, dim);
+  if (!A->cell) {
+    lattice_set_kref(A);
+    A->cell = dev_alloc(prec_bytes(A->prec) * ncells);
+    layout_changed(A);
+  }
+  const double scale = std::pow(1.0 / n, dim - 2);
+  const double *kd = kappa ? (const double *)kappa->d : nullptr;
+  if (A->prec == FLGPU_F64)
+    k_alpha<double><<<grid_for(ncells, 256), 256, 0, A->ctx->stream>>>(ncells, scale, kd,
+                                                                       (double *)A->cell);
+  else
+    k_alpha<float><<<grid_for(ncells, 256), 256, 0, A->ctx->stream>>>(ncells, scale, kd,
+                                                                      (float *)A->cell);
+  FLGPU_HIP(hipGetLastError());
+}
+
 // 3D Q1 with one coefficient value per cell (nk == n): the element matrix of
 // cell c is H kappa_c Kref, Kref = sum_q T_q, and by the reflection symmetry
 // of the cube Kref[a][b] = Kref[0][a xor b].  Stores alpha_c = H kappa_c and
 // Kref[0][.] so that the kernels apply A without streaming its values.
 static void lattice_set_alpha(flgpu_mat *A, const flgpu_vec *kappa, int nk) {
   int n = A->lat_n;
+  if (A->lat_order == 2) {
+    lattice_set_cell(A, kappa, nk);
+    return;
+  }
   if (A->lat_dim != 3 || A->lat_order != 1 || (kappa && nk != n)) {
     drop_alpha(A);
     return;
@@ -1017,7 +1074,8 @@ flgpu_mat *lattice_pattern(flgpu_ctx *ctx, int dim, int order, int n, int prec) 
 }
 
 flgpu_mat *lattice_assemble(flgpu_ctx *ctx, int dim, int order, int n, const flgpu_vec *kappa,
-                            int nk, double f, int prec, int mode, flgpu_vec **rhs) {
+                            int nk, double f, int prec, int mode, flgpu_vec **rhs,
+                            bool keep_elem) {
   check_lattice_args(dim, order, n);
   check_kappa(kappa, dim, n, nk);
   FLGPU_REQUIRE(mode == FLGPU_ASM_F64 || mode == FLGPU_ASM_MFMA, "unknown assembly mode");
@@ -1026,6 +1084,12 @@ flgpu_mat *lattice_assemble(flgpu_ctx *ctx, int dim, int order, int n, const flg
   flgpu_vec *b = nullptr;
   try {
     if (rhs) b = vec_new(ctx, A->nrows, prec);
+    if (keep_elem && order == 2 && kappa && nk != n) {
+      const int nloc = (int)ipow(3, dim);
+      const long cnt = ipow(n, dim) * nloc * row_pad(nloc, prec);
+      A->elem = dev_alloc(prec_bytes(prec) * cnt);
+      vfill(ctx, cnt, prec, A->elem, 0.0);  // the padding
+    }
     assemble_values(A, kappa, nk, mode, b ? b->d : nullptr);
     lattice_set_alpha(A, kappa, nk);
     mat_finish(A);
@@ -1075,7 +1139,7 @@ void lattice_dirichlet_identity(flgpu_mat *A, int dim, int order, int n) {
 void lattice_reassemble(flgpu_mat *A, const flgpu_vec *kappa, int nk, int mode) {
   check_kappa(kappa, A->lat_dim, A->lat_n, nk);
   assemble_values(A, kappa, nk, mode, nullptr);
-  if (A->alpha) lattice_set_alpha(A, kappa, nk);
+  if (A->alpha || A->cell) lattice_set_alpha(A, kappa, nk);
   mat_refresh_values(A);
 }
 
@@ -1427,7 +1491,7 @@ extern "C" int flgpu_lattice_element_matrices(flgpu_ctx *ctx, int dim, int order
     RefElement R = ref_element(dim, order);
     void *E = dev_alloc(prec_bytes(prec) * total * R.nloc2);
     try {
-      element_matrices(ctx, R, n, kappa, nk, mode, prec, E);
+      element_matrices(ctx, R, n, kappa, nk, mode, prec, E, R.nloc);
       long cnt = ncells * R.nloc2;
       if (prec == FLGPU_F64) {
         FLGPU_HIP(hipMemcpy(out, (double *)E + first_cell * R.nloc2, sizeof(double) * cnt,

@@ -665,7 +665,7 @@ static void smooth(flgpu_mg *mg, int l, bool post, bool last = false) {
     bool seen = !ssc || b == r;
     if (seen) ensure_residual(mg, l);
     for (int k = 0; k < steps; k++) {
-      block_sweep(L.A, ssc, p.omega, post && p.symmetric, x, b, r);
+      block_sweep(L.A, ssc, p.omega, post && p.symmetric, x, b, r, true);
       if (steps > 1 && seen) spmv(L.A, -1.0, x, 1.0, b, r);
     }
   } else {
@@ -1161,7 +1161,8 @@ extern "C" int flgpu_mg_create_lattice(flgpu_ctx *ctx, int dim, int order, int n
         bool bbox = params->transfer == FLGPU_TRANSFER_BLACKBOX;
         if (is_top || (!params->galerkin && !bbox)) {
           mg->lv[l].A = lattice_assemble(ctx, dim, order, n, kappa, nk, f, params->prec, asm_mode,
-                                         (is_top && rhs) ? &b : nullptr);
+                                         (is_top && rhs) ? &b : nullptr,
+                                         block_smoother(*params) && l > params->base_level);
         } else {
           if (bbox) lattice_blackbox(mg->lv[l + 1].A, mg->lv[l].I);
           mg->lv[l].A = lattice_galerkin(mg->lv[l].I, mg->lv[l + 1].A, dim, order, n);

@@ -270,6 +270,9 @@ void mat_free(flgpu_mat *A) {
   for (auto &s : A->colour_sell) sell_free(s);
   if (A->transpose) mat_free(A->transpose);
   dev_free(A->alpha);
+  dev_free(A->cell);
+  dev_free(A->kref);
+  dev_free(A->elem);
   dev_free(A->sor_ghost);
   dev_free(A->val27);
   dev_free(A->tp27);
@@ -292,6 +295,15 @@ void drop_alpha(flgpu_mat *A) {
   dev_free(A->alpha);
   A->alpha = nullptr;
   drop_sor_strips(A);
+}
+
+// new values that are no sum over the lattice's cells
+void drop_cells(flgpu_mat *A) {
+  if (A->cell || A->elem) layout_changed(A);
+  for (void **p : {&A->cell, &A->kref, &A->elem}) {
+    dev_free(*p);
+    *p = nullptr;
+  }
 }
 
 void mat_refresh_values(flgpu_mat *A) {
@@ -416,6 +428,13 @@ flgpu_mat *mat_convert(const flgpu_mat *A, int prec) {
     vcopy(ctx, nc, A->prec, A->alpha, prec, B->alpha);
     for (int j = 0; j < 8; j++) B->kt[j] = A->kt[j];
     sor_strips_alloc(B);
+  }
+  if (A->cell) {
+    long nc = 1;
+    for (int k = 0; k < A->lat_dim; k++) nc *= A->lat_n;
+    B->cell = dev_alloc(prec_bytes(prec) * nc);
+    vcopy(ctx, nc, A->prec, A->cell, prec, B->cell);
+    lattice_set_kref(B);
   }
   mat_finish(B);
   if (A->transpose) B->transpose = mat_convert(A->transpose, prec);
@@ -2757,6 +2776,8 @@ extern "C" int flgpu_galerkin_product(const flgpu_mat *P, const flgpu_mat *A, fl
     FLGPU_REQUIRE(P->ctx == A->ctx && A->ctx == Ac->ctx, "matrices of different contexts");
     CTX_LOCK(A->ctx);
     galerkin_product(P, A, Ac);
+    drop_alpha(Ac);  // Ac's forms that are sums over cells do not hold the new values
+    drop_cells(Ac);
     mat_refresh_values(Ac);
     FLGPU_HIP(hipStreamSynchronize(A->ctx->stream));
     return 0;
@@ -2804,6 +2825,7 @@ extern "C" int flgpu_csr_update_values(flgpu_mat *A, const double *vals) {
     FLGPU_REQUIRE(A && (vals || A->nnz == 0), "arguments must not be NULL");
     CTX_LOCK(A->ctx);
     drop_alpha(A);
+    drop_cells(A);
     upload_vals(A, vals);
     mat_refresh_values(A);
     FLGPU_HIP(hipStreamSynchronize(A->ctx->stream));
@@ -2851,7 +2873,10 @@ extern "C" int flgpu_mat_storage(flgpu_mat *A, int max_form, int *form) {
     FLGPU_REQUIRE(A, "matrix must not be NULL");
     CTX_LOCK(A->ctx);
     FLGPU_HIP(hipStreamSynchronize(A->ctx->stream));
-    if (max_form < FLGPU_STORAGE_CELL) drop_alpha(A);
+    if (max_form < FLGPU_STORAGE_CELL) {
+      drop_alpha(A);
+      drop_cells(A);
+    }
     if (max_form < FLGPU_STORAGE_STENCIL) {
       drop_stencil(A);
       tp_drop(A);

@@ -45,14 +45,6 @@ __device__ __forceinline__ short bf16_bits(float f) {
 // (16 voxels) times its four channel groups read 512 consecutive bytes wherever the tap shifts
 // them, so no tap has bank conflicts and every value is rounded to BF16 once per box instead of
 // once per tap.
-struct Div1 {  // n / d for d >= 1
-  FastDiv f;
-};
-inline Div1 div1(unsigned d) { return Div1{d >= 2 ? fast_div(d) : FastDiv{1u, 0u, 0}}; }
-__device__ __forceinline__ unsigned fdiv(unsigned n, Div1 d) {
-  return d.f.d == 1u ? n : fdiv(n, d.f);
-}
-
 struct ConvGeom {
   int n;                   // voxels per axis
   int bz, by, bx;          // box

@@ -230,3 +230,45 @@ def test_ssc_mixed_fcg_eager_matches_graphs():
         assert bb["true_residual"] / np.linalg.norm(b.numpy()) < 1e-10
         out.append((bb["steps"], bb["solution"].numpy()))
     assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("dim,n0,levels", [(1, 1, 4), (2, 1, 4), (2, 3, 3), (3, 1, 3), (3, 2, 2),
+                                           (3, 3, 2)])
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("kind", [F.SMOOTH_SSC, F.SMOOTH_PSC])
+def test_cell_sweeps_equal_csr_sweeps(dim, n0, levels, prec, kind):
+    """Cycles whose block sweeps read the matrices as sums over their cells (factors of the
+    reference matrix where the coefficient is constant per cell, element matrices on coarser
+    levels) against the same cycles on uploaded copies of the matrices, which sweep the CSR
+    rows; also after new coefficients, one constant per fine cell and one finer (no cell form
+    on the top level any more).  Lattices down to one cell, where every block meets the
+    boundary.  One cycle sums the same products in another order: the bounds are those of the
+    oracle comparisons in FP64 and FP32 above."""
+    say(f"cell sweeps dim={dim} n0={n0} levels={levels} prec={prec} kind={kind}")
+    n = n0 << (levels - 1)
+    rng = np.random.default_rng(dim * 100 + n0 * 10 + levels)
+    kaps = [np.exp(rng.normal(size=(n,) * dim)), None, np.exp(rng.normal(size=(n,) * dim)),
+            np.exp(rng.normal(size=(2 * n,) * dim))]
+    sm = it.GeometricSSC(0.9) if kind == F.SMOOTH_SSC else it.GeometricPSC(0.2)
+    H = None
+    for kap in kaps:
+        if H is None or kap is None:
+            cs, H = _hier(dim, 2, n0, levels, sm, 1, 1, 0, True, kap, prec)
+        else:
+            H.reassemble(kap)
+        A = []
+        for l in range(levels):
+            rp, ci, v = H.level_matrix(l).csr()
+            A.append(GpuSparseMatrix.from_csr(rp, ci, v, prec=prec))
+            lat.colour(A[-1], dim, 2, n0 << l)
+        I = [H.level_matrix(l, True) for l in range(levels - 1)]
+        U = it.Hierarchy.from_matrices(cs, A, I)
+        N = A[-1].nrows
+        b = rng.normal(size=N)
+        out = []
+        for h in (H, U):
+            x, bv, r = GpuVector(N, prec), GpuVector.from_array(b, prec), \
+                GpuVector.from_array(b, prec)
+            h.apply(x, bv, r)
+            out.append(x.numpy())
+        assert relerr(out[0], out[1]) < (1e-12 if prec == F.F64 else 2e-5)
