@@ -146,6 +146,7 @@ struct Sell {
   long *slice_ptr = nullptr;
   int *col = nullptr;
   void *val = nullptr;
+  void *span = nullptr;  // colour subsets swept from the CSR: the rows' bounds (int2)
   long nstored = 0;
   int maxw = 0;
 };
@@ -161,6 +162,7 @@ struct flgpu_mat {
   int *diagpos = nullptr;  // CSR position of the diagonal (-1 if absent)
   void *diag = nullptr;    // diagonal values (prec)
   Sell sell;
+  int lanes = 0;  // products read the CSR with this many lanes per row (0: SELL)
   int ncolours = 0;
   std::vector<Sell> colour_sell;
   flgpu_mat *transpose = nullptr;

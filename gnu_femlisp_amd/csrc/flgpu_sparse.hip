@@ -102,11 +102,17 @@ __global__ __launch_bounds__(64) void k_sell_fill_lds(int nrows, const int *__re
   }
 }
 
+static int csr_lanes(const flgpu_mat *A);
+// the CSR bounds of a colour's rows (below)
+__global__ void k_row_span(int nsub, const int *__restrict__ rows, const int *__restrict__ rowptr,
+                           int2 *__restrict__ span);
+
 void sell_free(Sell &s) {
   dev_free(s.rows);
   dev_free(s.slice_ptr);
   dev_free(s.col);
   dev_free(s.val);
+  dev_free(s.span);
   s = Sell();
 }
 
@@ -166,7 +172,18 @@ static Sell sell_build(flgpu_mat *A, const std::vector<int> *rows_host) {
   return s;
 }
 
-Sell sell_build_rows(flgpu_mat *A, const std::vector<int> &rows) { return sell_build(A, &rows); }
+// A colour's rows.  Sweeps of matrices with long or irregular rows read the CSR (csr_lanes, and
+// rows of over 27 entries): they take the rows' bounds.
+Sell sell_build_rows(flgpu_mat *A, const std::vector<int> &rows) {
+  Sell s = sell_build(A, &rows);
+  if (s.nrows > 0 && (A->lanes > 0 || s.maxw > 27)) {
+    s.span = dev_alloc(sizeof(int2) * (size_t)s.nrows);
+    k_row_span<<<grid_for(s.nrows, 256), 256, 0, A->ctx->stream>>>(s.nrows, s.rows, A->rowptr,
+                                                                   (int2 *)s.span);
+    FLGPU_HIP(hipGetLastError());
+  }
+  return s;
+}
 
 // ---- diagonal -----------------------------------------------------------------------
 
@@ -252,6 +269,7 @@ void mat_finish(flgpu_mat *A) {
     diag_refresh(A);
   }
   A->sell = sell_build(A, nullptr);
+  A->lanes = csr_lanes(A);
   if (is_q1_lattice(A)) {
     A->val27 = dev_alloc(prec_bytes(A->prec) * 27 * (size_t)A->nrows);
     stencil_refresh(A);
@@ -473,7 +491,7 @@ void set_colouring(flgpu_mat *A, int ncolours, const int *colour) {
   for (auto &s : A->colour_sell) sell_free(s);
   A->colour_sell.clear();
   layout_changed(A);
-  for (int c = 0; c < ncolours; c++) A->colour_sell.push_back(sell_build(A, &rows[c]));
+  for (int c = 0; c < ncolours; c++) A->colour_sell.push_back(sell_build_rows(A, rows[c]));
   A->ncolours = ncolours;
 }
 
@@ -543,6 +561,81 @@ __global__ __launch_bounds__(256) void k_sell_spmv(int nsub, int nslices, const 
   T acc = (beta == (T)0) ? (T)0 : beta * z[row];
   acc = sell_row<T>(val + base + lane, col + base + lane, w, alpha, x, acc);
   out[row] = acc;
+}
+
+// The sum over one CSR row [b, e) by the G lanes that share it (l: this lane's place): every lane
+// takes each G-th entry, four of them loaded before the x values they name, and the lanes' sums
+// are added by exchanges.  All G lanes return the row's sum of (alpha x_col) val.  FP32 sums
+// are formed in FP64 too: adding lane by lane, not on top of beta z, would otherwise lose up to a
+// fifth more to rounding than SELL's order where a residual cancels.
+template <class T, int G>
+__device__ __forceinline__ double csr_row(const int *__restrict__ col, const T *__restrict__ val, int b,
+                                     int e, int l, T alpha, const T *x) {
+  constexpr int U = 4;
+  double acc = 0;
+  for (int k = b + l; k < e; k += G * U) {
+    T a[U], xv[U];
+    int c[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int kk = min(k + u * G, e - 1);
+      a[u] = val[kk];
+      c[u] = col[kk];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) xv[u] = x[c[u]];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (k + u * G < e) acc += (double)(alpha * xv[u]) * (double)a[u];
+  }
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+  return acc;
+}
+
+// out[row] = beta z[row] + sum_k (alpha x[col]) val from the CSR rows, G lanes per row (csr_lanes).
+// Nothing is read for padding and a row of w entries costs w / G steps of a lane instead of w:
+// irregular matrices are bound by the longest row of every 64 in SELL.  300 007 rows of 18
+// entries on average (55 at most), FP64: 23.1 us, 3.4 TB/s of entries, 40.3 us from SELL;
+// Q2 12^3 (15 625 rows of 58): 4.1 against 16.7 us.
+template <class T, int G>
+__global__ __launch_bounds__(256) void k_csr_spmv(int nrows, const int *__restrict__ rowptr,
+                                                  const int *__restrict__ col,
+                                                  const T *__restrict__ val, T alpha,
+                                                  const T *__restrict__ x, T beta, const T *z,
+                                                  T *out) {
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int row = (int)lb * (256 / G) + threadIdx.x / G, l = threadIdx.x % G;
+  if (row >= nrows) return;  // the lanes of a row leave together
+  const double acc = csr_row<T, G>(col, val, rowptr[row], rowptr[row + 1], l, alpha, x);
+  if (l == 0) out[row] = beta == (T)0 ? (T)acc : (T)((double)beta * (double)z[row] + acc);
+}
+
+// Lanes per row of the products from the CSR, 0: SELL.  SELL streams a slice as wide as its
+// longest row, so it stays where that pads little, and for the lattice forms' matrices (order 1,
+// the trilinear transfers), whose other storage forms sum in its order.  Measured, SELL against
+// CSR with 4 / 8 / 16 lanes, us: 400 000 rows of 7 (padding 3.2) FP64 25.4 against 14.4 / 20.6 /
+// 36.6; of 23 (2.2) 71.5 against 42.0 / 37.9 / 40.3; Q2 2D 96^2, 37 249 rows of 16 (1.3) 5.7
+// against 3.5 / 3.7 / 5.4; Q2 3D (1.3), rows of 61: 24^3 FP64 31.1 against 24.8 / 20.2 / 20.1, but
+// 48^3 (912 673 rows), where SELL's loads fill the GPU, FP32 126 against 187 / 146 / 143.
+static int csr_lanes(const flgpu_mat *A) {
+  const double pad = A->nnz > 0 ? (double)A->sell.nstored / A->nnz : 1.0;
+  if (A->lat_order == 1 || A->tp_nc > 0 || A->sell.maxw <= 8 || pad <= 1.15) return 0;
+  if (pad <= 1.5 && A->nrows > 400000) return 0;
+  return A->nnz < 10L * A->nrows ? 4 : 8;
+}
+
+template <class T>
+static void launch_csr_spmv(const flgpu_mat *A, T alpha, const void *x, T beta, const void *z,
+                            void *out) {
+  const int G = A->lanes;
+  const unsigned g = xcd_grid(grid_for((long)A->nrows * G, 256));
+  auto launch = [&](auto kern) {
+    kern<<<g, 256, 0, A->ctx->stream>>>(A->nrows, A->rowptr, A->colidx, (const T *)A->vals, alpha,
+                                        (const T *)x, beta, (const T *)z, (T *)out);
+  };
+  launch(G == 4 ? k_csr_spmv<T, 4> : k_csr_spmv<T, 8>);
+  FLGPU_HIP(hipGetLastError());
 }
 
 template <class T>
@@ -1868,6 +1961,11 @@ void spmv(const flgpu_mat *A, double alpha, const void *x, double beta, const vo
                               (float *)out);
     return;
   }
+  if (A->lanes) {
+    if (A->prec == FLGPU_F64) launch_csr_spmv<double>(A, alpha, x, beta, z, out);
+    else launch_csr_spmv<float>(A, (float)alpha, x, (float)beta, z, out);
+    return;
+  }
   if (A->prec == FLGPU_F64) launch_spmv<double>(A->ctx, A->sell, alpha, x, beta, z, out);
   else launch_spmv<float>(A->ctx, A->sell, alpha, x, beta, z, out);
 }
@@ -2207,6 +2305,37 @@ __global__ __launch_bounds__(256) void k_sor_colour(int nsub, int nslices, const
   x[row] += omega * corr;
 }
 
+// The same from the CSR rows, eight lanes per row.  A colour's rows are few, so the length of a
+// row's chain of loads sets the time: 60 001 rows of 12 entries in nine colours, FP32: 3.1 us per
+// colour, 8.1 us from SELL.
+template <class T>
+__global__ __launch_bounds__(256) void k_sor_colour_csr(int nsub, const int *__restrict__ rows,
+                                                        const int2 *__restrict__ span,
+                                                        const int *__restrict__ col,
+                                                        const T *__restrict__ val,
+                                                        const T *__restrict__ diag, T omega, T *x,
+                                                        const T *b, T *r) {
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int li = (int)lb * 32 + threadIdx.x / 8, l = threadIdx.x % 8;
+  if (li >= nsub) return;  // the lanes of a row leave together
+  const int row = rows[li];
+  const int2 be = span[li];
+  const T bi = b[row], di = diag[row], xi = x[row];
+  T corr = (T)((double)bi + csr_row<T, 8>(col, val, be.x, be.y, l, (T)-1, x));
+  corr = corr / di;
+  if (l == 0) {
+    r[row] = corr;
+    x[row] = xi + omega * corr;
+  }
+}
+
+// the CSR bounds of a colour's rows
+__global__ void k_row_span(int nsub, const int *__restrict__ rows, const int *__restrict__ rowptr,
+                           int2 *__restrict__ span) {
+  const int li = blockIdx.x * blockDim.x + threadIdx.x;
+  if (li < nsub) span[li] = make_int2(rowptr[rows[li]], rowptr[rows[li] + 1]);
+}
+
 // LDS of the strip sweep (values): 128 KB in FP64, 64 KB in FP32
 constexpr int kSorCapF64 = 16384, kSorCapF32 = 16384;
 
@@ -2355,6 +2484,19 @@ void sor_sweep(const flgpu_mat *A, double omega, int backwards, void *x, const v
   for (int k = 0; k < A->ncolours; k++) {
     const Sell &s = A->colour_sell[backwards ? A->ncolours - 1 - k : k];
     if (s.nrows == 0) continue;
+    if (s.span) {
+      const unsigned gc = xcd_grid(grid_for(s.nrows, 32));
+      if (A->prec == FLGPU_F64)
+        k_sor_colour_csr<double><<<gc, 256, 0, A->ctx->stream>>>(
+            s.nrows, s.rows, (const int2 *)s.span, A->colidx, (const double *)A->vals,
+            (const double *)A->diag, omega, (double *)x, (const double *)b, (double *)r);
+      else
+        k_sor_colour_csr<float><<<gc, 256, 0, A->ctx->stream>>>(
+            s.nrows, s.rows, (const int2 *)s.span, A->colidx, (const float *)A->vals,
+            (const float *)A->diag, (float)omega, (float *)x, (const float *)b, (float *)r);
+      FLGPU_HIP(hipGetLastError());
+      continue;
+    }
     unsigned g = xcd_grid(grid_for(s.nslices, 4));
     if (A->prec == FLGPU_F64)
       k_sor_colour<double><<<g, 256, 0, A->ctx->stream>>>(

@@ -13,6 +13,7 @@ import scipy.sparse as sp
 from gnu_femlisp_amd import flgpu as F
 from gnu_femlisp_amd import iteration as it
 from gnu_femlisp_amd import lattice as lat
+from gnu_femlisp_amd.flgpu import check, lib
 from gnu_femlisp_amd.matlisp import (GpuSparseMatrix, GpuVector, compute_residual,
                                      default_context, dot, gemm, norm)
 from oracle import pyoracle as po
@@ -139,6 +140,63 @@ def test_empty_and_ragged_rows():
     x = GpuVector.from_array(np.full(5, 9.0))
     gemm(1.0, A, y, 0.0, x)
     assert np.array_equal(x.numpy(), [0.0, 1 + 6 + 15, 0.0, 8.0, 0.0])
+
+
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("nrows,ncols,mean,longest", [(1, 40, 40, 40), (65, 65, 5, 33),
+                                                      (130, 77, 3, 77), (200, 200, 12, 129),
+                                                      (333, 333, 40, 300)])
+def test_irregular_products_and_sweeps(nrows, ncols, mean, longest, prec):
+    """Products (nn, tn, residual) and a coloured <sor> sweep of matrices with empty, short and
+    very long rows, whose kernels read the CSR with 4 or 8 lanes per row: row lengths around the
+    lanes' steps (1 to 300), row counts that leave partial groups, rectangular matrices.  Bounds:
+    the sums of at most 300 products, 300 eps of the largest row's absolute sum."""
+    say(f"irregular {nrows}x{ncols} mean {mean} longest {longest} prec={prec}")
+    rng = np.random.default_rng(nrows + longest)
+    eps = 2.0 ** -52 if prec == F.F64 else 2.0 ** -23
+    lens = np.minimum(rng.geometric(1.0 / mean, nrows) - 1, ncols)
+    lens[0] = longest
+    lens[-1] = min(longest, ncols) if nrows == 1 else 0
+    rows = [np.sort(rng.choice(ncols, k, replace=False)) for k in lens]
+    S = sp.csr_matrix((rng.normal(size=lens.sum()), np.concatenate(rows),
+                       np.concatenate([[0], np.cumsum(lens)])), shape=(nrows, ncols))
+    if prec == F.F32:
+        S.data = S.data.astype(np.float32).astype(np.float64)
+    A = GpuSparseMatrix.from_scipy(S, prec=prec)
+
+    def vec(n):
+        v = rng.normal(size=n)
+        v = v if prec == F.F64 else v.astype(np.float32).astype(np.float64)
+        return v, GpuVector.from_array(v, prec)
+    for job, B in (("nn", S), ("tn", S.T.tocsr())):
+        (y, gy), (x, gx) = vec(B.shape[1]), vec(B.shape[0])
+        got = gemm(0.75, A, gy, -0.5, gx, job).numpy()
+        bound = 300 * eps * (abs(B) @ np.abs(y) + np.abs(x)).max()
+        assert np.abs(got - (0.75 * (B @ y) - 0.5 * x)).max() <= bound
+    if nrows != ncols:
+        return
+    # a diagonally dominant symmetric pattern: the sweep in (colour, index) order
+    D = (abs(S) + abs(S.T)).tocsr()
+    D = (D + sp.diags(np.asarray(D.sum(axis=1)).ravel() + 1.0)).tocsr()
+    D.sort_indices()
+    if prec == F.F32:
+        D.data = D.data.astype(np.float32).astype(np.float64)
+    A = GpuSparseMatrix.from_scipy(D, prec=prec)
+    A.colour_greedy()
+    colour = np.full(nrows, -1)
+    for i in range(nrows):
+        used = {colour[j] for j in D.indices[D.indptr[i]:D.indptr[i + 1]] if j != i}
+        colour[i] = next(k for k in range(nrows + 1) if k not in used)
+    (x, gx), (b, gb) = vec(nrows), vec(nrows)
+    r = GpuVector(nrows, prec)
+    check(lib().flgpu_sor_iterate(A.h, 0.9, 0, gx.h, gb.h, r.h))
+    ref, scale = x.copy(), np.abs(x).max() + np.abs(b).max()
+    for c in range(colour.max() + 1):
+        m = colour == c
+        ref[m] += 0.9 * ((b - D @ ref) / D.diagonal())[m]
+    # the sweep contracts errors (dominant diagonal): a row's rounding of 300 eps adds up over
+    # the colours at most
+    assert np.abs(gx.numpy() - ref).max() <= 300 * eps * scale * (colour.max() + 1)
 
 
 def test_csr_upload_rejects_bad_input():
