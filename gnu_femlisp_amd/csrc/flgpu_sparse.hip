@@ -1940,8 +1940,244 @@ void stage_first_step(const flgpu_mat *A, int rprec, const void *r, void *b, dou
   FLGPU_HIP(hipGetLastError());
 }
 
+// ---- order-2 lattices with a coefficient constant per cell: products without the matrix ------
+// out = beta z + alpha A x with A = sum over the cells of cell[c] Kref.  A workgroup owns the
+// DOFs 2c, 2c + 1 (per axis) of a box of cells; its 256 lanes take the box's cells and those one
+// below it per axis, which share DOFs with it.  Every lane applies the reference matrix to its
+// cell's 3^DIM values of x from an LDS patch (zero at Dirichlet points, as the eliminated columns
+// are) and leaves the scaled result in LDS; then every lane of the box adds up its 2^DIM rows,
+// cells in ascending order.  Dirichlet rows are identity rows.
+//
+// Kref is the sum of the tensor products of one 1-D stiffness matrix K and 1-D mass matrices M of
+// the reference interval.  Both are symmetric under reflection, so on (u0 + u2, u1, u0 - u2) they
+// are a 2 x 2 block and a scalar: 315 multiply-adds and 108 additions per 3D cell instead of the
+// 729 of the 27 x 27 matrix, with ten constants in scalar registers (the matrix itself, fetched by
+// scalar loads, took 21.5 us at Q2 48^3, FP64).
+// Bytes: 8 (FP32) or 16 per row instead of 62 matrix entries with their columns.  The latency of
+// the three phases bounds small lattices, the waves in flight (LDS) large ones.
+// Q2 48^3: FP64 15.2 us, FP32 14.2 us; 193 and 128 us from SELL.
+template <class T>
+struct Ref1D {  // a 1-D reference matrix on (sum, middle, difference): a, b; b, c; d
+  T a, b, c, d;
+};
+template <class T>
+__device__ __forceinline__ Ref1D<T> ref_mass() {  // 1/30 [4 2 -1; 2 16 2; -1 2 4]
+  return {(T)(1.5 / 30), (T)(2.0 / 30), (T)(16.0 / 30), (T)(2.5 / 30)};
+}
+template <class T>
+__device__ __forceinline__ Ref1D<T> ref_stiff() {  // 1/3 [7 -8 1; -8 16 -8; 1 -8 7]
+  return {(T)(4.0 / 3), (T)(-8.0 / 3), (T)(16.0 / 3), (T)1};
+}
+// (e, m, o) of the line through u with stride S -> the matrix's product, plus `add` if given
+template <class T>
+__device__ __forceinline__ void ref_apply(const Ref1D<T> &R, T e, T m, T o, T &p, T &q, T &r) {
+  p = R.a * e + R.b * m;
+  q = R.b * e + R.c * m;
+  r = R.d * o;
+}
+template <class T>
+__device__ __forceinline__ void ref_add(const Ref1D<T> &R, T e, T m, T o, T &p, T &q, T &r) {
+  p += R.a * e + R.b * m;
+  q += R.b * e + R.c * m;
+  r += R.d * o;
+}
+
+// v <- Kref v for the 3^DIM values of one cell, last axis fastest
+template <class T, int DIM>
+__device__ __forceinline__ void cell_matrix(T *v) {
+  constexpr int NL = DIM == 3 ? 27 : 9;
+  const Ref1D<T> Mm = ref_mass<T>(), Km = ref_stiff<T>();
+  // to (sum, middle, difference) along every axis
+#pragma unroll
+  for (int st = 1; st < NL; st *= 3)
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+      if ((i / st) % 3 == 0) {
+        const T u0 = v[i], u2 = v[i + 2 * st];
+        v[i] = u0 + u2;
+        v[i + 2 * st] = u0 - u2;
+      }
+  // last axis: a = M v, b = K v
+  T a[NL], b[NL];
+#pragma unroll
+  for (int i = 0; i < NL; i += 3) {
+    ref_apply(Mm, v[i], v[i + 1], v[i + 2], a[i], a[i + 1], a[i + 2]);
+    ref_apply(Km, v[i], v[i + 1], v[i + 2], b[i], b[i + 1], b[i + 2]);
+  }
+  // middle axis (the first in 2D): a <- M a, b <- K a + M b
+#pragma unroll
+  for (int i = 0; i < NL; i++)
+    if ((i / 3) % 3 == 0) {
+      T m0, m1, m2, k0, k1, k2;
+      if (DIM == 3) ref_apply(Mm, a[i], a[i + 3], a[i + 6], m0, m1, m2);
+      ref_apply(Km, a[i], a[i + 3], a[i + 6], k0, k1, k2);
+      ref_add(Mm, b[i], b[i + 3], b[i + 6], k0, k1, k2);
+      if (DIM == 3) {
+        a[i] = m0;
+        a[i + 3] = m1;
+        a[i + 6] = m2;
+      }
+      b[i] = k0;
+      b[i + 3] = k1;
+      b[i + 6] = k2;
+    }
+  // first axis: K a + M b
+  if (DIM == 3) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+      T k0, k1, k2;
+      ref_apply(Km, a[i], a[i + 9], a[i + 18], k0, k1, k2);
+      ref_add(Mm, b[i], b[i + 9], b[i + 18], k0, k1, k2);
+      b[i] = k0;
+      b[i + 9] = k1;
+      b[i + 18] = k2;
+    }
+  }
+  // back: first and last node from (half sum, middle, half difference)
+#pragma unroll
+  for (int st = 1; st < NL; st *= 3)
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+      if ((i / st) % 3 == 0) {
+        const T p = b[i], q = b[i + 2 * st];
+        b[i] = p + q;
+        b[i + 2 * st] = p - q;
+      }
+#pragma unroll
+  for (int i = 0; i < NL; i++) v[i] = b[i];
+}
+
+// Below this many rows the CSR product is faster: 15 625 rows (3D) 4.1 against 6.4 us, 9 409 (2D)
+// 3.6 against 3.8; above, 35 937 (3D) 7.5 against 6.5, 37 249 (2D) 3.6 against 3.7, 103 041 (2D)
+// 6.7 against 3.9, 117 649 (3D) 20.3 against 6.6 us (FP64).
+constexpr int kCellApplyRows = 30000;
+
+template <int DIM>
+struct CellBox;
+template <>
+struct CellBox<3> {
+  static constexpr int B[3] = {3, 7, 7};  // cells of the box: 4 x 8 x 8 lanes
+};
+template <>
+struct CellBox<2> {
+  static constexpr int B[3] = {0, 15, 15};  // 16 x 16 lanes
+};
+
+template <class T, int DIM>
+__global__ __launch_bounds__(256) void k_cell_apply(int n, Div1 dby, Div1 dbx,
+                                                    const T *__restrict__ cell, T alpha,
+                                                    const T *__restrict__ x, T beta, const T *z,
+                                                    T *out, unsigned nblk) {
+  constexpr int NL = DIM == 3 ? 27 : 9;
+  constexpr int PZ = DIM == 3 ? 2 * (CellBox<DIM>::B[0] + 1) + 1 : 1,
+                PY = 2 * (CellBox<DIM>::B[1] + 1) + 1, PX = 2 * (CellBox<DIM>::B[2] + 1) + 1;
+  constexpr int LX = CellBox<DIM>::B[2] + 1, LY = CellBox<DIM>::B[1] + 1;
+  __shared__ T px[PZ * PY * PX];
+  __shared__ T ye[NL * 256];
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  if (lb >= nblk) return;
+  const int tid = threadIdx.x, M = 2 * n + 1;
+  unsigned u = lb, q = fdiv(u, dbx);
+  const int cx0 = (int)(u - q * dbx.f.d) * CellBox<DIM>::B[2];
+  u = q;
+  q = fdiv(u, dby);
+  const int cy0 = (int)(u - q * dby.f.d) * CellBox<DIM>::B[1];
+  const int cz0 = DIM == 3 ? (int)q * CellBox<DIM>::B[0] : 0;
+  // the x patch [2 c0 - 2, 2 (c0 + B)] per axis
+  constexpr int NP = PZ * PY * PX, NS = (NP + 255) / 256;
+  T pv[NS];
+#pragma unroll
+  for (int k = 0; k < NS; k++) {
+    const int e = min(tid + k * 256, NP - 1);
+    const int qx = 2 * cx0 - 2 + e % PX, qy = 2 * cy0 - 2 + (e / PX) % PY,
+              qz = DIM == 3 ? 2 * cz0 - 2 + e / (PX * PY) : 1;
+    const bool in = qx > 0 && qx < M - 1 && qy > 0 && qy < M - 1 &&
+                    (DIM == 2 || (qz > 0 && qz < M - 1));
+    const long idx = DIM == 3 ? ((long)qz * M + qy) * M + qx : (long)qy * M + qx;
+    const T t = x[in ? idx : 0];
+    pv[k] = in ? t : (T)0;
+  }
+#pragma unroll
+  for (int k = 0; k < NS; k++)
+    if (tid + k * 256 < NP) px[tid + k * 256] = pv[k];
+  const int lx = tid % LX, ly = (tid / LX) % LY, lz = tid / (LX * LY);
+  const int cx = cx0 - 1 + lx, cy = cy0 - 1 + ly, cz = DIM == 3 ? cz0 - 1 + lz : 0;
+  const bool live = cx >= 0 && cx < n && cy >= 0 && cy < n && cz >= 0 && cz < n;
+  const T fac = cell[live ? ((long)cz * n + cy) * n + cx : 0];
+  // the rows 2c, 2c + 1 of this lane's cell; what they need besides the sums is loaded ahead
+  const bool own = lx > 0 && ly > 0 && (DIM == 2 || lz > 0) && cx <= n && cy <= n && cz <= n;
+  const long row0 = ((DIM == 3 ? (long)2 * cz * M : 0) + 2 * cy) * M + 2 * cx;
+  T zv[1 << DIM];
+#pragma unroll
+  for (int t = 0; t < (1 << DIM); t++) {
+    const int tx = t & 1, ty = (t >> 1) & 1, tz = DIM == 3 ? t >> 2 : 0;
+    const bool in = own && (cx < n || !tx) && (cy < n || !ty) && (DIM == 2 || cz < n || !tz);
+    if (beta != (T)0) zv[t] = z[in ? row0 + ((long)tz * M + ty) * M + tx : 0];
+  }
+  __syncthreads();
+  double xv[NL];  // FP64 for FP32 too: the same rate, and no rounding before the cells' sums
+  const int pb = ((DIM == 3 ? 2 * lz : 0) * PY + 2 * ly) * PX + 2 * lx;
+#pragma unroll
+  for (int j = 0; j < NL; j++) {
+    const int o = DIM == 3 ? ((j / 9) * PY + (j / 3) % 3) * PX + j % 3 : (j / 3) * PX + j % 3;
+    xv[j] = px[pb + o];
+  }
+  cell_matrix<double, DIM>(xv);
+#pragma unroll
+  for (int l = 0; l < NL; l++) ye[l * 256 + tid] = live ? (T)((double)fac * xv[l]) : (T)0;
+  __syncthreads();
+  if (!own) return;
+#pragma unroll
+  for (int t = 0; t < (1 << DIM); t++) {
+    const int tx = t & 1, ty = (t >> 1) & 1, tz = DIM == 3 ? t >> 2 : 0;
+    const int qx = 2 * cx + tx, qy = 2 * cy + ty, qz = 2 * cz + tz;
+    if (qx >= M || qy >= M || qz >= M) continue;
+    double s = 0;
+#pragma unroll
+    for (int c = 0; c < (1 << DIM); c++) {  // bit set: this lane's cell, else the one below
+      const int ux = c & 1, uy = (c >> 1) & 1, uz = DIM == 3 ? c >> 2 : 1;
+      if ((tx && !ux) || (ty && !uy) || (tz && !uz)) continue;  // interior node of this cell
+      const int jx = ux ? tx : 2, jy = uy ? ty : 2, jz = uz ? tz : 2;
+      const int l = DIM == 3 ? (jz * 3 + jy) * 3 + jx : jy * 3 + jx;
+      const int src = tid - (ux ? 0 : 1) - (uy ? 0 : LX) - (uz ? 0 : LX * LY);
+      s += (double)ye[l * 256 + src];
+    }
+    const long idx = row0 + ((long)tz * M + ty) * M + tx;
+    const bool dir = qx == 0 || qx == M - 1 || qy == 0 || qy == M - 1 ||
+                     (DIM == 3 && (qz == 0 || qz == M - 1));
+    if (dir) s = (double)x[idx];
+    s *= (double)alpha;
+    out[idx] = beta == (T)0 ? (T)s : (T)((double)beta * (double)zv[t] + s);
+  }
+}
+
+template <class T>
+static void launch_cell_apply(const flgpu_mat *A, T alpha, const void *x, T beta, const void *z,
+                              void *out) {
+  const int n = A->lat_n;
+  auto boxes = [&](int B) { return (unsigned)((n + 1 + B - 1) / B); };
+  if (A->lat_dim == 3) {
+    const unsigned bz = boxes(CellBox<3>::B[0]), by = boxes(CellBox<3>::B[1]),
+                   bx = boxes(CellBox<3>::B[2]), nb = bz * by * bx;
+    k_cell_apply<T, 3><<<xcd_grid(nb), 256, 0, A->ctx->stream>>>(
+        n, div1(by), div1(bx), (const T *)A->cell, alpha, (const T *)x, beta,
+        (const T *)z, (T *)out, nb);
+  } else {
+    const unsigned by = boxes(CellBox<2>::B[1]), bx = boxes(CellBox<2>::B[2]), nb = by * bx;
+    k_cell_apply<T, 2><<<xcd_grid(nb), 256, 0, A->ctx->stream>>>(
+        n, div1(by), div1(bx), (const T *)A->cell, alpha, (const T *)x, beta,
+        (const T *)z, (T *)out, nb);
+  }
+  FLGPU_HIP(hipGetLastError());
+}
+
 void spmv(const flgpu_mat *A, double alpha, const void *x, double beta, const void *z,
           void *out) {
+  if (A->cell && A->lat_dim >= 2 && A->nrows >= kCellApplyRows) {
+    if (A->prec == FLGPU_F64) launch_cell_apply<double>(A, alpha, x, beta, z, out);
+    else launch_cell_apply<float>(A, (float)alpha, x, (float)beta, z, out);
+    return;
+  }
   if (A->tp_kind) {
     if (A->prec == FLGPU_F64) launch_tp<double>(A, alpha, x, beta, z, out);
     else launch_tp<float>(A, (float)alpha, x, (float)beta, z, out);

@@ -264,6 +264,37 @@ def test_lattice_storage_matches_csr(prec, form):
         assert relerr(rs[0].numpy(), rs[1].numpy()) < 10 * tol
 
 
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("dim,n", [(3, 16), (3, 21), (2, 97), (2, 90)])
+def test_order2_cell_products(dim, n, prec):
+    """Products of order-2 lattice matrices with one coefficient per cell (and none), which are
+    applied cell by cell from 30000 rows on, against the same matrix's entries (SELL or CSR):
+    boxes that end at, before and beyond the lattice's last cell, alpha and beta, x random at
+    Dirichlet points too.  A row's terms are at most 125 products of entries rounded once:
+    125 eps of the row's absolute sum."""
+    say(f"order-2 cell products dim={dim} n={n} prec={prec}")
+    rng = np.random.default_rng(dim + n)
+    eps = 2.0 ** -52 if prec == F.F64 else 2.0 ** -23
+    for kap in (np.exp(rng.normal(scale=1.5, size=(n,) * dim)), None):
+        A, _ = lat.assemble(dim, 2, n, kap, prec=prec)
+        assert A.nrows >= 30000
+        B = A.convert(prec)
+        assert B.storage(F.STORAGE_SELL) == F.STORAGE_SELL
+        rp, ci, v = A.csr()
+        S = sp.csr_matrix((np.abs(v), ci, rp))
+        y, x = (rng.normal(size=A.nrows).astype(np.float32).astype(np.float64) for _ in range(2))
+        bound = 125 * eps * (S @ np.abs(y) + np.abs(x)).max()
+        for alpha, beta in ((-1.0, 1.0), (0.5, 0.0), (2.0, -0.25)):
+            got = [gemm(alpha, M, GpuVector.from_array(y, prec), beta,
+                        GpuVector.from_array(x, prec)).numpy() for M in (A, B)]
+            assert np.abs(got[0] - got[1]).max() <= bound
+        # new values are no sum over the cells: the entries are used from then on
+        A.update_values(2.0 * v)
+        z = gemm(1.0, A, GpuVector.from_array(y, prec), 0.0, A.make_image_vector()).numpy()
+        w = gemm(2.0, B, GpuVector.from_array(y, prec), 0.0, B.make_image_vector()).numpy()
+        assert np.abs(z - w).max() <= 2 * bound
+
+
 def test_vector_ops():
     say("vector ops")
     rng = np.random.default_rng(9)
