@@ -174,7 +174,7 @@ struct flgpu_mat {
   // by DOFs i and j), d = lattice offset; kernels apply A from alpha
   void *alpha = nullptr;  // n^3 cell factors (prec), nullptr if not available
   double kt[8] = {};      // Kref[0][b], b = bz*4 + by*2 + bx
-  // with alpha: the <sor> sweep's strips per plane (0: one launch per colour) and its copy of
+  // with val27: the <sor> sweep's strips per plane (0: one launch per colour) and its copy of
   // x and b around the strip boundaries, 2 (M (S - 1) 8 M) values (prec), nullptr if S < 2
   int sor_strips = 0, sor_h = 0;
   void *sor_ghost = nullptr;
@@ -223,7 +223,7 @@ void drop_alpha(flgpu_mat *A);
 void drop_cells(flgpu_mat *A);  // cell, kref, elem
 // entries of a row of n values padded to 16 bytes
 inline int row_pad(int n, int prec) { return prec == FLGPU_F64 ? (n + 1) & ~1 : (n + 3) & ~3; }
-// the strips and boundary copy of the per-cell <sor> sweep, after alpha is allocated
+// the strips and boundary copy of the stencil-form <sor> sweep
 void sor_strips_alloc(flgpu_mat *A);
 void tp_prepare(flgpu_mat *T);  // (re)fill tp27 of an interpolation or its transpose
 void tp_drop(flgpu_mat *A);     // products of A (and its transpose) go back to SELL
@@ -247,8 +247,6 @@ void spmv_t(const flgpu_mat *A, double alpha, const void *x, double beta,
 // applied in the per-cell form; false (nothing launched) otherwise
 bool spmv_dot(const flgpu_mat *A, const void *x, void *out, int slot);
 void jacobi_iterate(const flgpu_mat *A, double damp, void *x, void *r);
-void sor_sweep(const flgpu_mat *A, double omega, int backwards, void *x,
-               const void *b, void *r);
 // `steps` <jacobi> steps with fresh residuals, x ping-ponged through tmp; x_zero: x is zero
 // and need not be read (the first step is x = damp b / diag)
 // x64 (FP64, n values) may receive a copy of the final x: true when the last step wrote it
@@ -271,9 +269,12 @@ void blocks_prepare(flgpu_mat *A);
 void blocks_drop(flgpu_mat *A);
 void block_sweep(const flgpu_mat *A, bool ssc, double omega, int backwards, void *x,
                  const void *b, void *r, bool cells);
-// `steps` sweeps
-void sor_sweeps(const flgpu_mat *A, double omega, int steps, int backwards, void *x,
-                const void *b, void *r);
+bool sor_outplace(const flgpu_mat *A);  // its sweeps use a spare vector
+// `steps` <sor> sweeps.  tmp (n values): lets the per-cell form sweep out of place; x_zero: x is
+// zero and need not be stored; rmode: 1: r holds the last corrections, 0: r is not wanted, 2: r
+// is wanted as the residual, true when it is (b == r implies 1)
+bool sor_sweeps(const flgpu_mat *A, double omega, int steps, int backwards, void *x,
+                const void *b, void *r, void *tmp = nullptr, bool x_zero = false, int rmode = 1);
 
 // lattices (flgpu_lattice.hip)
 // keep_elem: keep the element matrices of an order-2 lattice (flgpu_mat::elem) when its

@@ -62,7 +62,7 @@ struct MGLevel {
   flgpu_mat *I = nullptr;  // owned: interpolation level -> level+1 (transpose attached)
   flgpu_mat *R = nullptr;  // owned, FAS only: projection level+1 -> level (:fas-r-vec)
   void *sol = nullptr, *rhs = nullptr, *res = nullptr;  // owned work vectors
-  void *tmp = nullptr;  // <jacobi> steps: the other half of x's ping-pong (smoother Jacobi)
+  void *tmp = nullptr;  // the other half of x's ping-pong (<jacobi>, per-cell <sor>)
   bool residual_p = false;
   bool x_zero = false;  // sol is zero but not stored: the next smoother step or coarse solve
                         // writes it instead of updating it
@@ -669,7 +669,14 @@ static void smooth(flgpu_mg *mg, int l, bool post, bool last = false) {
       if (steps > 1 && seen) spmv(L.A, -1.0, x, 1.0, b, r);
     }
   } else {
-    sor_sweeps(L.A, p.omega, steps, post && p.symmetric, x, b, r);
+    // nothing reads the corrections that a sweep leaves in r but the caller, at the top level;
+    // the pre-smoothing's r is overwritten by the residual
+    const int rmode = !post ? 2 : (l == mg->top ? 1 : 0);
+    const bool res = sor_sweeps(L.A, p.omega, steps, post && p.symmetric, x, b, r, L.tmp,
+                                L.x_zero, rmode);
+    L.x_zero = false;
+    L.residual_p = res;
+    return;
   }
   L.residual_p = false;  // residual-after nil
 }
@@ -694,7 +701,10 @@ static void lmgc(flgpu_mg *mg, int l) {
   // stored zero, and fused steps recompute the residual from rhs, so the restriction goes
   // straight into rhs there (the coarse solve reads only res)
   bool base = (l - 1 == mg->p.base_level);
-  bool fused = !add && mg->p.smoother == FLGPU_SMOOTH_JACOBI && C.tmp && mg->p.pre_steps > 0;
+  const bool pre = !add && mg->p.pre_steps > 0;
+  bool fused = pre && mg->p.smoother == FLGPU_SMOOTH_JACOBI && C.tmp;
+  // <sor> and <ssc> form their residuals from rhs too; <sor> takes x = 0 without reading it
+  bool sweeps = pre && (mg->p.smoother == FLGPU_SMOOTH_SOR || mg->p.smoother == FLGPU_SMOOTH_SSC);
   if (mg->p.fas) {
     // <fas> :after (multigrid.lisp:226-232): rhs_{l-1} = res_{l-1}, sol_{l-1} = R sol_l,
     // rhs_{l-1} += A_{l-1} sol_{l-1}, residual-p t
@@ -711,6 +721,11 @@ static void lmgc(flgpu_mg *mg, int l) {
     C.step1 = restrict_first_step(C.I->transpose, lres(mg, l), C.rhs, C.A, mg->p.omega, C.tmp);
     if (!C.step1) spmv(C.I->transpose, 1.0, lres(mg, l), 0.0, C.rhs, C.rhs);
     C.x_zero = true;
+    C.residual_p = false;
+  } else if (sweeps && !base) {
+    spmv(C.I->transpose, 1.0, lres(mg, l), 0.0, C.rhs, C.rhs);
+    C.x_zero = mg->p.smoother == FLGPU_SMOOTH_SOR;
+    if (!C.x_zero) vfill(mg->ctx, C.N, mg->p.prec, C.sol, 0.0);
     C.residual_p = false;
   } else {
     spmv(C.I->transpose, 1.0, lres(mg, l), 0.0, C.res, C.res);
@@ -833,7 +848,8 @@ static void mg_apply_zero(flgpu_mg *mg, int vprec, void *q, void *r, void *work,
   bool add = p.additive != 0;
   bool sweeps = p.smoother == FLGPU_SMOOTH_SOR || p.smoother == FLGPU_SMOOTH_SSC;
   bool reads_r = base_top || add || !(jac || (sweeps && p.pre_steps > 0));
-  bool zero = (jac && !add) || base_top;  // the first step writes x
+  bool sor = p.smoother == FLGPU_SMOOTH_SOR && p.pre_steps > 0;
+  bool zero = ((jac || sor) && !add) || base_top;  // the first step writes x
   FLGPU_REQUIRE(!staged || mg_stages_first(mg, vprec), "this cycle does not take a staged rhs");
   if (vprec == p.prec) {
     if (zero) T.x_zero = true;
@@ -960,7 +976,10 @@ static void mg_alloc_work(flgpu_mg *mg) {
     vfill(mg->ctx, L.N, mg->p.prec, L.sol, 0.0);
     vfill(mg->ctx, L.N, mg->p.prec, L.rhs, 0.0);
     vfill(mg->ctx, L.N, mg->p.prec, L.res, 0.0);
-    if (mg->p.smoother == FLGPU_SMOOTH_JACOBI) L.tmp = dev_alloc(b);
+    const int steps = std::max(mg->p.pre_steps, mg->p.post_steps);
+    if (mg->p.smoother == FLGPU_SMOOTH_JACOBI ||
+        (mg->p.smoother == FLGPU_SMOOTH_SOR && steps > 1 && sor_outplace(L.A)))
+      L.tmp = dev_alloc(b);
   }
   long N = mg->lv[mg->top].N;
   size_t b = prec_bytes(mg->p.prec) * N;

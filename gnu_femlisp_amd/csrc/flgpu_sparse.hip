@@ -273,7 +273,7 @@ void mat_finish(flgpu_mat *A) {
   if (is_q1_lattice(A)) {
     A->val27 = dev_alloc(prec_bytes(A->prec) * 27 * (size_t)A->nrows);
     stencil_refresh(A);
-    if (A->sor_strips == 0) sor_strips_alloc(A);
+    sor_strips_alloc(A);
   }
 }
 
@@ -299,9 +299,8 @@ void mat_free(flgpu_mat *A) {
   delete A;
 }
 
-// the strip <sor> sweeps' boundary copies, once neither lattice form is left
+// the stencil-form <sor> sweeps' boundary copies
 static void drop_sor_strips(flgpu_mat *A) {
-  if (A->alpha || A->val27) return;
   dev_free(A->sor_ghost);
   A->sor_ghost = nullptr;
   A->sor_strips = A->sor_h = 0;
@@ -312,7 +311,6 @@ void drop_alpha(flgpu_mat *A) {
   if (A->alpha) layout_changed(A);
   dev_free(A->alpha);
   A->alpha = nullptr;
-  drop_sor_strips(A);
 }
 
 // new values that are no sum over the lattice's cells
@@ -445,7 +443,6 @@ flgpu_mat *mat_convert(const flgpu_mat *A, int prec) {
     B->alpha = dev_alloc(prec_bytes(prec) * nc);
     vcopy(ctx, nc, A->prec, A->alpha, prec, B->alpha);
     for (int j = 0; j < 8; j++) B->kt[j] = A->kt[j];
-    sor_strips_alloc(B);
   }
   if (A->cell) {
     long nc = 1;
@@ -651,10 +648,6 @@ static void launch_spmv(flgpu_ctx *ctx, const Sell &s, double alpha, const void 
 
 // ---- 3D Q1 lattice with a per-cell coefficient: A applied from alpha ---------------
 
-struct Q1K {
-  double k[8];
-};
-
 // The neighbours along one axis (one nonzero offset): the Q1 stiffness of a cube couples the
 // nodes of a common edge with exactly 0, and kt holds the FP64 Gauss sum's residue, about
 // 1e-17 of kt[0]: such an entry is 1e-17 of the row's diagonal, far below the FP32 resolution
@@ -665,56 +658,6 @@ __device__ __forceinline__ constexpr bool q1_axis(int dz, int dy, int dx) {
   return sizeof(T) == 4 && (dz != 0) + (dy != 0) + (dx != 0) == 1;
 }
 
-// acc + sum over interior neighbours j of row i (ascending j) of (coef x_j) A_ij
-// with A_ij = kt[|dz|*4 + |dy|*2 + |dx|] * (sum of alpha over the cells shared
-// by i and j); *dii receives A_ii.  Row i = (z,y,x) must be interior.  All
-// loads are issued before the first product: a Dirichlet column (eliminated,
-// A_ij = 0) reads x_i and adds a zero product, so the sum keeps its order and
-// the row waits for one memory latency instead of one per neighbour.
-template <class T>
-__device__ __forceinline__ T q1_row(int M, int n, long i, int z, int y, int x,
-                                    const T *__restrict__ alpha, const Q1K &kt, T acc, T coef,
-                                    const T *__restrict__ xv, T *dii) {
-  T a[2][2][2];
-#pragma unroll
-  for (int p = 0; p < 2; p++)
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-#pragma unroll
-      for (int s = 0; s < 2; s++)
-        a[p][q][s] = alpha[((long)(z - 1 + p) * n + (y - 1 + q)) * n + (x - 1 + s)];
-  long M2 = (long)M * M;
-  bool lz[3] = {z - 1 != 0, true, z + 1 != M - 1}, ly[3] = {y - 1 != 0, true, y + 1 != M - 1},
-       lx[3] = {x - 1 != 0, true, x + 1 != M - 1};
-  T xn[27];
-#pragma unroll
-  for (int k = 0; k < 27; k++) {
-    int dz = k / 9 - 1, dy = (k / 3) % 3 - 1, dx = k % 3 - 1;
-    bool live = lz[dz + 1] && ly[dy + 1] && lx[dx + 1];
-    xn[k] = xv[live ? i + dz * M2 + dy * M + dx : i];
-  }
-#pragma unroll
-  for (int k = 0; k < 27; k++) {
-    int dz = k / 9 - 1, dy = (k / 3) % 3 - 1, dx = k % 3 - 1;
-    if (q1_axis<T>(dz, dy, dx)) continue;
-    int pz0 = dz > 0 ? 1 : 0, pz1 = dz < 0 ? 0 : 1;
-    int py0 = dy > 0 ? 1 : 0, py1 = dy < 0 ? 0 : 1;
-    int px0 = dx > 0 ? 1 : 0, px1 = dx < 0 ? 0 : 1;
-    T s = (T)0;
-#pragma unroll
-    for (int p = pz0; p <= pz1; p++)
-#pragma unroll
-      for (int q = py0; q <= py1; q++)
-#pragma unroll
-        for (int r = px0; r <= px1; r++) s += a[p][q][r];
-    T aij = (T)kt.k[(dz != 0) * 4 + (dy != 0) * 2 + (dx != 0)] * s;
-    if (k == 13) *dii = aij;
-    bool live = lz[dz + 1] && ly[dy + 1] && lx[dx + 1];
-    acc += (coef * xn[k]) * (live ? aij : (T)0);
-  }
-  return acc;
-}
-
 // ---- whole-lattice passes in the per-cell form, blocked along z ---------------------------
 // A thread owns QZB consecutive rows along z at one (y, x).  It loads its own x column of the
 // 3 lines y-1..y+1 over the QZB + 2 planes and its own cell-factor column of the lines y-1, y
@@ -722,8 +665,9 @@ __device__ __forceinline__ T q1_row(int M, int n, long i, int z, int y, int x,
 // the neighbouring lanes of its wave (DPP whole-wave shifts).  Each wave computes 62
 // consecutive positions; its two edge lanes only load the columns its first and last position
 // need.  Dirichlet values are zeroed as they are loaded, which is what the explicit zeros of
-// the eliminated columns contribute.  Each row is formed with exactly q1_row's arithmetic (same
-// terms, same order; the cell sums start from their first term, as alpha > 0).
+// the eliminated columns contribute.  Row i is the sum over its neighbours j, ascending, of
+// (coef x_j) A_ij with A_ij = kt[|dz| 4 + |dy| 2 + |dx|] (sum of alpha over the cells i and j
+// share, ascending).
 enum { Q1_SPMV = 0, Q1_JACOBI = 1 };
 
 template <class T> struct Q1KT {
@@ -849,7 +793,7 @@ __global__ __launch_bounds__(256) void k_q1_zblock(int M, int n, const T *__rest
   // cs[k][dy][dx]: the ordered sum over cell plane k of the cells an entry with in-plane
   // offset (dy, dx) shares; pl = kt * cs is the entry itself when the offset crosses planes
   // (dz = -1 of row k, dz = +1 of row k - 1).  An entry within a plane (dz = 0) continues
-  // row r's plane-r sum with the plane-(r + 1) cells, which is q1_row's order.
+  // row r's plane-r sum with the plane-(r + 1) cells.
   T cs[QZB + 1][3][3], pl[QZB + 1][3][3];
   auto prep_a = [&](int k) {
 #pragma unroll
@@ -984,269 +928,308 @@ static void launch_q1_pass(const flgpu_mat *A, T coef, T beta, const void *v, co
   FLGPU_HIP(hipGetLastError());
 }
 
-// one colour (cz, cy, cx) of a <sor> sweep from alpha
-template <class T>
-__global__ __launch_bounds__(256) void k_q1_sor(int M, int n, int cz, int cy, int cx,
-                                                const T *__restrict__ alpha, Q1K kt, T omega, T *x,
-                                                const T *b, T *r) {
-  int nx = (M - cx + 1) / 2, ny = (M - cy + 1) / 2, nz = (M - cz + 1) / 2;
-  unsigned lb = xcd_block(blockIdx.x, gridDim.x);
-  long t = (long)lb * blockDim.x + threadIdx.x;
-  if (t >= (long)nx * ny * nz) return;
-  int xx = 2 * (int)(t % nx) + cx, yy = 2 * (int)((t / nx) % ny) + cy,
-      zz = 2 * (int)(t / ((long)nx * ny)) + cz;
-  long i = ((long)zz * M + yy) * M + xx;
-  bool bd = xx == 0 || yy == 0 || zz == 0 || xx == M - 1 || yy == M - 1 || zz == M - 1;
-  T corr = b[i];
-  T d = (T)1;
-  if (bd) corr += (-x[i]) * (T)1;
-  else corr = q1_row<T>(M, n, i, zz, yy, xx, alpha, kt, corr, (T)-1, x, &d);
-  corr = corr / d;
-  r[i] = corr;
-  x[i] += omega * corr;
+// ---- the per-cell <sor> sweep --------------------------------------------------------------
+// The Q1 stiffness of a cube couples the nodes of a common edge with exactly 0 (kt's entries for
+// one nonzero offset are the Gauss sum's residue, 1e-17 of kt[0], and are left out here), so a
+// row couples only to rows that differ in at least two of the parities (z, y, x).  Of the eight
+// colours c = 4 z + 2 y + x in their order, 2k and 2k + 1 then do not see each other: a sweep
+// needs four steps, one for each (z, y) parity, and a step's rows are whole lines.  With the
+// edge terms gone a row is, per cell it shares with its neighbours,
+//   alpha_c (kt[6] x(z', y') + kt[5] x(z', x') + kt[7] x(z', y', x') + kt[3] x(y', x')),
+// ' marking the neighbour on the cell's side: 4 products a cell plane instead of the 9 entries'
+// sums and products.  A wave takes 62 consecutive positions of the lines (lanes 1..62, lanes 0
+// and 63 only load); a lane loads the x and cell columns of its own position and takes the x - 1
+// and x + 1 columns from its neighbouring lanes: a row's x - 1 and x + 1 are on its own line (a
+// line ends only at a Dirichlet row, which reads none).
+// Bound by the memory (x, the cells, b and the new x of a parity: 47 MB of FP64 a step at 129^3)
+// and, up to 65^3, by the launches.  A sweep in place, FP64: 129^3 29 us, 97^3 12.7; two launches
+// with eight in-plane colours in LDS, from a copy of the strips' edges, took 51 and 46.
+template <class T> struct SorCols {
+  T off[2][3];  // x at (z -+ 1, y - 1..y + 1)
+  T in[2];      // x at (z, y -+ 1)
+  T a[2][2];    // cells (z - 1.., y - 1..) of cell column x
+  T xi, b;
+};
+
+// OFF0: x is zero on the planes z -+ 1, IN0: on the lines y -+ 1 (or not wanted), ZERO: the row's
+// own x is zero; those are not read.  Indexes are clamped into the lattice.
+template <class T, bool OFF0, bool IN0, bool ZERO>
+__device__ __forceinline__ void sor_load(SorCols<T> &C, int M, int n, int z, int y, int xc,
+                                         const T *__restrict__ alpha, const T *xoff,
+                                         const T *xin, const T *b) {
+  const unsigned uM = (unsigned)M, un = (unsigned)n, ux = (unsigned)xc;
+  const int xcc = min(xc, n - 1);
+#pragma unroll
+  for (int p = 0; p < 2; p++) {
+    const unsigned zo = (unsigned)min(max(z - 1 + 2 * p, 0), M - 1) * uM;
+    const unsigned zc = (unsigned)min(max(z - 1 + p, 0), n - 1) * un;
+    if (!OFF0)
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+        C.off[p][d] = xoff[(zo + (unsigned)min(max(y + d - 1, 0), M - 1)) * uM + ux];
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+      C.a[p][q] = alpha[(zc + (unsigned)min(max(y - 1 + q, 0), n - 1)) * un + (unsigned)xcc];
+  }
+  if (!IN0)
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+      C.in[q] = xin[((unsigned)z * uM + (unsigned)min(max(y - 1 + 2 * q, 0), M - 1)) * uM + ux];
+  const unsigned i = ((unsigned)z * uM + (unsigned)y) * uM + ux;
+  C.xi = ZERO ? (T)0 : xin[i];
+  C.b = b[i];
 }
 
-// ---- the per-cell <sor> sweep in plane strips ----------------------------------------------
-// Colours 0-3 lie on the even z planes, 4-7 on the odd ones, and a row couples to the other z
-// parity only through the planes z - 1 and z + 1, which no row of its own parity changes.  So
-// one launch sweeps the four colours of one parity.  A block owns the lines [y0, y1) (whole
-// lines in x) of one interior plane z.  It stages the plane's x over the lines
-// [y0 - 4, y1 + 4), b plus the terms of the planes z - 1 and z + 1 for every row of
-// [y0 - 3, y1 + 3), and the cell factors of the cell planes z - 1 and z summed per cell column.
-// Then it runs the four in-plane colours with a barrier between them.  Colour j of the four
-// needs the in-plane values of the colours before it one line away, so the block computes it
-// on 3 - j lines beyond its own on each side.  It does so from the same values with the same
-// arithmetic as the block owning those lines, so the values it uses equal the owner's bit for
-// bit.  The owner overwrites those lines in the same launch, so a block reads them from a copy
-// that k_q1_sor_prep takes before the sweep (gx, gb: for every plane z and strip boundary
-// sb = 1..S-1 the lines sb H - 4 .. sb H + 3).  k_q1_sor_prep also updates the Dirichlet
-// planes z = 0 and z = M - 1, whose rows couple to nothing.  The row sums b, then the
-// neighbours of planes z - 1 and z + 1, then the in-plane ones, and divide by A_ii.  That is
-// q1_row's arithmetic (linit.lisp:309-318) with the in-plane cell sums taken over cell columns.
-// A row updated here gets r_i = corr and x_i += omega corr, as in k_q1_sor.  b may be r: every
-// row's b is read before its r is written, by the owner or from the copy.
-template <class T>
-__global__ __launch_bounds__(256) void k_q1_sor_prep(int M, int H, int S, FastDiv fM,
-                                                     FastDiv fS1, T omega, T *x, const T *b,
-                                                     T *r, T *gx, T *gb) {
-  const unsigned uM = (unsigned)M, M2 = uM * uM;
-  const unsigned nb = (unsigned)(M - 2) * (unsigned)(S - 1) * 8u * uM;  // boundary lines
-  const unsigned nt = nb + 2u * M2;
-  for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < nt; t += gridDim.x * blockDim.x) {
-    if (t < nb) {
-      unsigned u = fdiv(t, fM);
-      const unsigned xc = t - u * uM, k = u & 7u;
-      u >>= 3;  // (z - 1) (S - 1) + sb - 1
-      const unsigned zq = S > 2 ? fdiv(u, fS1) : u;
-      const int sb = (int)(u - zq * (unsigned)(S - 1)) + 1, z = (int)zq + 1;
-      const int y = sb * H - 4 + (int)k;
-      if (y < 0 || y >= M) continue;
-      // copy index ((z (S - 1) + sb - 1) 8 + k) M + xc, u = (z - 1) (S - 1) + sb - 1
-      const unsigned g = ((u + (unsigned)(S - 1)) * 8u + k) * uM + xc;
-      const unsigned i = ((unsigned)z * uM + (unsigned)y) * uM + xc;
-      gx[g] = x[i];
-      gb[g] = b[i];
-    } else {
-      const unsigned e = t - nb;
-      const unsigned i = (e < M2 ? 0u : (uM - 1u) * M2) + (e < M2 ? e : e - M2);
-      T corr = b[i];
-      corr += (-x[i]) * (T)1;
-      corr = corr / (T)1;
-      r[i] = corr;
-      x[i] += omega * corr;
+// b_i - (the terms of the planes z -+ 1), the cell columns' sums be over those planes.  Every
+// lane of the wave calls it (the shifts read all lanes); Dirichlet values are zeroed, which is
+// what their eliminated columns contribute.
+template <class T, bool OFF0>
+__device__ __forceinline__ T sor_off(const SorCols<T> &C, int M, int z, int y, bool xbd,
+                                     const Q1KT<T> &kt, T (&be)[2][2]) {
+  T acc = C.b;
+#pragma unroll
+  for (int p = 0; p < 2; p++) {
+    T xs[3][3], a[2][2];
+    if (!OFF0) {
+      const bool zbd = p ? z + 1 >= M - 1 : z - 1 <= 0;
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const bool bd = zbd || xbd || (d == 0 ? y - 1 <= 0 : d == 2 && y + 1 >= M - 1);
+        const T v = bd ? (T)0 : C.off[p][d];
+        xs[d][1] = v;
+        xs[d][0] = lane_up(v);
+        xs[d][2] = lane_down(v);
+      }
     }
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      a[q][1] = C.a[p][q];
+      a[q][0] = lane_up(C.a[p][q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        be[q][c] = p ? be[q][c] + a[q][c] : a[q][c];
+        if (!OFF0) {
+          const T s = kt.k[6] * xs[2 * q][1] + kt.k[5] * xs[1][2 * c] +
+                      kt.k[7] * xs[2 * q][2 * c];
+          acc -= a[q][c] * s;
+        }
+      }
+  }
+  return acc;
+}
+
+// the correction (b_i - sum_j A_ij x_j) / A_ii from sor_off's sum and the in-plane corners cn
+template <class T>
+__device__ __forceinline__ T sor_corr(T acc, T xi, const T (&be)[2][2], const T (&cn)[2][2],
+                                      const Q1KT<T> &kt) {
+  const T s = (be[0][0] * cn[0][0] + be[0][1] * cn[0][1]) +
+              (be[1][0] * cn[1][0] + be[1][1] * cn[1][1]);
+  const T d = kt.k[0] * ((be[0][0] + be[0][1]) + (be[1][0] + be[1][1]));
+  return (acc - kt.k[3] * s - d * xi) / d;
+}
+
+// the corners' values from the line columns of sor_load
+template <class T>
+__device__ __forceinline__ void sor_corners(const SorCols<T> &C, int M, int y, bool xbd,
+                                            T (&cn)[2][2]) {
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const T v = xbd || (q ? y + 1 >= M - 1 : y - 1 <= 0) ? (T)0 : C.in[q];
+    cn[q][0] = lane_up(v);
+    cn[q][1] = lane_down(v);
+  }
+}
+
+// One step of a sweep in place: the rows of parity (cz, cy).  b may be r: a row's b is read
+// before its r is written.  ZERO: the sweep starts from x = 0, which is not read (OFF0, IN0: as
+// in sor_load, for the sweep's first two steps and its first and third).
+template <class T, bool OFF0, bool IN0, bool ZERO>
+__global__ __launch_bounds__(256) void k_q1_sor_lines(int M, int n, int cz, int cy, int nyl,
+                                                      unsigned total, FastDiv fM, Div1 fny,
+                                                      const T *__restrict__ alpha, Q1KT<T> kt,
+                                                      T omega, T *x, const T *b, T *r) {
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int lane = threadIdx.x & 63;
+  const unsigned tw = (lb * 4 + (threadIdx.x >> 6)) * 62 + (unsigned)lane;  // position + 1
+  const unsigned t = tw == 0 ? 0u : min(tw - 1, total - 1);
+  const unsigned line = fdiv(t, fM), zi = fdiv(line, fny);
+  const int xc = (int)(t - line * (unsigned)M);
+  const int z = cz + 2 * (int)zi, y = cy + 2 * (int)(line - zi * (unsigned)nyl);
+  SorCols<T> C;
+  sor_load<T, OFF0, IN0, ZERO>(C, M, n, z, y, xc, alpha, x, x, b);
+  const bool xbd = xc == 0 || xc == M - 1;
+  T be[2][2], cn[2][2] = {};
+  const T acc = sor_off<T, OFF0>(C, M, z, y, xbd, kt, be);
+  if (!IN0) sor_corners<T>(C, M, y, xbd, cn);
+  if (lane < 1 || lane > 62 || tw > total) return;
+  const bool bd = xbd || y == 0 || y == M - 1 || z == 0 || z == M - 1;
+  const T corr = bd ? C.b - C.xi : sor_corr<T>(acc, C.xi, be, cn, kt);
+  const unsigned i = ((unsigned)z * (unsigned)M + (unsigned)y) * (unsigned)M + (unsigned)xc;
+  if (r) r[i] = corr;
+  x[i] = C.xi + omega * corr;
+}
+
+// Two steps of a sweep in one launch, out of place: the planes of one z parity, first the lines
+// of y parity ap, then the others.  xs is x before the sweep, xoff x on the other planes (xs in
+// the first launch, xd in the second), xd gets the new values.  A block owns the lines
+// [y0, y0 + H) of a plane; the first step is also done for the line on either side that the
+// second step reads, from the same values with the same arithmetic as by the block that owns
+// it, and reaches the second step through LDS.  b must not be r.
+template <class T, bool OFF0, bool ZERO>
+__global__ __launch_bounds__(256) void k_q1_sor_planes(int M, int n, int pz, int ap, int H,
+                                                       int S, int planes, FastDiv fM,
+                                                       const T *__restrict__ alpha, Q1KT<T> kt,
+                                                       T omega, const T *__restrict__ xs,
+                                                       const T *xoff, T *xd,
+                                                       const T *__restrict__ b, T *r) {
+  extern __shared__ char sor_lds[];
+  T *la = (T *)sor_lds;  // the first step's lines, Dirichlet values 0
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int zi = (int)(lb / (unsigned)S), s = (int)(lb - (unsigned)(zi * S));
+  if (zi >= planes) return;  // the grid's padding (whole blocks)
+  const int z = pz + 2 * zi, y0 = s * H, y1 = min(M, y0 + H);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool zbd = z == 0 || z == M - 1;
+  int a0 = max(0, y0 - 1);
+  a0 += (a0 ^ ap) & 1;
+  const int a1 = min(M - 1, y1), na = a1 >= a0 ? ((a1 - a0) / 2 + 1) * M : 0;
+  const int b0 = y0 + ((y0 ^ ap ^ 1) & 1), nb = b0 < y1 ? ((y1 - 1 - b0) / 2 + 1) * M : 0;
+  for (int c0 = wave * 62; c0 < na; c0 += 4 * 62) {
+    const int e = c0 + lane - 1, ec = min(max(e, 0), na - 1);
+    const int l = (int)fdiv((unsigned)ec, fM), xc = ec - l * M, y = a0 + 2 * l;
+    SorCols<T> C;
+    sor_load<T, OFF0, ZERO, ZERO>(C, M, n, z, y, xc, alpha, xoff, xs, b);
+    const bool xbd = xc == 0 || xc == M - 1;
+    T be[2][2], cn[2][2] = {};
+    const T acc = sor_off<T, OFF0>(C, M, z, y, xbd, kt, be);
+    if (!ZERO) sor_corners<T>(C, M, y, xbd, cn);
+    const bool bd = zbd || xbd || y == 0 || y == M - 1;
+    const T corr = bd ? C.b - C.xi : sor_corr<T>(acc, C.xi, be, cn, kt);
+    const T xn = C.xi + omega * corr;
+    if (lane >= 1 && lane <= 62 && e < na) {
+      la[e] = bd ? (T)0 : xn;
+      if (y >= y0 && y < y1) {
+        const unsigned i = ((unsigned)z * (unsigned)M + (unsigned)y) * (unsigned)M + (unsigned)xc;
+        xd[i] = xn;
+        if (r) r[i] = corr;
+      }
+    }
+  }
+  // the second step's loads are issued before the wait for the first step's lines
+  SorCols<T> C;
+  int c0 = wave * 62, e, l, xc;
+  auto place = [&] {
+    e = c0 + lane - 1;
+    const int ec = min(max(e, 0), nb - 1);
+    l = (int)fdiv((unsigned)ec, fM);
+    xc = ec - l * M;
+    sor_load<T, OFF0, true, ZERO>(C, M, n, z, b0 + 2 * l, xc, alpha, xoff, xs, b);
+  };
+  if (c0 < nb) place();
+  __syncthreads();
+  for (; c0 < nb;) {
+    const int y = b0 + 2 * l;
+    const bool xbd = xc == 0 || xc == M - 1;
+    T be[2][2];
+    const T acc = sor_off<T, OFF0>(C, M, z, y, xbd, kt, be);
+    if (lane >= 1 && lane <= 62 && e < nb) {
+      T corr = C.b - C.xi;
+      if (!(zbd || xbd || y == 0 || y == M - 1)) {
+        const T *up = la + ((y - 1 - a0) >> 1) * M + xc;
+        const T cn[2][2] = {{up[-1], up[1]}, {up[M - 1], up[M + 1]}};
+        corr = sor_corr<T>(acc, C.xi, be, cn, kt);
+      }
+      const unsigned i = ((unsigned)z * (unsigned)M + (unsigned)y) * (unsigned)M + (unsigned)xc;
+      xd[i] = C.xi + omega * corr;
+      if (r) r[i] = corr;
+    }
+    c0 += 4 * 62;
+    if (c0 < nb) place();
+  }
+}
+
+// All sweeps of a smoothing step on a lattice of at most 10^3 nodes by one block, a row per
+// thread (its cells, b and x in registers, x of the others in LDS).  Threads are laid out by the
+// rows' (z, y) parity, each parity starting a wave.  rmode 1: r = the last corrections, 2: r =
+// the residual after the sweeps, 0: r is not written.  Two sweeps of 9^3 nodes and the residual
+// take 4.7 us, by launches they took 32: the steps' chains of LDS reads bound it, not the rows.
+template <class T>
+__global__ __launch_bounds__(1024) void k_q1_sor_small(int M, int n, int steps, int backwards,
+                                                       int rmode, int zero,
+                                                       const T *__restrict__ alpha, Q1KT<T> kt,
+                                                       T omega, T *x, const T *b, T *r) {
+  __shared__ T xs[1000];
+  int cls = 0, t = (int)threadIdx.x, cnt = 0;
+  for (; cls < 4; cls++) {
+    cnt = ((M - (cls >> 1) + 1) / 2) * ((M - (cls & 1) + 1) / 2) * M;
+    const int pad = (cnt + 63) & ~63;
+    if (t < pad) break;
+    t -= pad;
+  }
+  const bool row = cls < 4 && t < cnt;
+  const int nyl = (M - (cls & 1) + 1) / 2;
+  const int line = row ? t / M : 0, xc = row ? t - line * M : 0;
+  const int zi = row ? line / nyl : 0;
+  const int z = (cls >> 1) + 2 * zi, y = (cls & 1) + 2 * (line - zi * nyl);
+  const int i = (z * M + y) * M + xc;
+  const bool in = row && xc > 0 && xc < M - 1 && y > 0 && y < M - 1 && z > 0 && z < M - 1;
+  T a[2][2][2] = {}, bi = (T)0, xi = (T)0, d = (T)1, corr = (T)0;
+  if (row) {
+    bi = b[i];
+    if (!zero) xi = x[i];
+    xs[i] = in ? xi : (T)0;  // the eliminated columns
+  }
+  if (in) {
+    T s = (T)0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int p = k >> 2, q = (k >> 1) & 1, c = k & 1;
+      a[p][q][c] = alpha[((z - 1 + p) * n + y - 1 + q) * n + xc - 1 + c];
+      s += a[p][q][c];
+    }
+    d = kt.k[0] * s;
+  }
+  const int M2 = M * M;
+  auto sum = [&] {  // b_i minus the neighbours' terms
+    T acc = bi, s3 = (T)0;
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+      const T *v = xs + i + (p ? M2 : -M2);
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          const int dy = q ? M : -M, dx = c ? 1 : -1;
+          acc -= a[p][q][c] * (kt.k[6] * v[dy] + kt.k[5] * v[dx] + kt.k[7] * v[dy + dx]);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+      for (int c = 0; c < 2; c++)
+        s3 += (a[0][q][c] + a[1][q][c]) * xs[i + (q ? M : -M) + (c ? 1 : -1)];
+    return acc - kt.k[3] * s3;
+  };
+  __syncthreads();
+  for (int k = 0; k < 4 * steps; k++) {
+    if (row && cls == (backwards ? 3 - (k & 3) : (k & 3))) {
+      corr = in ? (sum() - d * xi) / d : bi - xi;
+      xi += omega * corr;
+      if (in) xs[i] = xi;
+    }
+    __syncthreads();
+  }
+  if (row) {
+    x[i] = xi;
+    if (rmode == 1) r[i] = corr;
+    else if (rmode == 2) r[i] = in ? sum() - d * xi : bi - xi;
   }
 }
 
 constexpr int kSorBatch = 6;  // staged elements per thread and load batch
-
-// Index arithmetic is 32-bit (the lattice has fewer than 2^31 nodes) and divides by the
-// lattice widths through FastDiv (fM: M, fn: n, fx0 / fx1: the colour columns (M + 1) / 2 and
-// M / 2, 0 when that width is 1): a runtime integer division costs tens of VALU instructions,
-// and the kernel is bound by VALU issue.
-template <class T, int CAP>
-__global__ __launch_bounds__(1024) void k_q1_sor_strips(int M, int n, int pz, int H, int S,
-                                                        int backwards, FastDiv fM, FastDiv fn,
-                                                        FastDiv fx0, FastDiv fx1,
-                                                        const T *__restrict__ alpha, Q1K kt,
-                                                        T omega, T *__restrict__ x, const T *b,
-                                                        T *r, const T *__restrict__ gx,
-                                                        const T *__restrict__ gb) {
-  __shared__ T lds[CAP];
-  T *xs = lds;                   // x of plane z, line y0 - 4 + l
-  T *ps = xs + (H + 8) * M;      // b plus the off-plane terms, line y0 - 3 + l
-  T *bs = ps + (H + 6) * M;      // alpha(z - 1) + alpha(z) per cell column, cell line y0 - 4 + l
-  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
-  const int s = (int)(lb % S);
-  const int z = (pz == 0 ? 2 : 1) + 2 * (int)(lb / S);
-  if (z > M - 2) return;  // the grid's padding (whole blocks)
-  const int y0 = s * H, y1 = min(M, y0 + H);
-  const unsigned uM = (unsigned)M, un = (unsigned)n, M2 = uM * uM;
-  const unsigned zb = (unsigned)z * M2;                    // plane z
-  const unsigned cb0 = (unsigned)(z - 1) * un * un, cb1 = (unsigned)z * un * un;  // cell planes
-  // the copies of boundary s (lines y0 - 4 ..) and s + 1 (lines y1 - 4 ..); only read where
-  // that boundary exists
-  const unsigned ol = (unsigned)(z * (S - 1) + s - 1) * 8u * uM, ou = ol + 8u * uM;
-  // Staging is a chain of global loads; every thread issues its loads of x and of the cell
-  // columns for kSorBatch elements before it stores any, and the off-plane terms of two rows
-  // at a time, so that a block waits for a few memory latencies instead of one per element.
-  const int nxs = (H + 8) * M, nbs = (H + 7) * n;
-  for (int e0 = threadIdx.x; e0 < max(nxs, nbs); e0 += kSorBatch * blockDim.x) {
-    T xv[kSorBatch], bv[kSorBatch];
-#pragma unroll
-    for (int u = 0; u < kSorBatch; u++) {
-      const int e = e0 + u * blockDim.x;
-      xv[u] = (T)0;
-      bv[u] = (T)0;
-      if (e < nxs) {
-        const int l = (int)fdiv((unsigned)e, fM), xc = e - l * M, y = y0 - 4 + l;
-        if (y >= 0 && y < M) {
-          if (y < y0) xv[u] = gx[ol + (unsigned)((y - y0 + 4) * M + xc)];
-          else if (y >= y1) xv[u] = gx[ou + (unsigned)((y - y1 + 4) * M + xc)];
-          else xv[u] = x[zb + (unsigned)(y * M + xc)];
-        }
-      }
-      if (e < nbs) {
-        const int l = (int)fdiv((unsigned)e, fn), xc = e - l * n, yc = y0 - 4 + l;
-        if (yc >= 0 && yc < n) {
-          const unsigned o = (unsigned)(yc * n + xc);
-          bv[u] = alpha[cb0 + o] + alpha[cb1 + o];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kSorBatch; u++) {
-      const int e = e0 + u * blockDim.x;
-      if (e < nxs) xs[e] = xv[u];
-      if (e < nbs) bs[e] = bv[u];
-    }
-  }
-  // The off-plane terms: a wave takes 62 consecutive positions of the lines [y0 - 3, y1 + 3)
-  // (lanes 1..62; lanes 0 and 63 only load), each lane loading the x column and the cell
-  // column of its own position and taking the x - 1 / x + 1 columns from its neighbouring
-  // lanes (DPP shifts): 11 loads per row instead of 27.  A row's x - 1 and x + 1 are on its
-  // own line (a line ends only at a Dirichlet row, which reads none).  Every lane of a wave
-  // runs every iteration (the shifts read all lanes); loads are clamped into the lattice.
-  const bool lz[2] = {z - 1 != 0, z + 1 != M - 1};
-  const int nps = (H + 6) * M;
-  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-  for (int c0 = (threadIdx.x >> 6) * 62; c0 < nps; c0 += nw * 62) {
-    const int e = c0 + lane - 1;
-    const int ec = min(max(e, 0), nps - 1);
-    const int l = (int)fdiv((unsigned)ec, fM), xc = ec - l * M, y = y0 - 3 + l;
-    const int yl = min(max(y, 0), M - 1), xcc = min(xc, n - 1);
-    T xcol[2][3], acol[2][2];
-#pragma unroll
-    for (int p = 0; p < 2; p++) {
-#pragma unroll
-      for (int d = 0; d < 3; d++) {
-        const int yy = min(max(yl + d - 1, 0), M - 1);
-        xcol[p][d] = x[(p ? zb + M2 : zb - M2) + (unsigned)(yy * M + xc)];
-      }
-#pragma unroll
-      for (int q = 0; q < 2; q++) {
-        const int yc = min(max(yl - 1 + q, 0), n - 1);
-        acol[p][q] = alpha[(p ? cb1 : cb0) + (unsigned)(yc * n + xcc)];
-      }
-    }
-    const bool row = lane >= 1 && lane <= 62 && e < nps && y >= 0 && y < M;
-    T acc = (T)0;
-    if (row) {
-      const unsigned i = zb + (unsigned)(y * M + xc);
-      if (y < y0) acc = gb[ol + (unsigned)((y - y0 + 4) * M + xc)];
-      else if (y >= y1) acc = gb[ou + (unsigned)((y - y1 + 4) * M + xc)];
-      else acc = b[i];
-    }
-    T xn[2][3][3], a[2][2][2];
-#pragma unroll
-    for (int p = 0; p < 2; p++) {
-#pragma unroll
-      for (int d = 0; d < 3; d++) {
-        xn[p][d][1] = xcol[p][d];
-        xn[p][d][0] = lane_up(xcol[p][d]);
-        xn[p][d][2] = lane_down(xcol[p][d]);
-      }
-#pragma unroll
-      for (int q = 0; q < 2; q++) {
-        a[p][q][1] = acol[p][q];
-        a[p][q][0] = lane_up(acol[p][q]);
-      }
-    }
-    if (row && y != 0 && y != M - 1 && xc != 0 && xc != M - 1) {
-      const bool ly[3] = {y - 1 != 0, true, y + 1 != M - 1};
-      const bool lx[3] = {xc - 1 != 0, true, xc + 1 != M - 1};
-#pragma unroll
-      for (int p = 0; p < 2; p++)
-#pragma unroll
-        for (int k = 0; k < 9; k++) {
-          const int dy = k / 3 - 1, dx = k % 3 - 1;
-          const int q0 = dy > 0 ? 1 : 0, q1 = dy < 0 ? 0 : 1;
-          const int c0c = dx > 0 ? 1 : 0, c1c = dx < 0 ? 0 : 1;
-          T sum = (T)0;
-#pragma unroll
-          for (int q = q0; q <= q1; q++)
-#pragma unroll
-            for (int c = c0c; c <= c1c; c++) sum += a[p][q][c];
-          if (q1_axis<T>(1, dy, dx)) continue;
-          const T aij = (T)kt.k[4 + (dy != 0) * 2 + (dx != 0)] * sum;
-          const bool live = lz[p] && ly[dy + 1] && lx[dx + 1];
-          acc += ((T)-1 * xn[p][dy + 1][dx + 1]) * (live ? aij : (T)0);
-        }
-    }
-    if (row) ps[e] = acc;
-  }
-  __syncthreads();
-  for (int j = 0; j < 4; j++) {
-    const int c = backwards ? 3 - j : j;
-    const int cy = c >> 1, cx = c & 1;
-    int lo = max(0, y0 - (3 - j));
-    const int hi = min(M, y1 + (3 - j));
-    lo += (lo - cy) & 1;  // the first line of parity cy
-    const int nyl = hi > lo ? (hi - lo + 1) / 2 : 0, nxl = (M - cx + 1) / 2;
-    const FastDiv fx = cx ? fx1 : fx0;
-    for (int e = threadIdx.x; e < nyl * nxl; e += blockDim.x) {
-      const int ey = nxl > 1 ? (int)fdiv((unsigned)e, fx) : e;
-      const int y = lo + 2 * ey, xc = cx + 2 * (e - ey * nxl);
-      const int li = (y - y0 + 4) * M + xc;
-      const T xi = xs[li];
-      T acc = ps[(y - y0 + 3) * M + xc];
-      T d = (T)1;
-      if (y == 0 || y == M - 1 || xc == 0 || xc == M - 1) {
-        acc += (-xi) * (T)1;
-      } else {
-        const T *bc = bs + (y - y0 + 3) * n + (xc - 1);  // cell column (y - 1, xc - 1)
-        const T be[2][2] = {{bc[0], bc[1]}, {bc[n], bc[n + 1]}};
-        const bool ly[3] = {y - 1 != 0, true, y + 1 != M - 1};
-        const bool lx[3] = {xc - 1 != 0, true, xc + 1 != M - 1};
-#pragma unroll
-        for (int k = 0; k < 9; k++) {
-          const int dy = k / 3 - 1, dx = k % 3 - 1;
-          const int q0 = dy > 0 ? 1 : 0, q1 = dy < 0 ? 0 : 1;
-          const int c0 = dx > 0 ? 1 : 0, c1 = dx < 0 ? 0 : 1;
-          T sum = (T)0;
-#pragma unroll
-          for (int q = q0; q <= q1; q++)
-#pragma unroll
-            for (int cc = c0; cc <= c1; cc++) sum += be[q][cc];
-          if (q1_axis<T>(0, dy, dx)) continue;
-          const T aij = (T)kt.k[(dy != 0) * 2 + (dx != 0)] * sum;
-          if (k == 4) d = aij;
-          const bool live = ly[dy + 1] && lx[dx + 1];
-          acc += ((T)-1 * xs[live ? li + dy * M + dx : li]) * (live ? aij : (T)0);
-        }
-      }
-      const T corr = acc / d;
-      const T xnew = xi + omega * corr;
-      xs[li] = xnew;
-      if (y >= y0 && y < y1) {
-        const unsigned i = zb + (unsigned)(y * M + xc);
-        r[i] = corr;
-        x[i] = xnew;
-      }
-    }
-    __syncthreads();
-  }
-}
 
 // ---- 3D Q1 lattice matrices in 27-point stencil storage ------------------------------
 
@@ -1390,11 +1373,16 @@ __global__ __launch_bounds__(256) void k_st27_sor(int M, int cz, int cy, int cx,
 }
 
 // ---- the stencil-form <sor> sweep in plane strips --------------------------------------------
-// The decomposition of k_q1_sor_strips for matrices in 27-point stencil storage: one launch per
-// z parity sweeps the four in-plane colours of its planes (all of them, the boundary planes
-// included, since a stencil row is swept like any other), a block owns the whole lines
-// [y0, y1) of one plane and recomputes colour j on 3 - j lines beyond them, and the lines of a
-// neighbouring strip are read from the copies k_st27_sor_prep takes before the sweep.  Each row
+// Colours 0-3 lie on the even z planes, 4-7 on the odd ones, and a row couples to the other z
+// parity only through the planes z - 1 and z + 1, which no row of its own parity changes.  So
+// one launch sweeps the four in-plane colours of one parity's planes, with a barrier between
+// them.  A block owns the whole lines [y0, y1) of one plane.  Colour j of the four needs the
+// in-plane values of the colours before it one line away, so the block computes it on 3 - j
+// lines beyond its own on each side, from the same values with the same arithmetic as the block
+// owning those lines.  The owner overwrites those lines in the same launch, so a block reads
+// them from a copy that k_st27_sor_prep takes before the sweep (gx, gb: for every plane z and
+// strip boundary sb = 1..S-1 the lines sb H - 4 .. sb H + 3).  b may be r: every row's b is read
+// before its r is written, by the owner or from the copy.  Each row
 // is st27_row's sum in its order: b, then the terms k = 0..8 (plane z - 1), 9..17 (plane z),
 // 18..26 (plane z + 1), then the division by the diagonal entry.  The planes z - 1 and z + 1
 // have the other parity and do not change during the launch, so the first nine terms are
@@ -1645,12 +1633,6 @@ void drop_stencil(flgpu_mat *A) {
   A->val27 = nullptr;
   A->st_sym = false;
   drop_sor_strips(A);
-}
-
-static Q1K q1k(const flgpu_mat *A) {
-  Q1K k;
-  for (int j = 0; j < 8; j++) k.k[j] = A->kt[j];
-  return k;
 }
 
 // ---- 3D order-1 lattice interpolation with the pattern implied ------------------------------
@@ -2576,9 +2558,7 @@ __global__ void k_row_span(int nsub, const int *__restrict__ rows, const int *__
 constexpr int kSorCapF64 = 16384, kSorCapF32 = 16384;
 
 // values the strip sweep stages for strips of H lines on an M^3 lattice
-static long sor_strip_lds(int M, int H) {
-  return (long)(H + 8) * M + (long)(H + 6) * M + (long)(H + 7) * (M - 1);
-}
+static long sor_strip_lds(int M, int H) { return (long)(2 * H + 14) * M; }
 
 void sor_strips_alloc(flgpu_mat *A) {
   dev_free(A->sor_ghost);
@@ -2587,8 +2567,7 @@ void sor_strips_alloc(flgpu_mat *A) {
   const int M = A->lat_n + 1;
   if (A->lat_dim != 3 || A->lat_order != 1 || M < 3) return;
   const long cap = A->prec == FLGPU_F64 ? kSorCapF64 : kSorCapF32;
-  // about one block per CU and launch, strips of at least 8 lines, within the LDS (two blocks
-  // per CU in FP32 with strips half as high measured slower: 63 against 48 us at 129^3)
+  // about one block per CU and launch, strips of at least 8 lines, within the LDS
   const int planes = (M - 1) / 2;
   int S = std::max(1, std::min((256 + planes - 1) / planes, (M + 7) / 8));
   while (S <= M && sor_strip_lds(M, (M + S - 1) / S) > cap) S++;
@@ -2601,37 +2580,104 @@ void sor_strips_alloc(flgpu_mat *A) {
     A->sor_ghost = dev_alloc(prec_bytes(A->prec) * 2 * (size_t)M * (S - 1) * 8 * M);
 }
 
-template <class T, int CAP>
-static void q1_sor_strips(const flgpu_mat *A, T omega, int backwards, T *x, const T *b, T *r) {
-  const int M = A->lat_n + 1, S = A->sor_strips, H = A->sor_h;
-  FLGPU_REQUIRE(sor_strip_lds(M, H) <= CAP, "strip sweep: LDS size");
-  T *gx = (T *)A->sor_ghost, *gb = gx ? gx + (long)M * (S - 1) * 8 * M : nullptr;
-  const long prep = (long)(M - 2) * (S - 1) * 8 * M + 2L * M * M;
-  const FastDiv fS1 = S > 2 ? fast_div((unsigned)(S - 1)) : FastDiv{1, 0, 0};
-  k_q1_sor_prep<T><<<grid_for(prep, 256), 256, 0, A->ctx->stream>>>(
-      M, H, S, fast_div((unsigned)M), fS1, omega, x, b, r, gx, gb);
-  FLGPU_HIP(hipGetLastError());
-  for (int k = 0; k < 2; k++) {
-    const int pz = backwards ? 1 - k : k;
-    const int z0 = pz == 0 ? 2 : 1;
-    if (z0 > M - 2) continue;
-    const int planes = (M - 2 - z0) / 2 + 1;
-    const unsigned g = xcd_grid((unsigned)(planes * S));
-    const FastDiv fx1 = M / 2 > 1 ? fast_div((unsigned)(M / 2)) : FastDiv{1, 0, 0};
-    k_q1_sor_strips<T, CAP><<<g, 1024, 0, A->ctx->stream>>>(
-        M, A->lat_n, pz, H, S, backwards, fast_div((unsigned)M), fast_div((unsigned)A->lat_n),
-        fast_div((unsigned)((M + 1) / 2)), fx1, (const T *)A->alpha, q1k(A), omega, x, b, r, gx,
-        gb);
-    FLGPU_HIP(hipGetLastError());
+// lines of a block of k_q1_sor_planes
+constexpr int kSorLines = 8;
+// lattices of at most 65^3 nodes sweep out of place where a spare vector is there: a launch costs
+// 2.3 us at least, so two of 3.8 us beat four at 17^3 and 33^3 (7.6 against 11 us FP64), they are
+// equal at 65^3, and at 129^3 the halo lines and LDS cost more than the launches (33 against 29)
+constexpr int kSorOutplaceM = 65;
+
+bool sor_outplace(const flgpu_mat *A) { return A->alpha && A->lat_n < kSorOutplaceM; }
+
+template <class T>
+static Q1KT<T> q1kt(const flgpu_mat *A) {
+  Q1KT<T> k;
+  for (int j = 0; j < 8; j++) k.k[j] = (T)A->kt[j];
+  return k;
+}
+
+// a sweep in place, four launches
+template <class T>
+static void q1_sor_inplace(const flgpu_mat *A, T omega, int backwards, T *x, const T *b, T *r,
+                           bool zero) {
+  const int M = A->lat_n + 1;
+  const Q1KT<T> kt = q1kt<T>(A);
+  for (int k = 0; k < 4; k++) {
+    const int cz = backwards ? 1 - (k >> 1) : k >> 1, cy = backwards ? 1 - (k & 1) : k & 1;
+    const int nzl = (M - cz + 1) / 2, nyl = (M - cy + 1) / 2;
+    const unsigned total = (unsigned)nzl * (unsigned)nyl * (unsigned)M;
+    const unsigned g = xcd_grid((total + 4 * 62 - 1) / (4 * 62));
+    auto launch = [&](auto kern) {
+      kern<<<g, 256, 0, A->ctx->stream>>>(M, A->lat_n, cz, cy, nyl, total, fast_div((unsigned)M),
+                                          div1((unsigned)nyl), (const T *)A->alpha, kt, omega, x,
+                                          b, r);
+      FLGPU_HIP(hipGetLastError());
+    };
+    if (!zero) launch(k_q1_sor_lines<T, false, false, false>);
+    else if (k == 0) launch(k_q1_sor_lines<T, true, true, true>);
+    else if (k == 1) launch(k_q1_sor_lines<T, true, false, true>);
+    else if (k == 2) launch(k_q1_sor_lines<T, false, true, true>);
+    else launch(k_q1_sor_lines<T, false, false, true>);
   }
 }
 
+// a sweep from xs into xd, two launches
+template <class T>
+static void q1_sor_outplace(const flgpu_mat *A, T omega, int backwards, const T *xs, T *xd,
+                            const T *b, T *r, bool zero) {
+  const int M = A->lat_n + 1, H = kSorLines, S = (M + H - 1) / H;
+  const Q1KT<T> kt = q1kt<T>(A);
+  const size_t lds = sizeof(T) * (size_t)(H / 2 + 1) * M;
+  for (int k = 0; k < 2; k++) {
+    const int pz = backwards ? 1 - k : k, planes = (M - 1 - pz) / 2 + 1;
+    const unsigned g = xcd_grid((unsigned)planes * (unsigned)S);
+    auto launch = [&](auto kern) {
+      kern<<<g, 256, lds, A->ctx->stream>>>(M, A->lat_n, pz, backwards ? 1 : 0, H, S, planes,
+                                            fast_div((unsigned)M), (const T *)A->alpha, kt,
+                                            omega, xs, k == 0 ? xs : xd, xd, b, r);
+      FLGPU_HIP(hipGetLastError());
+    };
+    if (!zero) launch(k_q1_sor_planes<T, false, false>);
+    else if (k == 0) launch(k_q1_sor_planes<T, true, true>);
+    else launch(k_q1_sor_planes<T, false, true>);
+  }
+}
+
+// `steps` sweeps of the per-cell form; true when r holds the residual (rmode 2)
+template <class T>
+static bool q1_sor(const flgpu_mat *A, T omega, int steps, int backwards, T *x, const T *b, T *r,
+                   T *tmp, bool zero, int rmode) {
+  const int M = A->lat_n + 1;
+  if (b == r) rmode = 1;
+  if (M <= 10) {
+    const int per = b == r ? 1 : steps;  // each sweep reads the last one's r
+    for (int k = 0; k < steps; k += per, zero = false) {
+      k_q1_sor_small<T><<<1, 1024, 0, A->ctx->stream>>>(M, A->lat_n, per, backwards, rmode, zero,
+                                                        (const T *)A->alpha, q1kt<T>(A), omega,
+                                                        x, b, r);
+      FLGPU_HIP(hipGetLastError());
+    }
+    return rmode == 2;
+  }
+  int k = 0;
+  if (tmp && b != r && sor_outplace(A))
+    for (; k + 2 <= steps; k += 2, zero = false) {
+      q1_sor_outplace<T>(A, omega, backwards, x, tmp, b, nullptr, zero);
+      q1_sor_outplace<T>(A, omega, backwards, tmp, x, b, k + 2 == steps && rmode == 1 ? r : nullptr,
+                         false);
+    }
+  for (; k < steps; k++, zero = false)
+    q1_sor_inplace<T>(A, omega, backwards, x, b,
+                      b == r || (k + 1 == steps && rmode == 1) ? r : nullptr, zero);
+  return false;
+}
+
 // the stencil-form sweep in strips: the copies of the strip boundaries of every plane, then one
-// launch per z parity (the same strips as the per-cell sweep, whose LDS need is larger)
+// launch per z parity
 template <class T, int CAP>
 static void st27_sor_strips(const flgpu_mat *A, T omega, int backwards, T *x, const T *b, T *r) {
   const int M = A->lat_n + 1, S = A->sor_strips, H = A->sor_h;
-  FLGPU_REQUIRE((long)(2 * H + 14) * M <= CAP, "strip sweep: LDS size");
+  FLGPU_REQUIRE(sor_strip_lds(M, H) <= CAP, "strip sweep: LDS size");
   FLGPU_REQUIRE(27L * M * M * M < (1L << 32), "strip sweep: lattice too large");
   T *gx = (T *)A->sor_ghost, *gb = gx ? gx + (long)M * (S - 1) * 8 * M : nullptr;
   const FastDiv fM = fast_div((unsigned)M);
@@ -2658,17 +2704,9 @@ static void st27_sor_strips(const flgpu_mat *A, T omega, int backwards, T *x, co
   }
 }
 
-void sor_sweep(const flgpu_mat *A, double omega, int backwards, void *x, const void *b, void *r) {
-  if (A->alpha && A->sor_strips > 0) {
-    if (A->prec == FLGPU_F64)
-      q1_sor_strips<double, kSorCapF64>(A, omega, backwards, (double *)x, (const double *)b,
-                                        (double *)r);
-    else
-      q1_sor_strips<float, kSorCapF32>(A, (float)omega, backwards, (float *)x,
-                                       (const float *)b, (float *)r);
-    return;
-  }
-  if (!A->alpha && A->val27 && A->sor_strips > 0 && 27L * A->nrows < (1L << 32)) {
+static void sor_sweep(const flgpu_mat *A, double omega, int backwards, void *x, const void *b,
+                      void *r) {
+  if (A->val27 && A->sor_strips > 0 && 27L * A->nrows < (1L << 32)) {
     if (A->prec == FLGPU_F64)
       st27_sor_strips<double, kSorCapF64>(A, omega, backwards, (double *)x, (const double *)b,
                                           (double *)r);
@@ -2677,7 +2715,7 @@ void sor_sweep(const flgpu_mat *A, double omega, int backwards, void *x, const v
                                          (const float *)b, (float *)r);
     return;
   }
-  if (A->alpha || A->val27) {
+  if (A->val27) {
     // lattice colours in the order of the lattice colouring: cz*4 + cy*2 + cx
     int M = A->lat_n + 1;
     for (int k = 0; k < 8; k++) {
@@ -2685,33 +2723,22 @@ void sor_sweep(const flgpu_mat *A, double omega, int backwards, void *x, const v
       int cz = c >> 2, cy = (c >> 1) & 1, cx = c & 1;
       long cnt = (long)((M - cx + 1) / 2) * ((M - cy + 1) / 2) * ((M - cz + 1) / 2);
       unsigned g = xcd_grid(grid_for(cnt, 256));
-      if (!A->alpha) {
-        if (A->prec == FLGPU_F64 && A->st_sym)
-          k_st27_sor<double, true><<<g, 256, 0, A->ctx->stream>>>(
-              M, cz, cy, cx, (const double *)A->val27, omega, (double *)x, (const double *)b,
-              (double *)r);
-        else if (A->prec == FLGPU_F64)
-          k_st27_sor<double, false><<<g, 256, 0, A->ctx->stream>>>(
-              M, cz, cy, cx, (const double *)A->val27, omega, (double *)x, (const double *)b,
-              (double *)r);
-        else if (A->st_sym)
-          k_st27_sor<float, true><<<g, 256, 0, A->ctx->stream>>>(
-              M, cz, cy, cx, (const float *)A->val27, (float)omega, (float *)x, (const float *)b,
-              (float *)r);
-        else
-          k_st27_sor<float, false><<<g, 256, 0, A->ctx->stream>>>(
-              M, cz, cy, cx, (const float *)A->val27, (float)omega, (float *)x, (const float *)b,
-              (float *)r);
-      } else if (A->prec == FLGPU_F64)
-        k_q1_sor<double><<<g, 256, 0, A->ctx->stream>>>(M, A->lat_n, cz, cy, cx,
-                                                        (const double *)A->alpha, q1k(A), omega,
-                                                        (double *)x, (const double *)b,
-                                                        (double *)r);
+      if (A->prec == FLGPU_F64 && A->st_sym)
+        k_st27_sor<double, true><<<g, 256, 0, A->ctx->stream>>>(
+            M, cz, cy, cx, (const double *)A->val27, omega, (double *)x, (const double *)b,
+            (double *)r);
+      else if (A->prec == FLGPU_F64)
+        k_st27_sor<double, false><<<g, 256, 0, A->ctx->stream>>>(
+            M, cz, cy, cx, (const double *)A->val27, omega, (double *)x, (const double *)b,
+            (double *)r);
+      else if (A->st_sym)
+        k_st27_sor<float, true><<<g, 256, 0, A->ctx->stream>>>(
+            M, cz, cy, cx, (const float *)A->val27, (float)omega, (float *)x, (const float *)b,
+            (float *)r);
       else
-        k_q1_sor<float><<<g, 256, 0, A->ctx->stream>>>(M, A->lat_n, cz, cy, cx,
-                                                       (const float *)A->alpha, q1k(A),
-                                                       (float)omega, (float *)x, (const float *)b,
-                                                       (float *)r);
+        k_st27_sor<float, false><<<g, 256, 0, A->ctx->stream>>>(
+            M, cz, cy, cx, (const float *)A->val27, (float)omega, (float *)x, (const float *)b,
+            (float *)r);
       FLGPU_HIP(hipGetLastError());
     }
     return;
@@ -2747,9 +2774,18 @@ void sor_sweep(const flgpu_mat *A, double omega, int backwards, void *x, const v
 }
 
 // `steps` <sor> sweeps (the product-iterator of a smoother, linit.lisp:94-120)
-void sor_sweeps(const flgpu_mat *A, double omega, int steps, int backwards, void *x, const void *b,
-                void *r) {
+bool sor_sweeps(const flgpu_mat *A, double omega, int steps, int backwards, void *x, const void *b,
+                void *r, void *tmp, bool x_zero, int rmode) {
+  if (A->alpha) {
+    if (A->prec == FLGPU_F64)
+      return q1_sor<double>(A, omega, steps, backwards, (double *)x, (const double *)b,
+                            (double *)r, (double *)tmp, x_zero, rmode);
+    return q1_sor<float>(A, (float)omega, steps, backwards, (float *)x, (const float *)b,
+                         (float *)r, (float *)tmp, x_zero, rmode);
+  }
+  if (x_zero) vfill(A->ctx, A->nrows, A->prec, x, 0.0);
   for (int k = 0; k < steps; k++) sor_sweep(A, omega, backwards, x, b, r);
+  return false;
 }
 
 // ---- Galerkin product P^T A P (src/iteration/amg.lisp:247-280) ---------------------

@@ -435,3 +435,49 @@ def test_one_pass_q1_assembly_equals_element_gather(prec, mode, nk_factor):
     # the load vector of f = 1 against the oracle
     orp, oci, ov, ob = po.assemble(3, 1, n, kap, 1.0)
     assert relerr(b.numpy(), ob) < (1e-14 if prec == F.F64 else 1e-7)
+
+
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("m,levels,pre,post", [(2, 2, 2, 2), (9, 1, 3, 1), (5, 2, 1, 2),
+                                               (8, 3, 2, 3), (17, 3, 2, 1), (18, 3, 3, 2)])
+def test_cell_sor_cycles_equal_sell_cycles(m, levels, pre, post, prec):
+    """V-cycles whose <sor> steps sweep a level in the per-cell form (one block up to 10^3 nodes,
+    out of place up to 65^3, in place above, from zero on the coarse levels and under a Krylov
+    method, an odd last step) against the same cycles on the SELL matrices: a cycle from a random
+    x, one with rhs and residual one vector, and a solve.  Constant coefficient: every level is
+    per-cell.  Tolerance: a sweep differs by rounding alone (1e-13 and 2e-6 for two), a cycle
+    makes up to 30 of them over three levels and a coarse solve."""
+    say(f"cell sor cycles m={m} levels={levels} V({pre},{post}) prec={prec}")
+    rng = np.random.default_rng(m)
+    n = m * 2 ** (levels - 1)
+    tol = 2e-12 if prec == F.F64 else 4e-5
+    y, c = rng.uniform(-1, 1, (n + 1) ** 3), rng.uniform(-1, 1, (n + 1) ** 3)
+    outs = []
+    for form in (F.STORAGE_CELL, F.STORAGE_SELL):
+        cs = it.GeometricCS(it.SOR(1.1), pre, post, 0, symmetric=True, prec=prec)
+        if levels == 1:  # one smoothed level without a coarse one: the iterate alone
+            A, b = lat.assemble(3, 1, n, prec=prec)
+            assert A.storage(form) == form
+            x = GpuVector.from_array(y, prec)
+            r, bb = GpuVector(A.nrows, prec), GpuVector.from_array(c, prec)
+            for k in range(pre + post):
+                check(lib().flgpu_sor_iterate(A.h, 1.1, k & 1, x.h, bb.h, r.h))
+            outs.append([x.numpy(), r.numpy()])
+            continue
+        H = it.Hierarchy.lattice(cs, 3, 1, m, levels)
+        for l in range(levels):
+            assert H.level_matrix(l).storage(form) == form
+        res = []
+        for alias in (False, True):
+            x, r = GpuVector.from_array(y, prec), GpuVector.from_array(c, prec)
+            b = r if alias else GpuVector.from_array(c, prec)
+            check(lib().flgpu_mg_apply(H.h, x.h, b.h, r.h))
+            res += [x.numpy(), r.numpy()]
+        bb = it.solve(it.LinearSolver(it.FCG(cs), success_if=("<", "reduction", 1e-6),
+                                      failure_if=(">", "step", 50)),
+                      {"matrix": H.top_matrix(), "rhs": H.rhs, "hierarchy": H})
+        assert bb["status"] == "success"
+        res.append(np.array([bb["steps"]], float))
+        outs.append(res)
+    for a, s in zip(*outs):
+        assert relerr(a, s) < tol
