@@ -174,13 +174,10 @@ struct flgpu_mat {
   // by DOFs i and j), d = lattice offset; kernels apply A from alpha
   void *alpha = nullptr;  // n^3 cell factors (prec), nullptr if not available
   double kt[8] = {};      // Kref[0][b], b = bz*4 + by*2 + bx
-  // with val27: the <sor> sweep's strips per plane (0: one launch per colour) and its copy of
-  // x and b around the strip boundaries, 2 (M (S - 1) 8 M) values (prec), nullptr if S < 2
-  int sor_strips = 0, sor_h = 0;
-  void *sor_ghost = nullptr;
   // 3D Q1 lattice matrices otherwise: the 27 values of every row, SoA
   // val27[k][row], k = (dz+1)*9 + (dy+1)*3 + (dx+1); columns are implied
   void *val27 = nullptr;
+  void *sor_work = nullptr;  // with val27: the <sor> sweeps' spare x and copy of b (2 nrows)
   bool st_sym = false;  // val27 exactly symmetric: kernels stream 14 of the 27 planes
   // order-1 3D lattice interpolation from a (tp_nc+1)^3 to a (2 tp_nc+1)^3 lattice with the
   // full trilinear pattern (1: the interpolation, 2: its transpose): products read the CSR
@@ -223,8 +220,6 @@ void drop_alpha(flgpu_mat *A);
 void drop_cells(flgpu_mat *A);  // cell, kref, elem
 // entries of a row of n values padded to 16 bytes
 inline int row_pad(int n, int prec) { return prec == FLGPU_F64 ? (n + 1) & ~1 : (n + 3) & ~3; }
-// the strips and boundary copy of the stencil-form <sor> sweep
-void sor_strips_alloc(flgpu_mat *A);
 void tp_prepare(flgpu_mat *T);  // (re)fill tp27 of an interpolation or its transpose
 void tp_drop(flgpu_mat *A);     // products of A (and its transpose) go back to SELL
 bool is_q1_lattice(const flgpu_mat *A);
@@ -269,6 +264,8 @@ void blocks_prepare(flgpu_mat *A);
 void blocks_drop(flgpu_mat *A);
 void block_sweep(const flgpu_mat *A, bool ssc, double omega, int backwards, void *x,
                  const void *b, void *r, bool cells);
+// allocates the stencil form's sor_work: before its sweeps, outside a capture
+void sor_prepare(const flgpu_mat *A);
 bool sor_outplace(const flgpu_mat *A);  // its sweeps use a spare vector
 // `steps` <sor> sweeps.  tmp (n values): lets the per-cell form sweep out of place; x_zero: x is
 // zero and need not be stored; rmode: 1: r holds the last corrections, 0: r is not wanted, 2: r

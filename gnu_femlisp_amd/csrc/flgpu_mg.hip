@@ -904,6 +904,8 @@ static unsigned long mg_layout(const flgpu_mg *mg) {
 }
 
 static void mg_run_cached(flgpu_mg *mg, int mode, int vprec, void *x, void *b, void *r) {
+  if (mg->p.smoother == FLGPU_SMOOTH_SOR)
+    for (int l = mg->p.base_level + 1; l <= mg->top; l++) sor_prepare(mg->lv[l].A);
   if (!mg->use_graphs) {
     mg_run(mg, mode, vprec, x, b, r);
     return;

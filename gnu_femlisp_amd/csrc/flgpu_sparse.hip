@@ -273,7 +273,6 @@ void mat_finish(flgpu_mat *A) {
   if (is_q1_lattice(A)) {
     A->val27 = dev_alloc(prec_bytes(A->prec) * 27 * (size_t)A->nrows);
     stencil_refresh(A);
-    sor_strips_alloc(A);
   }
 }
 
@@ -291,19 +290,12 @@ void mat_free(flgpu_mat *A) {
   dev_free(A->cell);
   dev_free(A->kref);
   dev_free(A->elem);
-  dev_free(A->sor_ghost);
+  dev_free(A->sor_work);
   dev_free(A->val27);
   dev_free(A->tp27);
   dev_free(A->blk_inv);
   dev_free(A->dot_part);
   delete A;
-}
-
-// the stencil-form <sor> sweeps' boundary copies
-static void drop_sor_strips(flgpu_mat *A) {
-  dev_free(A->sor_ghost);
-  A->sor_ghost = nullptr;
-  A->sor_strips = A->sor_h = 0;
 }
 
 // values no longer follow the per-cell form (new values or another ordering)
@@ -1229,8 +1221,6 @@ __global__ __launch_bounds__(1024) void k_q1_sor_small(int M, int n, int steps, 
   }
 }
 
-constexpr int kSorBatch = 6;  // staged elements per thread and load batch
-
 // ---- 3D Q1 lattice matrices in 27-point stencil storage ------------------------------
 
 // val27[k][i] = A(i, i + off_k) for the CSR entries of row i, 0 elsewhere
@@ -1344,219 +1334,109 @@ __global__ __launch_bounds__(256) void k_st27_spmv(int M, const T *__restrict__ 
   out[i] = st27_row<T, SYM>(M, N, i, zz, yy, xx, val27, acc, coef, x, &d);
 }
 
-// <sor> update of the t-th row of colour (cz, cy, cx): corr = (b_i - sum_j A_ij x_j) / A_ii,
-// r_i = corr, x_i += omega corr
-template <class T, bool SYM>
-__device__ __forceinline__ void st27_sor_row(int M, int cz, int cy, int cx, int nx, int ny,
-                                             long t, const T *__restrict__ val27, T omega, T *x,
-                                             const T *b, T *r) {
-  int xx = 2 * (int)(t % nx) + cx, yy = 2 * (int)((t / nx) % ny) + cy,
-      zz = 2 * (int)(t / ((long)nx * ny)) + cz;
-  long N = (long)M * M * M;
-  long i = ((long)zz * M + yy) * M + xx;
-  T d = (T)1;
-  T corr = st27_row<T, SYM>(M, N, i, zz, yy, xx, val27, b[i], (T)-1, x, &d);
-  corr = corr / d;
-  r[i] = corr;
-  x[i] += omega * corr;
-}
-
-template <class T, bool SYM>
-__global__ __launch_bounds__(256) void k_st27_sor(int M, int cz, int cy, int cx,
-                                                  const T *__restrict__ val27, T omega, T *x,
-                                                  const T *b, T *r) {
-  int nx = (M - cx + 1) / 2, ny = (M - cy + 1) / 2, nz = (M - cz + 1) / 2;
-  unsigned lb = xcd_block(blockIdx.x, gridDim.x);
-  long t = (long)lb * blockDim.x + threadIdx.x;
-  if (t >= (long)nx * ny * nz) return;
-  st27_sor_row<T, SYM>(M, cz, cy, cx, nx, ny, t, val27, omega, x, b, r);
-}
-
-// ---- the stencil-form <sor> sweep in plane strips --------------------------------------------
+// ---- the stencil-form <sor> sweep in tiles ---------------------------------------------------
 // Colours 0-3 lie on the even z planes, 4-7 on the odd ones, and a row couples to the other z
-// parity only through the planes z - 1 and z + 1, which no row of its own parity changes.  So
-// one launch sweeps the four in-plane colours of one parity's planes, with a barrier between
-// them.  A block owns the whole lines [y0, y1) of one plane.  Colour j of the four needs the
-// in-plane values of the colours before it one line away, so the block computes it on 3 - j
-// lines beyond its own on each side, from the same values with the same arithmetic as the block
-// owning those lines.  The owner overwrites those lines in the same launch, so a block reads
-// them from a copy that k_st27_sor_prep takes before the sweep (gx, gb: for every plane z and
-// strip boundary sb = 1..S-1 the lines sb H - 4 .. sb H + 3).  b may be r: every row's b is read
-// before its r is written, by the owner or from the copy.  Each row
-// is st27_row's sum in its order: b, then the terms k = 0..8 (plane z - 1), 9..17 (plane z),
-// 18..26 (plane z + 1), then the division by the diagonal entry.  The planes z - 1 and z + 1
-// have the other parity and do not change during the launch, so the first nine terms are
-// summed for every staged row before the colour phases, and the last nine are loaded from
-// device memory in the row's colour phase.  A term whose neighbour lies outside the lattice
-// takes the row's own x, as st27_row does, which is the staged value: it still holds x_i
-// before the row's update.
-template <class T>
-__global__ __launch_bounds__(256) void k_st27_sor_prep(int M, int H, int S, FastDiv fM,
-                                                       FastDiv fS1, const T *x, const T *b,
-                                                       T *gx, T *gb) {
-  const unsigned uM = (unsigned)M;
-  const unsigned nb = uM * (unsigned)(S - 1) * 8u * uM;  // boundary lines of every plane
-  for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < nb; t += gridDim.x * blockDim.x) {
-    unsigned u = fdiv(t, fM);
-    const unsigned xc = t - u * uM, k = u & 7u;
-    u >>= 3;  // z (S - 1) + sb - 1
-    const unsigned z = S > 2 ? fdiv(u, fS1) : u;
-    const int sb = (int)(u - z * (unsigned)(S - 1)) + 1;
-    const int y = sb * H - 4 + (int)k;
-    if (y < 0 || y >= M) continue;
-    const unsigned g = (u * 8u + k) * uM + xc;  // the layout k_st27_sor_strips reads
-    const unsigned i = (z * uM + (unsigned)y) * uM + xc;
-    gx[g] = x[i];
-    gb[g] = b[i];
-  }
-}
+// parity only through the planes z - 1 and z + 1, which no row of its own parity changes.  So one
+// launch sweeps the four in-plane colours of one parity's planes, out of place (xs before the
+// sweep, xoff x on the other planes: xs in the first launch, xd in the second).  A block owns H
+// lines of W columns of one plane.  Colour j of the four needs the in-plane values of the
+// colours before it one node away, so the block computes it on 3 - j lines and columns beyond
+// its own on each side, from the same values with the same arithmetic as the block owning them,
+// and keeps x of the plane in LDS.  A thread has at most one row of a colour and 4 / G rows (G
+// groups of threads take every G-th colour): before the colour phases it loads their
+// coefficients, sums b and the terms of the planes z - 1 and z + 1 and keeps the nine in-plane
+// coefficients in registers, so that a phase waits for LDS only.  FP32 rows take
+// the three planes' sums and the diagonal term together in FP64 (their terms one by one cost as
+// much again as the loads).  b must not be r.
+// The coefficients' bytes bound it from 65^3 on (27 a row and once more for the rows beyond the
+// tile), their latency below.  A sweep in a cycle, FP64: 17^3 11, 33^3 12, 65^3 22 us; strips of
+// whole lines that loaded each colour's coefficients in its phase, and copies of the strips'
+// edges, took 19, 21 and 42.
+constexpr int kTileCols = 65;
+constexpr int kTileRows(int H) { return ((H + 7) / 2) * ((kTileCols + 7) / 2); }  // of a colour
 
-// rows per thread and load batch of the plane z - 1 terms
-template <class T> constexpr int sor_batch_p() { return sizeof(T) == 8 ? 2 : 4; }
-
-// st27_coef with 32-bit indices (27 N < 2^32) and every load issued (the neighbour's index
-// replaced by the row's own when the neighbour is outside the lattice), the value selected
-// afterwards
-template <class T, bool SYM>
-__device__ __forceinline__ T st27_coef_sel(const T *__restrict__ val27, unsigned N, int k,
-                                           unsigned i, int off, bool live) {
-  if (SYM && k < 13) {
-    const T v = val27[(unsigned)(26 - k) * N + (live ? i + (unsigned)off : i)];
-    return live ? v : (T)0;
-  }
-  return val27[(unsigned)k * N + i];
-}
-
-template <class T, bool SYM, int CAP>
-__global__ __launch_bounds__(1024) void k_st27_sor_strips(int M, int pz, int H, int S,
-                                                          int backwards, FastDiv fM, FastDiv fx0,
-                                                          FastDiv fx1,
-                                                          const T *__restrict__ val27, T omega,
-                                                          T *__restrict__ x, const T *b, T *r,
-                                                          const T *__restrict__ gx,
-                                                          const T *__restrict__ gb) {
-  __shared__ T lds[CAP];
-  T *xs = lds;               // x of plane z, line y0 - 4 + l
-  T *ps = xs + (H + 8) * M;  // b plus the plane z - 1 terms, line y0 - 3 + l
+// OFF0: x is zero on the planes z -+ 1, ZERO: on the plane itself; those are not read.
+template <class T, bool SYM, bool OFF0, bool ZERO, int H, int G>
+__global__ __launch_bounds__((kTileRows(H) + 63) / 64 * 64 * G) void k_st27_sor_tiles(int M, int pz, int W, int ntx, int nty,
+                                                        int planes, int backwards,
+                                                        const T *__restrict__ val27, T omega,
+                                                        const T *__restrict__ xs, const T *xoff,
+                                                        T *xd, const T *__restrict__ b, T *r) {
+  constexpr int LW = kTileCols + 8, P = (kTileRows(H) + 63) / 64 * 64;
+  __shared__ T lx[(H + 8) * LW];  // x of lines y0 - 4.., columns x0 - 4..; 0 outside the lattice
   const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
-  const int s = (int)(lb % S);
-  const int z = pz + 2 * (int)(lb / S);
-  if (z > M - 1) return;  // the grid's padding (whole blocks)
-  const int y0 = s * H, y1 = min(M, y0 + H);
+  const int tx = (int)(lb % (unsigned)ntx), tyz = (int)(lb / (unsigned)ntx);
+  const int ty = tyz % nty, zi = tyz / nty;
+  if (zi >= planes) return;  // the grid's padding (whole blocks)
+  const int z = pz + 2 * zi, y0 = ty * H, y1 = min(M, y0 + H), x0 = tx * W, x1 = min(M, x0 + W);
   const int M2 = M * M;
-  const unsigned N = (unsigned)M2 * (unsigned)M, zb = (unsigned)z * (unsigned)M2;
-  // the copies of boundary s (lines y0 - 4 ..) and s + 1 (lines y1 - 4 ..); only read where
-  // that boundary exists
-  const unsigned ol = (unsigned)(z * (S - 1) + s - 1) * 8u * (unsigned)M, ou = ol + 8u * M;
-  const int nxs = (H + 8) * M;
-  for (int e0 = threadIdx.x; e0 < nxs; e0 += kSorBatch * blockDim.x) {
-    T xv[kSorBatch];
+  const size_t N = (size_t)M2 * (size_t)M;
+  const T *val = val27;  // plane k: val + k N, uniform
+  constexpr int NE = ((H + 8) * LW + P * G - 1) / (P * G);
 #pragma unroll
-    for (int u = 0; u < kSorBatch; u++) {
-      const int e = e0 + u * blockDim.x;
-      xv[u] = (T)0;
-      if (e < nxs) {
-        const int l = (int)fdiv((unsigned)e, fM), xc = e - l * M, y = y0 - 4 + l;
-        if (y >= 0 && y < M) {
-          if (y < y0) xv[u] = gx[ol + (unsigned)((y - y0 + 4) * M + xc)];
-          else if (y >= y1) xv[u] = gx[ou + (unsigned)((y - y1 + 4) * M + xc)];
-          else xv[u] = x[zb + (unsigned)(y * M + xc)];
-        }
-      }
-    }
+  for (int u = 0; u < NE; u++) {
+    const int e = (int)threadIdx.x + u * P * G;
+    const int l = e / LW, y = y0 - 4 + l, x = x0 - 4 + e - l * LW;
+    if (e < (H + 8) * LW)
+      lx[e] = !ZERO && y >= 0 && y < M && x >= 0 && x < M
+                  ? xs[(unsigned)z * (unsigned)M2 + (unsigned)(y * M + x)] : (T)0;
+  }
+  constexpr int R = 4 / G;
+  const int g = (int)threadIdx.x / P, t = (int)threadIdx.x - g * P;
+  double acc[R];
+  T cf[R][9];
+  int li[R];          // the row's place in lx, -1: none
+  unsigned gi[R];     // its index, 0xffffffff: another block's
 #pragma unroll
-    for (int u = 0; u < kSorBatch; u++) {
-      const int e = e0 + u * blockDim.x;
-      if (e < nxs) xs[e] = xv[u];
+  for (int q = 0; q < R; q++) {
+    const int j = g + q * G, c = backwards ? 3 - j : j, cy = c >> 1, cx = c & 1, e = 3 - j;
+    int ya = max(0, y0 - e), xa = max(0, x0 - e);
+    ya += (ya ^ cy) & 1;
+    xa += (xa ^ cx) & 1;
+    const int ny = (min(M, y1 + e) - ya + 1) >> 1, nx = (min(M, x1 + e) - xa + 1) >> 1;
+    const int ey = nx > 0 ? t / nx : 0;
+    const int y = ya + 2 * ey, x = xa + 2 * (t - ey * nx);
+    li[q] = -1;
+    gi[q] = 0xffffffffu;
+    acc[q] = 0.0;
+    if (nx <= 0 || ey >= ny) continue;
+    li[q] = (y - y0 + 4) * LW + x - x0 + 4;
+    const unsigned i = (unsigned)z * (unsigned)M2 + (unsigned)(y * M + x);
+    if (y >= y0 && y < y1 && x >= x0 && x < x1) gi[q] = i;
+    const bool lz[3] = {z > 0, true, z < M - 1}, ly[3] = {y > 0, true, y < M - 1},
+               lxx[3] = {x > 0, true, x < M - 1};
+    const T bi = b[i];
+    T sd[2] = {};  // the planes' sums
+#pragma unroll
+    for (int k = 0; k < 27; k++) {
+      const int dz = k / 9 - 1, dy = (k / 3) % 3 - 1, dx = k % 3 - 1;
+      if (OFF0 && dz != 0) continue;
+      const bool live = lz[dz + 1] && ly[dy + 1] && lxx[dx + 1];
+      const unsigned in = live ? i + (unsigned)(dz * M2 + dy * M + dx) : i;
+      T v = SYM && k < 13 ? (val + (size_t)(26 - k) * N)[in] : (val + (size_t)k * N)[i];
+      if (SYM && k < 13) v = live ? v : (T)0;
+      if (dz == 0) cf[q][k - 9] = v;
+      else sd[dz > 0] += (live ? xoff[in] : (T)0) * v;
     }
+    acc[q] = ((double)bi - (double)sd[0]) - (double)sd[1];
   }
   __syncthreads();
-  // b plus the terms k = 0..8 for the rows of the lines [y0 - 3, y1 + 3)
-  const int nps = (H + 6) * M;
-  constexpr int BP = sor_batch_p<T>();
-  for (int e0 = threadIdx.x; e0 < nps; e0 += BP * blockDim.x) {
-    T acc[BP], av[BP][9], xn[BP][9];
-    int yq[BP], xq[BP];
 #pragma unroll
-    for (int u = 0; u < BP; u++) {
-      const int e = e0 + u * blockDim.x;
-      const int l = (int)fdiv((unsigned)min(e, nps - 1), fM);
-      xq[u] = min(e, nps - 1) - l * M;
-      const int y = y0 - 3 + l;
-      yq[u] = e < nps && y >= 0 && y < M ? y : -1;  // -1: no row
-      const int yc = min(max(y, 0), M - 1), xc = xq[u];
-      const unsigned i = zb + (unsigned)(yc * M + xc);
-      acc[u] = (T)0;
-      if (yq[u] >= 0) {
-        if (y < y0) acc[u] = gb[ol + (unsigned)((y - y0 + 4) * M + xc)];
-        else if (y >= y1) acc[u] = gb[ou + (unsigned)((y - y1 + 4) * M + xc)];
-        else acc[u] = b[i];
-      }
-      const bool ly[3] = {yc > 0, true, yc < M - 1}, lx[3] = {xc > 0, true, xc < M - 1};
-#pragma unroll
-      for (int k = 0; k < 9; k++) {
-        const int dy = k / 3 - 1, dx = k % 3 - 1;
-        const bool live = z > 0 && ly[dy + 1] && lx[dx + 1];
-        const int off = -M2 + dy * M + dx;
-        av[u][k] = st27_coef_sel<T, SYM>(val27, N, k, i, off, live);
-        xn[u][k] = x[live ? i + (unsigned)off : i];  // not used when the neighbour is outside
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < BP; u++) {
-      const int y = yq[u], xc = xq[u];
-      if (y < 0) continue;
-      const bool ly[3] = {y > 0, true, y < M - 1}, lx[3] = {xc > 0, true, xc < M - 1};
-      const T xi = xs[(y - y0 + 4) * M + xc];
-      T a = acc[u];
-#pragma unroll
-      for (int k = 0; k < 9; k++) {
-        const int dy = k / 3 - 1, dx = k % 3 - 1;
-        const bool live = z > 0 && ly[dy + 1] && lx[dx + 1];
-        a += ((T)-1 * (live ? xn[u][k] : xi)) * av[u][k];
-      }
-      ps[e0 + u * blockDim.x] = a;
-    }
-  }
-  __syncthreads();
   for (int j = 0; j < 4; j++) {
-    const int c = backwards ? 3 - j : j;
-    const int cy = c >> 1, cx = c & 1;
-    int lo = max(0, y0 - (3 - j));
-    const int hi = min(M, y1 + (3 - j));
-    lo += (lo - cy) & 1;  // the first line of parity cy
-    const int nyl = hi > lo ? (hi - lo + 1) / 2 : 0, nxl = (M - cx + 1) / 2;
-    const FastDiv fx = cx ? fx1 : fx0;
-    for (int e = threadIdx.x; e < nyl * nxl; e += blockDim.x) {
-      const int ey = nxl > 1 ? (int)fdiv((unsigned)e, fx) : e;
-      const int y = lo + 2 * ey, xc = cx + 2 * (e - ey * nxl);
-      const int li = (y - y0 + 4) * M + xc;
-      const unsigned i = zb + (unsigned)(y * M + xc);
-      const bool ly[3] = {y > 0, true, y < M - 1}, lx[3] = {xc > 0, true, xc < M - 1};
-      T av[18], xp[9];
+    const int q = j / G;
+    if (j % G == g && li[q] >= 0) {
+      const T *v = lx + li[q];
+      T sp = (T)0;
 #pragma unroll
-      for (int k = 9; k < 27; k++) {
-        const int dz = k / 9 - 1, dy = (k / 3) % 3 - 1, dx = k % 3 - 1;
-        const bool live = (dz == 0 || z < M - 1) && ly[dy + 1] && lx[dx + 1];
-        const int off = dz * M2 + dy * M + dx;
-        av[k - 9] = st27_coef_sel<T, SYM>(val27, N, k, i, off, live);
-        if (dz > 0) xp[k - 18] = x[live ? i + (unsigned)off : i];  // not used when outside
-      }
-      const T xi = xs[li];
-      T acc = ps[(y - y0 + 3) * M + xc];
-#pragma unroll
-      for (int k = 9; k < 27; k++) {
-        const int dz = k / 9 - 1, dy = (k / 3) % 3 - 1, dx = k % 3 - 1;
-        const bool live = (dz == 0 || z < M - 1) && ly[dy + 1] && lx[dx + 1];
-        const T xk = dz == 0 ? xs[live ? li + dy * M + dx : li] : (live ? xp[k - 18] : xi);
-        acc += ((T)-1 * xk) * av[k - 9];
-      }
-      const T corr = acc / av[13 - 9];
-      const T xnew = xi + omega * corr;
-      xs[li] = xnew;
-      if (y >= y0 && y < y1) {
-        r[i] = corr;
-        x[i] = xnew;
+      for (int k = 0; k < 9; k++)
+        if (k != 4) sp += v[(k / 3 - 1) * LW + k % 3 - 1] * cf[q][k];
+      const double a = (acc[q] - (double)sp) - (double)v[0] * (double)cf[q][4];
+      const T corr = (T)a / cf[q][4];
+      const T xn = v[0] + omega * corr;
+      lx[li[q]] = xn;
+      if (gi[q] != 0xffffffffu) {
+        xd[gi[q]] = xn;
+        if (r) r[gi[q]] = corr;
       }
     }
     __syncthreads();
@@ -1632,7 +1512,8 @@ void drop_stencil(flgpu_mat *A) {
   dev_free(A->val27);
   A->val27 = nullptr;
   A->st_sym = false;
-  drop_sor_strips(A);
+  dev_free(A->sor_work);
+  A->sor_work = nullptr;
 }
 
 // ---- 3D order-1 lattice interpolation with the pattern implied ------------------------------
@@ -2554,32 +2435,6 @@ __global__ void k_row_span(int nsub, const int *__restrict__ rows, const int *__
   if (li < nsub) span[li] = make_int2(rowptr[rows[li]], rowptr[rows[li] + 1]);
 }
 
-// LDS of the strip sweep (values): 128 KB in FP64, 64 KB in FP32
-constexpr int kSorCapF64 = 16384, kSorCapF32 = 16384;
-
-// values the strip sweep stages for strips of H lines on an M^3 lattice
-static long sor_strip_lds(int M, int H) { return (long)(2 * H + 14) * M; }
-
-void sor_strips_alloc(flgpu_mat *A) {
-  dev_free(A->sor_ghost);
-  A->sor_ghost = nullptr;
-  A->sor_strips = A->sor_h = 0;
-  const int M = A->lat_n + 1;
-  if (A->lat_dim != 3 || A->lat_order != 1 || M < 3) return;
-  const long cap = A->prec == FLGPU_F64 ? kSorCapF64 : kSorCapF32;
-  // about one block per CU and launch, strips of at least 8 lines, within the LDS
-  const int planes = (M - 1) / 2;
-  int S = std::max(1, std::min((256 + planes - 1) / planes, (M + 7) / 8));
-  while (S <= M && sor_strip_lds(M, (M + S - 1) / S) > cap) S++;
-  if (S > M) return;  // lattices this wide keep the colour launches
-  const int H = (M + S - 1) / S;
-  S = (M + H - 1) / H;  // no empty strip
-  A->sor_strips = S;
-  A->sor_h = H;
-  if (S > 1)
-    A->sor_ghost = dev_alloc(prec_bytes(A->prec) * 2 * (size_t)M * (S - 1) * 8 * M);
-}
-
 // lines of a block of k_q1_sor_planes
 constexpr int kSorLines = 8;
 // lattices of at most 65^3 nodes sweep out of place where a spare vector is there: a launch costs
@@ -2672,77 +2527,71 @@ static bool q1_sor(const flgpu_mat *A, T omega, int steps, int backwards, T *x, 
   return false;
 }
 
-// the stencil-form sweep in strips: the copies of the strip boundaries of every plane, then one
-// launch per z parity
-template <class T, int CAP>
-static void st27_sor_strips(const flgpu_mat *A, T omega, int backwards, T *x, const T *b, T *r) {
-  const int M = A->lat_n + 1, S = A->sor_strips, H = A->sor_h;
-  FLGPU_REQUIRE(sor_strip_lds(M, H) <= CAP, "strip sweep: LDS size");
-  FLGPU_REQUIRE(27L * M * M * M < (1L << 32), "strip sweep: lattice too large");
-  T *gx = (T *)A->sor_ghost, *gb = gx ? gx + (long)M * (S - 1) * 8 * M : nullptr;
-  const FastDiv fM = fast_div((unsigned)M);
-  if (S > 1) {
-    const long prep = (long)M * (S - 1) * 8 * M;
-    const FastDiv fS1 = S > 2 ? fast_div((unsigned)(S - 1)) : FastDiv{1, 0, 0};
-    k_st27_sor_prep<T><<<grid_for(prep, 256), 256, 0, A->ctx->stream>>>(M, H, S, fM, fS1, x, b,
-                                                                        gx, gb);
-    FLGPU_HIP(hipGetLastError());
-  }
-  const FastDiv fx0 = fast_div((unsigned)((M + 1) / 2));
-  const FastDiv fx1 = M / 2 > 1 ? fast_div((unsigned)(M / 2)) : FastDiv{1, 0, 0};
+// A sweep of the stencil form from xs into xd.  Small lattices leave the GPU idle and wait for
+// one row's loads: one row a thread.  On larger ones taller tiles recompute less (1.45 times the
+// rows with 8 lines, 1.3 with 12, 1.2 with 20).  Measured, us an iterate, 8 lines and 1 row a
+// thread / 12 and 2 / 20 and 4: 49^3 FP64 16.0 / 18.7 / 24.9; 65^3 28.6 / 24.2 / 33.8; 129^3 158 /
+// 151 / 165, FP32 114 / 86 / 91; 193^3 FP32 436 / 344 / 332.
+template <class T>
+static void st27_sor(const flgpu_mat *A, T omega, int backwards, const T *xs, T *xd, const T *b,
+                     T *r, bool zero) {
+  const int M = A->lat_n + 1;
+  const int ntx = (M + kTileCols - 1) / kTileCols, W = (M + ntx - 1) / ntx;
   for (int k = 0; k < 2; k++) {
-    const int pz = backwards ? 1 - k : k;
-    const int planes = (M - 1 - pz) / 2 + 1;
-    const unsigned g = xcd_grid((unsigned)(planes * S));
-    if (A->st_sym)
-      k_st27_sor_strips<T, true, CAP><<<g, 1024, 0, A->ctx->stream>>>(
-          M, pz, H, S, backwards, fM, fx0, fx1, (const T *)A->val27, omega, x, b, r, gx, gb);
-    else
-      k_st27_sor_strips<T, false, CAP><<<g, 1024, 0, A->ctx->stream>>>(
-          M, pz, H, S, backwards, fM, fx0, fx1, (const T *)A->val27, omega, x, b, r, gx, gb);
-    FLGPU_HIP(hipGetLastError());
+    const int pz = backwards ? 1 - k : k, planes = (M - 1 - pz) / 2 + 1;
+    auto launch = [&](auto sym, auto lines, auto grp) {
+      constexpr bool SYM = decltype(sym)::value;
+      constexpr int H = decltype(lines)::value, G = decltype(grp)::value;
+      constexpr int threads = (kTileRows(H) + 63) / 64 * 64 * G;
+      const int nty = (M + H - 1) / H;
+      const unsigned g = xcd_grid((unsigned)planes * (unsigned)(ntx * nty));
+      auto run = [&](auto kern) {
+        kern<<<g, threads, 0, A->ctx->stream>>>(M, pz, W, ntx, nty, planes, backwards,
+                                                (const T *)A->val27, omega, xs,
+                                                k == 0 ? xs : xd, xd, b, r);
+        FLGPU_HIP(hipGetLastError());
+      };
+      if (!zero) run(k_st27_sor_tiles<T, SYM, false, false, H, G>);
+      else if (k == 0) run(k_st27_sor_tiles<T, SYM, true, true, H, G>);
+      else run(k_st27_sor_tiles<T, SYM, false, true, H, G>);
+    };
+    auto shape = [&](auto sym) {
+      using std::integral_constant;
+      if (M <= 56) launch(sym, integral_constant<int, 8>(), integral_constant<int, 4>());
+      else if (M <= 160) launch(sym, integral_constant<int, 12>(), integral_constant<int, 2>());
+      else launch(sym, integral_constant<int, 20>(), integral_constant<int, 1>());
+    };
+    if (A->st_sym) shape(std::true_type());
+    else shape(std::false_type());
   }
+}
+
+template <class T>
+static void st27_sor_sweeps(const flgpu_mat *A, T omega, int steps, int backwards, T *x,
+                            const T *b, T *r, bool zero, int rmode) {
+  FLGPU_REQUIRE(A->sor_work, "stencil <sor> sweeps need sor_prepare");
+  const long N = A->nrows;
+  T *w = (T *)A->sor_work, *cur = x, *other = w;
+  for (int k = 0; k < steps; k++, zero = false) {
+    const T *bk = b;
+    if (b == r) {  // the sweep reads b beyond the rows whose r it writes
+      vcopy(A->ctx, N, A->prec, b, A->prec, w + N);
+      bk = w + N;
+    }
+    const bool wr = b == r || (rmode == 1 && k + 1 == steps);
+    st27_sor<T>(A, omega, backwards, cur, other, bk, wr ? r : nullptr, zero);
+    std::swap(cur, other);
+  }
+  if (cur != x) vcopy(A->ctx, N, A->prec, cur, A->prec, x);
+}
+
+void sor_prepare(const flgpu_mat *A) {
+  if (A->alpha || !A->val27 || A->sor_work) return;
+  const_cast<flgpu_mat *>(A)->sor_work = dev_alloc(prec_bytes(A->prec) * 2 * (size_t)A->nrows);
 }
 
 static void sor_sweep(const flgpu_mat *A, double omega, int backwards, void *x, const void *b,
                       void *r) {
-  if (A->val27 && A->sor_strips > 0 && 27L * A->nrows < (1L << 32)) {
-    if (A->prec == FLGPU_F64)
-      st27_sor_strips<double, kSorCapF64>(A, omega, backwards, (double *)x, (const double *)b,
-                                          (double *)r);
-    else
-      st27_sor_strips<float, kSorCapF32>(A, (float)omega, backwards, (float *)x,
-                                         (const float *)b, (float *)r);
-    return;
-  }
-  if (A->val27) {
-    // lattice colours in the order of the lattice colouring: cz*4 + cy*2 + cx
-    int M = A->lat_n + 1;
-    for (int k = 0; k < 8; k++) {
-      int c = backwards ? 7 - k : k;
-      int cz = c >> 2, cy = (c >> 1) & 1, cx = c & 1;
-      long cnt = (long)((M - cx + 1) / 2) * ((M - cy + 1) / 2) * ((M - cz + 1) / 2);
-      unsigned g = xcd_grid(grid_for(cnt, 256));
-      if (A->prec == FLGPU_F64 && A->st_sym)
-        k_st27_sor<double, true><<<g, 256, 0, A->ctx->stream>>>(
-            M, cz, cy, cx, (const double *)A->val27, omega, (double *)x, (const double *)b,
-            (double *)r);
-      else if (A->prec == FLGPU_F64)
-        k_st27_sor<double, false><<<g, 256, 0, A->ctx->stream>>>(
-            M, cz, cy, cx, (const double *)A->val27, omega, (double *)x, (const double *)b,
-            (double *)r);
-      else if (A->st_sym)
-        k_st27_sor<float, true><<<g, 256, 0, A->ctx->stream>>>(
-            M, cz, cy, cx, (const float *)A->val27, (float)omega, (float *)x, (const float *)b,
-            (float *)r);
-      else
-        k_st27_sor<float, false><<<g, 256, 0, A->ctx->stream>>>(
-            M, cz, cy, cx, (const float *)A->val27, (float)omega, (float *)x, (const float *)b,
-            (float *)r);
-      FLGPU_HIP(hipGetLastError());
-    }
-    return;
-  }
   FLGPU_REQUIRE(A->ncolours > 0, "<sor> needs a colouring of the matrix");
   for (int k = 0; k < A->ncolours; k++) {
     const Sell &s = A->colour_sell[backwards ? A->ncolours - 1 - k : k];
@@ -2782,6 +2631,15 @@ bool sor_sweeps(const flgpu_mat *A, double omega, int steps, int backwards, void
                             (double *)r, (double *)tmp, x_zero, rmode);
     return q1_sor<float>(A, (float)omega, steps, backwards, (float *)x, (const float *)b,
                          (float *)r, (float *)tmp, x_zero, rmode);
+  }
+  if (A->val27) {
+    if (A->prec == FLGPU_F64)
+      st27_sor_sweeps<double>(A, omega, steps, backwards, (double *)x, (const double *)b,
+                              (double *)r, x_zero, rmode);
+    else
+      st27_sor_sweeps<float>(A, (float)omega, steps, backwards, (float *)x, (const float *)b,
+                             (float *)r, x_zero, rmode);
+    return false;
   }
   if (x_zero) vfill(A->ctx, A->nrows, A->prec, x, 0.0);
   for (int k = 0; k < steps; k++) sor_sweep(A, omega, backwards, x, b, r);
@@ -3453,6 +3311,7 @@ extern "C" int flgpu_sor_iterate(const flgpu_mat *A, double omega, int backwards
     check_vec(A, b, A->nrows, "b");
     check_vec(A, r, A->nrows, "r");
     CTX_LOCK(A->ctx);
+    sor_prepare(A);
     sor_sweeps(A, omega, 1, backwards, x->d, b->d, r->d);
     return 0;
   });

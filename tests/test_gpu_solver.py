@@ -481,3 +481,63 @@ def test_cell_sor_cycles_equal_sell_cycles(m, levels, pre, post, prec):
         outs.append(res)
     for a, s in zip(*outs):
         assert relerr(a, s) < tol
+
+
+@pytest.mark.parametrize("n,prec,sym", [(1, F.F64, True), (2, F.F32, True), (5, F.F64, False),
+                                        (55, F.F32, False), (56, F.F64, False),
+                                        (65, F.F64, True), (160, F.F32, True)])
+def test_stencil_sor_tile_shapes(n, prec, sym):
+    """the stencil-form <sor> sweep at the edges of its tile shapes (8 lines up to 56 nodes a
+    side, 12 up to 160, 20 above; 65 columns; the smallest lattices) equals the SELL colour sweep,
+    forwards, backwards and with rhs and residual one vector"""
+    say(f"stencil sor tiles n={n} prec={prec} sym={sym}")
+    rng = np.random.default_rng(n)
+    kap = np.exp(rng.normal(size=(n, n, n)))
+    A, b = lat.assemble(3, 1, n, kap, prec=prec)
+    B, _ = lat.assemble(3, 1, n, kap, prec=prec)
+    if not sym:
+        v = A.csr()[2]
+        v = v * (1.0 + 0.1 * rng.uniform(-1, 1, v.size))
+        A.update_values(v)
+        B.update_values(v)
+    assert A.storage(F.STORAGE_STENCIL) == F.STORAGE_STENCIL
+    assert A.stencil_planes() == (14 if sym else 27)
+    assert B.storage(F.STORAGE_SELL) == F.STORAGE_SELL
+    tol = 1e-13 if prec == F.F64 else 2e-6
+    y, c = rng.uniform(-1, 1, A.nrows), rng.uniform(-1, 1, A.nrows)
+    for bw, alias in ((0, False), (1, False), (0, True)):
+        out = []
+        for M in (A, B):
+            x, r = GpuVector.from_array(y, prec), GpuVector.from_array(c, prec)
+            bv = r if alias else GpuVector.from_array(c, prec)
+            check(lib().flgpu_sor_iterate(M.h, 1.1, bw, x.h, bv.h, r.h))
+            out.append((x.numpy(), r.numpy()))
+        assert relerr(out[0][0], out[1][0]) < tol, (bw, alias)
+        assert relerr(out[0][1], out[1][1]) < 10 * tol, (bw, alias)
+
+
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("m,levels,pre,post", [(3, 2, 1, 2), (7, 3, 2, 3)])
+def test_stencil_sor_cycles_equal_sell_cycles(m, levels, pre, post, prec):
+    """V-cycles whose levels are in the stencil form (a coefficient finer than the lattice), with
+    odd and even numbers of out-of-place sweeps, sweeps from zero and rhs and residual one vector,
+    against the same cycles on the SELL matrices; tolerance as for the per-cell form's cycles"""
+    say(f"stencil sor cycles m={m} levels={levels} V({pre},{post}) prec={prec}")
+    rng = np.random.default_rng(m)
+    n = m * 2 ** (levels - 1)
+    kap = np.exp(rng.normal(size=(2 * n,) * 3))
+    tol = 2e-12 if prec == F.F64 else 4e-5
+    y, c = rng.uniform(-1, 1, (n + 1) ** 3), rng.uniform(-1, 1, (n + 1) ** 3)
+    outs = []
+    for form in (F.STORAGE_STENCIL, F.STORAGE_SELL):
+        cs = it.GeometricCS(it.SOR(1.1), pre, post, 0, symmetric=True, prec=prec)
+        H = it.Hierarchy.lattice(cs, 3, 1, m, levels, kappa=kap)
+        for l in range(levels):
+            assert H.level_matrix(l).storage(form) == form
+        for alias in (False, True):
+            x, r = GpuVector.from_array(y, prec), GpuVector.from_array(c, prec)
+            b = r if alias else GpuVector.from_array(c, prec)
+            check(lib().flgpu_mg_apply(H.h, x.h, b.h, r.h))
+            outs.append((form, x.numpy(), r.numpy()))
+    for (_, xa, ra), (_, xb, rb) in zip(outs[:2], outs[2:]):
+        assert relerr(xa, xb) < tol and relerr(ra, rb) < tol
