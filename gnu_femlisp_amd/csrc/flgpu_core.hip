@@ -152,8 +152,8 @@ __global__ __launch_bounds__(kRedThreads) void k_dot_partial_multi(long n, const
   }
 }
 
-// The CG/FCG step's dots q.r, r.r (and q.a for K = 3) with each vector loaded once: the same
-// products summed in the same order as k_dot_partial_multi over (q, r, q) x (r, r, a)
+// The CG/FCG step's dots q.r, r.r (and q.a for K = 3) with each vector loaded once, as
+// k_dot_partial_multi forms them
 template <typename T, int K, typename TQ = T>
 __global__ __launch_bounds__(kRedThreads) void k_dot_partial_qr(long n, const TQ *q, const T *r,
                                                                 const T *a, double *partial) {
@@ -314,24 +314,11 @@ void vdot_multi_dev(flgpu_ctx *ctx, long n, int prec, int count, const void *con
   const void *xx[3] = {x[0], count > 1 ? x[1] : x[0], count > 2 ? x[2] : x[0]};
   const void *yy[3] = {y[0], count > 1 ? y[1] : y[0], count > 2 ? y[2] : y[0]};
   hipStream_t st = ctx->stream;
-  // (q, r, q) x (r, r, a): the CG/FCG step's dots, each vector loaded once
-  const bool qr = count >= 2 && xx[1] == yy[0] && yy[1] == yy[0] && (count < 3 || xx[2] == xx[0]);
 #define FLGPU_DOTS(T, K)                                                                      \
   k_dot_partial_multi<T, K><<<kRedBlocks, kRedThreads, 0, st>>>(                              \
       n, (const T *)xx[0], (const T *)yy[0], (const T *)xx[1], (const T *)yy[1],              \
       (const T *)xx[2], (const T *)yy[2], ctx->red_partial)
-#define FLGPU_QR(T, K)                                                                        \
-  k_dot_partial_qr<T, K><<<kRedBlocks, kRedThreads, 0, st>>>(                                 \
-      n, (const T *)xx[0], (const T *)yy[0], (const T *)yy[2], ctx->red_partial)
-  if (qr) {
-    if (prec == FLGPU_F64) {
-      if (count == 2) FLGPU_QR(double, 2);
-      else FLGPU_QR(double, 3);
-    } else {
-      if (count == 2) FLGPU_QR(float, 2);
-      else FLGPU_QR(float, 3);
-    }
-  } else if (prec == FLGPU_F64) {
+  if (prec == FLGPU_F64) {
     if (count == 1) FLGPU_DOTS(double, 1);
     else if (count == 2) FLGPU_DOTS(double, 2);
     else FLGPU_DOTS(double, 3);
@@ -341,24 +328,63 @@ void vdot_multi_dev(flgpu_ctx *ctx, long n, int prec, int count, const void *con
     else FLGPU_DOTS(float, 3);
   }
 #undef FLGPU_DOTS
-#undef FLGPU_QR
   k_dot_final_multi<<<count, kRedBlocks, 0, st>>>(ctx->red_partial, kRedBlocks, ctx->red_out,
                                                   slots[0], count > 1 ? slots[1] : slots[0],
                                                   count > 2 ? slots[2] : slots[0]);
   FLGPU_HIP(hipGetLastError());
 }
 
-// the FCG step's dots z.r, r.r, z.a with z in FP32 (an FP32 cycle's output) and r, a in FP64:
-// the same products, summed in the same order, as vdot_multi_dev over the FP64 copy of z
-void vdot_qr_f32(flgpu_ctx *ctx, long n, const float *z, const double *r, const double *a,
-                 const int *slots) {
-  for (int k = 0; k < 3; k++)
-    FLGPU_REQUIRE(slots[k] >= 0 && slots[k] < kRedSlots, "reduction slot out of range");
-  k_dot_partial_qr<double, 3, float><<<kRedBlocks, kRedThreads, 0, ctx->stream>>>(
-      n, z, r, a, ctx->red_partial);
-  k_dot_final_multi<<<3, kRedBlocks, 0, ctx->stream>>>(ctx->red_partial, kRedBlocks, ctx->red_out,
-                                                       slots[0], slots[1], slots[2]);
+// the regions of red_partial: the dots of vdot_dev and vdot_multi_dev (and dot_parts_qr, whose
+// rows are read before another dot is queued), dot_parts, dot_parts_rr
+constexpr int kRedOwn = 3 * kRedBlocks, kRedAll = kRedOwn + kRedBlocks + kPartsMax;
+
+static unsigned red_blocks(long n) {
+  return (unsigned)std::min((long)kRedBlocks, std::max(1L, (n + kRedThreads - 1) / kRedThreads));
+}
+
+DotParts dot_parts(flgpu_ctx *ctx, long n, int prec, const void *x, const void *y) {
+  const unsigned g = red_blocks(n);
+  double *part = ctx->red_partial + kRedOwn;
+  if (prec == FLGPU_F64)
+    k_dot_partial<double><<<g, kRedThreads, 0, ctx->stream>>>(n, (const double *)x,
+                                                              (const double *)y, part);
+  else
+    k_dot_partial<float><<<g, kRedThreads, 0, ctx->stream>>>(n, (const float *)x,
+                                                             (const float *)y, part);
   FLGPU_HIP(hipGetLastError());
+  return DotParts{part, (int)g};
+}
+
+DotParts dot_parts_qr(flgpu_ctx *ctx, long n, int prec, int qprec, const void *q, const void *r,
+                      const void *a) {
+  const unsigned g = red_blocks(n);
+  double *part = ctx->red_partial;
+  hipStream_t s = ctx->stream;
+  const double *rd = (const double *)r, *ad = (const double *)a;
+  const float *rf = (const float *)r, *af = (const float *)a;
+  FLGPU_REQUIRE(qprec == prec || prec == FLGPU_F64, "dot_parts_qr: precisions");
+  if (prec == FLGPU_F64 && qprec == FLGPU_F32 && a)
+    k_dot_partial_qr<double, 3, float><<<g, kRedThreads, 0, s>>>(n, (const float *)q, rd, ad, part);
+  else if (prec == FLGPU_F64 && qprec == FLGPU_F32)
+    k_dot_partial_qr<double, 2, float><<<g, kRedThreads, 0, s>>>(n, (const float *)q, rd, rd, part);
+  else if (prec == FLGPU_F64 && a)
+    k_dot_partial_qr<double, 3><<<g, kRedThreads, 0, s>>>(n, (const double *)q, rd, ad, part);
+  else if (prec == FLGPU_F64)
+    k_dot_partial_qr<double, 2><<<g, kRedThreads, 0, s>>>(n, (const double *)q, rd, rd, part);
+  else if (a)
+    k_dot_partial_qr<float, 3><<<g, kRedThreads, 0, s>>>(n, (const float *)q, rf, af, part);
+  else
+    k_dot_partial_qr<float, 2><<<g, kRedThreads, 0, s>>>(n, (const float *)q, rf, rf, part);
+  FLGPU_HIP(hipGetLastError());
+  return DotParts{part, (int)g};
+}
+
+double *dot_parts_rr(flgpu_ctx *ctx) { return ctx->red_partial + kRedOwn + kRedBlocks; }
+
+DotParts dot_parts_bound(flgpu_ctx *ctx, const double *p, long np, int slot) {
+  if (np <= kPartsMax) return DotParts{p, (int)np};
+  dot_final(ctx, p, (int)np, slot);
+  return DotParts{ctx->red_out + slot, 1};
 }
 
 void fetch_slots(flgpu_ctx *ctx, int nslots) {
@@ -372,6 +398,8 @@ void fetch_slots_async(flgpu_ctx *ctx, int nslots) {
                            hipMemcpyDeviceToHost, ctx->stream));
   FLGPU_HIP(hipEventRecord(ctx->ev_fetch, ctx->stream));
 }
+
+void fetch_mark(flgpu_ctx *ctx) { FLGPU_HIP(hipEventRecord(ctx->ev_fetch, ctx->stream)); }
 
 void fetch_wait(flgpu_ctx *ctx) { FLGPU_HIP(hipEventSynchronize(ctx->ev_fetch)); }
 
@@ -442,7 +470,7 @@ extern "C" int flgpu_ctx_create(int device, flgpu_ctx **out) {
     c->cus = prop.multiProcessorCount;
     c->name = prop.gcnArchName;
     FLGPU_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    c->red_partial = (double *)dev_alloc(sizeof(double) * 3 * kRedBlocks);
+    c->red_partial = (double *)dev_alloc(sizeof(double) * kRedAll);
     c->red_out = (double *)dev_alloc(sizeof(double) * kRedSlots);
     FLGPU_HIP(hipHostMalloc((void **)&c->host_out, sizeof(double) * kRedSlots, hipHostMallocDefault));
     FLGPU_HIP(hipEventCreate(&c->ev_start));

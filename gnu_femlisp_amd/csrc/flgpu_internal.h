@@ -197,7 +197,7 @@ struct flgpu_mat {
   // lattice vertex order, blk_inv[v][i][j] = (A_BB^-1)_ij (prec, rows padded to 16 bytes);
   // nullptr until needed and for order 1, whose blocks are single DOFs
   void *blk_inv = nullptr;
-  // per-block partial sums of the per-cell product's fused dot (spmv_dot), dot_np entries
+  // per-block partial sums of a product's fused dot (spmv_dot), dot_np entries
   double *dot_part = nullptr;
   long dot_np = 0;
   // counts the changes of the buffers and forms the kernels read (a form dropped or built, a
@@ -238,9 +238,16 @@ void spmv(const flgpu_mat *A, double alpha, const void *x, double beta,
           const void *z, void *out);
 void spmv_t(const flgpu_mat *A, double alpha, const void *x, double beta,
             void *out);
-// out = A x and the dot (out, x) into reduction slot `slot` in one pass over A, when A is
-// applied in the per-cell form; false (nothing launched) otherwise
-bool spmv_dot(const flgpu_mat *A, const void *x, void *out, int slot);
+// Per-block partials of one or more dots, K rows of np values.  The kernel that needs a sum adds
+// its row up itself (parts_sum), in every block: 3072 values at most, cheaper than a launch.
+struct DotParts {
+  const double *p = nullptr;
+  int np = 0;
+};
+constexpr int kPartsMax = 3072;
+// out = A x and the partials of the dot (out, x): formed in the same pass where A's form does
+// that, else read from the vectors; `slot` as for dot_parts_bound
+DotParts spmv_dot(const flgpu_mat *A, const void *x, void *out, int slot);
 void jacobi_iterate(const flgpu_mat *A, double damp, void *x, void *r);
 // `steps` <jacobi> steps with fresh residuals, x ping-ponged through tmp; x_zero: x is zero
 // and need not be read (the first step is x = damp b / diag)
@@ -304,17 +311,65 @@ void vdot_dev(flgpu_ctx *ctx, long n, int prec, const void *x, const void *y,
               int slot);
 // the sum of np per-block partials into reduction slot `slot`
 void dot_final(flgpu_ctx *ctx, const double *partial, int np, int slot);
+// a dot's partials: of x y (kept apart from the others' until the next call), and of q.r, r.r and,
+// with a, q.a, with q in FP32 or the precision of r
+DotParts dot_parts(flgpu_ctx *ctx, long n, int prec, const void *x, const void *y);
+DotParts dot_parts_qr(flgpu_ctx *ctx, long n, int prec, int qprec, const void *q, const void *r,
+                      const void *a);
+double *dot_parts_rr(flgpu_ctx *ctx);  // kPartsMax values for a caller's own partials
+// np partials brought down to kPartsMax: by a reduction into slot `slot` where there are more
+DotParts dot_parts_bound(flgpu_ctx *ctx, const double *p, long np, int slot);
+
+// this block's share (256 threads, all of them here) of a dot
+__device__ __forceinline__ void block_part(double v, double *part) {
+  __shared__ double ws[4];
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = ((ws[0] + ws[1]) + ws[2]) + ws[3];
+}
+// the sums of K rows of partials, the same in every thread of every block of 256
+template <int K>
+__device__ __forceinline__ void parts_sum(const double *__restrict__ part, int np,
+                                          double (&out)[K]) {
+  __shared__ double ws[K][4];
+  constexpr int U = K == 1 ? kPartsMax / 256 : 4;  // all loads of one dot, or of 1024 partials
+  double acc[K] = {};
+  for (int i = threadIdx.x; i < np; i += U * 256) {
+    double v[K][U];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int j = i + u * 256;
+        v[k][u] = j < np ? part[(long)k * np + j] : 0.0;
+      }
+#pragma unroll
+    for (int k = 0; k < K; k++)
+#pragma unroll
+      for (int u = 0; u < U; u++) acc[k] += v[k][u];
+  }
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    for (int o = 32; o > 0; o >>= 1) acc[k] += __shfl_down(acc[k], o, 64);
+    if ((threadIdx.x & 63) == 0) ws[k][threadIdx.x >> 6] = acc[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K; k++) out[k] = ((ws[k][0] + ws[k][1]) + ws[k][2]) + ws[k][3];
+}
+
 // 1 to 3 dots in one pass, each identical to vdot_dev's
 void vdot_multi_dev(flgpu_ctx *ctx, long n, int prec, int count, const void *const *x,
                     const void *const *y, const int *slots);
-void vdot_qr_f32(flgpu_ctx *ctx, long n, const float *z, const double *r, const double *a,
-                 const int *slots);
 double vdot_host(flgpu_ctx *ctx, long n, int prec, const void *x,
                  const void *y);
 void fetch_slots(flgpu_ctx *ctx, int nslots);  // red_out[0..n) -> host_out
 // the same copy queued on the stream; host_out is valid after fetch_wait, while work queued
 // in between runs on
 void fetch_slots_async(flgpu_ctx *ctx, int nslots);
+// only the mark fetch_wait waits for: what kernels queued before it store to host_out is there
+void fetch_mark(flgpu_ctx *ctx);
 void fetch_wait(flgpu_ctx *ctx);
 
 }  // namespace flgpu

@@ -1040,50 +1040,144 @@ void mg_free(flgpu_mg *mg) {
 
 // ---- Krylov kernels with device scalars ----------------------------------------------------
 
-// p <- (a/b) p + q   (<cg>: scal! (/ new-alpha alpha) p, m+! q p)
-template <class T>
-__global__ void k_cg_p(long n, const double *a, const double *b, T *p, const T *__restrict__ q) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  T sc = (T)(*a / *b);
-  p[i] = sc * p[i] + q[i];
-}
+// The step's sums are added up from per-block partials by the kernels that need them (parts_sum)
+// instead of by launches of their own, and the block that is first writes them to the reduction
+// slots for the kernels after and, where host is given, to the host's copy.  A thread's vector
+// loads are issued before the sums' loads.  Bound by the vectors' bytes from 10^6 rows on (2.1
+// million FP64 rows: the update 17.6 us, 5.9 TB/s), by launches below.
 
-// p <- q + beta p, beta = -(q.a)/(a.p) (flexible CG): Polak-Ribiere's q.(r - r_old)/(q_old.r_old)
-// with r - r_old = -lam a and lam = (q_old.r_old)/(a.p), so that r_old need not be kept
-template <class T, class TQ = T>
-__global__ void k_fcg_p(long n, const double *qa, const double *ap, T *p,
-                        const TQ *__restrict__ q) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  T beta = (T)(-*qa / *ap);
-  p[i] = (T)q[i] + beta * p[i];
-}
-
-// <cg>'s update in one pass: x <- x + lam p, r <- r - lam a with lam = num / den rounded to T
-// once per sign (femlisp's axpy! with (/ alpha beta))
-// STAGE: also the next preconditioner call's staging pass on the new r (stage_first_step, for
-// an FP32 hierarchy under FP64 vectors): bs = (float)r, xo = damp (bs / diag), the values that
-// pass would write
-template <class T, bool STAGE = false>
-__global__ void k_cg_update(long n, const double *num, const double *den, const T *__restrict__ p,
-                            const T *__restrict__ a, T *__restrict__ x, T *__restrict__ r,
-                            float *__restrict__ bs = nullptr,
-                            const float *__restrict__ diag = nullptr, float damp = 0.0f,
-                            float *__restrict__ xo = nullptr) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double q = *num / *den;
-  T lp = (T)(1.0 * q), lm = (T)(-1.0 * q);
-  T ri = r[i];
-  x[i] = lp * p[i] + x[i];
-  T rn = lm * a[i] + ri;
-  r[i] = rn;
-  if (STAGE) {
-    float bi = (float)rn;
-    bs[i] = bi;
-    xo[i] = damp * (bi / diag[i]);
+// x <- x + lam p, r <- r - lam a with lam = num / (a.p) rounded to T once per sign (<cg>: femlisp's
+// axpy! with (/ alpha beta)).  STAGE: also the next preconditioner call's staging pass on the new
+// r (stage_first_step, for an FP32 hierarchy under FP64 vectors): bs = (float)r, xo = damp (bs /
+// diag), the values that pass would write.  RR: also the partials of r.r, one a block
+template <class T, int E, bool STAGE, bool RR>
+__global__ __launch_bounds__(256) void k_cg_update(long n, const double *num, DotParts ap,
+                                                   double *ap_out, const T *__restrict__ p,
+                                                   const T *__restrict__ a, T *__restrict__ x,
+                                                   T *__restrict__ r, double *rr,
+                                                   float *__restrict__ bs,
+                                                   const float *__restrict__ diag, float damp,
+                                                   float *__restrict__ xo) {
+  const long stride = (long)gridDim.x * (256 * E);
+  long i0 = (long)blockIdx.x * (256 * E) + threadIdx.x;
+  T pv[E], av[E], xv[E], rv[E];
+  auto load = [&] {
+#pragma unroll
+    for (int u = 0; u < E; u++) {
+      const long i = min(i0 + u * 256, n - 1);
+      pv[u] = p[i];
+      av[u] = a[i];
+      xv[u] = x[i];
+      rv[u] = r[i];
+    }
+  };
+  load();
+  double s[1];
+  parts_sum<1>(ap.p, ap.np, s);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *ap_out = s[0];
+  const double q = *num / s[0];
+  const T lp = (T)(1.0 * q), lm = (T)(-1.0 * q);
+  double acc = 0;
+  for (; i0 - (long)threadIdx.x < n;) {
+#pragma unroll
+    for (int u = 0; u < E; u++) {
+      const long i = i0 + u * 256;
+      if (i < n) {
+        x[i] = lp * pv[u] + xv[u];
+        const T rn = lm * av[u] + rv[u];
+        r[i] = rn;
+        if (RR) acc += (double)rn * (double)rn;
+        if (STAGE) {
+          const float bi = (float)rn;
+          bs[i] = bi;
+          xo[i] = damp * (bi / diag[i]);
+        }
+      }
+    }
+    i0 += stride;
+    if (i0 - (long)threadIdx.x < n) load();
   }
+  if (RR) block_part(acc, rr);
+}
+
+// The step's end from the partials d of q.r, r.r (K >= 2) and q.a (K = 3); K = 1 (no
+// preconditioner, q = r): of r.r alone.  slots[na] = q.r, slots[3] = r.r, slots[4] = q.a, also to
+// host.  <cg>: p <- (q.r / alpha) p + q (scal! (/ new-alpha alpha) p, m+! q p) with alpha =
+// slots[ca].  FCG: p <- q + beta p, beta = -(q.a)/(a.p): Polak-Ribiere's q.(r - r_old) /
+// (q_old.r_old) with r - r_old = -lam a and lam = (q_old.r_old)/(a.p), so that r_old need not be
+// kept
+template <class T, class TQ, int E, int K, bool FCG>
+__global__ __launch_bounds__(256) void k_cg_p(long n, DotParts d, double *slots, int na, int ca,
+                                              double *host, T *__restrict__ p,
+                                              const TQ *__restrict__ q) {
+  const long i0 = (long)blockIdx.x * (256 * E) + threadIdx.x;
+  T pv[E];
+  TQ qv[E];
+#pragma unroll
+  for (int u = 0; u < E; u++) {
+    const long i = min(i0 + u * 256, n - 1);
+    pv[u] = p[i];
+    qv[u] = q[i];
+  }
+  double s[K];
+  parts_sum<K>(d.p, d.np, s);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    slots[na] = s[0];
+    slots[3] = s[K > 1 ? 1 : 0];
+    if (K > 2) slots[4] = s[K - 1];
+    if (host) {
+      host[na] = s[0];
+      host[3] = s[K > 1 ? 1 : 0];
+    }
+  }
+  const T c = FCG ? (T)(-s[K - 1] / slots[1]) : (T)(s[0] / slots[ca]);
+#pragma unroll
+  for (int u = 0; u < E; u++) {
+    const long i = i0 + u * 256;
+    if (i < n) p[i] = FCG ? (T)qv[u] + c * pv[u] : c * pv[u] + (T)qv[u];
+  }
+}
+
+// rows per thread: four where that leaves two blocks a CU
+constexpr long kCgLong = 4L * 256 * 512;
+
+// blocks of the update, which bound the partials it leaves
+static unsigned cg_grid(long n) {
+  const long b = n >= kCgLong ? 1024 : 256;
+  return (unsigned)std::max(1L, std::min((long)kPartsMax, (n + b - 1) / b));
+}
+
+template <class T>
+static void cg_update(flgpu_ctx *ctx, long n, int ca, DotParts ap, const void *p, const void *a,
+                      void *x, void *r, double *rr, flgpu_mg *stage) {
+  const int E = n >= kCgLong ? 4 : 1;
+  const unsigned g = cg_grid(n);
+  double *slot = ctx->red_out;
+  MGLevel *S = stage ? &stage->lv[stage->top] : nullptr;
+  auto launch = [&](auto kern) {
+    kern<<<g, 256, 0, ctx->stream>>>(
+        n, slot + ca, ap, slot + 1, (const T *)p, (const T *)a, (T *)x, (T *)r, rr,
+        S ? (float *)stage->bs : nullptr, S ? (const float *)S->A->diag : nullptr,
+        S ? (float)stage->p.omega : 0.0f, S ? (float *)S->tmp : nullptr);
+    FLGPU_HIP(hipGetLastError());
+  };
+  if (S) launch(E == 4 ? k_cg_update<T, 4, true, false> : k_cg_update<T, 1, true, false>);
+  else if (rr) launch(E == 4 ? k_cg_update<T, 4, false, true> : k_cg_update<T, 1, false, true>);
+  else launch(E == 4 ? k_cg_update<T, 4, false, false> : k_cg_update<T, 1, false, false>);
+}
+
+template <class T, class TQ, int K, bool FCG>
+static void cg_p(flgpu_ctx *ctx, long n, DotParts d, int na, int ca, double *host, void *p,
+                 const void *q) {
+  const int E = n >= kCgLong ? 4 : 1;
+  const unsigned g = (unsigned)std::max(1L, (n + 256L * E - 1) / (256L * E));
+  if (E == 4)
+    k_cg_p<T, TQ, 4, K, FCG><<<g, 256, 0, ctx->stream>>>(n, d, ctx->red_out, na, ca, host, (T *)p,
+                                                         (const TQ *)q);
+  else
+    k_cg_p<T, TQ, 1, K, FCG><<<g, 256, 0, ctx->stream>>>(n, d, ctx->red_out, na, ca, host, (T *)p,
+                                                         (const TQ *)q);
+  FLGPU_HIP(hipGetLastError());
 }
 
 }  // namespace flgpu
@@ -1416,8 +1510,6 @@ extern "C" int flgpu_solve(flgpu_mg *mg, const flgpu_mat *A, const flgpu_solve_p
       }
       learned = mg->hook.get();
     }
-    double *slot = ctx->red_out;
-    unsigned g = grid_for(N, 256);
     auto t0 = std::chrono::steady_clock::now();
     vfill(ctx, N, prec, x->d, 0.0);  // initially: x := 0 (solve.lisp:126-132)
     bool residual_p = false, initialized = false;
@@ -1427,6 +1519,8 @@ extern "C" int flgpu_solve(flgpu_mg *mg, const flgpu_mat *A, const flgpu_solve_p
     // the iteration keeps, so they are queued ahead of the host's wait for the stopping
     // test and simply dropped when the iteration stops or restarts
     bool ap_ready = false;
+    DotParts ap;                  // a.p's partials, where ap_ready
+    constexpr int kApSlot = 20;   // its slot where they are too many
     // the current alpha's slot: 0 after a restart, then alternating 2 / 0 (the new alpha goes
     // to the other one, so no copy is needed between steps)
     int ca = 0;
@@ -1541,72 +1635,48 @@ extern "C" int flgpu_solve(flgpu_mg *mg, const flgpu_mat *A, const flgpu_solve_p
             initialized = true;
           }
           if (alpha != 0.0) {
-            if (!ap_ready && !spmv_dot(A, W.p, W.a, 1)) {
-              spmv(A, 1.0, W.p, 0.0, W.a, W.a);         // gemm! 1 A p 0 a
-              vdot_dev(ctx, N, prec, W.a, W.p, 1);       // beta = a.p
-            }
+            if (!ap_ready) ap = spmv_dot(A, W.p, W.a, kApSlot);  // a = A p, beta = a.p
             ap_ready = false;
             // x += (alpha/beta) p, r -= (alpha/beta) a (FCG keeps the old r first); for an
             // FP32 hierarchy under FP64 vectors the same pass stages the new r for the cycle
             const bool staged = pc && !p->alias && prec == FLGPU_F64 &&
                                 mg->p.prec == FLGPU_F32 && mg_stages_first(mg, prec);
-            if (staged) {
-              MGLevel &T = mg->lv[mg->top];
-              k_cg_update<double, true><<<g, 256, 0, s>>>(
-                  N, slot + ca, slot + 1, (const double *)W.p, (const double *)W.a,
-                  (double *)x->d, (double *)W.r, (float *)mg->bs, (const float *)T.A->diag,
-                  (float)mg->p.omega, (float *)T.tmp);
-            } else if (prec == FLGPU_F64)
-              k_cg_update<double><<<g, 256, 0, s>>>(N, slot + ca, slot + 1, (const double *)W.p,
-                                                    (const double *)W.a, (double *)x->d,
-                                                    (double *)W.r);
+            double *rr = pc ? nullptr : dot_parts_rr(ctx);
+            if (prec == FLGPU_F64)
+              cg_update<double>(ctx, N, ca, ap, W.p, W.a, x->d, W.r, rr, staged ? mg : nullptr);
             else
-              k_cg_update<float><<<g, 256, 0, s>>>(N, slot + ca, slot + 1, (const float *)W.p,
-                                                   (const float *)W.a, (float *)x->d,
-                                                   (float *)W.r);
-            FLGPU_HIP(hipGetLastError());
+              cg_update<float>(ctx, N, ca, ap, W.p, W.a, x->d, W.r, rr, nullptr);
             // FCG with an FP32 cycle under FP64 vectors reads the cycle's output in FP32 (the
             // same values as their FP64 copy, which is then not written)
             const bool z32 = pc && fcg && !learned && !p->alias && prec == FLGPU_F64 &&
                              mg->p.prec == FLGPU_F32;
-            if (pc) precondition(mg, p, W, W.r, W.q, learned, staged, z32);
-            else vcopy(ctx, N, prec, W.r, prec, W.q);
             const int na = 2 - ca;  // the new alpha's slot
-            if (z32) {  // new alpha = z.r, defect norm^2 = r.r, FCG's z.a: one pass
-              const int slots[3] = {na, 3, 4};
-              vdot_qr_f32(ctx, N, (const float *)mg->xs, (const double *)W.r,
-                          (const double *)W.a, slots);
-            } else {  // new alpha = q.r, defect norm^2 = r.r, FCG's q.a: one pass
-              const void *dx[3] = {W.q, W.r, W.q}, *dy[3] = {W.r, W.r, W.a};
-              const int slots[3] = {na, 3, 4};
-              vdot_multi_dev(ctx, N, prec, fcg ? 3 : 2, dx, dy, slots);
-            }
-            if (z32) {
-              k_fcg_p<double, float><<<g, 256, 0, s>>>(N, slot + 4, slot + 1, (double *)W.p,
-                                                       (const float *)mg->xs);
-            } else if (fcg) {
+            // with the network on, its decision (kLearnedFlag) comes along by a copy
+            double *host = learned ? nullptr : ctx->host_out;
+            if (!pc) {  // q = r: alpha and the defect norm^2 are r.r
+              const DotParts d{rr, (int)cg_grid(N)};
               if (prec == FLGPU_F64)
-                k_fcg_p<double><<<g, 256, 0, s>>>(N, slot + 4, slot + 1, (double *)W.p,
-                                                  (const double *)W.q);
+                cg_p<double, double, 1, false>(ctx, N, d, na, ca, host, W.p, W.r);
               else
-                k_fcg_p<float><<<g, 256, 0, s>>>(N, slot + 4, slot + 1, (float *)W.p,
-                                                 (const float *)W.q);
+                cg_p<float, float, 1, false>(ctx, N, d, na, ca, host, W.p, W.r);
             } else {
-              if (prec == FLGPU_F64)
-                k_cg_p<double><<<g, 256, 0, s>>>(N, slot + na, slot + ca, (double *)W.p,
-                                                 (const double *)W.q);
-              else
-                k_cg_p<float><<<g, 256, 0, s>>>(N, slot + na, slot + ca, (float *)W.p,
-                                                (const float *)W.q);
+              precondition(mg, p, W, W.r, W.q, learned, staged, z32);
+              // new alpha = q.r, defect norm^2 = r.r, FCG's q.a: one pass
+              const void *q = z32 ? mg->xs : W.q;
+              const DotParts d = dot_parts_qr(ctx, N, prec, z32 ? (int)FLGPU_F32 : prec, q, W.r,
+                                              fcg ? W.a : nullptr);
+              if (z32) cg_p<double, float, 3, true>(ctx, N, d, na, ca, host, W.p, q);
+              else if (fcg && prec == FLGPU_F64)
+                cg_p<double, double, 3, true>(ctx, N, d, na, ca, host, W.p, q);
+              else if (fcg) cg_p<float, float, 3, true>(ctx, N, d, na, ca, host, W.p, q);
+              else if (prec == FLGPU_F64)
+                cg_p<double, double, 2, false>(ctx, N, d, na, ca, host, W.p, q);
+              else cg_p<float, float, 2, false>(ctx, N, d, na, ca, host, W.p, q);
             }
-            FLGPU_HIP(hipGetLastError());
             ca = na;
-            // with the network on, its decision (kLearnedFlag) comes along
-            fetch_slots_async(ctx, learned ? kLearnedFlag + 1 : 4);
-            if (!spmv_dot(A, W.p, W.a, 1)) {  // the next step's product, ahead of the wait
-              spmv(A, 1.0, W.p, 0.0, W.a, W.a);
-              vdot_dev(ctx, N, prec, W.a, W.p, 1);
-            }
+            if (learned) fetch_slots_async(ctx, kLearnedFlag + 1);
+            else fetch_mark(ctx);
+            ap = spmv_dot(A, W.p, W.a, kApSlot);  // the next step's product, ahead of the wait
             ap_ready = true;
             fetch_wait(ctx);
             alpha = ctx->host_out[ca];

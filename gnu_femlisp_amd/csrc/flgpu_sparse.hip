@@ -530,26 +530,31 @@ __device__ __forceinline__ T sell_row(const T *__restrict__ vp, const int *__res
   return acc;
 }
 
-// out[row] = beta*z[row] + sum_k (alpha*x[col]) * val  over one SELL structure
-template <class T>
+// out[row] = beta*z[row] + sum_k (alpha*x[col]) * val  over one SELL structure.  DOT (here and in
+// the other products): also the block's share of sum_i out_i x_i to dpart (all rows, alpha 1,
+// beta 0); a pass over both vectors and a launch less for the conjugate gradients
+template <class T, bool DOT = false>
 __global__ __launch_bounds__(256) void k_sell_spmv(int nsub, int nslices, const int *__restrict__ rows,
                                                    const long *__restrict__ slice_ptr,
                                                    const int *__restrict__ col,
                                                    const T *__restrict__ val, T alpha,
                                                    const T *__restrict__ x, T beta, const T *z,
-                                                   T *out) {
+                                                   T *out, double *dpart = nullptr) {
   unsigned lb = xcd_block(blockIdx.x, gridDim.x);
   int s = (int)lb * 4 + (threadIdx.x >> 6);
-  if (s >= nslices) return;
   int lane = threadIdx.x & 63;
   int li = s * 64 + lane;
-  long base = slice_ptr[s];
-  int w = (int)((slice_ptr[s + 1] - base) >> 6);
-  if (li >= nsub) return;
-  int row = rows ? rows[li] : li;
-  T acc = (beta == (T)0) ? (T)0 : beta * z[row];
-  acc = sell_row<T>(val + base + lane, col + base + lane, w, alpha, x, acc);
-  out[row] = acc;
+  double d = 0;
+  if (s < nslices && li < nsub) {
+    long base = slice_ptr[s];
+    int w = (int)((slice_ptr[s + 1] - base) >> 6);
+    int row = rows ? rows[li] : li;
+    T acc = (beta == (T)0) ? (T)0 : beta * z[row];
+    acc = sell_row<T>(val + base + lane, col + base + lane, w, alpha, x, acc);
+    out[row] = acc;
+    if (DOT) d = (double)acc * (double)x[row];
+  }
+  if (DOT) block_part(d, dpart);
 }
 
 // The sum over one CSR row [b, e) by the G lanes that share it (l: this lane's place): every lane
@@ -587,17 +592,24 @@ __device__ __forceinline__ double csr_row(const int *__restrict__ col, const T *
 // irregular matrices are bound by the longest row of every 64 in SELL.  300 007 rows of 18
 // entries on average (55 at most), FP64: 23.1 us, 3.4 TB/s of entries, 40.3 us from SELL;
 // Q2 12^3 (15 625 rows of 58): 4.1 against 16.7 us.
-template <class T, int G>
+template <class T, int G, bool DOT = false>
 __global__ __launch_bounds__(256) void k_csr_spmv(int nrows, const int *__restrict__ rowptr,
                                                   const int *__restrict__ col,
                                                   const T *__restrict__ val, T alpha,
                                                   const T *__restrict__ x, T beta, const T *z,
-                                                  T *out) {
+                                                  T *out, double *dpart = nullptr) {
   const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
   const int row = (int)lb * (256 / G) + threadIdx.x / G, l = threadIdx.x % G;
-  if (row >= nrows) return;  // the lanes of a row leave together
-  const double acc = csr_row<T, G>(col, val, rowptr[row], rowptr[row + 1], l, alpha, x);
-  if (l == 0) out[row] = beta == (T)0 ? (T)acc : (T)((double)beta * (double)z[row] + acc);
+  double d = 0;
+  if (row < nrows) {  // the lanes of a row together
+    const double acc = csr_row<T, G>(col, val, rowptr[row], rowptr[row + 1], l, alpha, x);
+    if (l == 0) {
+      const T o = beta == (T)0 ? (T)acc : (T)((double)beta * (double)z[row] + acc);
+      out[row] = o;
+      if (DOT) d = (double)o * (double)x[row];
+    }
+  }
+  if (DOT) block_part(d, dpart);
 }
 
 // Lanes per row of the products from the CSR, 0: SELL.  SELL streams a slice as wide as its
@@ -616,25 +628,31 @@ static int csr_lanes(const flgpu_mat *A) {
 
 template <class T>
 static void launch_csr_spmv(const flgpu_mat *A, T alpha, const void *x, T beta, const void *z,
-                            void *out) {
+                            void *out, double *dpart = nullptr) {
   const int G = A->lanes;
   const unsigned g = xcd_grid(grid_for((long)A->nrows * G, 256));
   auto launch = [&](auto kern) {
     kern<<<g, 256, 0, A->ctx->stream>>>(A->nrows, A->rowptr, A->colidx, (const T *)A->vals, alpha,
-                                        (const T *)x, beta, (const T *)z, (T *)out);
+                                        (const T *)x, beta, (const T *)z, (T *)out, dpart);
   };
-  launch(G == 4 ? k_csr_spmv<T, 4> : k_csr_spmv<T, 8>);
+  if (dpart) launch(G == 4 ? k_csr_spmv<T, 4, true> : k_csr_spmv<T, 8, true>);
+  else launch(G == 4 ? k_csr_spmv<T, 4> : k_csr_spmv<T, 8>);
   FLGPU_HIP(hipGetLastError());
 }
 
 template <class T>
 static void launch_spmv(flgpu_ctx *ctx, const Sell &s, double alpha, const void *x, double beta,
-                        const void *z, void *out) {
+                        const void *z, void *out, double *dpart = nullptr) {
   if (s.nrows == 0) return;
   unsigned g = xcd_grid(grid_for(s.nslices, 4));
-  k_sell_spmv<T><<<g, 256, 0, ctx->stream>>>(s.nrows, s.nslices, s.rows, s.slice_ptr, s.col,
-                                             (const T *)s.val, (T)alpha, (const T *)x, (T)beta,
-                                             (const T *)z, (T *)out);
+  if (dpart)
+    k_sell_spmv<T, true><<<g, 256, 0, ctx->stream>>>(
+        s.nrows, s.nslices, s.rows, s.slice_ptr, s.col, (const T *)s.val, (T)alpha, (const T *)x,
+        (T)beta, (const T *)z, (T *)out, dpart);
+  else
+    k_sell_spmv<T><<<g, 256, 0, ctx->stream>>>(s.nrows, s.nslices, s.rows, s.slice_ptr, s.col,
+                                               (const T *)s.val, (T)alpha, (const T *)x, (T)beta,
+                                               (const T *)z, (T *)out);
   FLGPU_HIP(hipGetLastError());
 }
 
@@ -1320,18 +1338,23 @@ __device__ __forceinline__ T st27_row(int M, long N, long i, int z, int y, int x
   return acc;
 }
 
-template <class T, bool SYM>
+template <class T, bool SYM, bool DOT = false>
 __global__ __launch_bounds__(256) void k_st27_spmv(int M, const T *__restrict__ val27, T coef,
                                                    const T *__restrict__ x, T beta, const T *z,
-                                                   T *out) {
+                                                   T *out, double *dpart = nullptr) {
   unsigned lb = xcd_block(blockIdx.x, gridDim.x);
   long i = (long)lb * blockDim.x + threadIdx.x;
   long N = (long)M * M * M;
-  if (i >= N) return;
-  int xx = (int)(i % M), yy = (int)((i / M) % M), zz = (int)(i / ((long)M * M));
-  T acc = (beta == (T)0) ? (T)0 : beta * z[i];
-  T d;
-  out[i] = st27_row<T, SYM>(M, N, i, zz, yy, xx, val27, acc, coef, x, &d);
+  double dot = 0;
+  if (i < N) {
+    int xx = (int)(i % M), yy = (int)((i / M) % M), zz = (int)(i / ((long)M * M));
+    T acc = (beta == (T)0) ? (T)0 : beta * z[i];
+    T d;
+    acc = st27_row<T, SYM>(M, N, i, zz, yy, xx, val27, acc, coef, x, &d);
+    out[i] = acc;
+    if (DOT) dot = (double)acc * (double)x[i];
+  }
+  if (DOT) block_part(dot, dpart);
 }
 
 // ---- the stencil-form <sor> sweep in tiles ---------------------------------------------------
@@ -1744,15 +1767,14 @@ static void launch_tp(const flgpu_mat *A, T alpha, const void *x, T beta, const 
 }
 
 template <class T>
-static void launch_st27_spmv(const flgpu_mat *A, T alpha, const T *x, T beta, const T *z, T *out) {
-  int M = A->lat_n + 1;
-  unsigned g = xcd_grid(grid_for(A->nrows, 256));
-  if (A->st_sym)
-    k_st27_spmv<T, true><<<g, 256, 0, A->ctx->stream>>>(M, (const T *)A->val27, alpha, x, beta,
-                                                        z, out);
-  else
-    k_st27_spmv<T, false><<<g, 256, 0, A->ctx->stream>>>(M, (const T *)A->val27, alpha, x, beta,
-                                                         z, out);
+static void launch_st27_spmv(const flgpu_mat *A, T alpha, const T *x, T beta, const T *z, T *out,
+                             double *dpart = nullptr) {
+  auto launch = [&](auto kern) {
+    kern<<<xcd_grid(grid_for(A->nrows, 256)), 256, 0, A->ctx->stream>>>(
+        A->lat_n + 1, (const T *)A->val27, alpha, x, beta, z, out, dpart);
+  };
+  if (A->st_sym) launch(dpart ? k_st27_spmv<T, true, true> : k_st27_spmv<T, true>);
+  else launch(dpart ? k_st27_spmv<T, false, true> : k_st27_spmv<T, false>);
   FLGPU_HIP(hipGetLastError());
 }
 
@@ -1926,11 +1948,12 @@ struct CellBox<2> {
   static constexpr int B[3] = {0, 15, 15};  // 16 x 16 lanes
 };
 
-template <class T, int DIM>
+template <class T, int DIM, bool DOT = false>
 __global__ __launch_bounds__(256) void k_cell_apply(int n, Div1 dby, Div1 dbx,
                                                     const T *__restrict__ cell, T alpha,
                                                     const T *__restrict__ x, T beta, const T *z,
-                                                    T *out, unsigned nblk) {
+                                                    T *out, unsigned nblk,
+                                                    double *dpart = nullptr) {
   constexpr int NL = DIM == 3 ? 27 : 9;
   constexpr int PZ = DIM == 3 ? 2 * (CellBox<DIM>::B[0] + 1) + 1 : 1,
                 PY = 2 * (CellBox<DIM>::B[1] + 1) + 1, PX = 2 * (CellBox<DIM>::B[2] + 1) + 1;
@@ -1938,7 +1961,10 @@ __global__ __launch_bounds__(256) void k_cell_apply(int n, Div1 dby, Div1 dbx,
   __shared__ T px[PZ * PY * PX];
   __shared__ T ye[NL * 256];
   const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
-  if (lb >= nblk) return;
+  if (lb >= nblk) {
+    if (DOT && threadIdx.x == 0) dpart[blockIdx.x] = 0.0;
+    return;
+  }
   const int tid = threadIdx.x, M = 2 * n + 1;
   unsigned u = lb, q = fdiv(u, dbx);
   const int cx0 = (int)(u - q * dbx.f.d) * CellBox<DIM>::B[2];
@@ -1989,12 +2015,12 @@ __global__ __launch_bounds__(256) void k_cell_apply(int n, Div1 dby, Div1 dbx,
 #pragma unroll
   for (int l = 0; l < NL; l++) ye[l * 256 + tid] = live ? (T)((double)fac * xv[l]) : (T)0;
   __syncthreads();
-  if (!own) return;
+  double d = 0;
 #pragma unroll
   for (int t = 0; t < (1 << DIM); t++) {
     const int tx = t & 1, ty = (t >> 1) & 1, tz = DIM == 3 ? t >> 2 : 0;
     const int qx = 2 * cx + tx, qy = 2 * cy + ty, qz = 2 * cz + tz;
-    if (qx >= M || qy >= M || qz >= M) continue;
+    if (!own || qx >= M || qy >= M || qz >= M) continue;
     double s = 0;
 #pragma unroll
     for (int c = 0; c < (1 << DIM); c++) {  // bit set: this lane's cell, else the one below
@@ -2010,27 +2036,39 @@ __global__ __launch_bounds__(256) void k_cell_apply(int n, Div1 dby, Div1 dbx,
                      (DIM == 3 && (qz == 0 || qz == M - 1));
     if (dir) s = (double)x[idx];
     s *= (double)alpha;
-    out[idx] = beta == (T)0 ? (T)s : (T)((double)beta * (double)zv[t] + s);
+    const T o = beta == (T)0 ? (T)s : (T)((double)beta * (double)zv[t] + s);
+    out[idx] = o;
+    if (DOT) d += (double)o * (double)x[idx];
   }
+  if (DOT) block_part(d, dpart);
+}
+
+// the boxes of an A; per axis into by, bx
+static unsigned cell_boxes(const flgpu_mat *A, unsigned &by, unsigned &bx) {
+  const int n = A->lat_n;
+  auto boxes = [&](int B) { return (unsigned)((n + 1 + B - 1) / B); };
+  if (A->lat_dim == 3) {
+    by = boxes(CellBox<3>::B[1]);
+    bx = boxes(CellBox<3>::B[2]);
+    return boxes(CellBox<3>::B[0]) * by * bx;
+  }
+  by = boxes(CellBox<2>::B[1]);
+  bx = boxes(CellBox<2>::B[2]);
+  return by * bx;
 }
 
 template <class T>
 static void launch_cell_apply(const flgpu_mat *A, T alpha, const void *x, T beta, const void *z,
-                              void *out) {
-  const int n = A->lat_n;
-  auto boxes = [&](int B) { return (unsigned)((n + 1 + B - 1) / B); };
-  if (A->lat_dim == 3) {
-    const unsigned bz = boxes(CellBox<3>::B[0]), by = boxes(CellBox<3>::B[1]),
-                   bx = boxes(CellBox<3>::B[2]), nb = bz * by * bx;
-    k_cell_apply<T, 3><<<xcd_grid(nb), 256, 0, A->ctx->stream>>>(
-        n, div1(by), div1(bx), (const T *)A->cell, alpha, (const T *)x, beta,
-        (const T *)z, (T *)out, nb);
-  } else {
-    const unsigned by = boxes(CellBox<2>::B[1]), bx = boxes(CellBox<2>::B[2]), nb = by * bx;
-    k_cell_apply<T, 2><<<xcd_grid(nb), 256, 0, A->ctx->stream>>>(
-        n, div1(by), div1(bx), (const T *)A->cell, alpha, (const T *)x, beta,
-        (const T *)z, (T *)out, nb);
-  }
+                              void *out, double *dpart = nullptr) {
+  unsigned by, bx;
+  const unsigned nb = cell_boxes(A, by, bx);
+  auto launch = [&](auto kern) {
+    kern<<<xcd_grid(nb), 256, 0, A->ctx->stream>>>(A->lat_n, div1(by), div1(bx),
+                                                   (const T *)A->cell, alpha, (const T *)x, beta,
+                                                   (const T *)z, (T *)out, nb, dpart);
+  };
+  if (A->lat_dim == 3) launch(dpart ? k_cell_apply<T, 3, true> : k_cell_apply<T, 3>);
+  else launch(dpart ? k_cell_apply<T, 2, true> : k_cell_apply<T, 2>);
   FLGPU_HIP(hipGetLastError());
 }
 
@@ -2076,21 +2114,46 @@ static long q1_blocks(const flgpu_mat *A, int qzb) {
   return (long)xcd_grid(grid_for((total + 61) / 62 * 64, 256));
 }
 
-bool spmv_dot(const flgpu_mat *A, const void *x, void *out, int slot) {
-  if (!A->alpha || A->tp_kind) return false;
-  long nb = q1_blocks(A, A->prec == FLGPU_F64 ? FLGPU_QZB_F64_SPMV : FLGPU_QZB_F32);
+template <class T>
+static DotParts spmv_dot_t(const flgpu_mat *A, const void *x, void *out, int slot) {
+  // the blocks of the form that spmv would take, 0: the dot is read from the vectors
+  long nb = 0;
+  unsigned by, bx;
+  const bool cell = A->cell && A->lat_dim >= 2 && A->nrows >= kCellApplyRows;
+  if (cell) nb = (long)xcd_grid(cell_boxes(A, by, bx));
+  else if (A->tp_kind) nb = 0;
+  else if (A->alpha) nb = q1_blocks(A, sizeof(T) == 8 ? FLGPU_QZB_F64_SPMV : FLGPU_QZB_F32);
+  else if (A->val27) nb = (long)xcd_grid(grid_for(A->nrows, 256));
+  else if (A->lanes) nb = (long)xcd_grid(grid_for((long)A->nrows * A->lanes, 256));
+  else if (A->sell.nrows == A->nrows) nb = (long)xcd_grid(grid_for(A->sell.nslices, 4));
+  // a CSR product with more blocks than the consumer adds up needs a launch for the sum as well,
+  // and then a pass over the vectors costs no more: 300 007 rows 23 + 4.7 against 24 + 4.5 us
+  if (!cell && A->lanes && nb > kPartsMax) nb = 0;
+  if (nb == 0) {
+    spmv(A, 1.0, x, 0.0, out, out);
+    return dot_parts(A->ctx, A->nrows, A->prec, out, x);
+  }
   flgpu_mat *M = const_cast<flgpu_mat *>(A);
   if (M->dot_np < nb) {
     dev_free(M->dot_part);
+    M->dot_part = nullptr;
+    M->dot_np = 0;
     M->dot_part = (double *)dev_alloc(sizeof(double) * nb);
     M->dot_np = nb;
   }
-  if (A->prec == FLGPU_F64)
-    launch_q1_pass<double, Q1_SPMV>(A, 1.0, 0.0, out, x, out, nullptr, M->dot_part);
-  else
-    launch_q1_pass<float, Q1_SPMV>(A, 1.0f, 0.0f, out, x, out, nullptr, M->dot_part);
-  dot_final(A->ctx, M->dot_part, (int)nb, slot);
-  return true;
+  double *dp = M->dot_part;
+  if (cell) launch_cell_apply<T>(A, (T)1, x, (T)0, out, out, dp);
+  else if (A->alpha) launch_q1_pass<T, Q1_SPMV>(A, (T)1, (T)0, out, x, out, nullptr, dp);
+  else if (A->val27)
+    launch_st27_spmv<T>(A, (T)1, (const T *)x, (T)0, (const T *)out, (T *)out, dp);
+  else if (A->lanes) launch_csr_spmv<T>(A, (T)1, x, (T)0, out, out, dp);
+  else launch_spmv<T>(A->ctx, A->sell, 1.0, x, 0.0, out, out, dp);
+  return dot_parts_bound(A->ctx, dp, nb, slot);
+}
+
+DotParts spmv_dot(const flgpu_mat *A, const void *x, void *out, int slot) {
+  return A->prec == FLGPU_F64 ? spmv_dot_t<double>(A, x, out, slot)
+                              : spmv_dot_t<float>(A, x, out, slot);
 }
 
 void spmv_t(const flgpu_mat *A, double alpha, const void *x, double beta, void *out) {

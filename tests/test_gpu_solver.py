@@ -15,7 +15,7 @@ from gnu_femlisp_amd import flgpu as F
 from gnu_femlisp_amd import iteration as it
 from gnu_femlisp_amd import lattice as lat
 from gnu_femlisp_amd.flgpu import check, lib
-from gnu_femlisp_amd.matlisp import Context, GpuVector, gemm
+from gnu_femlisp_amd.matlisp import Context, GpuSparseMatrix, GpuVector, gemm
 from oracle import pyoracle as po
 
 pytestmark = pytest.mark.gpu
@@ -541,3 +541,67 @@ def test_stencil_sor_cycles_equal_sell_cycles(m, levels, pre, post, prec):
             outs.append((form, x.numpy(), r.numpy()))
     for (_, xa, ra), (_, xb, rb) in zip(outs[:2], outs[2:]):
         assert relerr(xa, xb) < tol and relerr(ra, rb) < tol
+
+
+@pytest.mark.parametrize("n,form,prec", [(2, F.STORAGE_SELL, F.F64), (13, F.STORAGE_CELL, F.F32),
+                                         (20, F.STORAGE_STENCIL, F.F64),
+                                         (80, F.STORAGE_CELL, F.F64), (81, F.STORAGE_SELL, F.F64),
+                                         (81, F.STORAGE_STENCIL, F.F32),
+                                         (93, F.STORAGE_STENCIL, F.F64)])
+def test_cg_recurrence_from_partial_sums(n, form, prec):
+    """plain <cg> with its sums added up from the products' and updates' per-block partials: one
+    or four rows a thread (524 288 rows), partials added up by the consumer or, above 3072 of
+    them, by a reduction; the defects of the first steps against the same recurrence on the host
+    (FP64: they agree to the rounding of a step's sums times the steps; FP32 to 1e-3)"""
+    say(f"cg partial sums n={n} form={form} prec={prec}")
+    rng = np.random.default_rng(n)
+    A, _ = lat.assemble(3, 1, n, np.exp(rng.normal(size=(n,) * 3)), prec=prec)
+    assert A.storage(form) == form
+    rp, ci, v = A.csr()
+    S = sp.csr_matrix((v.astype(float), ci, rp))
+    b = np.zeros((n + 1,) * 3)
+    b[1:n, 1:n, 1:n] = rng.uniform(-1, 1, (n - 1,) * 3)
+    bv = GpuVector.from_array(b.ravel(), prec)
+    steps = 12
+    bb = it.solve(it.LinearSolver(it.CG(), success_if=("<", "reduction", 1e-14),
+                                  failure_if=(">", "step", steps - 1)),
+                  {"matrix": A, "rhs": bv})
+    r = bv.numpy().astype(float)
+    p, x, al, want = r.copy(), np.zeros_like(r), r @ r, [np.sqrt(r @ r)]
+    while len(want) <= min(steps, len(bb["defnorms"]) - 1):
+        a = S @ p
+        lam = al / (a @ p)
+        x, r = x + lam * p, r - lam * a
+        new = r @ r
+        p, al = r + (new / al) * p, new
+        want.append(np.sqrt(new))
+    k = len(want) if n > 2 else 1  # one unknown: exact after a step
+    assert len(bb["defnorms"]) >= k
+    tol = 1e-9 if prec == F.F64 else 1e-3
+    assert np.allclose(bb["defnorms"][:k], want[:k], rtol=tol)
+    if n > 2:
+        assert relerr(bb["solution"].numpy(), x) < tol
+
+
+@pytest.mark.parametrize("order,n,outer", [(2, 24, "fcg"), (2, 24, "cg"), (1, 30, "fcg")])
+def test_krylov_dots_of_other_forms(order, n, outer):
+    """the fused product and dot of the order-2 cell form (2D, 16^2-lane boxes), and of SELL, CSR
+    rows: the same preconditioned solve with the top matrix in its form and as uploaded copy"""
+    say(f"krylov dots order={order} n={n} {outer}")
+    rng = np.random.default_rng(order)
+    kap = np.exp(rng.normal(size=(4 * n, 4 * n)))
+    sm = it.GeometricSSC(1.0) if order == 2 else it.Jacobi(0.6)
+    cs = it.GeometricCS(sm, 1, 1, 0, symmetric=True)
+    H = it.Hierarchy.lattice(cs, 2, order, n // 2, 4, kappa=kap)
+    A = H.top_matrix()
+    rp, ci, v = A.csr()
+    U = GpuSparseMatrix.from_csr(rp, ci, v)
+    itc = it.CG if outer == "cg" else it.FCG
+    res = []
+    for M in (A, U):
+        bb = it.solve(it.LinearSolver(itc(cs), failure_if=(">", "step", 60)),
+                      {"matrix": M, "rhs": H.rhs, "hierarchy": H})
+        assert bb["status"] == "success"
+        res.append(bb)
+    assert res[0]["steps"] == res[1]["steps"]
+    assert relerr(res[0]["solution"].numpy(), res[1]["solution"].numpy()) < 1e-9
