@@ -499,94 +499,93 @@ __global__ __launch_bounds__(256) void k_elem_mfma_bf16(long ncells, int nq, int
 
 // ---- gather (assembly of the global matrix from element matrices) -------------------
 
-// One thread per row: entry (P,Q) = sum over cells containing both DOFs, in
-// ascending cell order, of E[cell][loc(P)][loc(Q)]; then Dirichlet
-// elimination (identity on constrained rows, zeros in their columns) and the
-// load vector rhs_P = f H^d sum_cells m[loc(P)].
-template <class T, class TE>
-__global__ void k_gather(long N, int dim, int order, int n, DevTable pat, const int *rowptr,
-                         const TE *__restrict__ E, int nloc, int ld, T *vals, double rhs_scale,
-                         const double *__restrict__ mload, T *rhs) {
-  long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// Entry (P,Q) = sum over cells containing both DOFs, in ascending cell order, of
+// E[cell][loc(P)][loc(Q)]; then Dirichlet elimination (identity on constrained rows, zeros in
+// their columns) and the load vector rhs_P = f H^d sum_cells m[loc(P)].  G lanes form a row, each
+// every G-th entry: entries are independent, and a row's are stored side by side.  Bound by
+// the reads of E (one per entry and cell).  Order 2, 24^3 cells FP64 100 us, 3^3 cells 5;
+// a thread per row waited for each entry's reads in turn: 452 and 277.
+template <class T, class TE, int DIM, int G>
+__global__ __launch_bounds__(256) void k_gather(long N, int order, int n, DevTable pat,
+                                                const int *__restrict__ rowptr,
+                                                const TE *__restrict__ E, int nloc, int ld,
+                                                T *__restrict__ vals, double rhs_scale,
+                                                const double *__restrict__ mload, T *rhs) {
+  const long r = ((long)blockIdx.x * 256 + threadIdx.x) / G;
+  const int l = threadIdx.x % G;
   if (r >= N) return;
-  int M = pat.nr, nl1 = order + 1;
-  int P[kMaxDim], lo[kMaxDim], hi[kMaxDim], e[kMaxDim];
-  long q = r;
+  const int M = pat.nr, sh = order - 1;  // x / order = x >> sh (order 1 or 2)
+  int P[DIM], q0[DIM], w[DIM], W = 1;
+  unsigned q = (unsigned)r;
   bool rb = false;
-  for (int k = dim - 1; k >= 0; k--) {
-    P[k] = (int)(q % M);
-    q /= M;
-    lo[k] = pat.ptr[P[k]];
-    hi[k] = pat.ptr[P[k] + 1];
-    e[k] = lo[k];
-    if (P[k] == 0 || P[k] == M - 1) rb = true;
+#pragma unroll
+  for (int k = DIM - 1; k >= 0; k--) {
+    P[k] = (int)(q % (unsigned)M);
+    q /= (unsigned)M;
+    const int lo = pat.ptr[P[k]];
+    w[k] = pat.ptr[P[k] + 1] - lo;
+    q0[k] = pat.col[lo];  // a 1-D row's columns are consecutive
+    W *= w[k];
+    rb |= P[k] == 0 || P[k] == M - 1;
   }
-  long nloc2 = (long)nloc * ld;
-  long pos = rowptr[r];
-  for (;;) {
-    int Q[kMaxDim], clo[kMaxDim], chi[kMaxDim], c[kMaxDim];
+  const long nloc2 = (long)nloc * ld;
+  const long pos = rowptr[r];
+  for (int t = l; t < W; t += G) {
+    int Q[DIM], clo[DIM], chi[DIM], u = t;
     bool cb = false, diag = true;
-    for (int k = 0; k < dim; k++) {
-      Q[k] = pat.col[e[k]];
-      if (Q[k] == 0 || Q[k] == M - 1) cb = true;
-      if (Q[k] != P[k]) diag = false;
-      int mx = max(P[k], Q[k]), mn = min(P[k], Q[k]);
-      // cells c with order*c <= mn and mx <= order*c + order
-      clo[k] = (mx <= order) ? 0 : (mx - 1) / order;
-      chi[k] = min(mn / order, n - 1);
-      c[k] = clo[k];
+#pragma unroll
+    for (int k = DIM - 1; k >= 0; k--) {
+      const int uq = u / w[k];
+      Q[k] = q0[k] + u - uq * w[k];
+      u = uq;
+      cb |= Q[k] == 0 || Q[k] == M - 1;
+      diag &= Q[k] == P[k];
+      const int mx = max(P[k], Q[k]), mn = min(P[k], Q[k]);
+      // cells c with order*c <= mn and mx <= order*c + order: one or two
+      clo[k] = mx <= order ? 0 : (mx - 1) >> sh;
+      chi[k] = min(mn >> sh, n - 1);
     }
-    double acc = 0.0;
+    double acc = rb && diag ? 1.0 : 0.0;
     if (!(rb || cb)) {
-      for (;;) {
+      TE v[1 << DIM];
+      bool on[1 << DIM];
+#pragma unroll
+      for (int m = 0; m < (1 << DIM); m++) {
         long cell = 0;
         int la = 0, lb = 0;
-        for (int k = 0; k < dim; k++) {
-          cell = cell * n + c[k];
-          la = la * nl1 + (P[k] - order * c[k]);
-          lb = lb * nl1 + (Q[k] - order * c[k]);
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < DIM; k++) {
+          const int c = clo[k] + ((m >> (DIM - 1 - k)) & 1);
+          ok &= c <= chi[k];
+          cell = cell * n + c;
+          la = la * (order + 1) + (P[k] - order * c);
+          lb = lb * (order + 1) + (Q[k] - order * c);
         }
-        acc += (double)E[cell * nloc2 + (long)la * ld + lb];
-        int k = dim - 1;
-        while (k >= 0 && c[k] == chi[k]) {
-          c[k] = clo[k];
-          k--;
-        }
-        if (k < 0) break;
-        c[k]++;
+        on[m] = ok;
+        v[m] = E[ok ? cell * nloc2 + (long)la * ld + lb : 0];
       }
-    } else {
-      acc = (rb && diag) ? 1.0 : 0.0;
+      acc = 0.0;
+#pragma unroll
+      for (int m = 0; m < (1 << DIM); m++) acc = on[m] ? acc + (double)v[m] : acc;
     }
-    vals[pos++] = (T)acc;
-    int k = dim - 1;
-    while (k >= 0 && e[k] == hi[k] - 1) {
-      e[k] = lo[k];
-      k--;
-    }
-    if (k < 0) break;
-    e[k]++;
+    vals[pos + t] = (T)acc;
   }
-  if (rhs) {
+  if (rhs && l == 0) {
     double b = 0.0;
     if (!rb) {
-      int clo[kMaxDim], chi[kMaxDim], c[kMaxDim];
-      for (int k = 0; k < dim; k++) {
-        clo[k] = (P[k] % order == 0) ? max(P[k] / order - 1, 0) : P[k] / order;
-        chi[k] = (P[k] % order == 0) ? min(P[k] / order, n - 1) : P[k] / order;
-        c[k] = clo[k];
-      }
-      for (;;) {
+#pragma unroll
+      for (int m = 0; m < (1 << DIM); m++) {
         int la = 0;
-        for (int k = 0; k < dim; k++) la = la * nl1 + (P[k] - order * c[k]);
-        b += mload[la];
-        int k = dim - 1;
-        while (k >= 0 && c[k] == chi[k]) {
-          c[k] = clo[k];
-          k--;
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < DIM; k++) {
+          const bool edge = (P[k] & sh) == 0;  // P on a cell boundary: the cells below and above
+          const int hi = P[k] >> sh, c = (edge ? hi - 1 : hi) + ((m >> (DIM - 1 - k)) & 1);
+          ok &= c <= hi;
+          la = la * (order + 1) + (P[k] - order * c);
         }
-        if (k < 0) break;
-        c[k]++;
+        if (ok) b += mload[la];
       }
       b *= rhs_scale;
     }
@@ -935,14 +934,19 @@ static void assemble_values(flgpu_mat *A, const flgpu_vec *kappa, int nk, int mo
                            ctx->stream));
   double rscale = A->lat_f * std::pow(1.0 / n, dim);
   long N = A->nrows;
-  if (A->prec == FLGPU_F64)
-    k_gather<double, double><<<grid_for(N, 128), 128, 0, ctx->stream>>>(
-        N, dim, order, n, dpat, A->rowptr, (const double *)E, R.nloc, ld, (double *)A->vals, rscale,
-        dm, (double *)rhs_dev);
-  else
-    k_gather<float, float><<<grid_for(N, 128), 128, 0, ctx->stream>>>(
-        N, dim, order, n, dpat, A->rowptr, (const float *)E, R.nloc, ld, (float *)A->vals, rscale, dm,
-        (float *)rhs_dev);
+  auto gather = [&](auto t) {
+    using T = decltype(t);
+    auto launch = [&](auto kern, int G) {
+      kern<<<grid_for(N * G, 256), 256, 0, ctx->stream>>>(N, order, n, dpat, A->rowptr,
+                                                          (const T *)E, R.nloc, ld, (T *)A->vals,
+                                                          rscale, dm, (T *)rhs_dev);
+    };
+    if (dim == 3) launch(k_gather<T, T, 3, 64>, 64);
+    else if (dim == 2) launch(k_gather<T, T, 2, 16>, 16);
+    else launch(k_gather<T, T, 1, 4>, 4);
+  };
+  if (A->prec == FLGPU_F64) gather(0.0);
+  else gather(0.0f);
   FLGPU_HIP(hipGetLastError());
   FLGPU_HIP(hipStreamSynchronize(ctx->stream));
   free_table(dpat);

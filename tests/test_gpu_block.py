@@ -6,6 +6,7 @@ import sys
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from gnu_femlisp_amd import flgpu as F
 from gnu_femlisp_amd import iteration as it
@@ -272,3 +273,41 @@ def test_cell_sweeps_equal_csr_sweeps(dim, n0, levels, prec, kind):
             h.apply(x, bv, r)
             out.append(x.numpy())
         assert relerr(out[0], out[1]) < (1e-12 if prec == F.F64 else 2e-5)
+
+
+@pytest.mark.parametrize("dim,n", [(1, 1), (1, 2), (1, 7), (2, 1), (2, 2), (2, 5), (3, 1), (3, 2),
+                                   (3, 3)])
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+def test_order2_assembly_and_inverses_on_small_lattices(dim, n, prec):
+    """rows formed by several lanes (a coefficient finer than the cells) and block inverses in
+    registers, down to lattices whose blocks lie on the boundary only: values against the
+    oracle's, and y = A_BB^-1 r of every vertex block from one <geometric-psc> iterate against
+    numpy's solves (FP64 rounding times the blocks' condition, at most a few hundred)"""
+    say(f"order-2 assembly and inverses dim={dim} n={n} prec={prec}")
+    rng = np.random.default_rng(10 * dim + n)
+    kap = np.exp(rng.normal(size=(2 * n,) * dim))
+    A, b = lat.assemble(dim, 2, n, kap, prec=prec)
+    rp, ci, v = A.csr()
+    orp, oci, ov, ob = po.assemble(dim, 2, n, kap, 1.0)
+    assert np.array_equal(rp, orp) and np.array_equal(ci, oci)
+    tol = 1e-13 if prec == F.F64 else 1e-6
+    assert np.abs(v - ov).max() <= tol * np.abs(ov).max()
+    assert np.abs(b.numpy() - ob).max() <= tol * max(np.abs(ob).max(), 1e-300)
+    # <psc>: x += sum over blocks of A_BB^-1 r_B (omega 1), r = b - A x with x = 0
+    N, M = A.nrows, 2 * n + 1
+    r0 = rng.uniform(-1, 1, N)
+    x, r = GpuVector(N, prec), GpuVector.from_array(r0, prec)
+    bb = GpuVector.from_array(r0, prec)
+    check(lib().flgpu_block_iterate(A.h, F.SMOOTH_PSC, 1.0, 0, x.h, bb.h, r.h))
+    S = sp.csr_matrix((v.astype(float), ci, rp)).toarray()
+    idx = np.stack(np.unravel_index(np.arange(N), (M,) * dim), 1)
+    bd = ((idx == 0) | (idx == M - 1)).any(1)
+    want = np.zeros(N)
+    rr = r0 if prec == F.F64 else r0.astype(np.float32).astype(float)
+    for a in np.ndindex(*(n + 1,) * dim):
+        c = 2 * np.array(a)
+        near = (np.abs(idx - c) <= 1).all(1)
+        ks = np.flatnonzero(near & (~bd | (idx == c).all(1)))
+        want[ks] += np.linalg.solve(S[np.ix_(ks, ks)], rr[ks])
+    t = 1e-11 if prec == F.F64 else 1e-4
+    assert np.abs(x.numpy() - want).max() <= t * np.abs(want).max()
