@@ -240,81 +240,58 @@ __global__ void k_dense_gather(int m, int n, const int *__restrict__ cidx,
 constexpr int kGjB = 64;  // pivots per block
 typedef double v4d __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ double gj_lane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
 // D = C_KK^-1 (bs x bs, bs <= kGjB, zero-padded to kGjB x kGjB) by the unblocked elimination,
-// pivot by pivot; one workgroup.  Thread t holds the entries (t / 64 + 4 u, t % 64), u < 16, in
-// registers; per pivot k the holders of column k and row k publish their values before it
-// (LDS, two buffers by the parity of k, so one barrier per pivot), and every thread forms its
-// new entries with gj_row / gj_entry.
+// pivot by pivot; one workgroup.  Wave w holds the rows 16 w.., a lane a column, in registers.  Per
+// pivot k its row goes through LDS (two buffers, so one barrier a pivot); column k's entries of a
+// wave's rows are lane k's.  The pivots' chain (LDS, barrier, division) bounds it: 26 us, 47
+// with column k through LDS too and its row found by comparing 16 indexes.
 __global__ __launch_bounds__(256) void k_gj_diag(int m, int k0, int bs,
                                                  const double *__restrict__ C,
                                                  double *__restrict__ D, int *bad) {
-  __shared__ double colk[2][kGjB], rowk[2][kGjB];
+  __shared__ double rowk[2][kGjB];
   constexpr int kPer = kGjB * kGjB / 256;
-  const int b = threadIdx.x % kGjB, a0 = threadIdx.x / kGjB;
+  const int b = threadIdx.x % kGjB, w = threadIdx.x / kGjB, a0 = w * kPer;
   double v[kPer];
 #pragma unroll
   for (int u = 0; u < kPer; u++) {
-    const int a = a0 + 4 * u;
+    const int a = a0 + u;
     v[u] = (a < bs && b < bs) ? C[(long)(k0 + a) * m + k0 + b] : 0.0;
   }
-  for (int k = 0; k < bs; k++) {
-    const int par = k & 1;
-    if (b == k) {
+  for (int q = 0; q < kGjB / kPer; q++)
 #pragma unroll
-      for (int u = 0; u < kPer; u++) colk[par][a0 + 4 * u] = v[u];
-    }
-    if (a0 == (k & 3)) {
+    for (int j = 0; j < kPer; j++) {
+      const int k = q * kPer + j;
+      if (k >= bs) break;
+      if (w == q) rowk[j & 1][b] = v[j];
+      __syncthreads();
+      const double rk = rowk[j & 1][b], piv = gj_lane(rk, k);
+      if (threadIdx.x == 0 && piv == 0.0) *bad = 1;
+      const double rkb = gj_row(rk, piv, b == k);
 #pragma unroll
       for (int u = 0; u < kPer; u++)
-        if (u == (k >> 2)) rowk[par][b] = v[u];
+        v[u] = gj_entry(v[u], gj_lane(v[u], k), rkb, w == q && u == j, b == k);
     }
-    __syncthreads();
-    const double piv = colk[par][k];
-    if (threadIdx.x == 0 && piv == 0.0) *bad = 1;
-    const double rkb = gj_row(rowk[par][b], piv, b == k);
 #pragma unroll
-    for (int u = 0; u < kPer; u++) {
-      const int a = a0 + 4 * u;
-      v[u] = gj_entry(v[u], colk[par][a], rkb, a == k, b == k);
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < kPer; u++) D[(a0 + 4 * u) * kGjB + b] = v[u];
+  for (int u = 0; u < kPer; u++) D[(a0 + u) * kGjB + b] = v[u];
 }
 
-// U (m x kGjB) = C_iK D for the rows i outside K and D's rows inside K; R (kGjB x m) = C_KJ
-// before the update (rows and columns beyond bs are zero)
-__global__ __launch_bounds__(256) void k_gj_panels(int m, int k0, int bs,
-                                                   const double *__restrict__ C,
-                                                   const double *__restrict__ D,
-                                                   double *__restrict__ U, double *__restrict__ R) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long nu = (long)m * kGjB;
-  if (e < nu) {
-    const int i = (int)(e / kGjB), c = (int)(e % kGjB);
-    double v = 0.0;
-    if (i >= k0 && i < k0 + bs) {
-      v = D[(i - k0) * kGjB + c];
-    } else if (c < bs) {
-      for (int t = 0; t < bs; t++) v += C[(long)i * m + k0 + t] * D[t * kGjB + c];
-    }
-    U[e] = v;
-  } else if (e < 2 * nu) {
-    const long f = e - nu;
-    const int t = (int)(f / m), j = (int)(f - (long)t * m);
-    R[f] = t < bs ? C[(long)(k0 + t) * m + j] : 0.0;
-  }
-}
-
-// one kGjB x kGjB tile (I, J) of C per workgroup, K = the pivot block:
+// The pivots of the block K = kb, one kGjB x kGjB tile (I, J) of C per workgroup, from Ci into Co:
 //   J == K: C_iK = D_i (i in K) or -U_i (i outside K)
 //   J != K: C_iJ = D_i R_J (i in K) or C_iJ - U_i R_J (i outside K)
-// U_I R_J on FP64 MFMA 16x16x4 from LDS (lane l supplies A[l % 16][l / 16] and
-// B[l / 16][l % 16] and receives C[l / 16 + 4 v][l % 16]); wave w forms the 32 x 32 quarter
-// (w / 2, w % 2) of the tile
-__global__ __launch_bounds__(256) void k_gj_update(int m, int k0, const double *__restrict__ U,
-                                                   const double *__restrict__ R,
-                                                   double *__restrict__ C) {
+// with R = C_KJ before the update and U = C_iK D, which every tile of a row forms for itself (a
+// launch and its pass over C cost more).  Products on FP64 MFMA 16x16x4 (lane l supplies
+// A[l % 16][l / 16] and B[l / 16][l % 16] and receives C[l / 16 + 4 v][l % 16]); wave w forms the
+// 32 x 32 quarter (w / 2, w % 2) of a tile.  1331 unknowns: 23 us a block of pivots, 18 + 18 with
+// U and R by a launch of their own.
+__global__ __launch_bounds__(256) void k_gj_update(int m, int k0, int bs,
+                                                   const double *__restrict__ D,
+                                                   const double *__restrict__ Ci,
+                                                   double *__restrict__ Co) {
   __shared__ double us[kGjB][kGjB + 1];
   __shared__ double rs[kGjB][kGjB + 2];
   const int ntile = (m + kGjB - 1) / kGjB;
@@ -335,21 +312,28 @@ __global__ __launch_bounds__(256) void k_gj_update(int m, int k0, const double *
       for (int v = 0; v < 4; v++) {
         const int i = min(i0 + r0 + 16 * p + kg + 4 * v, m - 1);
         const int j = min(j0 + c0 + 16 * q + li, m - 1);
-        cv[p][q][v] = C[(long)i * m + j];
+        cv[p][q][v] = Ci[(long)i * m + j];
       }
+  // C_IK into us, D into rs; U = us rs into us, then R into rs
 #pragma unroll
   for (int u = 0; u < kPer; u++) {
     const int e = threadIdx.x + 256 * u, a = e / kGjB, b = e % kGjB;
-    us[a][b] = i0 + a < m ? U[(long)(i0 + a) * kGjB + b] : 0.0;
-    rs[a][b] = j0 + b < m ? R[(long)a * m + j0 + b] : 0.0;
+    us[a][b] = I == kb ? D[e] : i0 + a < m && b < bs ? Ci[(long)(i0 + a) * m + k0 + b] : 0.0;
+    if (I != kb) rs[a][b] = D[e];
+  }
+  double rv[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const int e = threadIdx.x + 256 * u, a = e / kGjB, b = e % kGjB;
+    rv[u] = a < bs && j0 + b < m ? Ci[(long)(k0 + a) * m + j0 + b] : 0.0;
   }
   __syncthreads();
   v4d acc[2][2];
+  auto product = [&] {
 #pragma unroll
-  for (int p = 0; p < 2; p++)
+    for (int p = 0; p < 2; p++)
 #pragma unroll
-    for (int q = 0; q < 2; q++) acc[p][q] = v4d{0.0, 0.0, 0.0, 0.0};
-  if (J != kb) {
+      for (int q = 0; q < 2; q++) acc[p][q] = v4d{0.0, 0.0, 0.0, 0.0};
     for (int k = 0; k < kGjB; k += 4)
 #pragma unroll
       for (int p = 0; p < 2; p++)
@@ -357,7 +341,24 @@ __global__ __launch_bounds__(256) void k_gj_update(int m, int k0, const double *
         for (int q = 0; q < 2; q++)
           acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(
               us[r0 + 16 * p + li][k + kg], rs[k + kg][c0 + 16 * q + li], acc[p][q], 0, 0, 0);
+  };
+  if (I != kb) {
+    product();
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) us[r0 + 16 * p + kg + 4 * v][c0 + 16 * q + li] = acc[p][q][v];
   }
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const int e = threadIdx.x + 256 * u;
+    rs[e / kGjB][e % kGjB] = rv[u];
+  }
+  __syncthreads();
+  if (J != kb) product();
 #pragma unroll
   for (int p = 0; p < 2; p++)
 #pragma unroll
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(256) void k_gj_update(int m, int k0, const double *
           double out;
           if (J == kb) out = I == kb ? us[a][b] : -us[a][b];
           else out = I == kb ? acc[p][q][v] : cv[p][q][v] - acc[p][q][v];
-          C[(long)i * m + j] = out;
+          Co[(long)i * m + j] = out;
         }
       }
 }
@@ -383,7 +384,7 @@ static DenseInverse dense_inverse_dev(const flgpu_mat *A) {
   const long nn = (long)n * n;
   hipStream_t s = A->ctx->stream;
   DenseInverse out;
-  double *M0 = nullptr, *D = nullptr, *U = nullptr, *R = nullptr;
+  double *M0 = nullptr, *D = nullptr, *C2 = nullptr;
   int *bad = nullptr, *dt = nullptr;
   try {
     if (n == 0) return out;
@@ -418,16 +419,15 @@ static DenseInverse dense_inverse_dev(const flgpu_mat *A) {
       k_dense_gather<<<grid_for(mm, 256), 256, 0, s>>>(m, n, out.cidx, M0, out.inv);
       FLGPU_HIP(hipGetLastError());
       D = (double *)dev_alloc(sizeof(double) * kGjB * kGjB);
-      U = (double *)dev_alloc(sizeof(double) * (size_t)m * kGjB);
-      R = (double *)dev_alloc(sizeof(double) * (size_t)m * kGjB);
+      C2 = (double *)dev_alloc(sizeof(double) * mm);
       bad = (int *)dev_alloc(sizeof(int));
       FLGPU_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
       const int ntile = (m + kGjB - 1) / kGjB;
       for (int k0 = 0; k0 < m; k0 += kGjB) {
         const int bs = std::min(kGjB, m - k0);
         k_gj_diag<<<1, 256, 0, s>>>(m, k0, bs, out.inv, D, bad);
-        k_gj_panels<<<grid_for(2L * m * kGjB, 256), 256, 0, s>>>(m, k0, bs, out.inv, D, U, R);
-        k_gj_update<<<(unsigned)(ntile * ntile), 256, 0, s>>>(m, k0, U, R, out.inv);
+        k_gj_update<<<(unsigned)(ntile * ntile), 256, 0, s>>>(m, k0, bs, D, out.inv, C2);
+        std::swap(out.inv, C2);
       }
       FLGPU_HIP(hipGetLastError());
       int hbad = 0;
@@ -440,8 +440,7 @@ static DenseInverse dense_inverse_dev(const flgpu_mat *A) {
     dev_free(M0);
     dev_free(dt);
     dev_free(D);
-    dev_free(U);
-    dev_free(R);
+    dev_free(C2);
     dev_free(bad);
     out.release();
     throw;
@@ -449,8 +448,7 @@ static DenseInverse dense_inverse_dev(const flgpu_mat *A) {
   dev_free(M0);
   dev_free(dt);
   dev_free(D);
-  dev_free(U);
-  dev_free(R);
+  dev_free(C2);
   dev_free(bad);
   return out;
 }

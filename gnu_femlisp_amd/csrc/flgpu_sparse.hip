@@ -2799,85 +2799,147 @@ __global__ __launch_bounds__(kRapB) void k_rap_lds(
   for (int j = 0; j < w; j++) acc[c0 + j] = sacc[j * kRapB + tid];
 }
 
-// The same product on 3D Q1 lattices, one thread per coarse entry (k, n): the fine matrix holds
-// the lattice pattern (every lattice neighbour, ascending), P the pattern of the lattice
-// interpolation (fine node m takes the coarse nodes floor(m / 2) and ceil(m / 2) per axis,
-// ascending) and the coarse matrix the coarse lattice pattern, so every position is computed
-// instead of searched, the row starts included.  The entry sums the contributions
-// (P_lk A_lm) P_mn of the fine l around 2k (ascending) and the m next to l and to 2n
-// (ascending): exactly the contributions, in the order, that k_rap's loops bring to this
-// entry, so the sums are equal bit for bit.
-__device__ __forceinline__ int lat_pos3(const int lo[3], const int cnt[3], int a, int b, int c) {
-  return ((a - lo[0]) * cnt[1] + (b - lo[1])) * cnt[2] + (c - lo[2]);
+// the contributions of one l (offset LE of the 27), entry by entry of A's row: which of its
+// entries, which entry c of the coarse row, which plane of t27
+struct RapList {
+  int n = 0;
+  signed char e[125] = {}, d[125] = {}, p[125] = {};
+};
+// The coarse entries (k, n), n >= k, are shared out to three threads of 343 to 486 contributions:
+// the diagonal, the faces' and the edges' and corners' neighbours
+constexpr int rap_group(int d) {
+  const int far = (d / 9 != 1) + ((d / 3) % 3 != 1) + (d % 3 != 1);
+  return far < 2 ? far : 2;
+}
+constexpr RapList rap_list(int le, int g) {
+  RapList q;
+  const int L[3] = {le / 9 - 1, (le / 3) % 3 - 1, le % 3 - 1};
+  for (int e = 0; e < 27; e++) {
+    const int E[3] = {e / 9 - 1, (e / 3) % 3 - 1, e % 3 - 1};
+    for (int d = 13; d < 27; d++) {
+      if (rap_group(d) != g) continue;
+      const int D[3] = {d / 9 - 1, (d / 3) % 3 - 1, d % 3 - 1};
+      bool near = true;
+      int plane = 0;
+      for (int a = 0; a < 3; a++) {
+        const int o = L[a] + E[a] - 2 * D[a];
+        near = near && o >= -1 && o <= 1;
+        plane = plane * 3 + o + 1;
+      }
+      if (!near) continue;
+      q.e[q.n] = (signed char)e;
+      q.d[q.n] = (signed char)d;
+      q.p[q.n] = (signed char)plane;
+      q.n++;
+    }
+  }
+  return q;
 }
 
-// the first entry of row (z, y, x) of a tensor product of 1-D patterns: pre[a] entries precede
-// the row's coordinate on axis a, which has cnt[a] entries; nnz1 per 1-D pattern
-__device__ __forceinline__ long tp_row_start(const long pre[3], const int cnt[3], long nnz1) {
-  return (pre[0] * nnz1 + cnt[0] * pre[1]) * nnz1 + (long)cnt[0] * cnt[1] * pre[2];
+// l = 2k + offset LE: its loads, then its contributions in order
+template <class T, int G, int LE, int... C>
+__device__ __forceinline__ void rap_step(int M, const int (&K)[3], unsigned k, unsigned i0,
+                                         size_t N, unsigned Nc, const T *a27, const T *t27,
+                                         const unsigned (&nn)[27], double (&s)[27],
+                                         std::integer_sequence<int, C...>) {
+  if constexpr (sizeof...(C) == 0) return;  // l reaches none of the group's entries
+  else {
+    constexpr RapList Q = rap_list(LE, G);
+    constexpr int L[3] = {LE / 9 - 1, (LE / 3) % 3 - 1, LE % 3 - 1};
+    bool in = true;
+#pragma unroll
+    for (int a = 0; a < 3; a++) in &= 2 * K[a] + L[a] >= 0 && 2 * K[a] + L[a] < M;
+    const unsigned l = in ? i0 + (unsigned)((L[0] * M + L[1]) * M + L[2]) : i0;
+    asm volatile("" ::: "memory");  // P's values are loaded for every l: kept, they'd spill
+    const double plk = in ? (double)t27[(size_t)LE * Nc + k] : 0.0;
+    T av[27];
+#pragma unroll
+    for (int e = 0; e < 27; e++) av[e] = a27[(size_t)e * N + l];
+    T pv[sizeof...(C)];
+    ((pv[C] = t27[(size_t)Q.p[C] * Nc + nn[(int)Q.d[C]]]), ...);
+    asm volatile("" ::: "memory");
+    ((s[(int)Q.d[C]] += (plk * (double)av[(int)Q.e[C]]) * (double)pv[C]), ...);
+    // the sums stay here: sunk to the stores, which are conditional, they'd keep every load alive
+#pragma unroll
+    for (int d = 13; d < 27; d++)
+      if (rap_group(d) == G) asm volatile("" : "+v"(s[d]));
+  }
+}
+
+// The same product on 3D Q1 lattices, a few threads per coarse node k: the fine matrix holds the
+// lattice pattern and its values as 27 planes (a27), P the pattern of the lattice interpolation
+// (fine node m takes the coarse nodes floor(m / 2) and ceil(m / 2) per axis) and its transpose's
+// values as 27 planes (t27: plane of offset e holds P(2c + e, c)), the coarse matrix the coarse
+// lattice pattern.  With l = 2k + a, m = l + b and n = k + c every offset is a constant of the
+// unrolled loops, so a contribution (P_lk A_lm) P_mn is two multiplications and its loads, which
+// neighbouring threads make side by side.  An entry sums its contributions in ascending l, then
+// m: the order that k_rap's loops bring them in, so the sums are equal bit for bit.  A and P are 0
+// where l or m is outside the lattice.  A is exactly symmetric: only entries n >= k are formed, and
+// written to (n, k) too.  Bound by the loads of P's values, one per contribution (1270 a row), and
+// the conversions to FP64; on small lattices by the 27 l's load latencies.  49^3 coarse nodes, FP32
+// 257 us, 7^3 21: a thread per entry that computed every position, the mirrored triangle and the
+// values took three launches, 1168 + 79 + 13 and 78 + 9 + 2.
+template <class T, int G, int... LE>
+__device__ __forceinline__ void rap_row(int Mc, unsigned k, const int (&K)[3], const T *a27,
+                                        const T *t27, const int *__restrict__ crp, T *cv,
+                                        std::integer_sequence<int, LE...>) {
+  const int M = 2 * Mc - 1;
+  const unsigned Nc = (unsigned)Mc * (unsigned)Mc * (unsigned)Mc;
+  const size_t N = (size_t)M * M * M;
+  const unsigned i0 = ((unsigned)(2 * K[0]) * (unsigned)M + (unsigned)(2 * K[1])) * (unsigned)M +
+                      (unsigned)(2 * K[2]);
+  unsigned nn[27];  // the coarse neighbours, k itself for those outside
+#pragma unroll
+  for (int d = 0; d < 27; d++) {
+    const int D[3] = {d / 9 - 1, (d / 3) % 3 - 1, d % 3 - 1};
+    bool in = true;
+#pragma unroll
+    for (int a = 0; a < 3; a++) in &= K[a] + D[a] >= 0 && K[a] + D[a] < Mc;
+    nn[d] = in ? k + (unsigned)((D[0] * Mc + D[1]) * Mc + D[2]) : k;
+  }
+  double s[27] = {};
+  (rap_step<T, G, LE>(M, K, k, i0, N, Nc, a27, t27, nn, s,
+                          std::make_integer_sequence<int, rap_list(LE, G).n>()),
+   ...);
+  // a coarse row's entries: the neighbours within the lattice, ascending
+  int cnt[3], lo[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    lo[a] = K[a] > 0 ? -1 : 0;
+    cnt[a] = (K[a] < Mc - 1 ? 1 : 0) - lo[a] + 1;
+  }
+  const int row = crp[k];
+#pragma unroll
+  for (int d = 13; d < 27; d++) {
+    if (rap_group(d) != G) continue;
+    const int D[3] = {d / 9 - 1, (d / 3) % 3 - 1, d % 3 - 1};
+    bool in = true;
+    int pos = 0, back = 0;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      const int n = K[a] + D[a];
+      in &= n >= 0 && n < Mc;
+      pos = pos * cnt[a] + D[a] - lo[a];
+      const int nlo = n > 0 ? -1 : 0;  // k's place in row n
+      back = back * ((n < Mc - 1 ? 1 : 0) - nlo + 1) - D[a] - nlo;
+    }
+    if (!in) continue;
+    cv[row + pos] = (T)s[d];
+    if (d > 13) cv[crp[nn[d]] + back] = (T)s[d];
+  }
 }
 
 template <class T>
-__global__ __launch_bounds__(256) void k_rap_q1(int Mc, int M, const T *__restrict__ av,
-                                                const T *__restrict__ pv,
-                                                const int *__restrict__ crp, double *acc,
-                                                int upper) {
-  // the 1-D patterns: A's row i holds i - 1, i, i + 1 within the lattice (3 M - 2 entries,
-  // 3 i - 1 of them before row i > 0); P's row i holds i / 2 and, for odd i, i / 2 + 1
-  // (3 Mc - 2 entries, i + i / 2 before row i)
-  const long nA = 3L * M - 2, nP = 3L * Mc - 2;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long Nc = (long)Mc * Mc * Mc;
-  if (t >= Nc * 27) return;
-  const int k = (int)(t / 27), d = (int)(t - (long)k * 27);
-  const int K[3] = {k / (Mc * Mc), (k / Mc) % Mc, k % Mc};
-  const int D[3] = {d / 9 - 1, (d / 3) % 3 - 1, d % 3 - 1};
-  int Nn[3], clo[3], ccnt[3];
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    Nn[a] = K[a] + D[a];
-    if (Nn[a] < 0 || Nn[a] >= Mc) return;
-    clo[a] = K[a] > 0 ? -1 : 0;
-    ccnt[a] = (K[a] < Mc - 1 ? 1 : 0) - clo[a] + 1;
-  }
-  const int n = (Nn[0] * Mc + Nn[1]) * Mc + Nn[2];
-  if (upper && n < k) return;  // the lower triangle is mirrored afterwards
-  double s = 0.0;
-  const int l0[3] = {max(2 * K[0] - 1, 0), max(2 * K[1] - 1, 0), max(2 * K[2] - 1, 0)};
-  const int l1[3] = {min(2 * K[0] + 1, M - 1), min(2 * K[1] + 1, M - 1), min(2 * K[2] + 1, M - 1)};
-  for (int lz = l0[0]; lz <= l1[0]; lz++)
-    for (int ly = l0[1]; ly <= l1[1]; ly++)
-      for (int lx = l0[2]; lx <= l1[2]; lx++) {
-        const int L[3] = {lz, ly, lx};
-        // P_lk: row l holds floor(l / 2) (and ceil(l / 2) on odd coordinates) per axis
-        int plo[3], pcnt[3], alo[3], acnt[3], m0[3], m1[3];
-        long ppre[3], apre[3];
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-          plo[a] = L[a] >> 1;
-          pcnt[a] = (L[a] & 1) + 1;
-          ppre[a] = L[a] + (L[a] >> 1);
-          alo[a] = L[a] > 0 ? L[a] - 1 : 0;
-          acnt[a] = min(L[a] + 1, M - 1) - alo[a] + 1;
-          apre[a] = L[a] > 0 ? 3L * L[a] - 1 : 0;
-          m0[a] = max(max(L[a] - 1, 2 * Nn[a] - 1), 0);
-          m1[a] = min(min(L[a] + 1, 2 * Nn[a] + 1), M - 1);
-        }
-        const double plk =
-            (double)pv[tp_row_start(ppre, pcnt, nP) + lat_pos3(plo, pcnt, K[0], K[1], K[2])];
-        const long ab = tp_row_start(apre, acnt, nA);
-        for (int mz = m0[0]; mz <= m1[0]; mz++)
-          for (int my = m0[1]; my <= m1[1]; my++)
-            for (int mx = m0[2]; mx <= m1[2]; mx++) {
-              const double w = plk * (double)av[ab + lat_pos3(alo, acnt, mz, my, mx)];
-              const int qlo[3] = {mz >> 1, my >> 1, mx >> 1};
-              const int qcnt[3] = {(mz & 1) + 1, (my & 1) + 1, (mx & 1) + 1};
-              const long qpre[3] = {mz + (mz >> 1), my + (my >> 1), mx + (mx >> 1)};
-              s += w * (double)pv[tp_row_start(qpre, qcnt, nP) +
-                                  lat_pos3(qlo, qcnt, Nn[0], Nn[1], Nn[2])];
-            }
-      }
-  acc[crp[k] + lat_pos3(clo, ccnt, D[0], D[1], D[2])] = s;
+__global__ __launch_bounds__(64, sizeof(T) == 4 ? 2 : 1) void k_rap_q1(
+    int Mc, FastDiv dMc, const T *a27, const T *t27, const int *__restrict__ crp, T *cv) {
+  const unsigned k = blockIdx.x * 64 + threadIdx.x;
+  if (k >= (unsigned)Mc * (unsigned)Mc * (unsigned)Mc) return;
+  int K[3];
+  lat_decode(k, dMc, K[0], K[1], K[2]);
+  const auto all = std::make_integer_sequence<int, 27>();
+  if (blockIdx.y == 0) rap_row<T, 0>(Mc, k, K, a27, t27, crp, cv, all);
+  else if (blockIdx.y == 1) rap_row<T, 1>(Mc, k, K, a27, t27, crp, cv, all);
+  else rap_row<T, 2>(Mc, k, K, a27, t27, crp, cv, all);
 }
 
 // the longest row: a grid of at most 1024 blocks strides over the rows, each block reduces its
@@ -3021,33 +3083,36 @@ void galerkin_product(const flgpu_mat *P, const flgpu_mat *A, flgpu_mat *Ac, boo
   FLGPU_REQUIRE(Ac->nrows == P->ncols && Ac->ncols == P->ncols, "galerkin: Ac does not match P");
   FLGPU_REQUIRE(P->prec == A->prec && A->prec == Ac->prec, "galerkin: precisions differ");
   flgpu_ctx *ctx = A->ctx;
+  const int nc = Ac->nrows;
+  // the structured product: 3D Q1, the fine lattice of an even n in stencil storage, whose values
+  // are exactly symmetric, the patterns' sizes as the lattices give them
+  const long nf = A->lat_n, ncl = nf / 2;
+  const flgpu_mat *PT = P->transpose;
+  if (lattice && is_q1_lattice(A) && A->val27 && A->st_sym && nf % 2 == 0 && PT && PT->tp_kind == 2 &&
+      PT->tp27 && PT->tp_nc == ncl && A->nnz == (3 * nf + 1) * (3 * nf + 1) * (3 * nf + 1) &&
+      Ac->nrows == (ncl + 1) * (ncl + 1) * (ncl + 1) &&
+      Ac->nnz == (3 * ncl + 1) * (3 * ncl + 1) * (3 * ncl + 1)) {
+    auto run = [&](auto t) {
+      using T = decltype(t);
+      k_rap_q1<T><<<dim3(grid_for(nc, 64), 3), 64, 0, ctx->stream>>>(
+          (int)ncl + 1, fast_div((unsigned)ncl + 1), (const T *)A->val27, (const T *)PT->tp27,
+          Ac->rowptr, (T *)Ac->vals);
+    };
+    if (A->prec == FLGPU_F64) run(0.0);
+    else run(0.0f);
+    FLGPU_HIP(hipGetLastError());
+    return;
+  }
   double *acc = (double *)dev_alloc(sizeof(double) * std::max<long>(Ac->nnz, 1));
   int *bad = (int *)dev_alloc(sizeof(int));
   FLGPU_HIP(hipMemsetAsync(bad, 0, sizeof(int), ctx->stream));
-  int nc = Ac->nrows;
   int *missing = (int *)dev_alloc(sizeof(int));
-  // the structured product: 3D Q1, the fine lattice of an even n, the patterns' sizes as the
-  // lattices give them
-  const long nf = A->lat_n, ncl = nf / 2;
-  const bool q1 = lattice && is_q1_lattice(A) && nf % 2 == 0 &&
-                  A->nnz == (3 * nf + 1) * (3 * nf + 1) * (3 * nf + 1) &&
-                  Ac->nrows == (ncl + 1) * (ncl + 1) * (ncl + 1) &&
-                  Ac->nnz == (3 * ncl + 1) * (3 * ncl + 1) * (3 * ncl + 1) &&
-                  P->nnz == (3 * ncl + 1) * (3 * ncl + 1) * (3 * ncl + 1);
-  if (!q1) mat_build_transpose(P);  // the general product walks the rows of P^T
-  const flgpu_mat *PT = P->transpose;
-  const bool lds = !q1 && max_row_length(Ac) <= kRapW;
+  mat_build_transpose(P);  // the product walks the rows of P^T
+  PT = P->transpose;
+  const bool lds = max_row_length(Ac) <= kRapW;
   auto rap = [&](int upper) {
     const unsigned gl = (unsigned)((nc + kRapB - 1) / kRapB);
-    if (q1 && A->prec == FLGPU_F64)
-      k_rap_q1<double><<<grid_for(27L * nc, 256), 256, 0, ctx->stream>>>(
-          (int)ncl + 1, (int)nf + 1, (const double *)A->vals, (const double *)P->vals,
-          Ac->rowptr, acc, upper);
-    else if (q1)
-      k_rap_q1<float><<<grid_for(27L * nc, 256), 256, 0, ctx->stream>>>(
-          (int)ncl + 1, (int)nf + 1, (const float *)A->vals, (const float *)P->vals,
-          Ac->rowptr, acc, upper);
-    else if (lds && A->prec == FLGPU_F64)
+    if (lds && A->prec == FLGPU_F64)
       k_rap_lds<double><<<gl, kRapB, 0, ctx->stream>>>(
           nc, PT->rowptr, PT->colidx, (const double *)PT->vals, A->rowptr, A->colidx,
           (const double *)A->vals, P->rowptr, P->colidx, (const double *)P->vals, Ac->rowptr,
@@ -3070,10 +3135,7 @@ void galerkin_product(const flgpu_mat *P, const flgpu_mat *A, flgpu_mat *Ac, boo
     FLGPU_HIP(hipGetLastError());
   };
   int hmiss = 1;
-  // a lattice matrix's stencil form records whether its values are exactly symmetric (the
-  // same comparison of A(i, j) with A(j, i) over the same entries, made when it was filled)
-  const bool sym = (q1 && A->val27) ? A->st_sym : csr_symmetric(A);
-  if (sym) {
+  if (csr_symmetric(A)) {
     FLGPU_HIP(hipMemsetAsync(missing, 0, sizeof(int), ctx->stream));
     rap(1);
     k_mirror<<<grid_for(nc, 128), 128, 0, ctx->stream>>>(nc, Ac->rowptr, Ac->colidx, acc,

@@ -605,3 +605,39 @@ def test_krylov_dots_of_other_forms(order, n, outer):
         res.append(bb)
     assert res[0]["steps"] == res[1]["steps"]
     assert relerr(res[0]["solution"].numpy(), res[1]["solution"].numpy()) < 1e-9
+
+
+@pytest.mark.parametrize("n,prec", [(2, F.F64), (4, F.F64), (5, F.F64), (6, F.F32), (9, F.F64)])
+def test_dense_inverse_block_edges(n, prec):
+    """the dense coarse inverse where a block of 64 pivots is one pivot (n = 2: one unknown), less
+    than a block (27), exactly one (64), just more than one (125: tiles of the second block, the
+    whole update out of place) and eight (512), against scipy's sparse LU on the matrix values"""
+    say(f"dense inverse n={n} prec={prec}")
+    rng = np.random.default_rng(n)
+    kap = np.exp(rng.normal(scale=1.5, size=(n,) * 3))
+    cs = it.GeometricCS(it.Jacobi(0.9), 2, 2, 0, prec=prec)
+    H = it.Hierarchy.lattice(cs, 3, 1, n, 1, kappa=kap)
+    A = H.top_matrix()
+    rp, ci, v = A.csr()
+    S = sp.csc_matrix(sp.csr_matrix((v.astype(float), ci, rp)))
+    b = rng.uniform(-1, 1, A.nrows).astype(np.float32).astype(float)
+    x, r, bv = GpuVector(A.nrows, prec), GpuVector.from_array(b, prec), GpuVector.from_array(b, prec)
+    check(lib().flgpu_mg_apply(H.h, x.h, bv.h, r.h))
+    assert relerr(x.numpy(), spla.splu(S).solve(b)) < (1e-11 if prec == F.F64 else 1e-5)
+
+
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("n", [2, 4, 6, 34])
+def test_blackbox_interpolation_on_edge_lattices(n, prec):
+    """the operator-dependent weights by the nodes' parities: lattices with one interior coarse
+    node or none, and one whose passes end inside a block, against the oracle"""
+    say(f"blackbox edges n={n} prec={prec}")
+    rng = np.random.default_rng(n)
+    A, _ = lat.assemble(3, 1, n, np.exp(rng.normal(scale=2.0, size=(n,) * 3)), prec=prec)
+    P = lat.interpolation(3, 1, n // 2, prec=prec)
+    lat.blackbox_interpolation(A, P)
+    rp, ci, v = A.csr()
+    brp, bci, bv = po.blackbox_interpolation(n, rp, ci, v.astype(np.float64))
+    prp, pci, pv = P.csr()
+    assert np.array_equal(prp, brp) and np.array_equal(pci, bci)
+    assert np.abs(pv - bv).max() <= (1e-13 if prec == F.F64 else 1e-6)
