@@ -30,6 +30,52 @@ void dev_free(void *p) {
   if (p) (void)hipFree(p);
 }
 
+void scratch_release(flgpu_ctx *ctx) {
+  for (auto &b : ctx->scratch_free) dev_free(b.second);
+  ctx->scratch_free.clear();
+  ctx->scratch_held = 0;
+}
+
+void *scratch_get(flgpu_ctx *ctx, size_t bytes) {
+  bytes = (std::max(bytes, (size_t)1) + 255) & ~(size_t)255;
+  auto &f = ctx->scratch_free;
+  // the smallest free block that holds it, unless most of that would lie idle
+  size_t best = f.size();
+  for (size_t i = 0; i < f.size(); i++)
+    if (f[i].first >= bytes && f[i].first <= 2 * bytes + 4096 &&
+        (best == f.size() || f[i].first < f[best].first))
+      best = i;
+  void *p = nullptr;
+  size_t n = bytes;
+  ctx->scratch_used.reserve(ctx->scratch_used.size() + 1);
+  if (best < f.size()) {
+    n = f[best].first;
+    p = f[best].second;
+    f[best] = f.back();
+    f.pop_back();
+    ctx->scratch_held -= n;
+  } else if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    scratch_release(ctx);
+    p = dev_alloc(bytes);
+  }
+  ctx->scratch_used[p] = n;
+  return p;
+}
+
+void scratch_put(flgpu_ctx *ctx, void *p) {
+  if (!p) return;
+  auto it = ctx->scratch_used.find(p);
+  const size_t n = it->second;
+  ctx->scratch_used.erase(it);
+  if (ctx->scratch_held + n > kScratchKeep) {
+    dev_free(p);
+    return;
+  }
+  ctx->scratch_free.emplace_back(n, p);
+  ctx->scratch_held += n;
+}
+
 constexpr int kRedBlocks = 1024;
 constexpr int kRedThreads = 256;
 constexpr int kRedSlots = 64;
@@ -489,6 +535,7 @@ extern "C" int flgpu_ctx_destroy(flgpu_ctx *ctx) {
     dev_free(ctx->red_partial);
     dev_free(ctx->red_out);
     dev_free(ctx->solve_buf);
+    scratch_release(ctx);
     if (ctx->host_out) (void)hipHostFree(ctx->host_out);
     if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
     if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);

@@ -6,6 +6,8 @@
 #include <cstdint>
 #include <mutex>
 #include <string>
+#include <unordered_map>
+#include <utility>
 #include <vector>
 
 #include "../../include/flgpu.h"
@@ -60,6 +62,23 @@ int guard(F &&f) {
 // ---- device buffers ---------------------------------------------------------
 
 void *dev_alloc(size_t bytes);
+// Device memory for work on ctx's stream, under its lock.  A block given back is handed out again
+// without waiting for the work that used it, since the next user's follows on the same stream.  At
+// most kScratchKeep bytes of free blocks are kept; they are released with the context, or when an
+// allocation fails.
+constexpr size_t kScratchKeep = (size_t)1 << 30;
+void *scratch_get(flgpu_ctx *ctx, size_t bytes);
+void scratch_put(flgpu_ctx *ctx, void *p);
+void scratch_release(flgpu_ctx *ctx);
+template <class T>
+struct Scratch {  // n values of T for a scope
+  flgpu_ctx *ctx;
+  T *p;
+  Scratch(flgpu_ctx *c, size_t n) : ctx(c), p((T *)scratch_get(c, sizeof(T) * n)) {}
+  ~Scratch() { scratch_put(ctx, p); }
+  Scratch(const Scratch &) = delete;
+  Scratch &operator=(const Scratch &) = delete;
+};
 void dev_free(void *p);
 inline size_t prec_bytes(int prec) { return prec == FLGPU_F64 ? 8 : 4; }
 
@@ -125,6 +144,11 @@ struct flgpu_ctx {
   // flgpu_solve's work vectors, kept between solves (the context lock serialises solves)
   void *solve_buf = nullptr;
   size_t solve_bytes = 0;
+  // temporaries of the assembly and the hierarchies' setup (scratch_get): blocks in use with
+  // their sizes, and free ones kept for the next call
+  std::unordered_map<void *, size_t> scratch_used;
+  std::vector<std::pair<size_t, void *>> scratch_free;
+  size_t scratch_held = 0;  // bytes in scratch_free
   std::string name;
 };
 

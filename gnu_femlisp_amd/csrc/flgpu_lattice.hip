@@ -102,7 +102,7 @@ struct RefElement {
   std::vector<double> m;  // [nloc]: sum_q w_q phi_a(q)  (load vector of f = 1)
 };
 
-static RefElement ref_element(int dim, int order) {
+static RefElement make_ref_element(int dim, int order) {
   RefElement R;
   R.dim = dim;
   R.order = order;
@@ -150,6 +150,14 @@ static RefElement ref_element(int dim, int order) {
     R.T[(size_t)R.nq * R.nloc2 + b] = sum;
   }
   return R;
+}
+
+// the tables of a dimension and order (1 to 3, 1 or 2), formed once
+static const RefElement &ref_element(int dim, int order) {
+  static const RefElement R[6] = {make_ref_element(1, 1), make_ref_element(1, 2),
+                                  make_ref_element(2, 1), make_ref_element(2, 2),
+                                  make_ref_element(3, 1), make_ref_element(3, 2)};
+  return R[2 * (dim - 1) + order - 1];
 }
 
 // ---- 1-D tables --------------------------------------------------------------------
@@ -506,7 +514,7 @@ __global__ __launch_bounds__(256) void k_elem_mfma_bf16(long ncells, int nq, int
 // the reads of E (one per entry and cell).  Order 2, 24^3 cells FP64 100 us, 3^3 cells 5;
 // a thread per row waited for each entry's reads in turn: 452 and 277.
 template <class T, class TE, int DIM, int G>
-__global__ __launch_bounds__(256) void k_gather(long N, int order, int n, DevTable pat,
+__global__ __launch_bounds__(256) void k_gather(long N, int order, int n,
                                                 const int *__restrict__ rowptr,
                                                 const TE *__restrict__ E, int nloc, int ld,
                                                 T *__restrict__ vals, double rhs_scale,
@@ -514,7 +522,7 @@ __global__ __launch_bounds__(256) void k_gather(long N, int order, int n, DevTab
   const long r = ((long)blockIdx.x * 256 + threadIdx.x) / G;
   const int l = threadIdx.x % G;
   if (r >= N) return;
-  const int M = pat.nr, sh = order - 1;  // x / order = x >> sh (order 1 or 2)
+  const int M = order * n + 1, sh = order - 1;  // x / order = x >> sh (order 1 or 2)
   int P[DIM], q0[DIM], w[DIM], W = 1;
   unsigned q = (unsigned)r;
   bool rb = false;
@@ -522,9 +530,10 @@ __global__ __launch_bounds__(256) void k_gather(long N, int order, int n, DevTab
   for (int k = DIM - 1; k >= 0; k--) {
     P[k] = (int)(q % (unsigned)M);
     q /= (unsigned)M;
-    const int lo = pat.ptr[P[k]];
-    w[k] = pat.ptr[P[k] + 1] - lo;
-    q0[k] = pat.col[lo];  // a 1-D row's columns are consecutive
+    // the nodes that share a cell with P: two away for a node on a cell boundary of order 2
+    const int reach = order == 2 && !(P[k] & 1) ? 2 : 1;
+    q0[k] = max(P[k] - reach, 0);
+    w[k] = min(P[k] + reach, M - 1) - q0[k] + 1;
     W *= w[k];
     rb |= P[k] == 0 || P[k] == M - 1;
   }
@@ -833,9 +842,9 @@ static void element_matrices(flgpu_ctx *ctx, const RefElement &R, int n, const f
   long ncells = ipow(n, dim);
   double H = 1.0 / n;
   double scale = std::pow(H, dim - 2);
-  double *dS = (double *)dev_alloc(sizeof(double) * ncells * R.nq);
-  double *dT = (double *)dev_alloc(sizeof(double) * R.T.size());
-  double *dg = (double *)dev_alloc(sizeof(double) * R.s);
+  Scratch<double> S(ctx, (size_t)ncells * R.nq), Tt(ctx, R.T.size()), pts(ctx, R.s);
+  double *dS = S.p, *dT = Tt.p, *dg = pts.p;
+  // R lives as long as the process: the copies need not be waited for
   FLGPU_HIP(hipMemcpyAsync(dT, R.T.data(), sizeof(double) * R.T.size(), hipMemcpyHostToDevice,
                            ctx->stream));
   FLGPU_HIP(hipMemcpyAsync(dg, R.pts, sizeof(double) * R.s, hipMemcpyHostToDevice, ctx->stream));
@@ -857,10 +866,6 @@ static void element_matrices(flgpu_ctx *ctx, const RefElement &R, int n, const f
           ncells, R.nq, R.nloc2, dS, dT, (float *)E, L);
   }
   FLGPU_HIP(hipGetLastError());
-  FLGPU_HIP(hipStreamSynchronize(ctx->stream));
-  dev_free(dS);
-  dev_free(dT);
-  dev_free(dg);
 }
 
 // 3D Q1: the one-pass assembly (k_asm_q1)
@@ -868,46 +873,30 @@ static void assemble_values_q1(flgpu_mat *A, const flgpu_vec *kappa, int nk, int
                                void *rhs_dev) {
   flgpu_ctx *ctx = A->ctx;
   const int n = A->lat_n;
-  RefElement R = ref_element(3, 1);
-  double *dT = (double *)dev_alloc(sizeof(double) * R.T.size());
-  double *dg = nullptr, *dm = nullptr;
-  try {
-    dg = (double *)dev_alloc(sizeof(double) * R.s);
-    dm = (double *)dev_alloc(sizeof(double) * R.nloc);
-    FLGPU_HIP(hipMemcpyAsync(dT, R.T.data(), sizeof(double) * R.T.size(), hipMemcpyHostToDevice,
-                             ctx->stream));
-    FLGPU_HIP(hipMemcpyAsync(dg, R.pts, sizeof(double) * R.s, hipMemcpyHostToDevice,
-                             ctx->stream));
-    FLGPU_HIP(hipMemcpyAsync(dm, R.m.data(), sizeof(double) * R.nloc, hipMemcpyHostToDevice,
-                             ctx->stream));
-    const int nbpa = (n + 1 + kAsmB - 1) / kAsmB;
-    const unsigned g = (unsigned)nbpa * nbpa * nbpa;
-    const double scale = 1.0 / n;  // H^(d-2)
-    const double rscale = A->lat_f * std::pow(1.0 / n, 3);
-    const double *kd = kappa ? (const double *)kappa->d : nullptr;
-    hipStream_t st = ctx->stream;
+  const RefElement &R = ref_element(3, 1);
+  Scratch<double> Tt(ctx, R.T.size()), pts(ctx, R.s), load(ctx, R.nloc);
+  double *dT = Tt.p, *dg = pts.p, *dm = load.p;
+  hipStream_t st = ctx->stream;
+  FLGPU_HIP(hipMemcpyAsync(dT, R.T.data(), sizeof(double) * R.T.size(), hipMemcpyHostToDevice, st));
+  FLGPU_HIP(hipMemcpyAsync(dg, R.pts, sizeof(double) * R.s, hipMemcpyHostToDevice, st));
+  FLGPU_HIP(hipMemcpyAsync(dm, R.m.data(), sizeof(double) * R.nloc, hipMemcpyHostToDevice, st));
+  const int nbpa = (n + 1 + kAsmB - 1) / kAsmB;
+  const unsigned g = (unsigned)nbpa * nbpa * nbpa;
+  const double scale = 1.0 / n;  // H^(d-2)
+  const double rscale = A->lat_f * std::pow(1.0 / n, 3);
+  const double *kd = kappa ? (const double *)kappa->d : nullptr;
 #define FLGPU_ASM(T, MODE)                                                                   \
   k_asm_q1<T, MODE><<<g, kAsmThreads, 0, st>>>(n, dg, kd, nk, scale, dT, A->rowptr, (T *)A->vals, \
                                        rscale, dm, (T *)rhs_dev)
-    if (A->prec == FLGPU_F64) {
-      if (mode == FLGPU_ASM_MFMA) FLGPU_ASM(double, ASM_MFMA64);
-      else FLGPU_ASM(double, ASM_FMA);
-    } else {
-      if (mode == FLGPU_ASM_MFMA) FLGPU_ASM(float, ASM_MFMA_BF16);
-      else FLGPU_ASM(float, ASM_FMA);
-    }
-#undef FLGPU_ASM
-    FLGPU_HIP(hipGetLastError());
-    FLGPU_HIP(hipStreamSynchronize(st));
-  } catch (...) {
-    dev_free(dT);
-    dev_free(dg);
-    dev_free(dm);
-    throw;
+  if (A->prec == FLGPU_F64) {
+    if (mode == FLGPU_ASM_MFMA) FLGPU_ASM(double, ASM_MFMA64);
+    else FLGPU_ASM(double, ASM_FMA);
+  } else {
+    if (mode == FLGPU_ASM_MFMA) FLGPU_ASM(float, ASM_MFMA_BF16);
+    else FLGPU_ASM(float, ASM_FMA);
   }
-  dev_free(dT);
-  dev_free(dg);
-  dev_free(dm);
+#undef FLGPU_ASM
+  FLGPU_HIP(hipGetLastError());
 }
 
 // values (and rhs) of a lattice matrix whose pattern is already built
@@ -919,17 +908,17 @@ static void assemble_values(flgpu_mat *A, const flgpu_vec *kappa, int nk, int mo
     assemble_values_q1(A, kappa, nk, mode, rhs_dev);
     return;
   }
-  RefElement R = ref_element(dim, order);
-  Table1D pat = table_pattern(order, n);
+  const RefElement &R = ref_element(dim, order);
   long ncells = ipow(n, dim);
   // E in FP64 for the FP64 path, FP32 for the FP32 (BF16-MFMA) path
   int eprec = A->prec;
   // a matrix that keeps its element matrices (elem) has them formed in place
   const int ld = A->elem ? row_pad(R.nloc, eprec) : R.nloc;
-  void *E = A->elem ? A->elem : dev_alloc(prec_bytes(eprec) * ncells * R.nloc2);
+  Scratch<char> elem(ctx, A->elem ? 1 : prec_bytes(eprec) * ncells * R.nloc2);
+  void *E = A->elem ? A->elem : elem.p;
   element_matrices(ctx, R, n, kappa, nk, mode, eprec, E, ld);
-  DevTable dpat = upload_table(ctx, pat);
-  double *dm = (double *)dev_alloc(sizeof(double) * R.nloc);
+  Scratch<double> load(ctx, R.nloc);
+  double *dm = load.p;
   FLGPU_HIP(hipMemcpyAsync(dm, R.m.data(), sizeof(double) * R.nloc, hipMemcpyHostToDevice,
                            ctx->stream));
   double rscale = A->lat_f * std::pow(1.0 / n, dim);
@@ -937,7 +926,7 @@ static void assemble_values(flgpu_mat *A, const flgpu_vec *kappa, int nk, int mo
   auto gather = [&](auto t) {
     using T = decltype(t);
     auto launch = [&](auto kern, int G) {
-      kern<<<grid_for(N * G, 256), 256, 0, ctx->stream>>>(N, order, n, dpat, A->rowptr,
+      kern<<<grid_for(N * G, 256), 256, 0, ctx->stream>>>(N, order, n, A->rowptr,
                                                           (const T *)E, R.nloc, ld, (T *)A->vals,
                                                           rscale, dm, (T *)rhs_dev);
     };
@@ -948,10 +937,6 @@ static void assemble_values(flgpu_mat *A, const flgpu_vec *kappa, int nk, int mo
   if (A->prec == FLGPU_F64) gather(0.0);
   else gather(0.0f);
   FLGPU_HIP(hipGetLastError());
-  FLGPU_HIP(hipStreamSynchronize(ctx->stream));
-  free_table(dpat);
-  dev_free(dm);
-  if (E != A->elem) dev_free(E);
 }
 
 template <class T>
@@ -962,7 +947,7 @@ __global__ void k_alpha(long ncells, double H, const double *__restrict__ kappa,
 
 // kref: the reference element matrix of a constant coefficient (sum_q T_q), padded rows
 void lattice_set_kref(flgpu_mat *A) {
-  RefElement R = ref_element(A->lat_dim, A->lat_order);
+  const RefElement &R = ref_element(A->lat_dim, A->lat_order);
   const int ld = row_pad(R.nloc, A->prec);
   std::vector<double> k((size_t)R.nloc * ld, 0.0);
   for (int a = 0; a < R.nloc; a++)
@@ -1014,7 +999,7 @@ static void lattice_set_alpha(flgpu_mat *A, const flgpu_vec *kappa, int nk) {
     drop_alpha(A);
     return;
   }
-  RefElement R = ref_element(3, 1);
+  const RefElement &R = ref_element(3, 1);
   for (int b = 0; b < 8; b++) A->kt[b] = R.T[(size_t)R.nq * R.nloc2 + b];  // sum_q T_q
   long ncells = (long)n * n * n;
   if (!A->alpha) {
@@ -1282,34 +1267,28 @@ void lattice_blackbox(const flgpu_mat *A, flgpu_mat *P) {
   FLGPU_REQUIRE(P->nrows == A->nrows && P->ncols == (long)Mc * Mc * Mc,
                 "the interpolation does not map the coarse lattice to the matrix's lattice");
   flgpu_ctx *ctx = A->ctx;
-  double *W = (double *)dev_alloc(sizeof(double) * 8 * (size_t)N);
-  try {
-    for (int pass = 0; pass <= 3; pass++) {
-      const long h = n / 2 + 1, most = pass == 0 ? h * h * h : pass == 1 ? h * h * (h - 1)
-                                     : pass == 2 ? h * (h - 1) * (h - 1)
-                                                 : (h - 1) * (h - 1) * (h - 1);
-      const dim3 g(grid_for(most, 256), pass == 1 || pass == 2 ? 3 : 1);
-      if (A->prec == FLGPU_F64)
-        k_bbox_pass<double><<<g, 256, 0, ctx->stream>>>(M, pass, A->rowptr,
-                                                        (const double *)A->vals, W);
-      else
-        k_bbox_pass<float><<<g, 256, 0, ctx->stream>>>(M, pass, A->rowptr,
-                                                       (const float *)A->vals, W);
-      FLGPU_HIP(hipGetLastError());
-    }
-    if (P->prec == FLGPU_F64)
-      k_bbox_write<double><<<grid_for(N, 256), 256, 0, ctx->stream>>>(
-          M, Mc, P->rowptr, P->colidx, W, (double *)P->vals);
+  Scratch<double> weights(ctx, 8 * (size_t)N);
+  double *W = weights.p;
+  for (int pass = 0; pass <= 3; pass++) {
+    const long h = n / 2 + 1, most = pass == 0 ? h * h * h : pass == 1 ? h * h * (h - 1)
+                                   : pass == 2 ? h * (h - 1) * (h - 1)
+                                               : (h - 1) * (h - 1) * (h - 1);
+    const dim3 g(grid_for(most, 256), pass == 1 || pass == 2 ? 3 : 1);
+    if (A->prec == FLGPU_F64)
+      k_bbox_pass<double><<<g, 256, 0, ctx->stream>>>(M, pass, A->rowptr,
+                                                      (const double *)A->vals, W);
     else
-      k_bbox_write<float><<<grid_for(N, 256), 256, 0, ctx->stream>>>(
-          M, Mc, P->rowptr, P->colidx, W, (float *)P->vals);
+      k_bbox_pass<float><<<g, 256, 0, ctx->stream>>>(M, pass, A->rowptr,
+                                                     (const float *)A->vals, W);
     FLGPU_HIP(hipGetLastError());
-    FLGPU_HIP(hipStreamSynchronize(ctx->stream));
-  } catch (...) {
-    dev_free(W);
-    throw;
   }
-  dev_free(W);
+  if (P->prec == FLGPU_F64)
+    k_bbox_write<double><<<grid_for(N, 256), 256, 0, ctx->stream>>>(
+        M, Mc, P->rowptr, P->colidx, W, (double *)P->vals);
+  else
+    k_bbox_write<float><<<grid_for(N, 256), 256, 0, ctx->stream>>>(
+        M, Mc, P->rowptr, P->colidx, W, (float *)P->vals);
+  FLGPU_HIP(hipGetLastError());
   mat_refresh_values(P);
 }
 
@@ -1520,10 +1499,11 @@ extern "C" int flgpu_lattice_element_matrices(flgpu_ctx *ctx, int dim, int order
     FLGPU_REQUIRE(first_cell >= 0 && ncells >= 0 && first_cell + ncells <= total,
                   "cell range out of bounds");
     CTX_LOCK(ctx);
-    RefElement R = ref_element(dim, order);
+    const RefElement &R = ref_element(dim, order);
     void *E = dev_alloc(prec_bytes(prec) * total * R.nloc2);
     try {
       element_matrices(ctx, R, n, kappa, nk, mode, prec, E, R.nloc);
+      FLGPU_HIP(hipStreamSynchronize(ctx->stream));
       long cnt = ncells * R.nloc2;
       if (prec == FLGPU_F64) {
         FLGPU_HIP(hipMemcpy(out, (double *)E + first_cell * R.nloc2, sizeof(double) * cnt,

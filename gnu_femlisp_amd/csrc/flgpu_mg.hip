@@ -40,14 +40,11 @@ struct DenseInverse {
   int *cidx = nullptr;  // the m non-trivial DOFs
   int *tidx = nullptr;  // the nt trivial DOFs
   int m = 0, nt = 0;
-  void release() {
-    dev_free(inv);
-    dev_free(tiles);
-    dev_free(tI);
-    dev_free(tJ);
-    dev_free(part);
-    dev_free(cidx);
-    dev_free(tidx);
+  flgpu_ctx *ctx = nullptr;
+  void release() {  // under ctx's lock
+    for (void *p : {(void *)inv, (void *)tiles, (void *)tI, (void *)tJ, (void *)part,
+                    (void *)cidx, (void *)tidx})
+      if (p) scratch_put(ctx, p);
     inv = nullptr;
     tiles = nullptr;
     tI = tJ = nullptr;
@@ -383,13 +380,16 @@ static DenseInverse dense_inverse_dev(const flgpu_mat *A) {
   const int n = A->nrows;
   const long nn = (long)n * n;
   hipStream_t s = A->ctx->stream;
+  flgpu_ctx *ctx = A->ctx;
   DenseInverse out;
-  double *M0 = nullptr, *D = nullptr, *C2 = nullptr;
-  int *bad = nullptr, *dt = nullptr;
+  out.ctx = ctx;
+  double *C2 = nullptr;
   try {
     if (n == 0) return out;
-    M0 = (double *)dev_alloc(sizeof(double) * nn);
-    dt = (int *)dev_alloc(sizeof(int) * n);
+    Scratch<double> full(ctx, nn), block(ctx, kGjB * kGjB);
+    Scratch<int> triv_p(ctx, n), bad_p(ctx, 1);
+    double *M0 = full.p, *D = block.p;
+    int *dt = triv_p.p, *bad = bad_p.p;
     k_dense_zero<<<grid_for(nn, 256), 256, 0, s>>>(nn, M0);
     if (A->prec == FLGPU_F64)
       k_dense_scatter<double><<<grid_for(n, 256), 256, 0, s>>>(n, A->rowptr, A->colidx,
@@ -407,20 +407,18 @@ static DenseInverse dense_inverse_dev(const flgpu_mat *A) {
     out.m = m;
     out.nt = (int)triv.size();
     if (out.nt > 0) {
-      out.tidx = (int *)dev_alloc(sizeof(int) * out.nt);
+      out.tidx = (int *)scratch_get(ctx, sizeof(int) * out.nt);
       FLGPU_HIP(hipMemcpyAsync(out.tidx, triv.data(), sizeof(int) * out.nt,
                                hipMemcpyHostToDevice, s));
     }
     if (m > 0) {
       const long mm = (long)m * m;
-      out.cidx = (int *)dev_alloc(sizeof(int) * m);
+      out.cidx = (int *)scratch_get(ctx, sizeof(int) * m);
       FLGPU_HIP(hipMemcpyAsync(out.cidx, piv.data(), sizeof(int) * m, hipMemcpyHostToDevice, s));
-      out.inv = (double *)dev_alloc(sizeof(double) * mm);
+      out.inv = (double *)scratch_get(ctx, sizeof(double) * mm);
       k_dense_gather<<<grid_for(mm, 256), 256, 0, s>>>(m, n, out.cidx, M0, out.inv);
       FLGPU_HIP(hipGetLastError());
-      D = (double *)dev_alloc(sizeof(double) * kGjB * kGjB);
-      C2 = (double *)dev_alloc(sizeof(double) * mm);
-      bad = (int *)dev_alloc(sizeof(int));
+      C2 = (double *)scratch_get(ctx, sizeof(double) * mm);
       FLGPU_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
       const int ntile = (m + kGjB - 1) / kGjB;
       for (int k0 = 0; k0 < m; k0 += kGjB) {
@@ -437,19 +435,11 @@ static DenseInverse dense_inverse_dev(const flgpu_mat *A) {
     }
     FLGPU_HIP(hipStreamSynchronize(s));
   } catch (...) {
-    dev_free(M0);
-    dev_free(dt);
-    dev_free(D);
-    dev_free(C2);
-    dev_free(bad);
+    scratch_put(ctx, C2);
     out.release();
     throw;
   }
-  dev_free(M0);
-  dev_free(dt);
-  dev_free(D);
-  dev_free(C2);
-  dev_free(bad);
+  scratch_put(ctx, C2);
   return out;
 }
 
@@ -600,16 +590,16 @@ static void coarse_setup(flgpu_mg *mg, MGLevel &L) {
         hJ.push_back(J);
       }
     const int nq = (int)hI.size();
-    D.tI = (int *)dev_alloc(sizeof(int) * nq);
-    D.tJ = (int *)dev_alloc(sizeof(int) * nq);
-    D.tiles = (float *)dev_alloc(sizeof(float) * (size_t)nq * kSymB * kSymB);
-    D.part = (double *)dev_alloc(sizeof(double) * (size_t)D.ntile * D.ntile * kSymB);
+    D.tI = (int *)scratch_get(mg->ctx, sizeof(int) * nq);
+    D.tJ = (int *)scratch_get(mg->ctx, sizeof(int) * nq);
+    D.tiles = (float *)scratch_get(mg->ctx, sizeof(float) * (size_t)nq * kSymB * kSymB);
+    D.part = (double *)scratch_get(mg->ctx, sizeof(double) * (size_t)D.ntile * D.ntile * kSymB);
     FLGPU_HIP(hipMemcpyAsync(D.tI, hI.data(), sizeof(int) * nq, hipMemcpyHostToDevice, s));
     FLGPU_HIP(hipMemcpyAsync(D.tJ, hJ.data(), sizeof(int) * nq, hipMemcpyHostToDevice, s));
     k_pack_sym<<<nq, 256, 0, s>>>(D.m, D.inv, D.tI, D.tJ, D.tiles);
     FLGPU_HIP(hipGetLastError());
     FLGPU_HIP(hipStreamSynchronize(s));
-    dev_free(D.inv);
+    scratch_put(mg->ctx, D.inv);
     D.inv = nullptr;
   }
 }

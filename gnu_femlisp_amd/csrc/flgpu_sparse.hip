@@ -1498,7 +1498,8 @@ void stencil_refresh(flgpu_mat *A) {
   if (!A->val27) return;
   int M = A->lat_n + 1;
   long N = A->nrows;
-  int *asym = (int *)dev_alloc(sizeof(int));
+  Scratch<int> flag(A->ctx, 1);
+  int *asym = flag.p;
   FLGPU_HIP(hipMemsetAsync(asym, 0, sizeof(int), A->ctx->stream));
   const bool lds = M >= 3 && A->sell.maxw <= 27;
   const unsigned gl = (unsigned)((N + kSt27Rows - 1) / kSt27Rows);
@@ -1525,7 +1526,6 @@ void stencil_refresh(flgpu_mat *A) {
   int h = 1;
   FLGPU_HIP(hipMemcpyAsync(&h, asym, sizeof(int), hipMemcpyDeviceToHost, A->ctx->stream));
   FLGPU_HIP(hipStreamSynchronize(A->ctx->stream));
-  dev_free(asym);
   if (A->st_sym != (h == 0)) layout_changed(A);
   A->st_sym = (h == 0);
 }

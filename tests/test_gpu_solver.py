@@ -641,3 +641,33 @@ def test_blackbox_interpolation_on_edge_lattices(n, prec):
     prp, pci, pv = P.csr()
     assert np.array_equal(prp, brp) and np.array_equal(pci, bci)
     assert np.abs(pv - bv).max() <= (1e-13 if prec == F.F64 else 1e-6)
+
+
+def test_setup_memory_reused_between_hierarchies():
+    """A context's setup memory serves hierarchies of different sizes, precisions and orders in
+    turn, the largest first and last, and ones destroyed in between: values and solves equal
+    those of fresh contexts bit for bit"""
+    say("setup memory reuse")
+    shared = Context(0)
+
+    def run(ctx, dim, order, m, levels, prec, transfer):
+        n = m << (levels - 1)
+        rng = np.random.default_rng(n)
+        ks = [(GpuVector.from_array(np.exp(rng.normal(size=n ** dim)), ctx=ctx), n)
+              for _ in range(2)]
+        sm = it.GeometricSSC(1.0) if order == 2 else it.Jacobi(0.8)
+        cs = it.GeometricCS(sm, 1, 1, 0, symmetric=True, prec=prec, transfer=transfer)
+        H = it.Hierarchy.lattice(cs, dim, order, m, levels, kappa=ks[0], ctx=ctx)
+        H.reassemble(ks[1])
+        x, r = (GpuVector.from_array(np.ones(H.top_matrix().nrows), prec, ctx=ctx)
+                for _ in range(2))
+        b = GpuVector.from_array(rng.uniform(-1, 1, H.top_matrix().nrows), prec, ctx=ctx)
+        check(lib().flgpu_mg_apply(H.h, x.h, b.h, r.h))
+        return [H.level_matrix(l).csr()[2] for l in range(levels)] + [x.numpy()]
+
+    cases = [(3, 1, 6, 3, F.F32, "blackbox"), (2, 2, 2, 4, F.F64, "geometric"),
+             (3, 1, 3, 2, F.F64, "blackbox"), (3, 2, 2, 2, F.F32, "geometric"),
+             (1, 2, 3, 3, F.F64, "geometric"), (3, 1, 6, 3, F.F64, "blackbox")]
+    for c in cases:
+        for a, b in zip(run(shared, *c), run(Context(0), *c)):
+            assert np.array_equal(a, b), c
