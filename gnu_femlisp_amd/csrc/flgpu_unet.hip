@@ -140,6 +140,72 @@ __device__ __forceinline__ void conv_stage(const ConvGeom &G, const ConvIn &in, 
   }
 }
 
+// The voxel of every position of the box at (b, z0, y0, x0) and its halo, -1 outside the grid; of
+// an upsampled input also the half grid's, behind them.
+__device__ __forceinline__ void conv_table(const ConvGeom &G, int up, int b, int z0, int y0,
+                                           int x0, int *tab) {
+  const int n = G.n, h = n >> 1;
+  for (int pos = threadIdx.x; pos < G.hvol; pos += 256) {
+    const unsigned t = fdiv((unsigned)pos, G.dhx), hz = fdiv(t, G.dhy);
+    const int x = x0 + pos - (int)(t * G.dhx.f.d) - 1, y = y0 + (int)(t - hz * G.dhy.f.d) - 1,
+              z = z0 + (int)hz - 1;
+    const bool in = (unsigned)z < (unsigned)n && (unsigned)y < (unsigned)n &&
+                    (unsigned)x < (unsigned)n;
+    tab[pos] = in ? ((b * n + z) * n + y) * n + x : -1;
+    if (up) tab[G.hvol + pos] = in ? ((b * h + (z >> 1)) * h + (y >> 1)) * h + (x >> 1) : 0;
+  }
+}
+
+// conv_stage of all chunks with the voxels from conv_table: several channel quads share a
+// position, whose division and multiplications are then formed once (the weight gradients, which
+// stage one chunk at a time, are faster without: 74 against 93 us)
+__device__ __forceinline__ void conv_stage_table(const ConvGeom &G, const ConvIn &in, int nch,
+                                                 Div1 dq, const int *tab, short *lds) {
+  const int Q = nch * 4, total = G.hvol * Q, ct = in.c0 + in.c1;
+  constexpr int U = 4;
+  auto run = [&](auto vec) {
+    for (int e0 = threadIdx.x; e0 < total; e0 += U * 256) {
+      float4 f[U];
+      int dst[U], left[U];  // channels from the entry's first on, 0: nothing there
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int e = e0 + u * 256;
+        const unsigned ec = (unsigned)min(e, total - 1);
+        const unsigned pos = fdiv(ec, dq), q = ec - pos * (unsigned)Q;
+        const int c = (int)q * 4, v = tab[pos];
+        dst[u] = e < total ? (int)(((q >> 2) * (unsigned)G.hvol + pos) * 16u + (q & 3u) * 4u) : -1;
+        const bool live = v >= 0 && c < ct, second = c >= in.c0;
+        left[u] = live ? ct - c : 0;
+        // unconditional loads, of the first values where there is nothing to load
+        const unsigned w = live ? (unsigned)(in.up && !second ? tab[G.hvol + pos] : v) : 0u;
+        const unsigned cs = (unsigned)(second ? in.c1 : in.c0),
+                       cc = live ? (unsigned)(second ? c - in.c0 : c) : 0u;
+        const float *src = (live && second ? in.p1 : in.p0) + (size_t)w * cs + cc;
+        if (vec) {
+          f[u] = *(const float4 *)src;
+        } else {  // channel counts that are no multiple of 4 (one source)
+          f[u].x = src[0];
+          f[u].y = src[left[u] > 1 ? 1 : 0];
+          f[u].z = src[left[u] > 2 ? 2 : 0];
+          f[u].w = src[left[u] > 3 ? 3 : 0];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (dst[u] >= 0) {
+          v4s s;
+          s[0] = left[u] > 0 ? bf16_bits(f[u].x) : (short)0;
+          s[1] = left[u] > 1 ? bf16_bits(f[u].y) : (short)0;
+          s[2] = left[u] > 2 ? bf16_bits(f[u].z) : (short)0;
+          s[3] = left[u] > 3 ? bf16_bits(f[u].w) : (short)0;
+          *(v4s *)(lds + dst[u]) = s;
+        }
+    }
+  };
+  if (((in.c0 | in.c1) & 3) == 0) run(std::true_type());
+  else run(std::false_type());
+}
+
 // ---- convolution forward / input gradient (implicit GEMM on MFMA) --------------------
 
 // out[v][o] = bias[o] + sum_t sum_c in[v + off(t) * sgn][c] * W[t][c][o]
@@ -153,8 +219,8 @@ __device__ __forceinline__ void conv_stage(const ConvGeom &G, const ConvIn &in, 
 // MT x NT tiles of 16 voxels x 16 channels, which share each voxel operand (LDS) and each weight
 // fragment (512 contiguous bytes, from L1/L2, fetched a group of iterations ahead).  Products
 // accumulate tap by tap and, within a tap, 16 channels at a time in ascending order.
-// Batch 32, 32^3, [32 up, 16 skip] -> 16 channels: 227 us, 96 TFLOP/s, bound by LDS reads and the
-// staging (2559 us and 215 us for the concatenation as one wave per 16 voxels without LDS, which
+// Batch 32, 32^3, [32 up, 16 skip] -> 16 channels: 189 us, 115 TFLOP/s (227 without conv_table),
+// bound by LDS reads and the staging (2559 us and 215 us for the concatenation as one wave per 16 voxels without LDS, which
 // rounded the inputs and fetched single 2-byte weights anew for each of the 27 taps).
 template <int MT, int NT>
 __global__ __launch_bounds__(256) void k_conv(ConvGeom G, ConvIn in, int nch, Div1 dq, int no,
@@ -168,7 +234,10 @@ __global__ __launch_bounds__(256) void k_conv(ConvGeom G, ConvIn in, int nch, Di
   if (box >= G.nbox) return;  // the whole block
   int b, z0, y0, x0;
   conv_box(G, box, b, z0, y0, x0);
-  conv_stage(G, in, 0, nch, dq, b, z0, y0, x0, lds);
+  int *tab = (int *)(lds + (long)nch * G.hvol * 16);
+  conv_table(G, in.up, b, z0, y0, x0, tab);
+  __syncthreads();
+  conv_stage_table(G, in, nch, dq, tab, lds);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int mw = w % wm, nw = w / wm;
   const int hx = (int)G.dhx.f.d, hy = (int)G.dhy.f.d;
@@ -807,7 +876,7 @@ template <int MT, int NT>
 static void conv_launch(flgpu_unet *u, const ConvPlan &p, const ConvIn &in, int no,
                         const short *wf, const float *bias, const float *mask, float *out,
                         int relu, int sgn) {
-  const size_t lds = (size_t)p.nch * p.g.hvol * 32;
+  const size_t lds = (size_t)p.g.hvol * (p.nch * 32 + (in.up ? 8 : 4));
   if (lds > 64 * 1024)
     FLGPU_HIP(hipFuncSetAttribute((const void *)k_conv<MT, NT>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
