@@ -187,6 +187,9 @@ struct flgpu_mat {
   void *diag = nullptr;    // diagonal values (prec)
   Sell sell;
   int lanes = 0;  // products read the CSR with this many lanes per row (0: SELL)
+  // 3D order-2 lattice interpolation from q2_nc^3 cells (q2t 1) or its transpose (2), as it was
+  // assembled: products take the weights from the nodes' positions; 0 once values are changed
+  int q2t = 0, q2_nc = 0;
   int ncolours = 0;
   std::vector<Sell> colour_sell;
   flgpu_mat *transpose = nullptr;
@@ -260,6 +263,8 @@ void galerkin_product(const flgpu_mat *P, const flgpu_mat *A, flgpu_mat *Ac, boo
 // out[row] = beta*z[row] + alpha*(A x)[row]  (z may be out; beta == 0 ignores z)
 void spmv(const flgpu_mat *A, double alpha, const void *x, double beta,
           const void *z, void *out);
+// out = A x and zero = 0 (nrows values)
+void spmv_zero(const flgpu_mat *A, const void *x, void *out, void *zero);
 void spmv_t(const flgpu_mat *A, double alpha, const void *x, double beta,
             void *out);
 // Per-block partials of one or more dots, K rows of np values.  The kernel that needs a sum adds

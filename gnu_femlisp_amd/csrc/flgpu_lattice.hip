@@ -1396,6 +1396,11 @@ flgpu_mat *lattice_interpolation(flgpu_ctx *ctx, int dim, int order, int nc, int
     mat_finish(P);
     mat_finish(PT);
     P->transpose = PT;
+    if (dim == 3 && order == 2) {
+      P->q2t = 1;
+      PT->q2t = 2;
+      P->q2_nc = PT->q2_nc = nc;
+    }
     if (dim == 3 && order == 1) {  // the trilinear pattern: products with implied columns
       P->tp_kind = 1;
       PT->tp_kind = 2;

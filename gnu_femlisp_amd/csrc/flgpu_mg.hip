@@ -711,9 +711,9 @@ static void lmgc(flgpu_mg *mg, int l) {
     C.x_zero = true;
     C.residual_p = false;
   } else if (sweeps && !base) {
-    spmv(C.I->transpose, 1.0, lres(mg, l), 0.0, C.rhs, C.rhs);
     C.x_zero = mg->p.smoother == FLGPU_SMOOTH_SOR;
-    if (!C.x_zero) vfill(mg->ctx, C.N, mg->p.prec, C.sol, 0.0);
+    if (C.x_zero) spmv(C.I->transpose, 1.0, lres(mg, l), 0.0, C.rhs, C.rhs);
+    else spmv_zero(C.I->transpose, lres(mg, l), C.rhs, C.sol);
     C.residual_p = false;
   } else {
     spmv(C.I->transpose, 1.0, lres(mg, l), 0.0, C.res, C.res);

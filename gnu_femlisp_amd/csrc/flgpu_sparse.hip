@@ -315,6 +315,8 @@ void drop_cells(flgpu_mat *A) {
 }
 
 void mat_refresh_values(flgpu_mat *A) {
+  if (A->q2t) layout_changed(A);
+  A->q2t = 0;  // other values than the interpolation's
   diag_refresh(A);
   stencil_refresh(A);
   if (A->tp_kind) tp_prepare(A);
@@ -430,6 +432,8 @@ flgpu_mat *mat_convert(const flgpu_mat *A, int prec) {
   B->lat_f = A->lat_f;
   B->tp_kind = A->tp_kind;
   B->tp_nc = A->tp_nc;
+  B->q2t = A->q2t;
+  B->q2_nc = A->q2_nc;
   if (A->alpha) {
     long nc = (long)A->lat_n * A->lat_n * A->lat_n;
     B->alpha = dev_alloc(prec_bytes(prec) * nc);
@@ -597,7 +601,8 @@ __global__ __launch_bounds__(256) void k_csr_spmv(int nrows, const int *__restri
                                                   const int *__restrict__ col,
                                                   const T *__restrict__ val, T alpha,
                                                   const T *__restrict__ x, T beta, const T *z,
-                                                  T *out, double *dpart = nullptr) {
+                                                  T *out, double *dpart = nullptr,
+                                                  T *zero = nullptr) {
   const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
   const int row = (int)lb * (256 / G) + threadIdx.x / G, l = threadIdx.x % G;
   double d = 0;
@@ -606,6 +611,7 @@ __global__ __launch_bounds__(256) void k_csr_spmv(int nrows, const int *__restri
     if (l == 0) {
       const T o = beta == (T)0 ? (T)acc : (T)((double)beta * (double)z[row] + acc);
       out[row] = o;
+      if (zero) zero[row] = (T)0;
       if (DOT) d = (double)o * (double)x[row];
     }
   }
@@ -628,12 +634,13 @@ static int csr_lanes(const flgpu_mat *A) {
 
 template <class T>
 static void launch_csr_spmv(const flgpu_mat *A, T alpha, const void *x, T beta, const void *z,
-                            void *out, double *dpart = nullptr) {
+                            void *out, double *dpart = nullptr, void *zero = nullptr) {
   const int G = A->lanes;
   const unsigned g = xcd_grid(grid_for((long)A->nrows * G, 256));
   auto launch = [&](auto kern) {
     kern<<<g, 256, 0, A->ctx->stream>>>(A->nrows, A->rowptr, A->colidx, (const T *)A->vals, alpha,
-                                        (const T *)x, beta, (const T *)z, (T *)out, dpart);
+                                        (const T *)x, beta, (const T *)z, (T *)out, dpart,
+                                        (T *)zero);
   };
   if (dpart) launch(G == 4 ? k_csr_spmv<T, 4, true> : k_csr_spmv<T, 8, true>);
   else launch(G == 4 ? k_csr_spmv<T, 4> : k_csr_spmv<T, 8>);
@@ -2072,8 +2079,165 @@ static void launch_cell_apply(const flgpu_mat *A, T alpha, const void *x, T beta
   FLGPU_HIP(hipGetLastError());
 }
 
+// ---- 3D order-2 lattice interpolation without its matrix -------------------------------------
+// A coarse Q2 node j lies on the fine node 2j.  Per axis a fine node i takes, for even i, the
+// coarse node i / 2 and, for odd i, the three nodes of its coarse cell i / 4 with the quadratic
+// shape functions at 1/4 or 3/4: 3/8, 3/4, -1/8 or the reverse.  Transposed, a coarse vertex j
+// (even) takes the fine nodes 2j - 3, 2j - 1, 2j, 2j + 1, 2j + 3 with -1/8, 3/8, 1, 3/8, -1/8 and a
+// mid node 2j - 1, 2j, 2j + 1 with 3/4, 1, 3/4.  Rows and columns on the boundary are zero
+// (constrained interpolation).  FP32 sums are formed in FP64, as the CSR products form them.
+// Bound by the vectors' bytes and, for the restriction, by a vertex's 125 reads.  48^3 cells, FP32:
+// 9.2 and 17.2 us; from the CSR 26.7 and 22.8, its 7.5 million entries.
+__device__ __forceinline__ double q2_weight(int r, int t) {  // r = i mod 4 in {1, 3}, tap t of 3
+  const double w[3] = {0.375, 0.75, -0.125};
+  return t == 1 ? w[1] : (r == 1) == (t == 0) ? w[0] : w[2];
+}
+
+template <class T>
+__global__ __launch_bounds__(256) void k_q2_prolong(int M, int Mc, FastDiv fM, T alpha,
+                                                    const T *__restrict__ x, T beta, const T *z,
+                                                    T *out) {
+  const unsigned i = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+  if (i >= (unsigned)M * (unsigned)M * (unsigned)M) return;
+  int q[3];
+  lat_decode(i, fM, q[0], q[1], q[2]);
+  const T zi = beta == (T)0 ? (T)0 : z[i];
+  // the taps of an axis: coarse nodes j0 + t with weights w[t]; 0 for those on the boundary
+  int j0[3];
+  double w[3][3];
+  bool in = true;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const bool odd = q[a] & 1;
+    j0[a] = odd ? 2 * (q[a] >> 2) : min(max((q[a] >> 1) - 1, 0), Mc - 3);
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+      const int j = j0[a] + t;
+      const double v = odd ? q2_weight(q[a] & 3, t) : j == q[a] >> 1 ? 1.0 : 0.0;
+      w[a][t] = j == 0 || j == Mc - 1 ? 0.0 : v;
+    }
+    in &= q[a] > 0 && q[a] < M - 1;
+  }
+  double s = 0;
+  if (in)
+#pragma unroll
+    for (int tz = 0; tz < 3; tz++) {
+      if (w[0][tz] == 0.0) continue;  // a plane's nodes alike
+      T v[3][3];
+#pragma unroll
+      for (int ty = 0; ty < 3; ty++) {
+        const T *p = x + ((unsigned)(j0[0] + tz) * (unsigned)Mc + (unsigned)(j0[1] + ty)) *
+                             (unsigned)Mc + (unsigned)j0[2];
+#pragma unroll
+        for (int u = 0; u < 3; u++) v[ty][u] = p[u];
+      }
+#pragma unroll
+      for (int ty = 0; ty < 3; ty++) {
+        double line = 0;
+#pragma unroll
+        for (int u = 0; u < 3; u++)
+          line += w[2][u] * (double)(w[1][ty] != 0.0 && w[2][u] != 0.0 ? v[ty][u] : (T)0);
+        s += w[0][tz] * w[1][ty] * line;
+      }
+    }
+  out[i] = (T)((double)beta * (double)zi + (double)alpha * s);
+}
+
+// tap t of 5 of the coarse coordinate q: its weight, 0 where there is none, and its fine coordinate
+// f (2q where there is none)
+__device__ __forceinline__ double q2_tap(int q, int t, int M, int &f) {
+  const int d = t == 2 ? 0 : t < 2 ? 2 * t - 3 : 2 * t - 5;  // -3, -1, 0, 1, 3
+  f = 2 * q + d;
+  const bool near = t == 1 || t == 3, ok = f > 0 && f < M - 1 && t < 5;
+  const double v = t == 2 ? 1.0 : q & 1 ? (near ? 0.75 : 0.0) : near ? 0.375 : -0.125;
+  if (!ok) f = 2 * q;
+  return ok ? v : 0.0;
+}
+
+// Eight lanes share a coarse row, each every eighth of its 25 lines of fine nodes: all of a lane's
+// loads are in flight together (one lane a row: 11 us on small lattices too).
+template <class T>
+__global__ __launch_bounds__(256) void k_q2_restrict(int M, int Mc, FastDiv fMc, T alpha,
+                                                     const T *__restrict__ x, T beta, const T *z,
+                                                     T *out, T *zero) {
+  const unsigned t0 = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+  const unsigned Nc = (unsigned)Mc * (unsigned)Mc * (unsigned)Mc;
+  const unsigned c = min(t0 >> 3, Nc - 1);
+  const int l = (int)(t0 & 7u);
+  int q[3];
+  lat_decode(c, fMc, q[0], q[1], q[2]);
+  bool in = true;
+#pragma unroll
+  for (int a = 0; a < 3; a++) in &= q[a] > 0 && q[a] < Mc - 1;
+  int fx[5];
+  double wx[5];
+#pragma unroll
+  for (int u = 0; u < 5; u++) wx[u] = q2_tap(q[2], u, M, fx[u]);
+  double w[4];
+  T v[4][5];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int t = l + 8 * k, tz = (t * 13) >> 6;  // t / 5 for t < 32
+    int fz, fy;
+    w[k] = q2_tap(q[0], tz, M, fz) * q2_tap(q[1], t - 5 * tz, M, fy);
+    const T *p = x + ((unsigned)fz * (unsigned)M + (unsigned)fy) * (unsigned)M;
+#pragma unroll
+    for (int u = 0; u < 5; u++) v[k][u] = p[fx[u]];
+  }
+  double s = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    double line = 0;
+#pragma unroll
+    for (int u = 0; u < 5; u++)
+      line += wx[u] * (double)(w[k] != 0.0 && wx[u] != 0.0 ? v[k][u] : (T)0);
+    s += w[k] * line;
+  }
+#pragma unroll
+  for (int o = 4; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (l != 0 || t0 >> 3 >= Nc) return;
+  if (!in) s = 0;
+  const T zi = beta == (T)0 ? (T)0 : z[c];
+  out[c] = (T)((double)beta * (double)zi + (double)alpha * s);
+  if (zero) zero[c] = (T)0;
+}
+
+template <class T>
+static void launch_q2t(const flgpu_mat *A, T alpha, const void *x, T beta, const void *z,
+                       void *out, void *zero = nullptr) {
+  const int M = 4 * A->q2_nc + 1, Mc = 2 * A->q2_nc + 1;
+  const unsigned g = xcd_grid(grid_for((long)A->nrows * (A->q2t == 1 ? 1 : 8), 256));
+  if (A->q2t == 1)
+    k_q2_prolong<T><<<g, 256, 0, A->ctx->stream>>>(M, Mc, fast_div((unsigned)M), alpha,
+                                                   (const T *)x, beta, (const T *)z, (T *)out);
+  else
+    k_q2_restrict<T><<<g, 256, 0, A->ctx->stream>>>(M, Mc, fast_div((unsigned)Mc), alpha,
+                                                    (const T *)x, beta, (const T *)z, (T *)out,
+                                                    (T *)zero);
+  FLGPU_HIP(hipGetLastError());
+}
+
+void spmv_zero(const flgpu_mat *A, const void *x, void *out, void *zero) {
+  const bool f64 = A->prec == FLGPU_F64;
+  if (A->q2t == 2) {
+    if (f64) launch_q2t<double>(A, 1.0, x, 0.0, out, out, zero);
+    else launch_q2t<float>(A, 1.0f, x, 0.0f, out, out, zero);
+  } else if (!A->tp_kind && !A->alpha && !A->val27 && !A->cell && A->lanes) {
+    if (f64) launch_csr_spmv<double>(A, 1.0, x, 0.0, out, out, nullptr, zero);
+    else launch_csr_spmv<float>(A, 1.0f, x, 0.0f, out, out, nullptr, zero);
+  } else {
+    spmv(A, 1.0, x, 0.0, out, out);
+    vfill(A->ctx, A->nrows, A->prec, zero, 0.0);
+  }
+}
+
 void spmv(const flgpu_mat *A, double alpha, const void *x, double beta, const void *z,
           void *out) {
+  if (A->q2t) {
+    if (A->prec == FLGPU_F64) launch_q2t<double>(A, alpha, x, beta, z, out);
+    else launch_q2t<float>(A, (float)alpha, x, (float)beta, z, out);
+    return;
+  }
   if (A->cell && A->lat_dim >= 2 && A->nrows >= kCellApplyRows) {
     if (A->prec == FLGPU_F64) launch_cell_apply<double>(A, alpha, x, beta, z, out);
     else launch_cell_apply<float>(A, (float)alpha, x, (float)beta, z, out);
@@ -2121,7 +2285,7 @@ static DotParts spmv_dot_t(const flgpu_mat *A, const void *x, void *out, int slo
   unsigned by, bx;
   const bool cell = A->cell && A->lat_dim >= 2 && A->nrows >= kCellApplyRows;
   if (cell) nb = (long)xcd_grid(cell_boxes(A, by, bx));
-  else if (A->tp_kind) nb = 0;
+  else if (A->tp_kind || A->q2t) nb = 0;
   else if (A->alpha) nb = q1_blocks(A, sizeof(T) == 8 ? FLGPU_QZB_F64_SPMV : FLGPU_QZB_F32);
   else if (A->val27) nb = (long)xcd_grid(grid_for(A->nrows, 256));
   else if (A->lanes) nb = (long)xcd_grid(grid_for((long)A->nrows * A->lanes, 256));

@@ -671,3 +671,62 @@ def test_setup_memory_reused_between_hierarchies():
     for c in cases:
         for a, b in zip(run(shared, *c), run(Context(0), *c)):
             assert np.array_equal(a, b), c
+
+
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("nc", [1, 2, 3, 6, 9])
+def test_order2_transfers_from_positions(nc, prec):
+    """3D order-2 interpolation and its transpose with the weights from the nodes' positions equal
+    the products of the assembled values (scipy, FP64), for several alpha and beta, on lattices
+    down to one cell; changed values go back to the stored ones"""
+    say(f"order-2 transfers nc={nc} prec={prec}")
+    rng = np.random.default_rng(nc)
+    P = lat.interpolation(3, 2, nc, prec=prec)
+    rp, ci, v = P.csr()
+    tol = 1e-14 if prec == F.F64 else 1e-6
+    x32 = lambda n: rng.uniform(-1, 1, n).astype(np.float32).astype(float)
+    xc, zf, yf, zc = x32(P.ncols), x32(P.nrows), x32(P.nrows), x32(P.ncols)
+
+    def check_products(v):
+        S = sp.csr_matrix((v.astype(float), ci, rp), shape=(P.nrows, P.ncols))
+        for alpha, beta in ((1.0, 0.0), (1.0, 1.0), (-0.5, 2.0)):
+            f = GpuVector.from_array(zf, prec)
+            gemm(alpha, P, GpuVector.from_array(xc, prec), beta, f)
+            assert np.abs(f.numpy() - (alpha * (S @ xc) + beta * zf)).max() <= 8 * tol
+            c = GpuVector.from_array(zc, prec)
+            gemm(alpha, P, GpuVector.from_array(yf, prec), beta, c, job="tn")
+            assert np.abs(c.numpy() - (alpha * (S.T @ yf) + beta * zc)).max() <= 64 * tol
+
+    check_products(v)
+    v2 = v * rng.uniform(0.5, 1.5, v.size).astype(np.float32)
+    v2 = v2.astype(np.float32).astype(float)
+    P.update_values(v2)
+    check_products(v2)
+
+
+@pytest.mark.parametrize("dim,m,levels,prec", [(2, 1, 4, F.F64), (2, 3, 3, F.F32),
+                                               (3, 1, 3, F.F64), (3, 2, 2, F.F32)])
+def test_ssc_cycles_from_zeroed_levels(dim, m, levels, prec):
+    """<ssc> cycles, whose restriction also clears the coarse level, equal the cycles of the same
+    hierarchy with transfers whose values were stored anew (the general products)"""
+    say(f"ssc zeroed levels dim={dim} m={m} prec={prec}")
+    rng = np.random.default_rng(m + dim)
+    n = m << (levels - 1)
+    kap = np.exp(rng.normal(size=(n,) * dim))
+    outs = []
+    for general in (False, True):
+        cs = it.GeometricCS(it.GeometricSSC(1.0), 1, 1, 0, symmetric=True, prec=prec)
+        H = it.Hierarchy.lattice(cs, dim, 2, m, levels, kappa=kap)
+        if general:
+            for l in range(levels - 1):
+                P = H.level_matrix(l, interp=True)
+                P.update_values(P.csr()[2])
+        N = H.top_matrix().nrows
+        x, r = GpuVector(N, prec), GpuVector(N, prec)
+        b = GpuVector.from_array(np.random.default_rng(1).uniform(-1, 1, N), prec)
+        gemm(1.0, H.top_matrix(), x, 0.0, r)
+        r = GpuVector.from_array(b.numpy(), prec)
+        for _ in range(2):
+            check(lib().flgpu_mg_apply(H.h, x.h, b.h, r.h))
+        outs.append(x.numpy())
+    assert relerr(outs[0], outs[1]) < (1e-12 if prec == F.F64 else 1e-5)
