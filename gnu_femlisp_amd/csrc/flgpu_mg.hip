@@ -76,6 +76,7 @@ struct flgpu_mg {
   flgpu_mg_params p{};
   std::vector<flgpu::MGLevel> lv;
   int top = 0;
+  int low = -1;  // the level below which one launch takes the cycle (low_top), -1: none
   // FP64 staging when an FP32 cycle is applied to FP64 vectors
   void *xs = nullptr, *bs = nullptr, *rs = nullptr;
   // active top-level pointers during one cycle
@@ -669,6 +670,254 @@ static void smooth(flgpu_mg *mg, int l, bool post, bool last = false) {
   L.residual_p = false;  // residual-after nil
 }
 
+// ---- the coarsest levels of a <jacobi> V-cycle in one workgroup ------------------------------
+// Levels of at most 1024 rows together (each started on a wave) take a launch of 2 us for every
+// smoothing step, residual and transfer.  Here a thread owns one row of one level for the whole
+// part of the cycle: its entries, its interpolation row and, with few entries a row, its
+// restriction row are loaded into registers at the start, all levels' in one memory round trip,
+// and the cycle runs on vectors in LDS with a barrier a step.  A step's operations are those of
+// the launches (x += damp ((b - A x) / A_ii), the first from zero; sums in FP64).  Bound by the
+// steps' chains of LDS reads, about 0.2 us each.  2D Poisson 32 x 32 cells, five levels of 289 to 4
+// rows: 11 us a cycle, 62 by launches.
+constexpr int kLowMax = 8, kLowRows = 1024;
+// rows in all of levels with more than 9 entries a row (3D): 27 of them fill the registers of more
+// waves, and with a level of 9^3 nodes the launches are as fast (<jacobi> cycles of 16^3 cells FP64:
+// 54 us, by launches 71, with 1024 rows 75)
+constexpr int kLowWide = 256;
+
+template <class T>
+struct LowLevel {
+  const int *rp, *ci;       // A
+  const T *av, *diag;
+  const int *prp, *pci;     // interpolation from the level below
+  const T *pv;
+  const int *rrp, *rci;     // restriction from the level above
+  const T *rv;
+  int n, off;               // rows, the first one's thread
+};
+template <class T>
+struct LowCycle {
+  LowLevel<T> lv[kLowMax];
+  int nl, pre, post;
+  T damp;
+  const T *rhs;             // the finest level's
+  T *sol;
+  const double *inv;        // the base level's inverse (m x m) or, in FP32, its one tile (64 wide)
+  const float *tile;
+  const int *cidx, *tidx;
+  int m, nt;
+};
+
+// W, PW: entries of a row and of an interpolation row at most.  RREG: the restriction rows (W
+// entries at most) are kept in registers
+template <class T, int W, int PW, bool RREG, int NT>
+__global__ __launch_bounds__(NT) void k_low_cycle(LowCycle<T> C) {
+  __shared__ T xs[2][NT], rs[NT];
+  const int t = threadIdx.x;
+  int k = -1;
+#pragma unroll
+  for (int l = 0; l < kLowMax; l++)
+    if (l < C.nl && t >= C.lv[l].off && t < C.lv[l].off + C.lv[l].n) k = l;
+  // wave-uniform, as levels start on waves; rows of none: k < 0
+  const int kw = __builtin_amdgcn_readfirstlane(max(k, 0));
+  const LowLevel<T> L = C.lv[kw];
+  const int row = k < 0 ? 0 : t - L.off;
+  const int below = kw > 0 ? C.lv[kw - 1].off : 0, above = kw + 1 < C.nl ? C.lv[kw + 1].off : 0;
+  T a[W], p[PW], r[RREG ? W : 1], d = (T)1, bi = (T)0, xi = (T)0;
+  int ai[W], pi[PW], ri[RREG ? W : 1], rb = 0, re = 0;
+#pragma unroll
+  for (int u = 0; u < W; u++) {
+    a[u] = (T)0;
+    ai[u] = t;
+  }
+#pragma unroll
+  for (int u = 0; u < PW; u++) {
+    p[u] = (T)0;
+    pi[u] = t;
+  }
+#pragma unroll
+  for (int u = 0; u < (RREG ? W : 1); u++) {
+    r[u] = (T)0;
+    ri[u] = t;
+  }
+  if (k > 0) {
+    const int b = L.rp[row], e = L.rp[row + 1], pb = L.prp[row], pe = L.prp[row + 1];
+    d = L.diag[row];
+#pragma unroll
+    for (int u = 0; u < W; u++)
+      if (b + u < e) {
+        a[u] = L.av[b + u];
+        ai[u] = L.off + L.ci[b + u];
+      }
+#pragma unroll
+    for (int u = 0; u < PW; u++)
+      if (pb + u < pe) {
+        p[u] = L.pv[pb + u];
+        pi[u] = below + L.pci[pb + u];
+      }
+  }
+  if (k >= 0 && k + 1 < C.nl) {
+    rb = L.rrp[row];
+    re = L.rrp[row + 1];
+    if (RREG)
+#pragma unroll
+      for (int u = 0; u < W; u++)
+        if (rb + u < re) {
+          r[u] = L.rv[rb + u];
+          ri[u] = above + L.rci[rb + u];
+        }
+  }
+  if (k >= 0 && k + 1 == C.nl) bi = C.rhs[row];
+  // b - A x from buffer q
+  auto residual = [&](int q) {
+    double s = (double)bi;
+#pragma unroll
+    for (int u = 0; u < W; u++) s -= (double)xs[q][ai[u]] * (double)a[u];
+    return s;
+  };
+  xs[0][t] = xs[1][t] = rs[t] = (T)0;
+  __syncthreads();
+  const int fin = (C.pre - 1) & 1;  // where the pre-smoothing ends
+  for (int l = C.nl - 1; l > 0; l--) {
+    if (k == l) {
+      xi = C.damp * (bi / d);
+      xs[0][t] = xi;
+    }
+    __syncthreads();
+    for (int s = 1; s < C.pre; s++) {
+      if (k == l) {
+        xi += C.damp * ((T)residual((s - 1) & 1) / d);
+        xs[s & 1][t] = xi;
+      }
+      __syncthreads();
+    }
+    if (k == l) rs[t] = (T)residual(fin);
+    __syncthreads();
+    if (k == l - 1) {
+      double s = 0;
+      if (RREG) {
+#pragma unroll
+        for (int u = 0; u < W; u++) s += (double)rs[ri[u]] * (double)r[u];
+      } else {
+        for (int e = rb; e < re; e++) s += (double)rs[above + L.rci[e]] * (double)L.rv[e];
+      }
+      bi = (T)s;
+    }
+  }
+  if (k == 0) rs[t] = bi;
+  __syncthreads();
+  if (k == 0) {  // the base level: its unit rows, then the others by the inverse
+    if (row < C.nt) xs[0][L.off + C.tidx[row]] = xs[1][L.off + C.tidx[row]] = rs[L.off + C.tidx[row]];
+    if (row < C.m) {
+      double s = 0;
+      for (int j = 0; j < C.m; j++)
+        s += (C.inv ? C.inv[row * C.m + j] : (double)C.tile[row * 64 + j]) *
+             (double)rs[L.off + C.cidx[j]];
+      const int o = L.off + C.cidx[row];
+      xs[0][o] = xs[1][o] = (T)s;
+    }
+  }
+  __syncthreads();
+  int from = 0;  // the buffer that holds the level below
+  for (int l = 1; l < C.nl; l++) {
+    if (k == l) {
+      double s = (double)xi;
+#pragma unroll
+      for (int u = 0; u < PW; u++) s += (double)xs[from][pi[u]] * (double)p[u];
+      xi = (T)s;
+      xs[fin][t] = xi;
+    }
+    __syncthreads();
+    for (int s = 0; s < C.post; s++) {
+      if (k == l) {
+        xi += C.damp * ((T)residual((fin + s) & 1) / d);
+        xs[(fin + s + 1) & 1][t] = xi;
+      }
+      __syncthreads();
+    }
+    from = (fin + C.post) & 1;
+  }
+  if (k >= 0 && k + 1 == C.nl) C.sol[row] = xi;
+}
+
+static bool low_wide(const flgpu_mat *A, const flgpu_mat *I) {
+  return A->sell.maxw > 9 || I->sell.maxw > 4 || I->transpose->sell.maxw > 9;
+}
+
+// The finest level of the part that k_low_cycle takes, -1: none.  One coarse cycle a level,
+// <jacobi> with a step before the restriction, the top level left out (its vectors are the
+// caller's), and rows that fit the registers.
+static int low_top(const flgpu_mg *mg) {
+  const flgpu_mg_params &p = mg->p;
+  if (p.smoother != FLGPU_SMOOTH_JACOBI || p.gamma != 1 || p.additive || p.fas ||
+      p.pre_steps < 1 || mg->lv[p.base_level].cinv.m > kSymB)
+    return -1;
+  int rows = 0, best = -1;
+  bool wide = false;
+  for (int l = p.base_level; l < mg->top && l - p.base_level < kLowMax; l++) {
+    const MGLevel &L = mg->lv[l];
+    rows += ((int)std::min(L.N, 2L * kLowRows) + 63) / 64 * 64;
+    if (l > p.base_level) {
+      const flgpu_mat *I = mg->lv[l - 1].I;
+      if (!L.A->diag || !I->transpose || L.A->sell.maxw > 27 || I->sell.maxw > 8) break;
+      wide = wide || low_wide(L.A, I);
+      if (rows > (wide ? kLowWide : kLowRows)) break;
+      best = l;
+    }
+  }
+  return best;
+}
+
+template <class T>
+static void low_cycle_t(flgpu_mg *mg, int lt) {
+  const flgpu_mg_params &p = mg->p;
+  const int base = p.base_level;
+  LowCycle<T> C{};
+  C.nl = lt - base + 1;
+  C.pre = p.pre_steps;
+  C.post = std::max(p.post_steps, 0);
+  C.damp = (T)p.omega;
+  C.rhs = (const T *)mg->lv[lt].rhs;
+  C.sol = (T *)mg->lv[lt].sol;
+  const DenseInverse &D = mg->lv[base].cinv;
+  C.inv = D.inv;
+  C.tile = D.tiles;
+  C.cidx = D.cidx;
+  C.tidx = D.tidx;
+  C.m = D.m;
+  C.nt = D.nt;
+  int off = 0;
+  bool wide = false;
+  for (int k = 0; k < C.nl; k++) {
+    const MGLevel &M = mg->lv[base + k];
+    LowLevel<T> &L = C.lv[k];
+    L.rp = M.A->rowptr;
+    L.ci = M.A->colidx;
+    L.av = (const T *)M.A->vals;
+    L.diag = (const T *)M.A->diag;
+    L.n = (int)M.N;
+    L.off = off;
+    off += (L.n + 63) / 64 * 64;
+    if (k > 0) {
+      const flgpu_mat *I = mg->lv[base + k - 1].I;
+      L.prp = I->rowptr;
+      L.pci = I->colidx;
+      L.pv = (const T *)I->vals;
+      wide = wide || low_wide(M.A, I);
+    }
+    if (k + 1 < C.nl) {
+      const flgpu_mat *R = M.I->transpose;
+      L.rrp = R->rowptr;
+      L.rci = R->colidx;
+      L.rv = (const T *)R->vals;
+    }
+  }
+  if (wide)
+    k_low_cycle<T, 27, 8, false, kLowWide><<<1, kLowWide, 0, mg->ctx->stream>>>(C);
+  else k_low_cycle<T, 9, 4, true, kLowRows><<<1, kLowRows, 0, mg->ctx->stream>>>(C);
+  FLGPU_HIP(hipGetLastError());
+}
+
 static void lmgc(flgpu_mg *mg, int l) {
   MGLevel &L = mg->lv[l];
   if (l == mg->p.base_level) {
@@ -703,6 +952,12 @@ static void lmgc(flgpu_mg *mg, int l) {
     C.x_zero = false;
     C.step1 = false;
     C.residual_p = true;
+  } else if (l - 1 == mg->low) {
+    // this level and those below by one launch
+    spmv(C.I->transpose, 1.0, lres(mg, l), 0.0, C.rhs, C.rhs);
+    if (mg->p.prec == FLGPU_F64) low_cycle_t<double>(mg, l - 1);
+    else low_cycle_t<float>(mg, l - 1);
+    C.x_zero = C.step1 = C.residual_p = false;
   } else if (fused && !base) {
     // the first coarse <jacobi> step from zero is pointwise in rhs: taken in the same pass
     // where the transfer allows it
@@ -731,7 +986,7 @@ static void lmgc(flgpu_mg *mg, int l) {
   // here every path that reads it recomputes it first (the smoothers' residual-before, the
   // restriction's ensure-mg-residual), so that step is left out.
   int reps = mg->p.gamma == 0 ? 0 : (base ? 1 : mg->p.gamma);
-  for (int i = 0; i < reps; i++) lmgc(mg, l - 1);
+  for (int i = 0; i < reps && l - 1 != mg->low; i++) lmgc(mg, l - 1);
   if (reps == 0) {  // the coarse correction is zero: sol_{l-1} must hold it
     if (C.x_zero) vfill(mg->ctx, C.N, mg->p.prec, C.sol, 0.0);
     C.x_zero = false;
@@ -757,6 +1012,7 @@ static void mg_cycle(flgpu_mg *mg, void *x, void *b, void *r) {
   mg->rhs_top = b;
   mg->res_top = r;
   mg->lv[mg->top].residual_p = true;
+  mg->low = low_top(mg);
   lmgc(mg, mg->top);
 }
 

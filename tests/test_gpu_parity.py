@@ -875,3 +875,30 @@ def test_mixed_precision_fcg():
                     pre_steps=2, post_steps=2, base_level=1, symmetric=1, tol=1e-12, maxsteps=100)
     _, xo, _, _ = oh.solve(prm)
     assert relerr(bb["solution"].numpy(), xo) < 1e-9
+
+
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("dim,order,n0,levels,pre,post,base",
+                         [(1, 1, 1, 5, 1, 0, 0), (1, 2, 1, 9, 2, 1, 0), (2, 1, 1, 6, 2, 2, 0),
+                          (2, 1, 3, 4, 1, 3, 1), (2, 1, 8, 3, 2, 1, 0), (2, 2, 1, 4, 3, 2, 0),
+                          (3, 1, 1, 5, 1, 2, 0), (3, 1, 2, 4, 2, 1, 1), (3, 2, 1, 3, 1, 1, 0)])
+def test_low_levels_in_one_launch(dim, order, n0, levels, pre, post, base, prec):
+    """<jacobi> V-cycles whose coarsest levels run in one launch (rows of at most 9 entries: up
+    to 1024 rows; wider ones 256), with one to three steps, none after the prolongation,
+    a base level of boundary rows only and one solved by its inverse, against the oracle's; FP32
+    to its rounding over the levels' steps"""
+    say(f"low levels dim={dim} order={order} n0={n0} levels={levels} V({pre},{post}) prec={prec}")
+    rng = np.random.default_rng(levels)
+    n = n0 << (levels - 1)
+    kap = np.exp(rng.normal(size=(n,) * dim))
+    cs, H = _gpu_hier(dim, order, n0, levels, po.SMOOTH_JACOBI, 0.7, pre, post, base, kappa=kap,
+                      prec=prec)
+    oh = po.Hierarchy(dim, order, n0, levels, kappa=kap)
+    prm = po.params(smoother=po.SMOOTH_JACOBI, omega=0.7, pre_steps=pre, post_steps=post,
+                    base_level=base)
+    r = rng.uniform(-1, 1, oh.ndofs()).astype(np.float32).astype(float)
+    r[po.boundary(dim, order, n)] = 0
+    ref = oh.apply(prm, r)
+    q = GpuVector(len(r), prec)
+    H.apply(q, GpuVector.from_array(r, prec), GpuVector.from_array(r, prec))
+    assert relerr(q.numpy(), ref) < (1e-12 if prec == F.F64 else 2e-5)
