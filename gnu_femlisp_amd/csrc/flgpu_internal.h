@@ -210,6 +210,7 @@ struct flgpu_mat {
   // full trilinear pattern (1: the interpolation, 2: its transpose): products read the CSR
   // values with the columns and row starts implied by the pattern (0: not such a matrix)
   int tp_kind = 0, tp_nc = 0;
+  bool tp_geo = false;  // the trilinear weights as assembled: products read no values
   // the values again as 27 planes over the coarse nodes c: for the transpose (tp_kind 2)
   // tp27[k][c], k = (dz+1)*9 + (dy+1)*3 + (dx+1), the entry of fine neighbour 2c + d; for the
   // interpolation (tp_kind 1) the entries of the fine nodes of c's block by parity class

@@ -1404,6 +1404,7 @@ flgpu_mat *lattice_interpolation(flgpu_ctx *ctx, int dim, int order, int nc, int
     if (dim == 3 && order == 1) {  // the trilinear pattern: products with implied columns
       P->tp_kind = 1;
       PT->tp_kind = 2;
+      P->tp_geo = PT->tp_geo = true;
       tp_prepare(P);
       tp_prepare(PT);
     }

@@ -315,8 +315,9 @@ void drop_cells(flgpu_mat *A) {
 }
 
 void mat_refresh_values(flgpu_mat *A) {
-  if (A->q2t) layout_changed(A);
+  if (A->q2t || A->tp_geo) layout_changed(A);
   A->q2t = 0;  // other values than the interpolation's
+  A->tp_geo = false;
   diag_refresh(A);
   stencil_refresh(A);
   if (A->tp_kind) tp_prepare(A);
@@ -433,6 +434,7 @@ flgpu_mat *mat_convert(const flgpu_mat *A, int prec) {
   B->tp_kind = A->tp_kind;
   B->tp_nc = A->tp_nc;
   B->q2t = A->q2t;
+  B->tp_geo = A->tp_geo;
   B->q2_nc = A->q2_nc;
   if (A->alpha) {
     long nc = (long)A->lat_n * A->lat_n * A->lat_n;
@@ -1599,7 +1601,9 @@ __global__ void k_tp8_fill(int nc, const T *__restrict__ vals, T *__restrict__ p
 
 // out = beta z + alpha P x: one thread per coarse node c writes the fine nodes of c's block
 // from the 8 coarse values of the cell [c, c + 1]^3 and the 27 planes
-template <class T>
+// GEO: the weights of the trilinear interpolation, powers of 1/2 per odd axis and 0 in the rows and
+// columns on the boundary, the same bits as the stored ones: 129^3 FP64 8.8 us, 18.0 with them
+template <class T, bool GEO>
 __global__ __launch_bounds__(256) void k_tp_prolong(int nc, FastDiv dMc,
                                                     const T *__restrict__ p27, T alpha,
                                                     const T *__restrict__ x, T beta,
@@ -1618,8 +1622,31 @@ __global__ __launch_bounds__(256) void k_tp_prolong(int nc, FastDiv dMc,
     if ((!pz || uz) && (!py || uy) && (!px || ux))
       xc[q] = x[c + ((unsigned)pz * Mc + (unsigned)py) * Mc + (unsigned)px];
   }
+  if (GEO) {
+    const int cc[3] = {cz, cy, cx};
+    T wa[3][3];  // per axis: even node; odd node's lower and upper neighbour
 #pragma unroll
-  for (int k = 0; k < 27; k++) w[k] = p27[(unsigned long)k * Nc + c];
+    for (int k = 0; k < 3; k++) {
+      wa[k][0] = cc[k] == 0 || cc[k] == nc ? (T)0 : (T)1;
+      wa[k][1] = cc[k] == 0 ? (T)0 : (T)0.5;
+      wa[k][2] = cc[k] + 1 == nc ? (T)0 : (T)0.5;
+    }
+#pragma unroll
+    for (int cls = 0; cls < 8; cls++) {
+      const int a = cls >> 2, b = (cls >> 1) & 1, e = cls & 1;
+#pragma unroll
+      for (int pz = 0; pz <= a; pz++)
+#pragma unroll
+        for (int py = 0; py <= b; py++)
+#pragma unroll
+          for (int px = 0; px <= e; px++)
+            w[tp_class_base(cls) + (pz * (b + 1) + py) * (e + 1) + px] =
+                wa[0][a + pz] * wa[1][b + py] * wa[2][e + px];
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 27; k++) w[k] = p27[(unsigned long)k * Nc + c];
+  }
   const unsigned f0 = ((unsigned)(2 * cz) * Mf + (unsigned)(2 * cy)) * Mf + (unsigned)(2 * cx);
 #pragma unroll
   for (int cls = 0; cls < 8; cls++) {
@@ -1685,7 +1712,7 @@ __global__ void k_tp27_fill(int nc, const T *__restrict__ tvals, T *__restrict__
 // out = beta z + alpha P^T r (coarse rows; t27 = the transpose's values as 27 planes).  FIRST:
 // also the first <jacobi> step from zero on the coarse level, xo = damp (out / diag), as
 // k_jacobi_zero forms it
-template <class T, bool FIRST = false>
+template <class T, bool GEO, bool FIRST = false>
 __global__ __launch_bounds__(256) void k_tp_restrict(int nc, FastDiv dMc,
                                                      const T *__restrict__ t27, T alpha,
                                                      const T *__restrict__ r, T beta,
@@ -1703,12 +1730,15 @@ __global__ __launch_bounds__(256) void k_tp_restrict(int nc, FastDiv dMc,
   const bool vz[3] = {cz > 0, true, cz < nc}, vy[3] = {cy > 0, true, cy < nc},
              vx[3] = {cx > 0, true, cx < nc};
   const unsigned f0 = ((unsigned)(2 * cz) * Mf + (unsigned)(2 * cy)) * Mf + (unsigned)(2 * cx);
+  // GEO: as in k_tp_prolong (129^3 FP64 7.0 us, 15.0 with the values)
+  const T inner = cz > 0 && cy > 0 && cx > 0 && cz < nc && cy < nc && cx < nc ? (T)1 : (T)0;
   T a[27], rv[27];
 #pragma unroll
   for (int e = 0; e < 27; e++) {
     const int dz = e / 9 - 1, dy = (e / 3) % 3 - 1, dx = e % 3 - 1;
     const bool live = vz[dz + 1] && vy[dy + 1] && vx[dx + 1];
-    a[e] = t27[(long)e * Nc + c];
+    a[e] = GEO ? inner * (dz ? (T)0.5 : (T)1) * (dy ? (T)0.5 : (T)1) * (dx ? (T)0.5 : (T)1)
+               : t27[(long)e * Nc + c];
     if (live) rv[e] = r[f0 + (unsigned)((dz * (int)Mf + dy) * (int)Mf + dx)];
   }
   T acc = (beta == (T)0) ? (T)0 : beta * z[c];
@@ -1762,14 +1792,17 @@ static void launch_tp(const flgpu_mat *A, T alpha, const void *x, T beta, const 
   const int nc = A->tp_nc;
   const long Nc = (long)(nc + 1) * (nc + 1) * (nc + 1);
   unsigned g = xcd_grid(grid_for(Nc, 256));
-  if (A->tp_kind == 1)
-    k_tp_prolong<T><<<g, 256, 0, A->ctx->stream>>>(nc, fast_div(nc + 1), (const T *)A->tp27,
-                                                   alpha, (const T *)x, beta, (const T *)z,
-                                                   (T *)out);
-  else
-    k_tp_restrict<T><<<g, 256, 0, A->ctx->stream>>>(nc, fast_div(nc + 1), (const T *)A->tp27,
-                                                    alpha, (const T *)x, beta, (const T *)z,
-                                                    (T *)out);
+  auto launch = [&](auto kern) {
+    kern<<<g, 256, 0, A->ctx->stream>>>(nc, fast_div(nc + 1), (const T *)A->tp27, alpha,
+                                        (const T *)x, beta, (const T *)z, (T *)out);
+  };
+  auto restricts = [&](auto kern) {
+    kern<<<g, 256, 0, A->ctx->stream>>>(nc, fast_div(nc + 1), (const T *)A->tp27, alpha,
+                                        (const T *)x, beta, (const T *)z, (T *)out, nullptr, (T)0,
+                                        nullptr);
+  };
+  if (A->tp_kind == 1) launch(A->tp_geo ? k_tp_prolong<T, true> : k_tp_prolong<T, false>);
+  else restricts(A->tp_geo ? k_tp_restrict<T, true> : k_tp_restrict<T, false>);
   FLGPU_HIP(hipGetLastError());
 }
 
@@ -1791,14 +1824,17 @@ bool restrict_first_step(const flgpu_mat *PT, const void *r, void *rhs, const fl
   const int nc = PT->tp_nc;
   const long Nc = (long)(nc + 1) * (nc + 1) * (nc + 1);
   unsigned g = xcd_grid(grid_for(Nc, 256));
-  if (PT->prec == FLGPU_F64)
-    k_tp_restrict<double, true><<<g, 256, 0, PT->ctx->stream>>>(
-        nc, fast_div(nc + 1), (const double *)PT->tp27, 1.0, (const double *)r, 0.0,
-        (const double *)rhs, (double *)rhs, (const double *)Ac->diag, damp, (double *)xo);
-  else
-    k_tp_restrict<float, true><<<g, 256, 0, PT->ctx->stream>>>(
-        nc, fast_div(nc + 1), (const float *)PT->tp27, 1.0f, (const float *)r, 0.0f,
-        (const float *)rhs, (float *)rhs, (const float *)Ac->diag, (float)damp, (float *)xo);
+  auto run = [&](auto t) {
+    using T = decltype(t);
+    auto launch = [&](auto kern) {
+      kern<<<g, 256, 0, PT->ctx->stream>>>(nc, fast_div(nc + 1), (const T *)PT->tp27, (T)1,
+                                           (const T *)r, (T)0, (const T *)rhs, (T *)rhs,
+                                           (const T *)Ac->diag, (T)damp, (T *)xo);
+    };
+    launch(PT->tp_geo ? k_tp_restrict<T, true, true> : k_tp_restrict<T, false, true>);
+  };
+  if (PT->prec == FLGPU_F64) run(0.0);
+  else run(0.0f);
   FLGPU_HIP(hipGetLastError());
   return true;
 }

@@ -730,3 +730,27 @@ def test_ssc_cycles_from_zeroed_levels(dim, m, levels, prec):
             check(lib().flgpu_mg_apply(H.h, x.h, b.h, r.h))
         outs.append(x.numpy())
     assert relerr(outs[0], outs[1]) < (1e-12 if prec == F.F64 else 1e-5)
+
+
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("nc", [1, 2, 7])
+def test_trilinear_transfers_follow_changed_values(nc, prec):
+    """the trilinear interpolation's products, which read no values, equal scipy's with the
+    assembled values, and with other values after those were changed (converted copies too)"""
+    say(f"trilinear transfers nc={nc} prec={prec}")
+    rng = np.random.default_rng(nc)
+    P = lat.interpolation(3, 1, nc, prec=prec)
+    rp, ci, v = P.csr()
+    xc = rng.uniform(-1, 1, P.ncols).astype(np.float32).astype(float)
+    yf = rng.uniform(-1, 1, P.nrows).astype(np.float32).astype(float)
+    tol = 1e-14 if prec == F.F64 else 2e-6
+    for changed in (False, True):
+        if changed:
+            v = (v * rng.uniform(0.5, 1.5, v.size)).astype(np.float32).astype(float)
+            P.update_values(v)
+        S = sp.csr_matrix((v.astype(float), ci, rp), shape=(P.nrows, P.ncols))
+        f, c = GpuVector(P.nrows, prec), GpuVector(P.ncols, prec)
+        gemm(1.0, P, GpuVector.from_array(xc, prec), 0.0, f)
+        gemm(1.0, P, GpuVector.from_array(yf, prec), 0.0, c, job="tn")
+        assert np.abs(f.numpy() - S @ xc).max() <= 8 * tol
+        assert np.abs(c.numpy() - S.T @ yf).max() <= 8 * tol
