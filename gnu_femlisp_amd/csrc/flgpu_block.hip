@@ -321,9 +321,9 @@ __device__ __forceinline__ void blk_runs(const int *__restrict__ colidx,
 // residual), then x_B += omega A_BB^-1 r_B.  <psc>: x_B += omega A_BB^-1 r_B with r as given.
 // b may be r.  The memory reads of a block are issued in batches of independent loads: the
 // row bounds; the CSR entries of the runs, 64 at a time and every lane its own entry; the x
-// values they name; then the block inverse, while the partial sums are reduced.  Every lane adds its products into per-slot
-// partial sums, and the 64 partials of each slot are summed in lane order through LDS by the
-// slot's own lane.
+// values they name; then the block inverse, while the partial sums are reduced.  Every lane adds
+// its products into per-slot partial sums, and the 64 partials of each slot are summed in lane
+// order through LDS by the slot's own lane.
 template <class T, bool SSC, int DIM>
 __global__ __launch_bounds__(64 * kBlkWaves) void k_blk_sweep(BlkGeom g, long cnt,
                                                               const int *__restrict__ rowptr,

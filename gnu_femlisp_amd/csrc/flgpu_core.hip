@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kRedThreads) void k_dot_partial(long n, const T *x,
   }
 }
 
-// up to three dots in one pass over the vectors: dot k's per-block partial is formed exactly
+// K <= 3 dots in one pass over the vectors: dot k's per-block partial is formed exactly
 // as k_dot_partial forms it (same grid, same order), into partial[k * gridDim.x + block]
 template <class T, int K>
 __global__ __launch_bounds__(kRedThreads) void k_dot_partial_multi(long n, const T *x0, const T *y0,
@@ -351,32 +351,22 @@ void dot_final(flgpu_ctx *ctx, const double *partial, int np, int slot) {
   FLGPU_HIP(hipGetLastError());
 }
 
-// dots (x[k], y[k]) into slots[k], k < count <= 3, in one pass; each equals vdot_dev's result
-void vdot_multi_dev(flgpu_ctx *ctx, long n, int prec, int count, const void *const *x,
+// dots (x[k], y[k]) into slots[k], k < 3, in one pass; each equals vdot_dev's result
+void vdot_multi_dev(flgpu_ctx *ctx, long n, int prec, const void *const *x,
                     const void *const *y, const int *slots) {
-  FLGPU_REQUIRE(count >= 1 && count <= 3, "vdot_multi_dev takes 1 to 3 dots");
-  for (int k = 0; k < count; k++)
+  for (int k = 0; k < 3; k++)
     FLGPU_REQUIRE(slots[k] >= 0 && slots[k] < kRedSlots, "reduction slot out of range");
-  const void *xx[3] = {x[0], count > 1 ? x[1] : x[0], count > 2 ? x[2] : x[0]};
-  const void *yy[3] = {y[0], count > 1 ? y[1] : y[0], count > 2 ? y[2] : y[0]};
   hipStream_t st = ctx->stream;
-#define FLGPU_DOTS(T, K)                                                                      \
-  k_dot_partial_multi<T, K><<<kRedBlocks, kRedThreads, 0, st>>>(                              \
-      n, (const T *)xx[0], (const T *)yy[0], (const T *)xx[1], (const T *)yy[1],              \
-      (const T *)xx[2], (const T *)yy[2], ctx->red_partial)
-  if (prec == FLGPU_F64) {
-    if (count == 1) FLGPU_DOTS(double, 1);
-    else if (count == 2) FLGPU_DOTS(double, 2);
-    else FLGPU_DOTS(double, 3);
-  } else {
-    if (count == 1) FLGPU_DOTS(float, 1);
-    else if (count == 2) FLGPU_DOTS(float, 2);
-    else FLGPU_DOTS(float, 3);
-  }
-#undef FLGPU_DOTS
-  k_dot_final_multi<<<count, kRedBlocks, 0, st>>>(ctx->red_partial, kRedBlocks, ctx->red_out,
-                                                  slots[0], count > 1 ? slots[1] : slots[0],
-                                                  count > 2 ? slots[2] : slots[0]);
+  if (prec == FLGPU_F64)
+    k_dot_partial_multi<double, 3><<<kRedBlocks, kRedThreads, 0, st>>>(
+        n, (const double *)x[0], (const double *)y[0], (const double *)x[1],
+        (const double *)y[1], (const double *)x[2], (const double *)y[2], ctx->red_partial);
+  else
+    k_dot_partial_multi<float, 3><<<kRedBlocks, kRedThreads, 0, st>>>(
+        n, (const float *)x[0], (const float *)y[0], (const float *)x[1], (const float *)y[1],
+        (const float *)x[2], (const float *)y[2], ctx->red_partial);
+  k_dot_final_multi<<<3, kRedBlocks, 0, st>>>(ctx->red_partial, kRedBlocks, ctx->red_out,
+                                              slots[0], slots[1], slots[2]);
   FLGPU_HIP(hipGetLastError());
 }
 

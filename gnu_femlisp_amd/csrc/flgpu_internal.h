@@ -389,8 +389,8 @@ __device__ __forceinline__ void parts_sum(const double *__restrict__ part, int n
   for (int k = 0; k < K; k++) out[k] = ((ws[k][0] + ws[k][1]) + ws[k][2]) + ws[k][3];
 }
 
-// 1 to 3 dots in one pass, each identical to vdot_dev's
-void vdot_multi_dev(flgpu_ctx *ctx, long n, int prec, int count, const void *const *x,
+// three dots in one pass, each identical to vdot_dev's
+void vdot_multi_dev(flgpu_ctx *ctx, long n, int prec, const void *const *x,
                     const void *const *y, const int *slots);
 double vdot_host(flgpu_ctx *ctx, long n, int prec, const void *x,
                  const void *y);

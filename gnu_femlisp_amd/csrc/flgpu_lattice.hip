@@ -1170,8 +1170,8 @@ flgpu_mat *lattice_galerkin(const flgpu_mat *P, const flgpu_mat *Afine, int dim,
 // The weights of node i = (z, y, x) with the parities (OZ, OY, OX): every offset is a constant, so
 // the neighbours' weights are loaded together and only those that exist (a node has one weight on
 // an even axis, two on an odd one).  Bound by the divisions and the rows' 27 entries.  Three
-// passes at 97^3 FP32 75 us, 12 on small lattices; with a loop over the entries, each waiting for its weights, and all
-// nodes' threads in every pass 493 and 148.
+// passes at 97^3 FP32 75 us, 12 on small lattices; with a loop over the entries, each waiting for
+// its weights, and all nodes' threads in every pass 493 and 148.
 template <class T, int OZ, int OY, int OX>
 __device__ __forceinline__ void bbox_node(int M, int z, int y, int x,
                                           const int *__restrict__ rowptr,

@@ -1389,11 +1389,10 @@ constexpr int kTileRows(int H) { return ((H + 7) / 2) * ((kTileCols + 7) / 2); }
 
 // OFF0: x is zero on the planes z -+ 1, ZERO: on the plane itself; those are not read.
 template <class T, bool SYM, bool OFF0, bool ZERO, int H, int G>
-__global__ __launch_bounds__((kTileRows(H) + 63) / 64 * 64 * G) void k_st27_sor_tiles(int M, int pz, int W, int ntx, int nty,
-                                                        int planes, int backwards,
-                                                        const T *__restrict__ val27, T omega,
-                                                        const T *__restrict__ xs, const T *xoff,
-                                                        T *xd, const T *__restrict__ b, T *r) {
+__global__ __launch_bounds__((kTileRows(H) + 63) / 64 * 64 * G) void k_st27_sor_tiles(
+    int M, int pz, int W, int ntx, int nty, int planes, int backwards,
+    const T *__restrict__ val27, T omega, const T *__restrict__ xs, const T *xoff, T *xd,
+    const T *__restrict__ b, T *r) {
   constexpr int LW = kTileCols + 8, P = (kTileRows(H) + 63) / 64 * 64;
   __shared__ T lx[(H + 8) * LW];  // x of lines y0 - 4.., columns x0 - 4..; 0 outside the lattice
   const unsigned lb = xcd_block(blockIdx.x, gridDim.x);

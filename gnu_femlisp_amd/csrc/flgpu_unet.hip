@@ -220,8 +220,9 @@ __device__ __forceinline__ void conv_stage_table(const ConvGeom &G, const ConvIn
 // fragment (512 contiguous bytes, from L1/L2, fetched a group of iterations ahead).  Products
 // accumulate tap by tap and, within a tap, 16 channels at a time in ascending order.
 // Batch 32, 32^3, [32 up, 16 skip] -> 16 channels: 189 us, 115 TFLOP/s (227 without conv_table),
-// bound by LDS reads and the staging (2559 us and 215 us for the concatenation as one wave per 16 voxels without LDS, which
-// rounded the inputs and fetched single 2-byte weights anew for each of the 27 taps).
+// bound by LDS reads and the staging (2559 us and 215 us for the concatenation as one wave per
+// 16 voxels without LDS, which rounded the inputs and fetched single 2-byte weights anew for each
+// of the 27 taps).
 template <int MT, int NT>
 __global__ __launch_bounds__(256) void k_conv(ConvGeom G, ConvIn in, int nch, Div1 dq, int no,
                                               int ntt, const short *__restrict__ wf,
@@ -1365,7 +1366,7 @@ struct UnetHook : LearnedHook {
     {  // c . r1, c . A c and the cycle step's z1 . r, one pass
       const void *dx[3] = {c, c, q}, *dy[3] = {r1, Ac, r};
       const int slots[3] = {11, 12, 13};
-      vdot_multi_dev(ctx, N, prec, 3, dx, dy, slots);
+      vdot_multi_dev(ctx, N, prec, dx, dy, slots);
     }
     k_add_opt<double><<<grid_for(N, 256), 256, 0, s>>>(N, ctx->red_out + 11, min_gain,
                                                        ctx->red_out + flag, (const double *)c,
