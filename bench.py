@@ -387,17 +387,17 @@ def main():
                 del M
             # the structured transfers between this level and the one below: prolongation with
             # beta 1, as the V-cycle adds the correction; restriction into its own vector.
-            # Algorithmic bytes: the 27 value planes over the coarse nodes, the coarse vector,
-            # the fine vector read (and, for the prolongation, written)
+            # Algorithmic bytes: the coarse vector and the fine vector read (and, for the
+            # prolongation, written); the geometric weights are not read
             P = lat.interpolation(3, 1, n // 2, prec=prec)
             Nc, Nf = P.ncols, P.nrows
             xc = GpuVector.from_array(np.random.default_rng(1).uniform(-1, 1, Nc), prec)
             yf = GpuVector.from_array(np.random.default_rng(2).uniform(-1, 1, Nf), prec)
             rc = GpuVector(Nc, prec)
             for name, fn, byt in (
-                    (f"tp_prolong_{tag}", lambda: gemm(1.0, P, xc, 1.0, yf), (28 * Nc + 2 * Nf) * vb),
+                    (f"tp_prolong_{tag}", lambda: gemm(1.0, P, xc, 1.0, yf), (Nc + 2 * Nf) * vb),
                     (f"tp_restrict_{tag}", lambda: gemm(1.0, P, yf, 0.0, rc, job="tn"),
-                     (28 * Nc + Nf) * vb)):
+                     (Nc + Nf) * vb)):
                 fn()
                 ctx.timer_start()
                 for _ in range(reps):
