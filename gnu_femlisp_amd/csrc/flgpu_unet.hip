@@ -161,23 +161,30 @@ __device__ __forceinline__ void conv_table(const ConvGeom &G, int up, int b, int
 // stage one chunk at a time, are faster without: 74 against 93 us)
 __device__ __forceinline__ void conv_stage_table(const ConvGeom &G, const ConvIn &in, int nch,
                                                  Div1 dq, const int *tab, short *lds) {
-  const int Q = nch * 4, total = G.hvol * Q, ct = in.c0 + in.c1;
+  const int Q = nch * 4, total = G.hvol * Q, ct = in.c0 + in.c1, hv = in.up ? G.hvol : 0;
   constexpr int U = 4;
   auto run = [&](auto vec) {
     for (int e0 = threadIdx.x; e0 < total; e0 += U * 256) {
       float4 f[U];
       int dst[U], left[U];  // channels from the entry's first on, 0: nothing there
+      int vox[U], vup[U];   // read together, without a branch
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const unsigned pos = fdiv((unsigned)min(e0 + u * 256, total - 1), dq);
+        vox[u] = tab[pos];
+        vup[u] = tab[hv + pos];
+      }
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const int e = e0 + u * 256;
         const unsigned ec = (unsigned)min(e, total - 1);
         const unsigned pos = fdiv(ec, dq), q = ec - pos * (unsigned)Q;
-        const int c = (int)q * 4, v = tab[pos];
+        const int c = (int)q * 4, v = vox[u];
         dst[u] = e < total ? (int)(((q >> 2) * (unsigned)G.hvol + pos) * 16u + (q & 3u) * 4u) : -1;
         const bool live = v >= 0 && c < ct, second = c >= in.c0;
         left[u] = live ? ct - c : 0;
         // unconditional loads, of the first values where there is nothing to load
-        const unsigned w = live ? (unsigned)(in.up && !second ? tab[G.hvol + pos] : v) : 0u;
+        const unsigned w = live ? (unsigned)(second ? v : vup[u]) : 0u;
         const unsigned cs = (unsigned)(second ? in.c1 : in.c0),
                        cc = live ? (unsigned)(second ? c - in.c0 : c) : 0u;
         const float *src = (live && second ? in.p1 : in.p0) + (size_t)w * cs + cc;
@@ -219,7 +226,7 @@ __device__ __forceinline__ void conv_stage_table(const ConvGeom &G, const ConvIn
 // MT x NT tiles of 16 voxels x 16 channels, which share each voxel operand (LDS) and each weight
 // fragment (512 contiguous bytes, from L1/L2, fetched a group of iterations ahead).  Products
 // accumulate tap by tap and, within a tap, 16 channels at a time in ascending order.
-// Batch 32, 32^3, [32 up, 16 skip] -> 16 channels: 189 us, 115 TFLOP/s (227 without conv_table),
+// Batch 32, 32^3, [32 up, 16 skip] -> 16 channels: 178 us, 244 TFLOP/s (227 us without conv_table),
 // bound by LDS reads and the staging (2559 us and 215 us for the concatenation as one wave per
 // 16 voxels without LDS, which rounded the inputs and fetched single 2-byte weights anew for each
 // of the 27 taps).
@@ -267,6 +274,11 @@ __global__ __launch_bounds__(256) void k_conv(ConvGeom G, ConvIn in, int nch, Di
   const v4s *wp = (const v4s *)wf + (long)nw * NT * 64 + lane;
   // weight fragments of PF iterations (tap, chunk) are in flight ahead of their use
   constexpr int PF = MT == 1 || NT == 1 ? 9 : 3;  // divides the 27 taps
+  // iterations whose voxels are read from LDS together: read one by one, a wave with one tile
+  // waits for LDS at every product (one sample of 32^3: convolutions of 10.4..12.9 us, together
+  // 9.5..11.0; more weights ahead, or fetched before the staging, gave nothing)
+  constexpr int PA = MT == 1 ? 9 : 3;
+  static_assert(PF % PA == 0, "a group of weights holds whole groups of voxels");
   v4s bw[PF][NT];
 #pragma unroll
   for (int u = 0; u < PF; u++)
@@ -276,29 +288,35 @@ __global__ __launch_bounds__(256) void k_conv(ConvGeom G, ConvIn in, int nch, Di
   int tz = -1, ty = -1, tx = -1, ch = 0;  // offset of the tap, channel chunk
   for (int it = 0; it < nit; it += PF) {
 #pragma unroll
-    for (int u = 0; u < PF; u++) {
-      const int off = (((tz * hy + ty) * hx + tx) * sgn + ch * G.hvol) * 16;
-      v4s a[MT];
+    for (int u0 = 0; u0 < PF; u0 += PA) {
+      v4s a[PA][MT];
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) a[mt] = *(const v4s *)(lds + abase[mt] + off);
+      for (int u = 0; u < PA; u++) {
+        const int off = (((tz * hy + ty) * hx + tx) * sgn + ch * G.hvol) * 16;
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-          acc[mt][t] =
-              __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bw[u][t], a[mt], acc[mt][t], 0, 0, 0);
-      const int nx = min(it + u + PF, nit - 1);
-#pragma unroll
-      for (int t = 0; t < NT; t++) bw[u][t] = wp[((long)nx * ntt + t) * 64];
-      if (++ch == nch) {
-        ch = 0;
-        if (++tx == 2) {
-          tx = -1;
-          if (++ty == 2) {
-            ty = -1;
-            tz++;
+        for (int mt = 0; mt < MT; mt++) a[u][mt] = *(const v4s *)(lds + abase[mt] + off);
+        if (++ch == nch) {
+          ch = 0;
+          if (++tx == 2) {
+            tx = -1;
+            if (++ty == 2) {
+              ty = -1;
+              tz++;
+            }
           }
         }
+      }
+#pragma unroll
+      for (int u = 0; u < PA; u++) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+          for (int t = 0; t < NT; t++)
+            acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bw[u0 + u][t], a[u][mt],
+                                                                   acc[mt][t], 0, 0, 0);
+        const int nx = min(it + u0 + u + PF, nit - 1);
+#pragma unroll
+        for (int t = 0; t < NT; t++) bw[u0 + u][t] = wp[((long)nx * ntt + t) * 64];
       }
     }
   }
