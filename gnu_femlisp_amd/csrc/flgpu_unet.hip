@@ -89,55 +89,56 @@ __device__ __forceinline__ void conv_box(const ConvGeom &G, int t, int &b, int &
 __device__ __forceinline__ void conv_stage(const ConvGeom &G, const ConvIn &in, int ch0, int nch,
                                            Div1 dq, int b, int z0, int y0, int x0, short *lds) {
   const int Q = nch * 4, total = G.hvol * Q, ct = in.c0 + in.c1, n = G.n, h = n >> 1;
-  const bool vec = ((in.c0 | in.c1) & 3) == 0;
   constexpr int U = 4;
-  for (int e0 = threadIdx.x; e0 < total; e0 += U * 256) {
-    float f[U][4];
-    int dst[U];
-    bool live[U];
+  auto run = [&](auto vec) {
+    for (int e0 = threadIdx.x; e0 < total; e0 += U * 256) {
+      float4 f[U];
+      int dst[U], left[U];  // channels from the entry's first on, 0: nothing there
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int e = e0 + u * 256;
-      const unsigned ec = (unsigned)min(e, total - 1);
-      const unsigned pos = fdiv(ec, dq), q = ec - pos * (unsigned)Q;
-      const unsigned t = fdiv(pos, G.dhx);
-      const int hx = (int)(pos - t * G.dhx.f.d);
-      const unsigned hz = fdiv(t, G.dhy);
-      const int hy = (int)(t - hz * G.dhy.f.d);
-      const int z = z0 + (int)hz - 1, y = y0 + hy - 1, x = x0 + hx - 1;
-      const int c = ch0 * 16 + (int)q * 4;
-      dst[u] = e < total ? (int)(((q >> 2) * (unsigned)G.hvol + pos) * 16u + (q & 3u) * 4u) : -1;
-      live[u] = z >= 0 && y >= 0 && x >= 0 && z < n && y < n && x < n && c < ct;
-      const bool second = c >= in.c0;
-      const int cs = second ? in.c1 : in.c0, cc = second ? c - in.c0 : c;
-      const float *src = second ? in.p1 : in.p0;
-      long vox;
-      if (in.up && !second)
-        vox = (((long)b * h + (z >> 1)) * h + (y >> 1)) * h + (x >> 1);
-      else
-        vox = (((long)b * n + z) * n + y) * n + x;
-      if (vec) {
-        const float4 v = live[u] ? *(const float4 *)(src + vox * cs + cc)
-                                 : make_float4(0.f, 0.f, 0.f, 0.f);
-        f[u][0] = v.x;
-        f[u][1] = v.y;
-        f[u][2] = v.z;
-        f[u][3] = v.w;
-      } else {  // channel counts that are no multiple of 4 (one source)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          f[u][j] = live[u] && c + j < ct ? in.p0[vox * in.c0 + c + j] : 0.f;
+      for (int u = 0; u < U; u++) {
+        const int e = e0 + u * 256;
+        const unsigned ec = (unsigned)min(e, total - 1);
+        const unsigned pos = fdiv(ec, dq), q = ec - pos * (unsigned)Q;
+        const unsigned t = fdiv(pos, G.dhx);
+        const int hx = (int)(pos - t * G.dhx.f.d);
+        const unsigned hz = fdiv(t, G.dhy);
+        const int hy = (int)(t - hz * G.dhy.f.d);
+        const int z = z0 + (int)hz - 1, y = y0 + hy - 1, x = x0 + hx - 1;
+        const int c = ch0 * 16 + (int)q * 4;
+        dst[u] = e < total ? (int)(((q >> 2) * (unsigned)G.hvol + pos) * 16u + (q & 3u) * 4u) : -1;
+        const bool live = (unsigned)z < (unsigned)n && (unsigned)y < (unsigned)n &&
+                          (unsigned)x < (unsigned)n && c < ct;
+        left[u] = live ? ct - c : 0;
+        // unconditional loads, of the first values where there is nothing to load: a load in a
+        // branch of its own waits for the one before it
+        const bool second = live && c >= in.c0;
+        const int cs = second ? in.c1 : in.c0, cc = second ? c - in.c0 : c;
+        const int sh = in.up && !second ? 1 : 0, m = sh ? h : n;
+        const long vox = (((long)b * m + (z >> sh)) * m + (y >> sh)) * m + (x >> sh);
+        const float *src = (second ? in.p1 : in.p0) + (live ? vox * cs + cc : 0);
+        if (vec) {
+          f[u] = *(const float4 *)src;
+        } else {  // channel counts that are no multiple of 4 (one source)
+          f[u].x = src[0];
+          f[u].y = src[left[u] > 1 ? 1 : 0];
+          f[u].z = src[left[u] > 2 ? 2 : 0];
+          f[u].w = src[left[u] > 3 ? 3 : 0];
+        }
       }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (dst[u] >= 0) {
+          v4s s;
+          s[0] = left[u] > 0 ? bf16_bits(f[u].x) : (short)0;
+          s[1] = left[u] > 1 ? bf16_bits(f[u].y) : (short)0;
+          s[2] = left[u] > 2 ? bf16_bits(f[u].z) : (short)0;
+          s[3] = left[u] > 3 ? bf16_bits(f[u].w) : (short)0;
+          *(v4s *)(lds + dst[u]) = s;
+        }
     }
-#pragma unroll
-    for (int u = 0; u < U; u++)
-      if (dst[u] >= 0) {
-        v4s s;
-#pragma unroll
-        for (int j = 0; j < 4; j++) s[j] = bf16_bits(f[u][j]);
-        *(v4s *)(lds + dst[u]) = s;
-      }
-  }
+  };
+  if (((in.c0 | in.c1) & 3) == 0) run(std::true_type());
+  else run(std::false_type());
 }
 
 // The voxel of every position of the box at (b, z0, y0, x0) and its halo, -1 outside the grid; of
@@ -376,7 +377,10 @@ __global__ __launch_bounds__(256) void k_conv(ConvGeom G, ConvIn in, int nch, Di
 // wave's gradient operand serves its seven taps.  The blocks of the first channel chunk also sum
 // gout in FP32 (the bias gradient).  Every block writes its sums as a partial
 // [block][27 ci co + co]; k_wgrad_reduce adds them in a fixed order.
-// Batch 32, 32^3, 48 x 16 channels: 213 us (3592 us with one tap per block, which read the
+// Bound by latency: four blocks a CU (128 registers a thread; with three 208 us), whose staging
+// loads are issued four at a time and whose seven taps' operands are read together.
+// Batch 32, 32^3, 48 x 16 channels: 185 us, 16 x 16 channels 66 (213 and 73 with every staging
+// load and every operand waited for by itself; 3592 us with one tap per block, which read the
 // inputs 27 times and gathered the operands from LDS two bytes at a time).
 
 constexpr int kWgVox = 256;  // voxels of a box, 16 K steps
@@ -387,9 +391,9 @@ __device__ __forceinline__ v4s lds_read_tr(const short *p) {
 }
 
 template <int NTO>
-__global__ __launch_bounds__(256) void k_conv_wgrad(ConvGeom G, ConvIn in, int ncc, int co,
-                                                    const float *__restrict__ gout, int P,
-                                                    float *__restrict__ partial) {
+__global__ __launch_bounds__(256, NTO <= 2 ? 4 : 2) void k_conv_wgrad(
+    ConvGeom G, ConvIn in, int ncc, int co, const float *__restrict__ gout, int P,
+    float *__restrict__ partial) {
   extern __shared__ __align__(16) short lds[];
   constexpr int Q = NTO * 4;
   short *sa = lds;                                // [halo voxel][16]
@@ -420,37 +424,51 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(ConvGeom G, ConvIn in, int n
     // the output gradients: thread tid takes the channels 4 (tid % Q) .. + 3 of every box voxel
     // tid / Q + k 256 / Q
     const int q = tid % Q;
-#pragma unroll 4
-    for (int m = tid / Q; m < kWgVox; m += 256 / Q) {
-      const unsigned mc = (unsigned)(m < G.vol ? m : 0), t = fdiv(mc, G.dbx);
-      const int xx = (int)(mc - t * G.dbx.f.d);
-      const unsigned zz = fdiv(t, G.dby);
-      const int yy = (int)(t - zz * G.dby.f.d);
-      const int z = z0 + (int)zz, y = y0 + yy, x = x0 + xx;
-      const bool ok = m < G.vol && z < G.n && y < G.n && x < G.n;
-      const long v = (((long)b * G.n + z) * G.n + y) * G.n + x;
-      float f[4];
-      if ((co & 3) == 0) {
-        const float4 r = ok && 4 * q < co ? *(const float4 *)(gout + v * co + 4 * q)
-                                          : make_float4(0.f, 0.f, 0.f, 0.f);
-        f[0] = r.x;
-        f[1] = r.y;
-        f[2] = r.z;
-        f[3] = r.w;
-      } else {
+    constexpr int U = 4;  // loads in flight together
+    auto run = [&](auto vec) {
+      for (int m0 = tid / Q; m0 < kWgVox; m0 += U * (256 / Q)) {
+        float4 fr[U];
+        int hp[U];  // the voxel's halo position, -1: outside the grid
 #pragma unroll
-        for (int j = 0; j < 4; j++) f[j] = ok && 4 * q + j < co ? gout[v * co + 4 * q + j] : 0.f;
-      }
-      v4s s;
+        for (int u = 0; u < U; u++) {
+          const int m = m0 + u * (256 / Q);
+          const unsigned mc = (unsigned)(m < G.vol ? m : 0), t = fdiv(mc, G.dbx);
+          const int xx = (int)(mc - t * G.dbx.f.d);
+          const unsigned zz = fdiv(t, G.dby);
+          const int yy = (int)(t - zz * G.dby.f.d);
+          const int z = z0 + (int)zz, y = y0 + yy, x = x0 + xx;
+          const bool ok = m < G.vol && z < G.n && y < G.n && x < G.n;
+          const long v = (((long)b * G.n + z) * G.n + y) * G.n + x;
+          hp[u] = ok ? (((int)zz + 1) * hy + yy + 1) * hx + xx + 1 : -1;
+          const int left = ok ? co - 4 * q : 0;
+          const float *src = gout + (left > 0 ? v * co + 4 * q : 0);
+          if (vec) {
+            fr[u] = *(const float4 *)src;
+          } else {
+            fr[u].x = src[0];
+            fr[u].y = src[left > 1 ? 1 : 0];
+            fr[u].z = src[left > 2 ? 2 : 0];
+            fr[u].w = src[left > 3 ? 3 : 0];
+          }
+        }
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        bs[j] += f[j];
-        s[j] = bf16_bits(f[j]);
+        for (int u = 0; u < U; u++) {
+          const int m = m0 + u * (256 / Q), left = hp[u] >= 0 ? co - 4 * q : 0;
+          const float f[4] = {left > 0 ? fr[u].x : 0.f, left > 1 ? fr[u].y : 0.f,
+                              left > 2 ? fr[u].z : 0.f, left > 3 ? fr[u].w : 0.f};
+          v4s s;
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            bs[j] += f[j];
+            s[j] = bf16_bits(f[j]);
+          }
+          *(v4s *)(sg + ((long)(q >> 2) * kWgVox + m) * 16 + (q & 3) * 4) = s;
+          if (q == 0) pt[m] = hp[u] >= 0 ? (unsigned short)hp[u] : (unsigned short)0xffff;
+        }
       }
-      *(v4s *)(sg + ((long)(q >> 2) * kWgVox + m) * 16 + (q & 3) * 4) = s;
-      if (q == 0)
-        pt[m] = ok ? (unsigned short)((((int)zz + 1) * hy + yy + 1) * hx + xx + 1) : 0xffff;
-    }
+    };
+    if ((co & 3) == 0) run(std::true_type());
+    else run(std::false_type());
     __syncthreads();
 #pragma unroll 2
     for (int ks = 0; ks < kWgVox; ks += 16) {
@@ -461,13 +479,15 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(ConvGeom G, ConvIn in, int n
 #pragma unroll
       for (int k = 0; k < NTO; k++)
         bb[k] = lds_read_tr(sg + ((long)k * kWgVox + m) * 16 + 4 * (l16 & 3));
+      v4s a[7];
 #pragma unroll
-      for (int t = 0; t < 7; t++) {
-        const v4s a = lds_read_tr(pos == 0xffffu ? sz : ab + toff[t]);
+      for (int t = 0; t < 7; t++) a[t] = lds_read_tr(pos == 0xffffu ? sz : ab + toff[t]);
+      __builtin_amdgcn_sched_barrier(0);  // else each is read when its product needs it
+#pragma unroll
+      for (int t = 0; t < 7; t++)
 #pragma unroll
         for (int k = 0; k < NTO; k++)
-          acc[t][k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb[k], acc[t][k], 0, 0, 0);
-      }
+          acc[t][k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[t], bb[k], acc[t][k], 0, 0, 0);
     }
   }
   const long npair = (long)ct * co, stride = 27 * npair + co;
