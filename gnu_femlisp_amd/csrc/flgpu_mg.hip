@@ -1057,7 +1057,10 @@ void mg_apply_ptr(flgpu_mg *mg, int vprec, void *x, void *b, void *r) {
 // bookkeeping restarts at every cycle), so it is captured once per vector
 // triple into a HIP graph and replayed: one launch instead of ~40 per level.
 // The cycle clears with fill kernels, never with memset nodes.
+// A replay may still be queued (flgpu_mg_apply returns before its cycle has run): the stream is
+// waited for before an executable graph goes.
 static void graphs_clear(flgpu_mg *mg) {
+  if (!mg->graphs.empty()) (void)hipStreamSynchronize(mg->ctx->stream);
   for (auto &g : mg->graphs) (void)hipGraphExecDestroy(g.exec);
   mg->graphs.clear();
 }
