@@ -4,6 +4,7 @@
 // (src/matlisp/vector.lisp:224-326, src/matlisp/sparse-vector.lisp:248-280):
 // fill!/x<-0, copy!, scal!, axpy!, dot, norm.  Dots are reduced in FP64 in a
 // fixed order (fixed grid, fixed tree) so results are bit-reproducible.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -19,9 +20,26 @@ static thread_local std::string g_last_error;
 void set_error(const std::string &msg) { g_last_error = msg; }
 void clear_error() { g_last_error.clear(); }
 
+// The contexts, whose free blocks any allocation may need (never destroyed: a context may be given
+// up while the process ends).  Taken before a context's scratch_mu.
+static std::mutex &pools_mu() {
+  static std::mutex *m = new std::mutex;
+  return *m;
+}
+static std::vector<flgpu_ctx *> &pools() {
+  static std::vector<flgpu_ctx *> *v = new std::vector<flgpu_ctx *>;
+  return *v;
+}
+
 void *dev_alloc(size_t bytes) {
   void *p = nullptr;
   if (bytes == 0) bytes = 8;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  {  // the memory that the contexts keep for their next setup, whoever needs it
+    std::lock_guard<std::mutex> g(pools_mu());
+    for (flgpu_ctx *c : pools()) scratch_release(c);
+  }
   FLGPU_HIP(hipMalloc(&p, bytes));
   return p;
 }
@@ -31,34 +49,36 @@ void dev_free(void *p) {
 }
 
 void scratch_release(flgpu_ctx *ctx) {
-  for (auto &b : ctx->scratch_free) dev_free(b.second);
+  std::lock_guard<std::mutex> g(ctx->scratch_mu);
+  for (auto &b : ctx->scratch_free) dev_free(b.second);  // waits for the work that used it
   ctx->scratch_free.clear();
   ctx->scratch_held = 0;
 }
 
 void *scratch_get(flgpu_ctx *ctx, size_t bytes) {
   bytes = (std::max(bytes, (size_t)1) + 255) & ~(size_t)255;
-  auto &f = ctx->scratch_free;
-  // the smallest free block that holds it, unless most of that would lie idle
-  size_t best = f.size();
-  for (size_t i = 0; i < f.size(); i++)
-    if (f[i].first >= bytes && f[i].first <= 2 * bytes + 4096 &&
-        (best == f.size() || f[i].first < f[best].first))
-      best = i;
   void *p = nullptr;
   size_t n = bytes;
   ctx->scratch_used.reserve(ctx->scratch_used.size() + 1);
-  if (best < f.size()) {
-    n = f[best].first;
-    p = f[best].second;
-    f[best] = f.back();
-    f.pop_back();
-    ctx->scratch_held -= n;
-  } else if (hipMalloc(&p, bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    scratch_release(ctx);
-    p = dev_alloc(bytes);
+  {
+    std::lock_guard<std::mutex> g(ctx->scratch_mu);
+    auto &f = ctx->scratch_free;
+    f.reserve(f.size() + ctx->scratch_used.size() + 1);  // scratch_put allocates nothing
+    // the smallest free block that holds it, unless most of that would lie idle
+    size_t best = f.size();
+    for (size_t i = 0; i < f.size(); i++)
+      if (f[i].first >= bytes && f[i].first <= 2 * bytes + 4096 &&
+          (best == f.size() || f[i].first < f[best].first))
+        best = i;
+    if (best < f.size()) {
+      n = f[best].first;
+      p = f[best].second;
+      f[best] = f.back();
+      f.pop_back();
+      ctx->scratch_held -= n;
+    }
   }
+  if (!p) p = dev_alloc(bytes);
   ctx->scratch_used[p] = n;
   return p;
 }
@@ -68,12 +88,15 @@ void scratch_put(flgpu_ctx *ctx, void *p) {
   auto it = ctx->scratch_used.find(p);
   const size_t n = it->second;
   ctx->scratch_used.erase(it);
-  if (ctx->scratch_held + n > kScratchKeep) {
-    dev_free(p);
-    return;
+  {
+    std::lock_guard<std::mutex> g(ctx->scratch_mu);
+    if (ctx->scratch_held + n <= kScratchKeep) {
+      ctx->scratch_free.emplace_back(n, p);
+      ctx->scratch_held += n;
+      return;
+    }
   }
-  ctx->scratch_free.emplace_back(n, p);
-  ctx->scratch_held += n;
+  dev_free(p);
 }
 
 constexpr int kRedBlocks = 1024;
@@ -512,6 +535,10 @@ extern "C" int flgpu_ctx_create(int device, flgpu_ctx **out) {
     FLGPU_HIP(hipEventCreate(&c->ev_start));
     FLGPU_HIP(hipEventCreate(&c->ev_stop));
     FLGPU_HIP(hipEventCreateWithFlags(&c->ev_fetch, hipEventDisableTiming));
+    {
+      std::lock_guard<std::mutex> g(pools_mu());
+      pools().push_back(c);
+    }
     *out = c;
     return 0;
   });
@@ -520,6 +547,11 @@ extern "C" int flgpu_ctx_create(int device, flgpu_ctx **out) {
 extern "C" int flgpu_ctx_destroy(flgpu_ctx *ctx) {
   return guard([&] {
     if (!ctx) return 0;
+    {
+      std::lock_guard<std::mutex> g(pools_mu());
+      auto &v = pools();
+      v.erase(std::remove(v.begin(), v.end(), ctx), v.end());
+    }
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     dev_free(ctx->red_partial);

@@ -61,11 +61,12 @@ int guard(F &&f) {
 
 // ---- device buffers ---------------------------------------------------------
 
+// Where there is no memory left, every context's free blocks (below) are released first.
 void *dev_alloc(size_t bytes);
 // Device memory for work on ctx's stream, under its lock.  A block given back is handed out again
 // without waiting for the work that used it, since the next user's follows on the same stream.  At
 // most kScratchKeep bytes of free blocks are kept; they are released with the context, or when an
-// allocation fails.
+// allocation of any kind (dev_alloc), of any context, fails.
 constexpr size_t kScratchKeep = (size_t)1 << 30;
 void *scratch_get(flgpu_ctx *ctx, size_t bytes);
 void scratch_put(flgpu_ctx *ctx, void *p);
@@ -145,8 +146,10 @@ struct flgpu_ctx {
   void *solve_buf = nullptr;
   size_t solve_bytes = 0;
   // temporaries of the assembly and the hierarchies' setup (scratch_get): blocks in use with
-  // their sizes, and free ones kept for the next call
+  // their sizes, and free ones kept for the next call (scratch_mu: another context's allocation
+  // may release them)
   std::unordered_map<void *, size_t> scratch_used;
+  std::mutex scratch_mu;
   std::vector<std::pair<size_t, void *>> scratch_free;
   size_t scratch_held = 0;  // bytes in scratch_free
   std::string name;

@@ -70,3 +70,49 @@ del Hy
 assert gone() > g
 assert H.host_hip_destroyed_in_flight() == 0
 """, dim, order, smoother)
+
+
+@pytest.mark.parametrize("kind", ["vector", "matrix", "hierarchy", "other context"])
+def test_kept_blocks_are_given_back_to_any_allocation(host_hip, kind):
+    """the blocks that a context keeps for its next setup do not make another allocation fail:
+    of its own vectors, matrices and hierarchies, or of another context's"""
+    run(host_hip, """
+kind = sys.argv[3]
+ctx = ml.default_context()
+other = ml.Context(0)
+before = H.host_hip_live()
+A = lat.assemble(3, 2, 12, rhs=False)[0]
+del A
+kept = H.host_hip_live() - before  # the assembly's temporaries
+assert kept > 8 * MB, kept
+# what the allocation takes by itself, and then with no more memory than that
+def get(c):
+    if kind == "matrix":
+        return lat.assemble(3, 1, 24, rhs=False, ctx=c)[0]
+    if kind == "hierarchy":
+        return it.Hierarchy.lattice(it.GeometricCS(it.Jacobi(0.5)), 3, 1, 3, 4, ctx=c)
+    return ml.GpuVector(4 * kept // 5 // 8, ctx=c)
+c = other if kind == "other context" else ctx
+H.host_hip_limit(H.host_hip_live() + kept // 2)
+try:
+    v = get(c)
+finally:
+    H.host_hip_limit(1 << 60)
+assert H.host_hip_live() < before + kept + kept // 2
+del v
+""", kind)
+
+
+def test_kept_blocks_end_with_their_context(host_hip):
+    """all memory is given back when the objects and their contexts are gone"""
+    run(host_hip, """
+start = H.host_hip_live()
+c = ml.Context(0)
+A = lat.assemble(3, 2, 6, ctx=c)
+Hy = it.Hierarchy.lattice(it.GeometricCS(it.GeometricSSC(1.0)), 3, 2, 1, 3, ctx=c)
+del A, Hy
+assert H.host_hip_live() > start
+ml.check(L.flgpu_ctx_destroy(c.h))
+c.h = None
+assert H.host_hip_live() == start
+""")
