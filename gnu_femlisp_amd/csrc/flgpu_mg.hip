@@ -31,25 +31,42 @@ namespace flgpu {
 // C whose inverse is kept (FP64, row-major).
 // For an FP32 cycle the inverse is kept as FP32 64 x 64 tiles of its upper triangle (tiles
 // (I, J), I <= J, in the order of tI / tJ; inv freed), applied by two passes through part.
+// The arrays are the inverse's own, of its size, and a new inverse of that size is written into
+// them (reassemblies); work space comes from the context's kept blocks.
 struct DenseInverse {
-  double *inv = nullptr;
-  float *tiles = nullptr;
-  int *tI = nullptr, *tJ = nullptr;  // the tiles' block row and column
-  double *part = nullptr;            // ntile x ntile x 64 partial products
+  template <class T>
+  struct Array {
+    T *p = nullptr;
+    size_t n = 0;
+    T *resize(size_t k) {
+      if (k != n) release();
+      if (!p) p = (T *)dev_alloc(sizeof(T) * k);
+      n = k;
+      return p;
+    }
+    void release() {
+      dev_free(p);
+      p = nullptr;
+      n = 0;
+    }
+    operator T *() const { return p; }
+  };
+  Array<double> inv;
+  Array<float> tiles;
+  Array<int> tI, tJ;   // the tiles' block row and column
+  Array<double> part;  // ntile x ntile x 64 partial products
   int ntile = 0;
-  int *cidx = nullptr;  // the m non-trivial DOFs
-  int *tidx = nullptr;  // the nt trivial DOFs
+  Array<int> cidx;  // the m non-trivial DOFs
+  Array<int> tidx;  // the nt trivial DOFs
   int m = 0, nt = 0;
-  flgpu_ctx *ctx = nullptr;
-  void release() {  // under ctx's lock
-    for (void *p : {(void *)inv, (void *)tiles, (void *)tI, (void *)tJ, (void *)part,
-                    (void *)cidx, (void *)tidx})
-      if (p) scratch_put(ctx, p);
-    inv = nullptr;
-    tiles = nullptr;
-    tI = tJ = nullptr;
-    part = nullptr;
-    cidx = tidx = nullptr;
+  void release() {
+    inv.release();
+    tiles.release();
+    tI.release();
+    tJ.release();
+    part.release();
+    cidx.release();
+    tidx.release();
     m = nt = ntile = 0;
   }
 };
@@ -374,74 +391,67 @@ __global__ __launch_bounds__(256) void k_gj_update(int m, int k0, int bs,
       }
 }
 
-// A^-1 of a square matrix of at most 8192 rows, compressed
-static DenseInverse dense_inverse_dev(const flgpu_mat *A) {
+// out = A^-1 of a square matrix of at most 8192 rows, compressed; inv (m x m) in out.inv or, when
+// `block` is given, in a block of the context's that it receives
+static void dense_inverse_dev(const flgpu_mat *A, DenseInverse &out,
+                              std::unique_ptr<Scratch<double>> *block) {
   FLGPU_REQUIRE(A->nrows == A->ncols, "dense inverse of a non-square matrix");
   FLGPU_REQUIRE(A->nrows <= 8192, "matrix too large for the dense inverse (> 8192 rows)");
   const int n = A->nrows;
   const long nn = (long)n * n;
   hipStream_t s = A->ctx->stream;
   flgpu_ctx *ctx = A->ctx;
-  DenseInverse out;
-  out.ctx = ctx;
-  double *C2 = nullptr;
-  try {
-    if (n == 0) return out;
-    Scratch<double> full(ctx, nn), block(ctx, kGjB * kGjB);
-    Scratch<int> triv_p(ctx, n), bad_p(ctx, 1);
-    double *M0 = full.p, *D = block.p;
-    int *dt = triv_p.p, *bad = bad_p.p;
-    k_dense_zero<<<grid_for(nn, 256), 256, 0, s>>>(nn, M0);
-    if (A->prec == FLGPU_F64)
-      k_dense_scatter<double><<<grid_for(n, 256), 256, 0, s>>>(n, A->rowptr, A->colidx,
-                                                               (const double *)A->vals, M0);
-    else
-      k_dense_scatter<float><<<grid_for(n, 256), 256, 0, s>>>(n, A->rowptr, A->colidx,
-                                                              (const float *)A->vals, M0);
-    k_dense_trivial<<<n, 256, 0, s>>>(n, M0, dt);
+  out.m = out.nt = out.ntile = 0;
+  if (n == 0) return;
+  Scratch<double> full(ctx, nn), pivots(ctx, kGjB * kGjB);
+  Scratch<int> triv_p(ctx, n), bad_p(ctx, 1);
+  double *M0 = full.p, *D = pivots.p;
+  int *dt = triv_p.p, *bad = bad_p.p;
+  k_dense_zero<<<grid_for(nn, 256), 256, 0, s>>>(nn, M0);
+  if (A->prec == FLGPU_F64)
+    k_dense_scatter<double><<<grid_for(n, 256), 256, 0, s>>>(n, A->rowptr, A->colidx,
+                                                             (const double *)A->vals, M0);
+  else
+    k_dense_scatter<float><<<grid_for(n, 256), 256, 0, s>>>(n, A->rowptr, A->colidx,
+                                                            (const float *)A->vals, M0);
+  k_dense_trivial<<<n, 256, 0, s>>>(n, M0, dt);
+  FLGPU_HIP(hipGetLastError());
+  std::vector<int> trivial(n, 0), piv, triv;
+  FLGPU_HIP(hipMemcpyAsync(trivial.data(), dt, sizeof(int) * n, hipMemcpyDeviceToHost, s));
+  FLGPU_HIP(hipStreamSynchronize(s));
+  for (int k = 0; k < n; k++) (trivial[k] ? triv : piv).push_back(k);
+  const int m = (int)piv.size(), nt = (int)triv.size();
+  if (nt > 0)
+    FLGPU_HIP(hipMemcpyAsync(out.tidx.resize(nt), triv.data(), sizeof(int) * nt,
+                             hipMemcpyHostToDevice, s));
+  if (m > 0) {
+    const long mm = (long)m * m;
+    FLGPU_HIP(hipMemcpyAsync(out.cidx.resize(m), piv.data(), sizeof(int) * m,
+                             hipMemcpyHostToDevice, s));
+    if (block) block->reset(new Scratch<double>(ctx, mm));
+    double *result = block ? (*block)->p : out.inv.resize(mm);
+    Scratch<double> other(ctx, mm);
+    // every block of pivots writes the other array; the last one writes `result`
+    const int steps = (m + kGjB - 1) / kGjB, ntile = steps;
+    double *C = steps % 2 ? other.p : result, *C2 = steps % 2 ? result : other.p;
+    k_dense_gather<<<grid_for(mm, 256), 256, 0, s>>>(m, n, out.cidx, M0, C);
     FLGPU_HIP(hipGetLastError());
-    std::vector<int> trivial(n, 0), piv, triv;
-    FLGPU_HIP(hipMemcpyAsync(trivial.data(), dt, sizeof(int) * n, hipMemcpyDeviceToHost, s));
-    FLGPU_HIP(hipStreamSynchronize(s));
-    for (int k = 0; k < n; k++) (trivial[k] ? triv : piv).push_back(k);
-    const int m = (int)piv.size();
-    out.m = m;
-    out.nt = (int)triv.size();
-    if (out.nt > 0) {
-      out.tidx = (int *)scratch_get(ctx, sizeof(int) * out.nt);
-      FLGPU_HIP(hipMemcpyAsync(out.tidx, triv.data(), sizeof(int) * out.nt,
-                               hipMemcpyHostToDevice, s));
+    FLGPU_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
+    for (int k0 = 0; k0 < m; k0 += kGjB) {
+      const int bs = std::min(kGjB, m - k0);
+      k_gj_diag<<<1, 256, 0, s>>>(m, k0, bs, C, D, bad);
+      k_gj_update<<<(unsigned)(ntile * ntile), 256, 0, s>>>(m, k0, bs, D, C, C2);
+      std::swap(C, C2);
     }
-    if (m > 0) {
-      const long mm = (long)m * m;
-      out.cidx = (int *)scratch_get(ctx, sizeof(int) * m);
-      FLGPU_HIP(hipMemcpyAsync(out.cidx, piv.data(), sizeof(int) * m, hipMemcpyHostToDevice, s));
-      out.inv = (double *)scratch_get(ctx, sizeof(double) * mm);
-      k_dense_gather<<<grid_for(mm, 256), 256, 0, s>>>(m, n, out.cidx, M0, out.inv);
-      FLGPU_HIP(hipGetLastError());
-      C2 = (double *)scratch_get(ctx, sizeof(double) * mm);
-      FLGPU_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
-      const int ntile = (m + kGjB - 1) / kGjB;
-      for (int k0 = 0; k0 < m; k0 += kGjB) {
-        const int bs = std::min(kGjB, m - k0);
-        k_gj_diag<<<1, 256, 0, s>>>(m, k0, bs, out.inv, D, bad);
-        k_gj_update<<<(unsigned)(ntile * ntile), 256, 0, s>>>(m, k0, bs, D, out.inv, C2);
-        std::swap(out.inv, C2);
-      }
-      FLGPU_HIP(hipGetLastError());
-      int hbad = 0;
-      FLGPU_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
-      FLGPU_HIP(hipStreamSynchronize(s));
-      FLGPU_REQUIRE(hbad == 0, "matrix is singular (zero pivot in the dense inverse)");
-    }
+    FLGPU_HIP(hipGetLastError());
+    int hbad = 0;
+    FLGPU_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
     FLGPU_HIP(hipStreamSynchronize(s));
-  } catch (...) {
-    scratch_put(ctx, C2);
-    out.release();
-    throw;
+    FLGPU_REQUIRE(hbad == 0, "matrix is singular (zero pivot in the dense inverse)");
   }
-  scratch_put(ctx, C2);
-  return out;
+  FLGPU_HIP(hipStreamSynchronize(s));
+  out.m = m;
+  out.nt = nt;
 }
 
 // The symmetric inverse from the tiles of its upper triangle, pass 1: one workgroup per tile
@@ -536,7 +546,7 @@ __global__ __launch_bounds__(256) void k_coarse_sym2(int m, int ntile,
 // x = A^-1 r (x_zero) or x += A^-1 r
 static void dense_inverse_apply(hipStream_t s, const DenseInverse &D, int prec, const void *r,
                                 void *x, int x_zero) {
-  if (D.tiles) {
+  if (D.ntile > 0) {
     FLGPU_REQUIRE(prec == FLGPU_F32, "the FP32 tiles of the inverse are for FP32 vectors");
     const int nq = D.ntile * (D.ntile + 1) / 2;
     k_coarse_sym1<float><<<nq, 256, 0, s>>>(D.m, D.ntile, D.tiles, D.tI, D.tJ, D.cidx,
@@ -579,29 +589,32 @@ __global__ void k_pack_sym(int m, const double *__restrict__ inv, const int *__r
 static void coarse_setup(flgpu_mg *mg, MGLevel &L) {
   FLGPU_REQUIRE(L.A->nrows <= 8192,
                 "base level too large for the dense coarse solve (> 8192 DOFs)");
-  L.cinv = dense_inverse_dev(L.A);
   DenseInverse &D = L.cinv;
-  if (mg->p.prec == FLGPU_F32 && D.m > 0) {
+  std::unique_ptr<Scratch<double>> inv;
+  const bool f32 = mg->p.prec == FLGPU_F32;
+  dense_inverse_dev(L.A, D, f32 ? &inv : nullptr);
+  if (f32 && D.m > 0) {
     hipStream_t s = mg->ctx->stream;
-    D.ntile = (D.m + kSymB - 1) / kSymB;
+    const int m = D.m, ntile = (m + kSymB - 1) / kSymB;
+    D.m = 0;  // no inverse until its tiles are there
     std::vector<int> hI, hJ;
-    for (int I = 0; I < D.ntile; I++)
-      for (int J = I; J < D.ntile; J++) {
+    for (int I = 0; I < ntile; I++)
+      for (int J = I; J < ntile; J++) {
         hI.push_back(I);
         hJ.push_back(J);
       }
     const int nq = (int)hI.size();
-    D.tI = (int *)scratch_get(mg->ctx, sizeof(int) * nq);
-    D.tJ = (int *)scratch_get(mg->ctx, sizeof(int) * nq);
-    D.tiles = (float *)scratch_get(mg->ctx, sizeof(float) * (size_t)nq * kSymB * kSymB);
-    D.part = (double *)scratch_get(mg->ctx, sizeof(double) * (size_t)D.ntile * D.ntile * kSymB);
+    D.tI.resize(nq);
+    D.tJ.resize(nq);
+    D.tiles.resize((size_t)nq * kSymB * kSymB);
+    D.part.resize((size_t)ntile * ntile * kSymB);
     FLGPU_HIP(hipMemcpyAsync(D.tI, hI.data(), sizeof(int) * nq, hipMemcpyHostToDevice, s));
     FLGPU_HIP(hipMemcpyAsync(D.tJ, hJ.data(), sizeof(int) * nq, hipMemcpyHostToDevice, s));
-    k_pack_sym<<<nq, 256, 0, s>>>(D.m, D.inv, D.tI, D.tJ, D.tiles);
+    k_pack_sym<<<nq, 256, 0, s>>>(m, inv->p, D.tI, D.tJ, D.tiles);
     FLGPU_HIP(hipGetLastError());
     FLGPU_HIP(hipStreamSynchronize(s));
-    scratch_put(mg->ctx, D.inv);
-    D.inv = nullptr;
+    D.ntile = ntile;
+    D.m = m;
   }
 }
 
@@ -1565,10 +1578,8 @@ extern "C" int flgpu_mg_reassemble(flgpu_mg *mg, const flgpu_vec *kappa, int nk)
         mat_refresh_values(L.A);
       }
     }
-    graphs_clear(mg);  // the coarse inverse is reallocated below
-    MGLevel &B = mg->lv[mg->p.base_level];
-    B.cinv.release();
-    coarse_setup(mg, B);
+    graphs_clear(mg);  // the coarse inverse may get other arrays below
+    coarse_setup(mg, mg->lv[mg->p.base_level]);
     FLGPU_HIP(hipStreamSynchronize(mg->ctx->stream));
     return 0;
   });
@@ -1824,7 +1835,7 @@ extern "C" int flgpu_solve(flgpu_mg *mg, const flgpu_mat *A, const flgpu_solve_p
         }
         // the iterator becomes <lu>'s; the step count and the residual at hand stay
         fallback_p = true;
-        lu_inv.d = dense_inverse_dev(A);
+        dense_inverse_dev(A, lu_inv.d, nullptr);
       }
       if (fallback_p) {  // <lu> iterate (linit.lisp:150-160): x += A^-1 r, residual-after nil
         dense_inverse_apply(s, lu_inv.d, prec, W.r, x->d, 0);

@@ -1,6 +1,6 @@
-// A HIP runtime for tests of the library's host code where there is no GPU: device memory is host
-// memory, kernels do nothing, streams run at once, and what the library must wait for or give
-// back is recorded.  Loaded into a process (RTLD_GLOBAL) before libflgpu.so, whose calls it takes.
+// A HIP runtime for tests of the library's host code where there is no GPU: kernels and copies do
+// nothing and device memory reads as zero; what the library must wait for and what memory it
+// holds is recorded.  Loaded into a process (RTLD_GLOBAL) before libflgpu.so, whose calls it takes.
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
 
@@ -61,20 +61,18 @@ hipError_t hipHostFree(void *p) {
   std::free(p);
   return hipSuccess;
 }
-hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
-  if (n) std::memcpy(d, s, n);
+// what comes back from the device is zero, whatever went there
+hipError_t hipMemcpyAsync(void *d, const void *, size_t n, hipMemcpyKind k, hipStream_t) {
+  if (n && k == hipMemcpyDeviceToHost) std::memset(d, 0, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) {
+  (void)hipMemcpyAsync(d, s, n, k, nullptr);
   std::lock_guard<std::mutex> g(mu);
   idle();
   return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
-  if (n) std::memcpy(d, s, n);
-  return hipSuccess;
-}
-hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) {
-  if (n) std::memset(d, v, n);
-  return hipSuccess;
-}
+hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) {
   *f = *t = (size_t)1 << 38;
   return hipSuccess;

@@ -1,6 +1,6 @@
 """The library's host code over a HIP runtime without a GPU (host_hip.cpp): what it waits for and
-what memory it gives back.  Kernels do nothing there, so no values are looked at; every check runs
-in a process of its own."""
+what memory it gives back.  Device memory reads as zero there, so no values are looked at; every
+check runs in a process of its own."""
 import os
 import subprocess
 import sys
@@ -116,3 +116,39 @@ ml.check(L.flgpu_ctx_destroy(c.h))
 c.h = None
 assert H.host_hip_live() == start
 """)
+
+
+@pytest.mark.parametrize("prec", ["F64", "F32"])
+def test_a_hierarchy_keeps_no_larger_block_than_it_needs(host_hip, prec):
+    """the memory that a hierarchy holds does not depend on the blocks that its context had kept
+    from other work, and a reassembly leaves it as it is"""
+    run(host_hip, """
+prec = getattr(F, sys.argv[3])
+def free_kept():  # an allocation that fails releases every kept block
+    H.host_hip_limit(H.host_hip_live())
+    try:
+        ml.GpuVector(MB)
+    except Exception:
+        pass
+    H.host_hip_limit(1 << 60)
+def held(work):
+    c = ml.Context(0)
+    for n in work:
+        del_me = lat.assemble(3, 2, n, rhs=False, prec=prec, ctx=c)[0]
+        del del_me
+    before = H.host_hip_live()
+    Hy = it.Hierarchy.lattice(it.GeometricCS(it.Jacobi(0.5), prec=prec), 3, 1, 4, 2, ctx=c)
+    out = []
+    for k in range(3):
+        free_kept()
+        out.append(H.host_hip_live())
+        ml.check(L.flgpu_mg_reassemble(Hy.h, None, 0))
+    del Hy
+    free_kept()
+    out = [o - H.host_hip_live() for o in out]
+    return out
+alone = held([])
+assert alone[0] == alone[1] == alone[2], alone
+for work in ([3], [2, 3, 4], [3, 5, 6, 3]):
+    assert held(work) == alone, (work, held(work), alone)
+""", prec)
