@@ -1071,9 +1071,9 @@ void mg_apply_ptr(flgpu_mg *mg, int vprec, void *x, void *b, void *r) {
 // triple into a HIP graph and replayed: one launch instead of ~40 per level.
 // The cycle clears with fill kernels, never with memset nodes.
 // A replay may still be queued (flgpu_mg_apply returns before its cycle has run): the stream is
-// waited for before an executable graph goes.
-static void graphs_clear(flgpu_mg *mg) {
-  if (!mg->graphs.empty()) (void)hipStreamSynchronize(mg->ctx->stream);
+// waited for before an executable graph goes, unless the caller has (waited).
+static void graphs_clear(flgpu_mg *mg, bool waited = false) {
+  if (!waited && !mg->graphs.empty()) (void)hipStreamSynchronize(mg->ctx->stream);
   for (auto &g : mg->graphs) (void)hipGraphExecDestroy(g.exec);
   mg->graphs.clear();
 }
@@ -1566,6 +1566,9 @@ extern "C" int flgpu_mg_reassemble(flgpu_mg *mg, const flgpu_vec *kappa, int nk)
     FLGPU_REQUIRE(mg->lat_dim > 0, "the hierarchy was not assembled on a lattice");
     FLGPU_REQUIRE(!kappa || kappa->ctx == mg->ctx, "kappa belongs to another context");
     CTX_LOCK(mg->ctx);
+    // the captured cycles queued so far are waited for alone, so that they are dropped while the
+    // assembly runs (with the GPU idle: 1 % of Q2 24^3 cells)
+    fetch_mark(mg->ctx);
     for (int l = mg->top; l >= 0; l--) {
       MGLevel &L = mg->lv[l];
       bool bbox = mg->p.transfer == FLGPU_TRANSFER_BLACKBOX;
@@ -1578,7 +1581,9 @@ extern "C" int flgpu_mg_reassemble(flgpu_mg *mg, const flgpu_vec *kappa, int nk)
         mat_refresh_values(L.A);
       }
     }
-    graphs_clear(mg);  // the coarse inverse may get other arrays below
+    // the coarse inverse may get other arrays: no captured cycle is kept
+    fetch_wait(mg->ctx);
+    graphs_clear(mg, true);
     coarse_setup(mg, mg->lv[mg->p.base_level]);
     FLGPU_HIP(hipStreamSynchronize(mg->ctx->stream));
     return 0;

@@ -16,6 +16,7 @@ std::map<void *, size_t> blocks;
 size_t live = 0, limit = (size_t)-1;
 int nmalloc = 0;
 std::set<void *> queued;  // executable graphs launched and not waited for
+std::map<void *, std::set<void *>> marked;  // those that an event waits for
 int destroyed_in_flight = 0, graphs_destroyed = 0;
 dim3 grid_, block_;
 size_t shmem_;
@@ -119,8 +120,16 @@ hipError_t hipEventDestroy(hipEvent_t e) {
   std::free((void *)e);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  std::lock_guard<std::mutex> g(mu);
+  marked[(void *)e] = queued;
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  std::lock_guard<std::mutex> g(mu);
+  for (void *q : marked[(void *)e]) queued.erase(q);
+  return hipSuccess;
+}
 hipError_t hipEventElapsedTime(float *t, hipEvent_t, hipEvent_t) {
   *t = 0.f;
   return hipSuccess;
