@@ -3141,6 +3141,85 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 2 : 1) void k_rap_q1(
   else rap_row<T, 2>(Mc, k, K, a27, t27, crp, cv, all);
 }
 
+// The same from the CSRs, one thread per coarse entry (k, n), for matrices that hold no 27 planes
+// (capped to SELL) or are not exactly symmetric and for interpolations without planes: every
+// position is computed, the row starts included.  Same contributions in the same order.  Bound by
+// the position arithmetic (49^3 coarse nodes FP32 1168 us).  A black-box hierarchy of six levels
+// to 96^3 cells, FP32, capped to SELL, reassembles in 5.6 ms, 16.5 with k_rap_lds, which searches
+// the positions; of five levels to 32^3 cells in 1.7, 9.3.
+__device__ __forceinline__ int lat_pos3(const int lo[3], const int cnt[3], int a, int b, int c) {
+  return ((a - lo[0]) * cnt[1] + (b - lo[1])) * cnt[2] + (c - lo[2]);
+}
+
+// the first entry of row (z, y, x) of a tensor product of 1-D patterns: pre[a] entries precede
+// the row's coordinate on axis a, which has cnt[a] entries; nnz1 per 1-D pattern
+__device__ __forceinline__ long pat_row_start(const long pre[3], const int cnt[3], long nnz1) {
+  return (pre[0] * nnz1 + cnt[0] * pre[1]) * nnz1 + (long)cnt[0] * cnt[1] * pre[2];
+}
+
+template <class T>
+__global__ __launch_bounds__(256) void k_rap_entry(int Mc, int M, const T *__restrict__ av,
+                                                   const T *__restrict__ pv,
+                                                   const int *__restrict__ crp, double *acc,
+                                                   int upper) {
+  // the 1-D patterns: A's row i holds i - 1, i, i + 1 within the lattice (3 M - 2 entries,
+  // 3 i - 1 of them before row i > 0); P's row i holds i / 2 and, for odd i, i / 2 + 1
+  // (3 Mc - 2 entries, i + i / 2 before row i)
+  const long nA = 3L * M - 2, nP = 3L * Mc - 2;
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long Nc = (long)Mc * Mc * Mc;
+  if (t >= Nc * 27) return;
+  const int k = (int)(t / 27), d = (int)(t - (long)k * 27);
+  const int K[3] = {k / (Mc * Mc), (k / Mc) % Mc, k % Mc};
+  const int D[3] = {d / 9 - 1, (d / 3) % 3 - 1, d % 3 - 1};
+  int Nn[3], clo[3], ccnt[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    Nn[a] = K[a] + D[a];
+    if (Nn[a] < 0 || Nn[a] >= Mc) return;
+    clo[a] = K[a] > 0 ? -1 : 0;
+    ccnt[a] = (K[a] < Mc - 1 ? 1 : 0) - clo[a] + 1;
+  }
+  const int n = (Nn[0] * Mc + Nn[1]) * Mc + Nn[2];
+  if (upper && n < k) return;  // the lower triangle is mirrored afterwards
+  double s = 0.0;
+  const int l0[3] = {max(2 * K[0] - 1, 0), max(2 * K[1] - 1, 0), max(2 * K[2] - 1, 0)};
+  const int l1[3] = {min(2 * K[0] + 1, M - 1), min(2 * K[1] + 1, M - 1), min(2 * K[2] + 1, M - 1)};
+  for (int lz = l0[0]; lz <= l1[0]; lz++)
+    for (int ly = l0[1]; ly <= l1[1]; ly++)
+      for (int lx = l0[2]; lx <= l1[2]; lx++) {
+        const int L[3] = {lz, ly, lx};
+        // P_lk: row l holds floor(l / 2) (and ceil(l / 2) on odd coordinates) per axis
+        int plo[3], pcnt[3], alo[3], acnt[3], m0[3], m1[3];
+        long ppre[3], apre[3];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+          plo[a] = L[a] >> 1;
+          pcnt[a] = (L[a] & 1) + 1;
+          ppre[a] = L[a] + (L[a] >> 1);
+          alo[a] = L[a] > 0 ? L[a] - 1 : 0;
+          acnt[a] = min(L[a] + 1, M - 1) - alo[a] + 1;
+          apre[a] = L[a] > 0 ? 3L * L[a] - 1 : 0;
+          m0[a] = max(max(L[a] - 1, 2 * Nn[a] - 1), 0);
+          m1[a] = min(min(L[a] + 1, 2 * Nn[a] + 1), M - 1);
+        }
+        const double plk =
+            (double)pv[pat_row_start(ppre, pcnt, nP) + lat_pos3(plo, pcnt, K[0], K[1], K[2])];
+        const long ab = pat_row_start(apre, acnt, nA);
+        for (int mz = m0[0]; mz <= m1[0]; mz++)
+          for (int my = m0[1]; my <= m1[1]; my++)
+            for (int mx = m0[2]; mx <= m1[2]; mx++) {
+              const double w = plk * (double)av[ab + lat_pos3(alo, acnt, mz, my, mx)];
+              const int qlo[3] = {mz >> 1, my >> 1, mx >> 1};
+              const int qcnt[3] = {(mz & 1) + 1, (my & 1) + 1, (mx & 1) + 1};
+              const long qpre[3] = {mz + (mz >> 1), my + (my >> 1), mx + (mx >> 1)};
+              s += w * (double)pv[pat_row_start(qpre, qcnt, nP) +
+                                  lat_pos3(qlo, qcnt, Nn[0], Nn[1], Nn[2])];
+            }
+      }
+  acc[crp[k] + lat_pos3(clo, ccnt, D[0], D[1], D[2])] = s;
+}
+
 // the longest row: a grid of at most 1024 blocks strides over the rows, each block reduces its
 // maximum in LDS and issues one atomic (atomics to one address are serialised)
 constexpr int kMaxRowBlocks = 1024;
@@ -3283,14 +3362,17 @@ void galerkin_product(const flgpu_mat *P, const flgpu_mat *A, flgpu_mat *Ac, boo
   FLGPU_REQUIRE(P->prec == A->prec && A->prec == Ac->prec, "galerkin: precisions differ");
   flgpu_ctx *ctx = A->ctx;
   const int nc = Ac->nrows;
-  // the structured product: 3D Q1, the fine lattice of an even n in stencil storage, whose values
-  // are exactly symmetric, the patterns' sizes as the lattices give them
+  // the structured products: 3D Q1, the fine lattice of an even n, the patterns' sizes as the
+  // lattices give them
   const long nf = A->lat_n, ncl = nf / 2;
+  const bool q1 = lattice && is_q1_lattice(A) && nf % 2 == 0 &&
+                  A->nnz == (3 * nf + 1) * (3 * nf + 1) * (3 * nf + 1) &&
+                  Ac->nrows == (ncl + 1) * (ncl + 1) * (ncl + 1) &&
+                  Ac->nnz == (3 * ncl + 1) * (3 * ncl + 1) * (3 * ncl + 1) &&
+                  P->nnz == (3 * ncl + 1) * (3 * ncl + 1) * (3 * ncl + 1);
   const flgpu_mat *PT = P->transpose;
-  if (lattice && is_q1_lattice(A) && A->val27 && A->st_sym && nf % 2 == 0 && PT && PT->tp_kind == 2 &&
-      PT->tp27 && PT->tp_nc == ncl && A->nnz == (3 * nf + 1) * (3 * nf + 1) * (3 * nf + 1) &&
-      Ac->nrows == (ncl + 1) * (ncl + 1) * (ncl + 1) &&
-      Ac->nnz == (3 * ncl + 1) * (3 * ncl + 1) * (3 * ncl + 1)) {
+  // from the planes: A exactly symmetric
+  if (q1 && A->val27 && A->st_sym && PT && PT->tp_kind == 2 && PT->tp27 && PT->tp_nc == ncl) {
     auto run = [&](auto t) {
       using T = decltype(t);
       k_rap_q1<T><<<dim3(grid_for(nc, 64), 3), 64, 0, ctx->stream>>>(
@@ -3306,12 +3388,20 @@ void galerkin_product(const flgpu_mat *P, const flgpu_mat *A, flgpu_mat *Ac, boo
   int *bad = (int *)dev_alloc(sizeof(int));
   FLGPU_HIP(hipMemsetAsync(bad, 0, sizeof(int), ctx->stream));
   int *missing = (int *)dev_alloc(sizeof(int));
-  mat_build_transpose(P);  // the product walks the rows of P^T
+  if (!q1) mat_build_transpose(P);  // the general product walks the rows of P^T
   PT = P->transpose;
-  const bool lds = max_row_length(Ac) <= kRapW;
+  const bool lds = !q1 && max_row_length(Ac) <= kRapW;
   auto rap = [&](int upper) {
     const unsigned gl = (unsigned)((nc + kRapB - 1) / kRapB);
-    if (lds && A->prec == FLGPU_F64)
+    if (q1 && A->prec == FLGPU_F64)
+      k_rap_entry<double><<<grid_for(27L * nc, 256), 256, 0, ctx->stream>>>(
+          (int)ncl + 1, (int)nf + 1, (const double *)A->vals, (const double *)P->vals,
+          Ac->rowptr, acc, upper);
+    else if (q1)
+      k_rap_entry<float><<<grid_for(27L * nc, 256), 256, 0, ctx->stream>>>(
+          (int)ncl + 1, (int)nf + 1, (const float *)A->vals, (const float *)P->vals, Ac->rowptr,
+          acc, upper);
+    else if (lds && A->prec == FLGPU_F64)
       k_rap_lds<double><<<gl, kRapB, 0, ctx->stream>>>(
           nc, PT->rowptr, PT->colidx, (const double *)PT->vals, A->rowptr, A->colidx,
           (const double *)A->vals, P->rowptr, P->colidx, (const double *)P->vals, Ac->rowptr,
@@ -3334,7 +3424,8 @@ void galerkin_product(const flgpu_mat *P, const flgpu_mat *A, flgpu_mat *Ac, boo
     FLGPU_HIP(hipGetLastError());
   };
   int hmiss = 1;
-  if (csr_symmetric(A)) {
+  // a lattice matrix's stencil form records whether its values are exactly symmetric
+  if (q1 && A->val27 ? A->st_sym : csr_symmetric(A)) {
     FLGPU_HIP(hipMemsetAsync(missing, 0, sizeof(int), ctx->stream));
     rap(1);
     k_mirror<<<grid_for(nc, 128), 128, 0, ctx->stream>>>(nc, Ac->rowptr, Ac->colidx, acc,

@@ -9,6 +9,7 @@
 #include <map>
 #include <mutex>
 #include <set>
+#include <string>
 
 namespace {
 std::mutex mu;
@@ -17,6 +18,8 @@ size_t live = 0, limit = (size_t)-1;
 int nmalloc = 0;
 std::set<void *> queued;  // executable graphs launched and not waited for
 std::map<void *, std::set<void *>> marked;  // those that an event waits for
+std::map<const void *, std::string> kernels;  // by their host stub: mangled name
+std::map<std::string, int> launches;
 int destroyed_in_flight = 0, graphs_destroyed = 0;
 dim3 grid_, block_;
 size_t shmem_;
@@ -33,6 +36,12 @@ size_t host_hip_live() { return live; }
 int host_hip_mallocs() { return nmalloc; }
 int host_hip_destroyed_in_flight() { return destroyed_in_flight; }
 int host_hip_graphs_destroyed() { return graphs_destroyed; }
+int host_hip_launches(const char *part) {  // of kernels whose mangled name contains part
+  int n = 0;
+  for (auto &k : launches)
+    if (k.first.find(part) != std::string::npos) n += k.second;
+  return n;
+}
 
 hipError_t hipMalloc(void **p, size_t n) {
   std::lock_guard<std::mutex> g(mu);
@@ -162,7 +171,9 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
 }
 
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t) {
+  std::lock_guard<std::mutex> g(mu);
+  launches[kernels[f]]++;
   return hipSuccess;
 }
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t n, hipStream_t s) {
@@ -180,8 +191,10 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *n, hipStream_t *s
   return hipSuccess;
 }
 void **__hipRegisterFatBinary(const void *) { return (void **)&live; }
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *,
-                           dim3 *, dim3 *, int *) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *,
+                           void *, dim3 *, dim3 *, int *) {
+  kernels[f] = name;
+}
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void **) {}
 

@@ -5,6 +5,7 @@ import sys
 import numpy as np
 import pytest
 
+from gnu_femlisp_amd import flgpu as F
 from gnu_femlisp_amd import iteration as it
 from gnu_femlisp_amd.flgpu import check, lib
 from gnu_femlisp_amd.matlisp import GpuVector, compute_residual
@@ -52,3 +53,27 @@ def test_reassembly_right_after_a_queued_cycle(dim, order, smoother):
         check(lib().flgpu_mg_apply(G.h, y.h, b.h, q.h))
         y.numpy()
     assert relerr(x.numpy(), y.numpy()) < 1e-13
+
+
+@pytest.mark.parametrize("prec", [F.F64, F.F32])
+@pytest.mark.parametrize("capped", ["levels", "interpolations"])
+@pytest.mark.parametrize("m,levels", [(1, 4), (3, 3)])
+def test_galerkin_levels_of_capped_hierarchies(m, levels, capped, prec):
+    """reassembled black-box hierarchies hold the same level matrices, bit for bit, where the
+    levels or their interpolations were capped to SELL and their products read the CSRs"""
+    say(f"galerkin levels capped m={m} levels={levels} {capped} prec={prec}")
+    n = m << (levels - 1)
+    rng = np.random.default_rng(n)
+    kap = [np.exp(rng.normal(size=(n,) * 3)) for _ in range(2)]
+    vals = []
+    for cap in (False, True):
+        cs = it.GeometricCS(it.Jacobi(0.6), 1, 1, 0, prec=prec, transfer="blackbox")
+        H = it.Hierarchy.lattice(cs, 3, 1, m, levels, kappa=kap[0])
+        if cap:
+            for l in range(levels - (capped == "interpolations")):
+                M = H.level_matrix(l, interp=capped == "interpolations")
+                assert M.storage(F.STORAGE_SELL) == F.STORAGE_SELL
+        H.reassemble(kap[1])
+        vals.append([H.level_matrix(l).csr()[2] for l in range(levels)])
+    for a, b in zip(*vals):
+        assert np.array_equal(a, b)

@@ -152,3 +152,23 @@ assert alone[0] == alone[1] == alone[2], alone
 for work in ([3], [2, 3, 4], [3, 5, 6, 3]):
     assert held(work) == alone, (work, held(work), alone)
 """, prec)
+
+
+@pytest.mark.parametrize("cap,kernel", [("CELL", b"k_rap_q1"), ("STENCIL", b"k_rap_q1"),
+                                        ("SELL", b"k_rap_entry")])
+def test_galerkin_levels_of_a_lattice_take_a_lattice_product(host_hip, cap, kernel):
+    """the Galerkin products of a reassembly compute their positions also where the levels'
+    storage was capped; the product that searches the rows is for other matrices"""
+    run(host_hip, """
+cs = it.GeometricCS(it.Jacobi(0.5), transfer="blackbox")
+Hy = it.Hierarchy.lattice(cs, 3, 1, 2, 3)
+for l in range(3):
+    Hy.level_matrix(l).storage(getattr(F, "STORAGE_" + sys.argv[3]))
+kap = ml.GpuVector(8 ** 3)
+count = lambda k: H.host_hip_launches(k)
+a, b = count(sys.argv[4].encode()), count(b"k_rap")
+ml.check(L.flgpu_mg_reassemble(Hy.h, kap.h, 8))
+assert count(sys.argv[4].encode()) == a + 2
+assert count(b"k_rap") == b + 2
+del Hy
+""", cap, kernel.decode())
