@@ -333,7 +333,12 @@ __global__ __launch_bounds__(64 * kBlkWaves) void k_blk_sweep(BlkGeom g, long cn
                                                               T *x, const T *b, T *r) {
   constexpr int W = pow_i(3, DIM), NRUN = W / 3;
   typedef BlkInverse<T, W, 64> Inv;
-  __shared__ __align__(16) T part[kBlkWaves][64 * (W + 1)];
+  // the partial sums, then r (32 values) and the inverse's products.  <psc> has no partial sums:
+  // with room for them only ten waves a CU were resident, and at Q2 32^3 FP64 an iterate took 73
+  // us instead of 60
+  constexpr int kPart = SSC ? 64 * (W + 1) : 32 + (Inv::NC + Inv::VL - 1) / Inv::VL * Inv::VL;
+  static_assert(kPart >= 32 + Inv::NC && Inv::WP <= 32, "r and the products fit");
+  __shared__ __align__(16) T part[kBlkWaves][kPart];
   unsigned lb = xcd_block(blockIdx.x, gridDim.x);
   const int wv = threadIdx.x >> 6;
   long w = (long)lb * kBlkWaves + wv;
