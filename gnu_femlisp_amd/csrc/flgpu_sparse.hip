@@ -2791,9 +2791,13 @@ static bool q1_sor(const flgpu_mat *A, T omega, int steps, int backwards, T *x, 
 
 // A sweep of the stencil form from xs into xd.  Small lattices leave the GPU idle and wait for
 // one row's loads: one row a thread.  On larger ones taller tiles recompute less (1.45 times the
-// rows with 8 lines, 1.3 with 12, 1.2 with 20).  Measured, us an iterate, 8 lines and 1 row a
-// thread / 12 and 2 / 20 and 4: 49^3 FP64 16.0 / 18.7 / 24.9; 65^3 28.6 / 24.2 / 33.8; 129^3 158 /
-// 151 / 165, FP32 114 / 86 / 91; 193^3 FP32 436 / 344 / 332.
+// rows with 8 lines, 1.3 with 12, 1.25 with 16, 1.2 with 20).  Measured, us an iterate, 8 lines
+// and 1 row a thread / 12 and 2 / 20 and 4: 49^3 FP64 16.0 / 18.7 / 24.9; 65^3 28.6 / 24.2 / 33.8;
+// 129^3 158 / 151 / 165, FP32 114 / 86 / 91.  Above, 12 and 2 / 16 and 2 / 20 and 4, FP64: 137^3
+// 223 / 204 / 198, 153^3 313 / 296 / 310, 177^3 457 / 464 / 467, 201^3 699 / 654 / 700; FP32, where
+// the last tile's idle lines decide, 12 and 2 / 16 and 4 / 20 and 4: 137^3 108 / 106 / 100, 153^3
+// 153 / 148 / 153, 177^3 258 / 259 / 253, 185^3 299 / 286 / 295, 193^3 340 / 335 / 327, 201^3 405 /
+// 386 / 399.
 template <class T>
 static void st27_sor(const flgpu_mat *A, T omega, int backwards, const T *xs, T *xd, const T *b,
                      T *r, bool zero) {
@@ -2819,8 +2823,12 @@ static void st27_sor(const flgpu_mat *A, T omega, int backwards, const T *xs, T 
     };
     auto shape = [&](auto sym) {
       using std::integral_constant;
+      constexpr int G = sizeof(T) == 8 ? 2 : 1;
+      auto idle = [&](int H) { return (M + H - 1) / H * H - M; };
       if (M <= 56) launch(sym, integral_constant<int, 8>(), integral_constant<int, 4>());
-      else if (M <= 160) launch(sym, integral_constant<int, 12>(), integral_constant<int, 2>());
+      else if (M <= 132) launch(sym, integral_constant<int, 12>(), integral_constant<int, 2>());
+      else if (G == 2 || idle(16) <= idle(20))
+        launch(sym, integral_constant<int, 16>(), integral_constant<int, G>());
       else launch(sym, integral_constant<int, 20>(), integral_constant<int, 1>());
     };
     if (A->st_sym) shape(std::true_type());
