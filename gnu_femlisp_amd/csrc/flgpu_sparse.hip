@@ -1785,6 +1785,13 @@ void tp_drop(flgpu_mat *A) {
   A->tp_kind = 0;
 }
 
+// the same for order 2: products of A and its transpose from their stored values
+static void q2t_drop(flgpu_mat *A) {
+  if (A->q2t == 1 && A->transpose) q2t_drop(A->transpose);
+  if (A->q2t) layout_changed(A);
+  A->q2t = 0;
+}
+
 template <class T>
 static void launch_tp(const flgpu_mat *A, T alpha, const void *x, T beta, const void *z,
                       void *out) {
@@ -3575,6 +3582,7 @@ extern "C" int flgpu_mat_storage(flgpu_mat *A, int max_form, int *form) {
     if (max_form < FLGPU_STORAGE_STENCIL) {
       drop_stencil(A);
       tp_drop(A);
+      q2t_drop(A);
     }
     long lat_rows = 1;
     for (int k = 0; k < A->lat_dim; k++) lat_rows *= (long)A->lat_order * A->lat_n + 1;

@@ -113,12 +113,19 @@ int flgpu_mat_convert(const flgpu_mat *A, int prec, flgpu_mat **out);
  *                          (A_ij = Kref-entry x sum of the factors of the cells
  *                          shared by i and j), no matrix values streamed;
  *   FLGPU_STORAGE_STENCIL  3D Q1 lattice matrix: the 27 values of each row
- *                          (SoA), columns implied by the lattice;
- *   FLGPU_STORAGE_SELL     any matrix: SELL-64 values and column indices.
+ *                          (SoA), columns implied by the lattice; 3D Q1
+ *                          interpolation: weights implied or in 27 planes;
+ *   FLGPU_STORAGE_SELL     any matrix: SELL-64 values and column indices, or
+ *                          the CSR where rows are long or irregular.
  * Lattice matrices get the richest form that applies.  max_form caps it
  * (forms are only ever dropped); *form receives the form in use.  New
  * values drop the per-cell form; a caller's colouring drops both lattice
- * forms (their sweeps follow the lattice colouring). */
+ * forms (their sweeps follow the lattice colouring).
+ * Order 2 is reported as FLGPU_STORAGE_SELL throughout, and max_form caps what
+ * its lattice matrices use beside the CSR: below FLGPU_STORAGE_CELL, products
+ * and block sweeps from the cells (one factor per cell, or in a hierarchy the
+ * cells' element matrices); below FLGPU_STORAGE_STENCIL, a 3D interpolation's
+ * products from the nodes' positions. */
 #define FLGPU_STORAGE_SELL 0
 #define FLGPU_STORAGE_STENCIL 1
 #define FLGPU_STORAGE_CELL 2

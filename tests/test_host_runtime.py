@@ -172,3 +172,40 @@ assert count(sys.argv[4].encode()) == a + 2
 assert count(b"k_rap") == b + 2
 del Hy
 """, cap, kernel.decode())
+
+
+@pytest.mark.parametrize("dim,order", [(3, 1), (3, 2), (2, 2)])
+def test_a_storage_cap_reaches_the_interpolation(host_hip, dim, order):
+    """capped to SELL, an interpolation, its transpose and its copies stream their stored values,
+    and a captured cycle that had read the positions instead is dropped"""
+    run(host_hip, """
+dim, order = int(sys.argv[3]), int(sys.argv[4])
+lattice_products = lambda: H.host_hip_launches(b"k_q2_") + H.host_hip_launches(b"k_tp_")
+def products(P):
+    c, f = ml.GpuVector(P.ncols, P.prec), ml.GpuVector(P.nrows, P.prec)
+    n = lattice_products()
+    ml.gemm(1.0, P, c, 0.0, f)
+    ml.gemm(1.0, P, f, 0.0, c, job="tn")
+    return lattice_products() - n
+P = lat.interpolation(dim, order, 2)
+own = 2 if dim == 3 else 0
+assert products(P) == products(P.convert(F.F32)) == own
+if order == 2:
+    P.storage(F.STORAGE_STENCIL)
+    assert products(P) == own
+assert P.storage(F.STORAGE_SELL) == F.STORAGE_SELL
+assert products(P) == products(P.convert(F.F32)) == 0
+sm = it.Jacobi(0.5) if order == 1 else it.GeometricSSC(1.0)
+Hy = it.Hierarchy.lattice(it.GeometricCS(sm), dim, order, 1, 3)
+x, b, r = (ml.GpuVector(Hy.top_matrix().nrows) for _ in range(3))
+n = lattice_products()
+Hy.apply(x, b, r)
+assert (lattice_products() > n) == (dim == 3)
+for l in range(2):
+    Hy.level_matrix(l, interp=True).storage(F.STORAGE_SELL)
+g, n = H.host_hip_graphs_destroyed(), lattice_products()
+Hy.apply(x, b, r)
+assert lattice_products() == n
+assert H.host_hip_graphs_destroyed() == g + (dim == 3)
+del Hy
+""", dim, order)
