@@ -1440,6 +1440,60 @@ static void cg_p(flgpu_ctx *ctx, long n, DotParts d, int na, int ca, double *hos
   FLGPU_HIP(hipGetLastError());
 }
 
+// ---- hierarchies on lattices ----------------------------------------------------------------
+
+// the hierarchy on lattices; keep_elem: its order-2 levels may keep their element matrices
+static flgpu_mg *mg_build_lattice(flgpu_ctx *ctx, int dim, int order, int n0, int nlevels,
+                                  const flgpu_vec *kappa, int nk, double f, int asm_mode,
+                                  const flgpu_mg_params *params, bool keep_elem,
+                                  flgpu_vec **rhs) {
+  flgpu_mg *mg = new flgpu_mg;
+  mg->ctx = ctx;
+  mg->p = *params;
+  mg->top = nlevels - 1;
+  mg->lv.resize(nlevels);
+  mg->lat_dim = dim;
+  mg->lat_order = order;
+  mg->lat_n0 = n0;
+  mg->asm_mode = asm_mode;
+  flgpu_vec *b = nullptr;
+  try {
+    for (int l = 0; l < nlevels; l++) {
+      int n = n0 << l;
+      bool is_top = (l == nlevels - 1);
+      if (!is_top) mg->lv[l].I = lattice_interpolation(ctx, dim, order, n, params->prec);
+      if (!is_top && params->fas)
+        mg->lv[l].R = lattice_projection(ctx, dim, order, n, params->prec);
+    }
+    for (int l = nlevels - 1; l >= 0; l--) {
+      int n = n0 << l;
+      bool is_top = (l == nlevels - 1);
+      bool bbox = params->transfer == FLGPU_TRANSFER_BLACKBOX;
+      if (is_top || (!params->galerkin && !bbox)) {
+        mg->lv[l].A = lattice_assemble(ctx, dim, order, n, kappa, nk, f, params->prec, asm_mode,
+                                       (is_top && rhs) ? &b : nullptr,
+                                       keep_elem && block_smoother(*params) &&
+                                           l > params->base_level);
+      } else {
+        if (bbox) lattice_blackbox(mg->lv[l + 1].A, mg->lv[l].I);
+        mg->lv[l].A = lattice_galerkin(mg->lv[l].I, mg->lv[l + 1].A, dim, order, n);
+      }
+      // matrices in the per-cell form sweep the lattice colours directly
+      if (params->smoother == FLGPU_SMOOTH_SOR && l > params->base_level &&
+          !mg->lv[l].A->alpha && !mg->lv[l].A->val27)
+        lattice_colouring(mg->lv[l].A, dim, order, n);
+      if (block_smoother(*params) && l > params->base_level) blocks_prepare(mg->lv[l].A);
+    }
+    mg_alloc_work(mg);
+  } catch (...) {
+    vec_free(b);
+    mg_free(mg);
+    throw;
+  }
+  if (rhs) *rhs = b;
+  return mg;
+}
+
 }  // namespace flgpu
 
 using namespace flgpu;
@@ -1512,50 +1566,16 @@ extern "C" int flgpu_mg_create_lattice(flgpu_ctx *ctx, int dim, int order, int n
     FLGPU_REQUIRE(params->transfer == FLGPU_TRANSFER_GEOMETRIC || (dim == 3 && order == 1),
                   "black-box transfers are defined for 3D Q1 lattices");
     CTX_LOCK(ctx);
-    flgpu_mg *mg = new flgpu_mg;
-    mg->ctx = ctx;
-    mg->p = *params;
-    mg->top = nlevels - 1;
-    mg->lv.resize(nlevels);
-    mg->lat_dim = dim;
-    mg->lat_order = order;
-    mg->lat_n0 = n0;
-    mg->asm_mode = asm_mode;
-    flgpu_vec *b = nullptr;
     try {
-      for (int l = 0; l < nlevels; l++) {
-        int n = n0 << l;
-        bool is_top = (l == nlevels - 1);
-        if (!is_top) mg->lv[l].I = lattice_interpolation(ctx, dim, order, n, params->prec);
-        if (!is_top && params->fas)
-          mg->lv[l].R = lattice_projection(ctx, dim, order, n, params->prec);
-      }
-      for (int l = nlevels - 1; l >= 0; l--) {
-        int n = n0 << l;
-        bool is_top = (l == nlevels - 1);
-        bool bbox = params->transfer == FLGPU_TRANSFER_BLACKBOX;
-        if (is_top || (!params->galerkin && !bbox)) {
-          mg->lv[l].A = lattice_assemble(ctx, dim, order, n, kappa, nk, f, params->prec, asm_mode,
-                                         (is_top && rhs) ? &b : nullptr,
-                                         block_smoother(*params) && l > params->base_level);
-        } else {
-          if (bbox) lattice_blackbox(mg->lv[l + 1].A, mg->lv[l].I);
-          mg->lv[l].A = lattice_galerkin(mg->lv[l].I, mg->lv[l + 1].A, dim, order, n);
-        }
-        // matrices in the per-cell form sweep the lattice colours directly
-        if (params->smoother == FLGPU_SMOOTH_SOR && l > params->base_level &&
-            !mg->lv[l].A->alpha && !mg->lv[l].A->val27)
-          lattice_colouring(mg->lv[l].A, dim, order, n);
-        if (block_smoother(*params) && l > params->base_level) blocks_prepare(mg->lv[l].A);
-      }
-      mg_alloc_work(mg);
-    } catch (...) {
-      vec_free(b);
-      mg_free(mg);
-      throw;
+      *out = mg_build_lattice(ctx, dim, order, n0, nlevels, kappa, nk, f, asm_mode, params, true,
+                              rhs);
+    } catch (const Error &e) {
+      // the element matrices (order 2, a coefficient finer than the lattice) take a third more
+      // memory: where there is not enough, the sweeps read the rows instead
+      if (e.code != -2 || order != 2 || !kappa || !block_smoother(*params)) throw;
+      *out = mg_build_lattice(ctx, dim, order, n0, nlevels, kappa, nk, f, asm_mode, params, false,
+                              rhs);
     }
-    if (rhs) *rhs = b;
-    *out = mg;
     return 0;
   });
 }

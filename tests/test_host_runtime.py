@@ -209,3 +209,44 @@ assert lattice_products() == n
 assert H.host_hip_graphs_destroyed() == g + (dim == 3)
 del Hy
 """, dim, order)
+
+
+@pytest.mark.parametrize("dim,smoother", [(2, "GeometricSSC"), (3, "GeometricSSC"),
+                                          (3, "GeometricPSC")])
+def test_a_hierarchy_is_built_where_only_its_rows_fit(host_hip, dim, smoother):
+    """with a coefficient finer than the lattice an order-2 hierarchy keeps its element matrices
+    if there is memory for them; with no more than one per cell takes, it is built without them"""
+    run(host_hip, """
+dim, sm = int(sys.argv[3]), getattr(it, sys.argv[4])
+cs = it.GeometricCS(sm(0.5), 1, 1, 0)
+n = 24 if dim == 2 else 8
+kaps = {nk: ml.GpuVector(nk ** dim) for nk in (n, 2 * n)}
+start = H.host_hip_live()
+def build(nk, room):
+    H.host_hip_limit(start + room)
+    try:
+        return it.Hierarchy.lattice(cs, dim, 2, n // 4, 3, kappa=(kaps[nk], nk))
+    finally:
+        H.host_hip_limit(1 << 60)
+def fits(nk, room):
+    try:
+        build(nk, room)
+        return True
+    except Exception:
+        return False
+def least(nk):  # memory, to 1 %
+    lo, hi = 0, 1 << 32
+    while hi > lo * 1.01 + 4096:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if fits(nk, mid) else (mid, hi)
+    return hi
+room = 1.03 * least(n)  # one factor per cell on the top level
+assert fits(2 * n, int(room))
+def sweeps(Hy):
+    x, b, r = (ml.GpuVector(Hy.top_matrix().nrows) for _ in range(3))
+    k = [H.host_hip_launches(q) for q in (b"k_blk_cell", b"k_blk_sweep")]
+    Hy.apply(x, b, r)
+    return [H.host_hip_launches(q) > o for q, o in zip((b"k_blk_cell", b"k_blk_sweep"), k)]
+assert sweeps(build(2 * n, int(room))) == [False, True]  # from the rows
+assert sweeps(build(2 * n, 1 << 32)) == [True, False]  # from the element matrices
+""", dim, smoother)
