@@ -102,6 +102,7 @@ __global__ __launch_bounds__(64) void k_sell_fill_lds(int nrows, const int *__re
   }
 }
 
+static bool csr_irregular(const flgpu_mat *A);
 static int csr_lanes(const flgpu_mat *A);
 // the CSR bounds of a colour's rows (below)
 __global__ void k_row_span(int nsub, const int *__restrict__ rows, const int *__restrict__ rowptr,
@@ -172,11 +173,11 @@ static Sell sell_build(flgpu_mat *A, const std::vector<int> *rows_host) {
   return s;
 }
 
-// A colour's rows.  Sweeps of matrices with long or irregular rows read the CSR (csr_lanes, and
-// rows of over 27 entries): they take the rows' bounds.
+// A colour's rows.  Sweeps of matrices with long or irregular rows read the CSR (csr_irregular,
+// and rows of over 27 entries): they take the rows' bounds.
 Sell sell_build_rows(flgpu_mat *A, const std::vector<int> &rows) {
   Sell s = sell_build(A, &rows);
-  if (s.nrows > 0 && (A->lanes > 0 || s.maxw > 27)) {
+  if (s.nrows > 0 && (csr_irregular(A) || s.maxw > 27)) {
     s.span = dev_alloc(sizeof(int2) * (size_t)s.nrows);
     k_row_span<<<grid_for(s.nrows, 256), 256, 0, A->ctx->stream>>>(s.nrows, s.rows, A->rowptr,
                                                                    (int2 *)s.span);
@@ -620,18 +621,34 @@ __global__ __launch_bounds__(256) void k_csr_spmv(int nrows, const int *__restri
   if (DOT) block_part(d, dpart);
 }
 
-// Lanes per row of the products from the CSR, 0: SELL.  SELL streams a slice as wide as its
-// longest row, so it stays where that pads little, and for the lattice forms' matrices (order 1,
-// the trilinear transfers), whose other storage forms sum in its order.  Measured, SELL against
-// CSR with 4 / 8 / 16 lanes, us: 400 000 rows of 7 (padding 3.2) FP64 25.4 against 14.4 / 20.6 /
-// 36.6; of 23 (2.2) 71.5 against 42.0 / 37.9 / 40.3; Q2 2D 96^2, 37 249 rows of 16 (1.3) 5.7
-// against 3.5 / 3.7 / 5.4; Q2 3D (1.3), rows of 61: 24^3 FP64 31.1 against 24.8 / 20.2 / 20.1, but
-// 48^3 (912 673 rows), where SELL's loads fill the GPU, FP32 126 against 187 / 146 / 143.
-static int csr_lanes(const flgpu_mat *A) {
+// long or irregular rows, where SELL pads: the sweeps' colours are read from the CSR (eight lanes a
+// row, a colour's rows being few), the products if csr_lanes finds that faster.  The lattice
+// forms' matrices (order 1, the trilinear transfers) stay with SELL, whose order their other
+// storage forms sum in.
+static bool csr_irregular(const flgpu_mat *A) {
   const double pad = A->nnz > 0 ? (double)A->sell.nstored / A->nnz : 1.0;
-  if (A->lat_order == 1 || A->tp_nc > 0 || A->sell.maxw <= 8 || pad <= 1.15) return 0;
-  if (pad <= 1.5 && A->nrows > 400000) return 0;
-  return A->nnz < 10L * A->nrows ? 4 : 8;
+  return !(A->lat_order == 1 || A->tp_nc > 0 || A->sell.maxw <= 8 || pad <= 1.15 ||
+           (pad <= 1.5 && A->nrows > 400000));
+}
+
+// Lanes per row of the products from the CSR, 0: SELL.  A lane takes four entries at a time, so
+// four lanes cost the same up to 16 entries and eight up to 32; SELL's time goes with the entries
+// it stores.  Up to 100 000 rows the longest row's chain decides, and the CSR is as fast or
+// faster throughout.  Above, SELL against 4 / 8 lanes, us: 390 000 rows of 7 (12 entries stored a
+// row) FP64 12.5 against 11.8 / 19.7; of 11 (15) 14.6 against 13.6 / 20.5; of 15 (18 stored, 18
+// the longest) 16.8 against 20.7 / 21.5; of 18 (29) 28.5 against 24.6 / 21.6; of 24 (29) 26.7
+// against 29.9 / 26.7, (43) 42.8 against 37.7 / 36.8; of 40 (48) 43.4 against 52.1 / 49.0, (71) 77.6
+// against 66.0 / 59.8; FP32 0.7..0.8 of these.  Rows of 18 on average and 55 at most, 300 007 of
+// them: 40.3 against 23.1 with eight.  Order 2: 2D, 314 721 rows of 16, FP32 11.3 against 10.8 /
+// 12.9; 3D, rows of 61: 117 649 FP64 30.8 against 25.1 / 20.1, 456 533 96.7 against 113.9 / 93.9 and
+// FP32 69.2 against 55.5 / 47.7, 912 673 (there SELL's loads fill the GPU) 196 against 231 / 191
+// and 123 against 163 / 137.
+static int csr_lanes(const flgpu_mat *A) {
+  if (!csr_irregular(A)) return 0;
+  const double len = (double)A->nnz / A->nrows, stored = (double)A->sell.nstored / A->nrows;
+  if (A->nrows > 300000 && stored <= 1.25 * len) return 0;
+  if (A->nrows > 100000 && stored < (len < 10 || A->sell.maxw <= 16 ? 11.5 : 19.5)) return 0;
+  return len < 17 ? 4 : 8;
 }
 
 template <class T>
