@@ -634,11 +634,11 @@ static bool csr_irregular(const flgpu_mat *A) {
 // Lanes per row of the products from the CSR, 0: SELL.  A lane takes four entries at a time, so
 // four lanes cost the same up to 16 entries and eight up to 32; SELL's time goes with the entries
 // it stores.  Up to 100 000 rows the longest row's chain decides, and the CSR is as fast or
-// faster throughout.  Above, SELL against 4 / 8 lanes, us: 390 000 rows of 7 (12 entries stored a
-// row) FP64 12.5 against 11.8 / 19.7; of 11 (15) 14.6 against 13.6 / 20.5; of 15 (18 stored, 18
-// the longest) 16.8 against 20.7 / 21.5; of 18 (29) 28.5 against 24.6 / 21.6; of 24 (29) 26.7
-// against 29.9 / 26.7, (43) 42.8 against 37.7 / 36.8; of 40 (48) 43.4 against 52.1 / 49.0, (71) 77.6
-// against 66.0 / 59.8; FP32 0.7..0.8 of these.  Rows of 18 on average and 55 at most, 300 007 of
+// faster throughout.  Above, SELL against 4 / 8 lanes, us: 390 000 rows of 7 (11 entries stored a
+// row) FP64 11.0 against 11.9 / 19.5, (13) 12.9 against 11.9 / 19.7; of 11 (15) 14.6 against 13.6 /
+// 20.5, (18) 17.2 against 18.5 / 20.4; of 15 (18) 16.8 against 20.7 / 21.5; of 18 (29) 27.9 against
+// 25.2 / 23.3; of 24 (29) 26.7 against 30.1 / 26.7, (43) 42.8 against 37.6 / 36.8; of 40 (48) 43.4
+// against 52.1 / 49.0, (71) 77.6 against 66.2 / 59.6; FP32 0.7..0.8 of these.  Rows of 18 on average and 55 at most, 300 007 of
 // them: 40.3 against 23.1 with eight.  Order 2: 2D, 314 721 rows of 16, FP32 11.3 against 10.8 /
 // 12.9; 3D, rows of 61: 117 649 FP64 30.8 against 25.1 / 20.1, 456 533 96.7 against 113.9 / 93.9 and
 // FP32 69.2 against 55.5 / 47.7, 912 673 (there SELL's loads fill the GPU) 196 against 231 / 191
