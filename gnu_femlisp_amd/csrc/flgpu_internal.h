@@ -217,7 +217,7 @@ struct flgpu_mat {
   // the values again as 27 planes over the coarse nodes c: for the transpose (tp_kind 2)
   // tp27[k][c], k = (dz+1)*9 + (dy+1)*3 + (dx+1), the entry of fine neighbour 2c + d; for the
   // interpolation (tp_kind 1) the entries of the fine nodes of c's block by parity class
-  // (k_tp8_fill); 0 where there is no such entry
+  // (k_tp8_fill); 0 where there is no such entry.  An interpolation with tp_geo has none
   void *tp27 = nullptr;
   // order-2 lattice matrices as sums over their cells (prec, rows padded to 16 bytes: row_pad):
   // with a coefficient constant per cell the factors cell[c] of one reference element matrix

@@ -1405,8 +1405,7 @@ flgpu_mat *lattice_interpolation(flgpu_ctx *ctx, int dim, int order, int nc, int
       P->tp_kind = 1;
       PT->tp_kind = 2;
       P->tp_geo = PT->tp_geo = true;
-      tp_prepare(P);
-      tp_prepare(PT);
+      tp_prepare(PT);  // P^T's planes: the Galerkin product reads them; the transfers read none
     }
   } catch (...) {
     mat_free(P);

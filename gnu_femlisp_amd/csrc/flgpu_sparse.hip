@@ -452,7 +452,7 @@ flgpu_mat *mat_convert(const flgpu_mat *A, int prec) {
   }
   mat_finish(B);
   if (A->transpose) B->transpose = mat_convert(A->transpose, prec);
-  if (B->tp_kind) tp_prepare(B);
+  if (B->tp_kind && !(B->tp_kind == 1 && B->tp_geo)) tp_prepare(B);
   if (A->ncolours > 0) {
     // rebuild the colour subsets from A's row lists
     std::vector<int> colour(A->nrows, 0);

@@ -250,3 +250,20 @@ def sweeps(Hy):
 assert sweeps(build(2 * n, int(room))) == [False, True]  # from the rows
 assert sweeps(build(2 * n, 1 << 32)) == [True, False]  # from the element matrices
 """, dim, smoother)
+
+
+def test_geometric_interpolations_hold_no_value_planes(host_hip):
+    """the planes that products of changed values read are made when the values change, not for
+    the trilinear weights, which no product reads; a converted copy follows"""
+    run(host_hip, """
+fills = lambda: H.host_hip_launches(b"k_tp8_fill")
+P = lat.interpolation(3, 1, 6)
+Q = P.convert(F.F32)
+Hy = it.Hierarchy.lattice(it.GeometricCS(it.Jacobi(0.5)), 3, 1, 1, 3)
+assert fills() == 0
+P.update_values(np.ones(P.nnz))
+assert fills() == 1
+R = P.convert(F.F32)
+assert fills() == 2
+del Hy
+""")
