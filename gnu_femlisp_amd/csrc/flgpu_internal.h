@@ -173,7 +173,7 @@ struct Sell {
   long *slice_ptr = nullptr;
   int *col = nullptr;
   void *val = nullptr;
-  void *span = nullptr;  // colour subsets swept from the CSR: the rows' bounds (int2)
+  void *span = nullptr;  // colour subsets swept from the CSR: the rows' bounds (int2), nothing stored
   long nstored = 0;
   int maxw = 0;
 };

@@ -119,7 +119,7 @@ void sell_free(Sell &s) {
 
 template <class T>
 static void sell_fill(flgpu_ctx *ctx, const flgpu_mat *A, Sell &s, int fill_cols) {
-  if (s.nrows == 0) return;
+  if (s.nrows == 0 || s.span) return;
   if (!s.rows && s.maxw <= kSellLdsW) {
     k_sell_fill_lds<T><<<s.nslices, 64, 0, ctx->stream>>>(s.nrows, A->rowptr, A->colidx,
                                                           (const T *)A->vals, s.slice_ptr, s.col,
@@ -134,7 +134,9 @@ static void sell_fill(flgpu_ctx *ctx, const flgpu_mat *A, Sell &s, int fill_cols
   FLGPU_HIP(hipGetLastError());
 }
 
-// rows_host: row ids of the subset (nullptr: all rows)
+// rows_host: row ids of the subset (nullptr: all rows).  A colour's rows that are long or irregular
+// (csr_irregular, or over 27 entries) are swept from the CSR: they get their bounds (span) instead
+// of stored entries.
 static Sell sell_build(flgpu_mat *A, const std::vector<int> *rows_host) {
   flgpu_ctx *ctx = A->ctx;
   Sell s;
@@ -161,6 +163,13 @@ static Sell sell_build(flgpu_mat *A, const std::vector<int> *rows_host) {
     sp[i + 1] = sp[i] + 64L * w[i];
     s.maxw = std::max(s.maxw, w[i]);
   }
+  if (rows_host && s.nrows > 0 && (csr_irregular(A) || s.maxw > 27)) {
+    s.span = dev_alloc(sizeof(int2) * (size_t)s.nrows);
+    k_row_span<<<grid_for(s.nrows, 256), 256, 0, ctx->stream>>>(s.nrows, s.rows, A->rowptr,
+                                                                (int2 *)s.span);
+    FLGPU_HIP(hipGetLastError());
+    return s;
+  }
   s.nstored = sp[s.nslices];
   s.slice_ptr = (long *)dev_alloc(sizeof(long) * (s.nslices + 1));
   FLGPU_HIP(hipMemcpyAsync(s.slice_ptr, sp.data(), sizeof(long) * (s.nslices + 1),
@@ -173,18 +182,7 @@ static Sell sell_build(flgpu_mat *A, const std::vector<int> *rows_host) {
   return s;
 }
 
-// A colour's rows.  Sweeps of matrices with long or irregular rows read the CSR (csr_irregular,
-// and rows of over 27 entries): they take the rows' bounds.
-Sell sell_build_rows(flgpu_mat *A, const std::vector<int> &rows) {
-  Sell s = sell_build(A, &rows);
-  if (s.nrows > 0 && (csr_irregular(A) || s.maxw > 27)) {
-    s.span = dev_alloc(sizeof(int2) * (size_t)s.nrows);
-    k_row_span<<<grid_for(s.nrows, 256), 256, 0, A->ctx->stream>>>(s.nrows, s.rows, A->rowptr,
-                                                                   (int2 *)s.span);
-    FLGPU_HIP(hipGetLastError());
-  }
-  return s;
-}
+Sell sell_build_rows(flgpu_mat *A, const std::vector<int> &rows) { return sell_build(A, &rows); }
 
 // ---- diagonal -----------------------------------------------------------------------
 
